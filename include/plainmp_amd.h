@@ -132,9 +132,10 @@ typedef struct pmp_schedule {
   int32_t block;            /* threads per workgroup (multiple of 64), 0 = default  */
   int32_t waves_per_cu;     /* persistent waves per compute unit, 0 = default       */
   int32_t eval_whole_chunks;  /* evaluate / trajectory batches of at least this many
-                                 64-configuration chunks walk each configuration as one
-                                 unit, smaller ones split it per sphere block and self
-                                 pair; 0 = default (512)                               */
+                                 64-configuration chunks hand out whole sphere blocks to
+                                 the waves of a workgroup, smaller ones slices of a
+                                 block's primitives; 0 = default (slices up to 16,384
+                                 configurations)                                      */
   int32_t pair_shares;      /* pair distances: the primitives are split into this many
                                shares, each walked by its own waves (more stores in
                                flight for a small batch); 0 = default (about four

@@ -5,8 +5,8 @@ Two knobs decide how the persistent kernels map onto the MI355X:
 * ``block`` / ``waves_per_cu`` of the edge kernel: workgroup size and how many
   persistent waves each CU holds (the grid never exceeds one wave per edge);
 * ``eval_whole_chunks``: from how many 64-configuration chunks on an evaluate
-  or trajectory batch walks each configuration as one unit instead of
-  splitting it per sphere block and self pair;
+  or trajectory batch hands out whole sphere blocks instead of slices of a
+  block's primitives;
 * ``pair_shares``: into how many shares the pair-distance launch splits the
   primitives (grid z), each share walked by its own waves.
 

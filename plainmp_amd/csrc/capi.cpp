@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -90,6 +91,27 @@ struct DevBuf {
   }
 };
 
+// Tables that go to the device together: one buffer, one copy.  Pointers are
+// set when the tables are sent.
+class TablePack {
+ public:
+  template <class T, class... P>
+  void add(const std::vector<T>& v, P*... targets) {
+    const size_t at = (host_.size() + 255) & ~(size_t)255;
+    host_.resize(at + std::max<size_t>(v.size() * sizeof(T), 16));
+    if (!v.empty()) std::memcpy(host_.data() + at, v.data(), v.size() * sizeof(T));
+    (put_.push_back([=](unsigned char* base) { *targets = (const T*)(base + at); }), ...);
+  }
+  void send(DevBuf& buf, hipStream_t st) {
+    unsigned char* base = buf.upload(host_, st);
+    for (auto& f : put_) f(base);
+  }
+
+ private:
+  std::vector<unsigned char> host_;
+  std::vector<std::function<void(unsigned char*)>> put_;
+};
+
 // Device buffers of one edge launch setup: the direct calls of a context
 // share one set; every captured graph owns its own, so that later calls
 // cannot change what a replay reads.
@@ -157,17 +179,17 @@ struct pmp_context {
   int max_lds = 65536;  // LDS bytes per workgroup on this device
   // robot
   bool has_robot = false;
-  DevBuf nodes32, nodes64, sph32, sph64, meta, pairs, blocks, items, units, unit_all, ws_vjp;
+  DevBuf robot_tables, ws_vjp;
   KinArgs<float> k32{};
   KinArgs<double> k64{};
   int n_spheres = 0, n_groups = 0, n_cols = 0, n_nodes = 0;
-  DevBuf rad_out;  // sphere radius by group-order index (FP32)
+  const float* rad_out = nullptr;  // sphere radius by group-order index
   // host copies for the cull table (rebuilt whenever robot, scene or band change)
   std::vector<DevSphereBlock> h_blocks;
   std::vector<int> h_block_node;
   std::vector<NodeReach> h_reach;
   // scene
-  DevBuf prims32, prims64, vprims32, vprims64, supers, tiles32, tiles64, tileB, pts64;
+  DevBuf scene_tables, supers, tiles32, tiles64, tileB, pts64;
   DevBuf cloud_stage, cloud_scratch;  // points of one cloud and the sort keys of its tile build
   SceneArgs<float> s32{};
   SceneArgs<double> s64{};
@@ -175,7 +197,7 @@ struct pmp_context {
   std::vector<CloudRange> clouds;
   std::vector<DevPrim<double>> h_vprims;  // kind-sorted, FP64 bounds
   int h_vrange[kNumKinds + 1] = {0};
-  DevBuf cull, cull_range, ecull, ecull_range, vorig;
+  DevBuf cull_tables;
   std::vector<int32_t> h_vorig;
   // misc
   DevBuf traj_off, traj_w2;
@@ -387,6 +409,20 @@ void build_cull(pmp_context* ctx, double margin, std::vector<CullEntry>& ent, st
   }
 }
 
+// Every block's candidates in runs of at most kSliceCands (a block without
+// candidates gets one empty slice), last block first: the distal links come
+// last in node order and have the most candidates.
+std::vector<DevCullSlice> cull_slices(const std::vector<CullRange>& rng, int n_blocks) {
+  std::vector<DevCullSlice> out;
+  for (int b = n_blocks - 1; b >= 0; --b) {
+    const int lo = rng[b].at[0], hi = rng[b].at[kKindCloud];
+    const int n = std::max(1, (hi - lo + kSliceCands - 1) / kSliceCands);
+    for (int k = 0; k < n; ++k)
+      out.push_back({b, lo + (int)((int64_t)(hi - lo) * k / n), lo + (int)((int64_t)(hi - lo) * (k + 1) / n), k == 0});
+  }
+  return out;
+}
+
 // The validity table (boxes grown by the band) and the evaluate table (by
 // the 0.1 m cutoff of evaluate_ext_collision's prefilter).
 void rebuild_cull(pmp_context* ctx) {
@@ -395,15 +431,17 @@ void rebuild_cull(pmp_context* ctx) {
   std::vector<CullRange> rng;
   hipStream_t s0 = st(ctx);
   build_cull(ctx, (double)ctx->band, ent, rng);
-  const CullEntry* c = ctx->cull.upload(ent, s0);
-  const CullRange* cr = ctx->cull_range.upload(rng, s0);
-  ctx->s32.cull = ctx->s64.cull = c;
-  ctx->s32.cull_range = ctx->s64.cull_range = cr;
+  TablePack pk;
+  pk.add(ent, &ctx->s32.cull, &ctx->s64.cull);
+  pk.add(rng, &ctx->s32.cull_range, &ctx->s64.cull_range);
   build_cull(ctx, 0.1, ent, rng);
-  c = ctx->ecull.upload(ent, s0);
-  cr = ctx->ecull_range.upload(rng, s0);
-  ctx->s32.ecull = ctx->s64.ecull = c;
-  ctx->s32.ecull_range = ctx->s64.ecull_range = cr;
+  pk.add(ent, &ctx->s32.ecull, &ctx->s64.ecull);
+  pk.add(rng, &ctx->s32.ecull_range, &ctx->s64.ecull_range);
+  ctx->s32.n_ecull = ctx->s64.n_ecull = (int32_t)ent.size();
+  const std::vector<DevCullSlice> sl = cull_slices(rng, (int)ctx->h_blocks.size());
+  pk.add(sl, &ctx->s32.eslices, &ctx->s64.eslices);
+  ctx->s32.n_eslices = ctx->s64.n_eslices = (int32_t)sl.size();
+  pk.send(ctx->cull_tables, s0);
 }
 
 template <class T>
@@ -533,11 +571,10 @@ pmp_status pmp_destroy(pmp_context* ctx) {
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     (void)hipDeviceSynchronize();
-    for (DevBuf* b : {&ctx->nodes32, &ctx->nodes64, &ctx->sph32, &ctx->sph64, &ctx->meta, &ctx->pairs, &ctx->blocks, &ctx->items, &ctx->units, &ctx->unit_all, &ctx->ws_vjp,
-                      &ctx->vprims32, &ctx->vprims64, &ctx->supers, &ctx->cull, &ctx->ecull, &ctx->ecull_range, &ctx->vorig, &ctx->cull_range, &ctx->rad_out,
-                      &ctx->prims32, &ctx->prims64, &ctx->tiles32, &ctx->tiles64, &ctx->tileB, &ctx->pts64, &ctx->seq,
-                      &ctx->tmp_prims, &ctx->tmp_cloud, &ctx->ws_cen, &ctx->cloud_stage, &ctx->cloud_scratch, &ctx->ws_vunit,
-                      &ctx->ws_cloud, &ctx->ws_flags, &ctx->traj_off, &ctx->traj_w2, &ctx->sqp_rows, &ctx->sqp_tables})
+    for (DevBuf* b : {&ctx->robot_tables, &ctx->scene_tables, &ctx->cull_tables, &ctx->ws_vjp, &ctx->supers,
+                      &ctx->tiles32, &ctx->tiles64, &ctx->tileB, &ctx->pts64, &ctx->seq, &ctx->tmp_prims, &ctx->tmp_cloud,
+                      &ctx->ws_cen, &ctx->cloud_stage, &ctx->cloud_scratch, &ctx->ws_vunit, &ctx->ws_cloud, &ctx->ws_flags,
+                      &ctx->traj_off, &ctx->traj_w2, &ctx->sqp_rows, &ctx->sqp_tables})
       b->release();
     ctx->eb.release();
     if (ctx->capture_stream) (void)hipStreamDestroy(ctx->capture_stream);
@@ -705,6 +742,58 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
       meta[k] = {s, ext ? n_ext : -1, r->sphere_node[s], g};
       n_ext += ext;
     }
+    // Staged kernels' paths: one from the root to every sphere-carrying node
+    // that has none below it; the first path through a sphere-carrying or a
+    // joint node writes its pose.
+    std::vector<int> pose_of(N, -1);
+    std::vector<DevPathNode> path;
+    std::vector<int32_t> path_at{0};
+    std::vector<DevJoint> joints;
+    std::vector<DevColumn> columns(n_q, DevColumn{{0.f, 0.f, 0.f}, -1});
+    int n_poses = 0;
+    bool staged = true;
+    {
+      std::vector<bool> has(N, false), below(N, false);
+      std::vector<int> joint_of(N, -1);
+      for (int s = 0; s < S; ++s) has[r->sphere_node[s]] = true;
+      for (int i = N - 1; i > 0; --i)
+        if (has[i] || below[i]) below[r->node_parent[i]] = true;
+      for (int leaf = 0; leaf < N; ++leaf) {
+        if (!has[leaf] || below[leaf]) continue;
+        std::vector<int> chain;
+        for (int a = leaf; a >= 0; a = a == 0 ? -1 : r->node_parent[a]) chain.push_back(a);
+        for (auto it = chain.rbegin(); it != chain.rend(); ++it) {
+          const int i = *it;
+          DevPathNode e{};
+          for (int k = 0; k < 4; ++k) e.quat[k] = (float)r->node_quat[4 * i + k];
+          for (int k = 0; k < 3; ++k) {
+            e.trans[k] = (float)r->node_trans[3 * i + k];
+            e.axis[k] = (float)r->node_axis[3 * i + k];
+          }
+          e.kind = r->node_kind[i];
+          e.identity = r->node_identity[i] ? 1 : 0;
+          e.pose = -1;
+          const bool joint = e.kind == PMP_NODE_REVOLUTE || e.kind == PMP_NODE_PRISMATIC;
+          if ((has[i] || joint) && pose_of[i] < 0) e.pose = pose_of[i] = n_poses++;
+          if (joint && joint_of[i] < 0) {
+            joint_of[i] = (int)joints.size();
+            DevJoint j{};
+            for (int k = 0; k < 4; ++k) j.quat[k] = e.quat[k];
+            for (int k = 0; k < 3; ++k) j.axis[k] = e.axis[k];
+            j.q_col = r->node_q_col[i];
+            j.identity = e.identity;
+            j.revolute = e.kind == PMP_NODE_REVOLUTE;
+            joints.push_back(j);
+            DevColumn& col = columns[j.q_col];
+            staged = staged && col.pose < 0;
+            col = {{e.axis[0], e.axis[1], e.axis[2]}, pose_of[i]};
+          }
+          e.joint = joint ? joint_of[i] : 0;
+          path.push_back(e);
+        }
+        path_at.push_back((int32_t)path.size());
+      }
+    }
     // Sphere blocks: per node, its primitive-checked spheres sorted along
     // their longest extent and cut into runs of at most kBlockSpheres, each
     // with a bounding sphere (rounded up to FP32) in the link frame.
@@ -733,6 +822,9 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
           const int a = m * q / nblk, z = m * (q + 1) / nblk;
           DevSphereBlock bk{};
           bk.n = z - a;
+          bk.pose = pose_of[i];
+          bk.n2_lo = (float)reach[i].n2_lo;
+          bk.n2_hi = (float)reach[i].n2_hi;
           double blo[3] = {INFINITY, INFINITY, INFINITY}, bhi[3] = {-INFINITY, -INFINITY, -INFINITY};
           for (int t = a; t < z; ++t)
             for (int d = 0; d < 3; ++d) {
@@ -747,6 +839,8 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
             G = std::max(G, std::sqrt(ex * ex + ey * ey + ez * ez) + sp64[k].r);
             bk.ext[t - a] = meta[k].ext;
             bk.sph[t - a] = k;
+            bk.group[t - a] = meta[k].group;
+            bk.out[t - a] = meta[k].out;
             bk.s[t - a][0] = sp32[k].x;
             bk.s[t - a][1] = sp32[k].y;
             bk.s[t - a][2] = sp32[k].z;
@@ -832,6 +926,9 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
       bound(pr.begin2, pr.end2, pr.bound2);
       pr.node1 = group_node[g1];
       pr.node2 = group_node[g2];
+      staged = staged && pr.end1 - pr.begin1 <= 2048 && pr.end2 - pr.begin2 <= 2048;  // self keys' position bits
+      pr.pose1 = pose_of[pr.node1];
+      pr.pose2 = pose_of[pr.node2];
       pr.slot1 = slot[pr.node1];
       pr.slot2 = slot[pr.node2];
       PMP_REQUIRE(pr.slot1 >= 0 && pr.slot2 >= 0, "internal: self-pair pose not kept");
@@ -841,31 +938,45 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
     hipStream_t s0 = st(ctx);
     KinArgs<float> a{};
     KinArgs<double> d{};
-    a.nodes = ctx->nodes32.upload(n32, s0);
-    d.nodes = ctx->nodes64.upload(n64, s0);
-    a.spheres = ctx->sph32.upload(sp32, s0);
-    d.spheres = ctx->sph64.upload(sp64, s0);
-    a.meta = d.meta = ctx->meta.upload(meta, s0);
-    a.pairs = d.pairs = ctx->pairs.upload(pairs, s0);
-    a.blocks = d.blocks = ctx->blocks.upload(blocks, s0);
+    TablePack pk;
+    pk.add(n32, &a.nodes);
+    pk.add(n64, &d.nodes);
+    pk.add(sp32, &a.spheres);
+    pk.add(sp64, &d.spheres);
+    pk.add(meta, &a.meta, &d.meta);
+    pk.add(pairs, &a.pairs, &d.pairs);
+    pk.add(blocks, &a.blocks, &d.blocks);
     std::vector<DevSphereItem> items;
     for (int i = 0; i < N; ++i)
       for (int b0 = n32[i].sphere_begin; b0 < n32[i].sphere_end; b0 += kItemSpheres)
-        items.push_back({i, b0, std::min(b0 + kItemSpheres, n32[i].sphere_end), 0});
-    a.items = d.items = ctx->items.upload(items, s0);
+        items.push_back({i, b0, std::min(b0 + kItemSpheres, n32[i].sphere_end), pose_of[i]});
+    pk.add(items, &a.items, &d.items);
     a.n_items = d.n_items = (int32_t)items.size();
+    pk.add(path, &a.path, &d.path);
+    std::vector<DevSphereRow> rows(S);
+    for (int k = 0; k < S; ++k)
+      rows[meta[k].out] = {sp32[k].x, sp32[k].y, sp32[k].z, pose_of[meta[k].node], mask[meta[k].node], 0};
+    pk.add(rows, &a.rows, &d.rows);
+    pk.add(path_at, &a.path_at, &d.path_at);
+    a.n_paths = d.n_paths = (int32_t)path_at.size() - 1;
+    a.n_poses = d.n_poses = n_poses;
+    pk.add(joints, &a.joints, &d.joints);
+    pk.add(columns, &a.columns, &d.columns);
+    a.n_joints = d.n_joints = (int32_t)joints.size();
+    a.staged = d.staged = staged ? 1 : 0;
     // evaluate units: one per sphere item, then one per self pair; and the whole configuration
     std::vector<DevEvalUnit> units;
     for (int b = 0; b < (int)blocks.size(); ++b) units.push_back({b, b + 1, 0, 0, block_node[b], {0, 0, 0}});
     for (int k = 0; k < (int)pairs.size(); ++k)
       units.push_back({0, 0, k, k + 1, std::max(pairs[k].node1, pairs[k].node2), {0, 0, 0}});
     std::vector<DevEvalUnit> whole{{0, (int32_t)blocks.size(), 0, (int32_t)pairs.size(), N - 1, {0, 0, 0}}};
-    a.units = d.units = ctx->units.upload(units, s0);
+    pk.add(units, &a.units, &d.units);
     a.n_units = d.n_units = (int32_t)units.size();
-    a.unit_all = d.unit_all = ctx->unit_all.upload(whole, s0);
+    pk.add(whole, &a.unit_all, &d.unit_all);
     std::vector<float> rad(std::max(S, 1), 0.f);
     for (int s2 = 0; s2 < S; ++s2) rad[s2] = (float)r->sphere_radius[s2];
-    ctx->rad_out.upload(rad, s0);
+    pk.add(rad, &ctx->rad_out);
+    pk.send(ctx->robot_tables, s0);
     a.n_nodes = d.n_nodes = N;
     a.n_spheres = d.n_spheres = S;
     a.n_pairs = d.n_pairs = (int)pairs.size();
@@ -959,12 +1070,14 @@ pmp_status pmp_upload_scene(pmp_context* ctx, const pmp_scene_desc* sc) {
     hipStream_t s0 = st(ctx);
     SceneArgs<float> a{};
     SceneArgs<double> d{};
-    a.prims = ctx->prims32.upload(p32, s0);
-    a.vprims = ctx->vprims32.upload(v32, s0);
-    d.vprims = ctx->vprims64.upload(v64, s0);
-    a.vorig = d.vorig = ctx->vorig.upload(vorig, s0);
+    TablePack pk;
+    pk.add(p32, &a.prims);
+    pk.add(p64, &d.prims);
+    pk.add(v32, &a.vprims);
+    pk.add(v64, &d.vprims);
+    pk.add(vorig, &a.vorig, &d.vorig);
+    pk.send(ctx->scene_tables, s0);
     for (int k = 0; k <= kNumKinds; ++k) a.vrange[k] = d.vrange[k] = vrange[k];
-    d.prims = ctx->prims64.upload(p64, s0);
     CloudTile* t32 = (CloudTile*)ctx->tiles32.get(std::max<size_t>(n_tiles * sizeof(CloudTile), 16));
     CloudTile64* t64 = (CloudTile64*)ctx->tiles64.get(std::max<size_t>(n_tiles * sizeof(CloudTile64), 16));
     float* tb = (float*)ctx->tileB.get(std::max<size_t>(n_tiles * 4 * kCloudTile * sizeof(float), 16));
@@ -1169,7 +1282,7 @@ pmp_status pmp_sphere_clearance_batch(pmp_context* ctx, const double* q, int64_t
     for (const CloudRange& c : ctx->clouds) {  // nearest point of every cloud, no cap
       float* d2 = (float*)ctx->ws_cloud.get(sizeof(float) * Q);
       PMP_HIP(launch_cloud_min(ctx->s32.tiles, ctx->s32.tileB, ctx->s32.supers, c, cen, nullptr, B, Q, d2, st(ctx)));
-      PMP_HIP(launch_cloud_clearance(clearance, d2, (const float*)ctx->rad_out.ptr, c.radius, B, S, st(ctx)));
+      PMP_HIP(launch_cloud_clearance(clearance, d2, ctx->rad_out, c.radius, B, S, st(ctx)));
     }
   });
 }

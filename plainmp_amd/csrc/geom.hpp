@@ -288,6 +288,48 @@ PMP_HD T sdf_eval_kind(const DevPrim<T>& p, V3<T> c) {
   }
 }
 
+// The hardware's square root, within an ulp.
+__device__ __forceinline__ float approx_sqrt(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_sqrtf(x);
+#else
+  return sqrtf(x);  // host pass: never executed, only type-checked
+#endif
+}
+
+// False only when sdf_eval_kind<K>(p, c) > lim for certain (clouds excluded):
+// a test without correctly rounded square roots, its margins (1e-4 of the
+// squared distance, 1e-5 m) far above the FP32 rounding of either form within
+// a few metres.
+template <int K>
+__device__ __forceinline__ bool sdf_may_reach(const DevPrim<float>& p, V3<float> c, float lim) {
+  const float dx = c.x - p.pos[0], dy = c.y - p.pos[1], dz = c.z - p.pos[2];
+  float m2, L = lim;
+  if constexpr (K == kKindBoxAA || K == kKindBoxRot) {
+    V3<float> d{dx, dy, dz};
+    if constexpr (K == kKindBoxRot) d = mv(load_m3(p.Rinv), d);
+    const float sx = fmaxf(fabsf(d.x) - p.p0, 0.0f), sy = fmaxf(fabsf(d.y) - p.p1, 0.0f),
+                sz = fmaxf(fabsf(d.z) - p.p2, 0.0f);
+    m2 = sx * sx + sy * sy + sz * sz;
+  } else if constexpr (K == kKindCylZ || K == kKindCylRot) {
+    float z = dz, x = dx, y = dy;
+    if constexpr (K == kKindCylRot) {
+      z = dx * p.R[2] + dy * p.R[5] + dz * p.R[8];
+      x = dx * p.R[0] + dy * p.R[3] + dz * p.R[6];
+      y = dx * p.R[1] + dy * p.R[4] + dz * p.R[7];
+    }
+    const float rs = fmaxf(approx_sqrt(x * x + y * y) - p.p0, 0.0f), zs = fmaxf(fabsf(z) - p.p1, 0.0f);
+    m2 = rs * rs + zs * zs;
+  } else if constexpr (K == kKindSphere) {
+    m2 = dx * dx + dy * dy + dz * dz;
+    L += p.p0;
+  } else {  // ground
+    return !(c.z + p.p0 > lim + 1e-5f);
+  }
+  L = fmaxf(L, 0.0f) + 1e-5f;
+  return !(m2 > L * L * 1.0001f);
+}
+
 // Gradient of sdf_eval with respect to the point (clouds excluded).  At kinks
 // the branch taken follows the evaluate() formula's active terms.
 template <class T>

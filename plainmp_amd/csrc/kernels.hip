@@ -8,192 +8,14 @@
 #include <float.h>
 #include <limits.h>
 
-#include "fk.hpp"
+#include "device.hpp"
 #include "launch.h"
 
 namespace pmp {
 
-constexpr float kCutoff = 0.1f;  // SphereCollisionCst::cutoff_dist_ (primitive_sphere_collision.hpp:115)
-// Evaluate batches of at least this many 64-configuration chunks walk each
-// configuration as one unit (the launch is large enough without splitting).
-constexpr int64_t kWholeUnitChunks = 512;
 // Edges are walked 64 states at a time; an edge needing more states than this
 // (a step ratio below 2^-24) is reported invalid with n_checked = -1 instead.
 constexpr double kMaxEdgeStates = 16777216.0;
-
-template <class T>
-__device__ __forceinline__ DevPrim<T> prim_at(const SceneArgs<T>& sc, int p) {
-  return cload(reinterpret_cast<const DevPrim<T>*>(sc.prims), p);
-}
-
-__device__ __forceinline__ int64_t gid() { return (int64_t)blockIdx.x * blockDim.x + threadIdx.x; }
-
-// Squared distance from c to the box [lb, ub] (0 inside).
-__device__ __forceinline__ float box_dist2(const float (&lb)[3], const float (&ub)[3], V3<float> c) {
-  const float dx = fmaxf(fmaxf(lb[0] - c.x, c.x - ub[0]), 0.f);
-  const float dy = fmaxf(fmaxf(lb[1] - c.y, c.y - ub[1]), 0.f);
-  const float dz = fmaxf(fmaxf(lb[2] - c.z, c.z - ub[2]), 0.f);
-  return dx * dx + dy * dy + dz * dz;
-}
-
-// Squared distance between the boxes [lb, ub] and [l, u] (0 when they meet).
-__device__ __forceinline__ float box_box_dist2(const float (&lb)[3], const float (&ub)[3], V3<float> l, V3<float> u) {
-  const float dx = fmaxf(fmaxf(lb[0] - u.x, l.x - ub[0]), 0.f);
-  const float dy = fmaxf(fmaxf(lb[1] - u.y, l.y - ub[1]), 0.f);
-  const float dz = fmaxf(fmaxf(lb[2] - u.z, l.z - ub[2]), 0.f);
-  return dx * dx + dy * dy + dz * dz;
-}
-
-// Minimum / maximum of v over the wave (every lane active; wave-uniform).
-__device__ __forceinline__ float wave_minf(float v) {
-#pragma unroll
-  for (int s = 32; s > 0; s >>= 1) v = fminf(v, __shfl_xor(v, s, 64));
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-__device__ __forceinline__ float wave_maxf(float v) {
-#pragma unroll
-  for (int s = 32; s > 0; s >>= 1) v = fmaxf(v, __shfl_xor(v, s, 64));
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-
-// Minimum of v over the wave (every lane active; wave-uniform result).
-__device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-  for (int s = 32; s > 0; s >>= 1) v = min(v, __shfl_xor(v, s, 64));
-  return __builtin_amdgcn_readfirstlane(v);
-}
-
-// Maximum of v over the wave's active lanes (wave-uniform result).
-__device__ __forceinline__ int wave_max_i(int v) {
-  for (int m = 32; m > 0; m >>= 1) v = max(v, __shfl_xor(v, m, 64));
-  return __builtin_amdgcn_readfirstlane(v);
-}
-
-// Four consecutive floats of a table read as one wave-uniform load.
-struct alignas(16) Quad4 {
-  float v[4];
-};
-
-// One kept tile t of cloud_block_min: the spheres' minima over its points.
-template <bool kBounds>
-__device__ __forceinline__ void cloud_tile_min(const SceneArgs<float>& sc, int t, const CloudTile& T,
-                                               const V3<float> (&c)[kBlockSpheres], int n,
-                                               float (&best)[kBlockSpheres], float (&lo)[kBlockSpheres]) {
-  V3<float> cl[kBlockSpheres];
-  float tb[kBlockSpheres];
-#pragma unroll
-  for (int k = 0; k < kBlockSpheres; ++k) {
-    cl[k] = V3<float>{c[k].x - T.o[0], c[k].y - T.o[1], c[k].z - T.o[2]};
-    tb[k] = FLT_MAX;
-  }
-  const Quad4* Bt = reinterpret_cast<const Quad4*>(sc.tileB + (int64_t)t * 4 * kCloudTile);
-  for (int m = 0; m < 4; ++m) {
-    for (int j4 = 0; j4 < 4; ++j4) {
-      // points 16 m + 4 j4 .. + 3: components x, y, z, |p'|^2
-      const Quad4 X = cload(Bt, m * 16 + 0 * 4 + j4), Y = cload(Bt, m * 16 + 1 * 4 + j4);
-      const Quad4 Z = cload(Bt, m * 16 + 2 * 4 + j4), W = cload(Bt, m * 16 + 3 * 4 + j4);
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-#pragma unroll
-        for (int k = 0; k < kBlockSpheres; ++k) {
-          if (k < n)
-            tb[k] = fminf(tb[k], fmaf(X.v[jj], cl[k].x, fmaf(Y.v[jj], cl[k].y, fmaf(Z.v[jj], cl[k].z, W.v[jj]))));
-        }
-      }
-    }
-  }
-  const float rho2 = kBounds ? tile_rho2(T) : 0.f;
-#pragma unroll
-  for (int k = 0; k < kBlockSpheres; ++k) {
-    const float off = dot(cl[k], cl[k]);
-    if constexpr (kBounds) {
-      const float err = kCloudGemmErr * (off + rho2);
-      best[k] = fminf(best[k], tb[k] + off + err);
-      lo[k] = fminf(lo[k], tb[k] + off - err);
-    } else {
-      best[k] = fminf(best[k], tb[k] + off);
-    }
-  }
-}
-
-// Per sphere k < n of a block, min |c_k - p|^2 over the points of cloud oc
-// that lie in tiles within sqrt(reach2) of the block's bounding centre g
-// (FLT_MAX when none).  Super-tiles, then tiles, are skipped for the whole
-// wave when no `live` lane's g reaches their box: 64 of them at a time are
-// first tested against the box around the live lanes' g, a box a lane, and
-// the survivors of that ballot are tested lane by lane.  A kept tile's points
-// are compared in tile-local coordinates, |c - p|^2 = |c'|^2 + (|p'|^2 -
-// 2 c'.p'), from the matrix-core pass's operands (-2 p', |p'|^2).  With
-// kBounds the minimum is bracketed: best = min over tiles of (d2 + err), lo =
-// min over tiles of (d2 - err), err = kCloudGemmErr (|c'|^2 + rho^2) of the
-// tile.
-template <bool kBounds>
-__device__ __forceinline__ void cloud_block_min(const SceneArgs<float>& sc, int oc, const V3<float> (&c)[kBlockSpheres],
-                                                int n, V3<float> g, float reach2, bool live,
-                                                float (&best)[kBlockSpheres], float (&lo)[kBlockSpheres]) {
-#pragma unroll
-  for (int k = 0; k < kBlockSpheres; ++k) best[k] = lo[k] = FLT_MAX;
-  if (!wave_any(live)) return;
-  const V3<float> gl{wave_minf(live ? g.x : FLT_MAX), wave_minf(live ? g.y : FLT_MAX), wave_minf(live ? g.z : FLT_MAX)};
-  const V3<float> gu{wave_maxf(live ? g.x : -FLT_MAX), wave_maxf(live ? g.y : -FLT_MAX),
-                     wave_maxf(live ? g.z : -FLT_MAX)};
-  const int lane = threadIdx.x & 63;
-  const int s_end = sc.super_at[oc + 1];
-  for (int s0 = sc.super_at[oc]; s0 < s_end; s0 += 64) {
-    bool snear = false;
-    if (s0 + lane < s_end) {
-      const CloudSuper Sv = sc.supers[s0 + lane];  // a super-tile a lane: vector loads
-      snear = box_box_dist2(Sv.lb, Sv.ub, gl, gu) <= reach2;
-    }
-    for (uint64_t smask = __ballot(snear); smask; smask &= smask - 1) {
-      const CloudSuper S = cload(sc.supers, s0 + __builtin_ctzll(smask));
-      if (!wave_any(live && box_dist2(S.lb, S.ub, g) <= reach2)) continue;
-      const int t_end = S.first + S.count;
-      for (int t0 = S.first; t0 < t_end; t0 += 64) {
-        bool tnear = false;
-        if (t0 + lane < t_end) {
-          const CloudTile Tv = sc.tiles[t0 + lane];
-          tnear = box_box_dist2(Tv.lb, Tv.ub, gl, gu) <= reach2;
-        }
-        for (uint64_t tmask = __ballot(tnear); tmask; tmask &= tmask - 1) {
-          const int t = t0 + __builtin_ctzll(tmask);
-          const CloudTile T = cload(sc.tiles, t);
-          if (!wave_any(live && box_dist2(T.lb, T.ub, g) <= reach2)) continue;
-          cloud_tile_min<kBounds>(sc, t, T, c, n, best, lo);
-        }
-      }
-    }
-  }
-}
-
-// The nearest point of cloud oc to c, per lane (an exhaustive search over
-// the tiles, skipping those whose box is farther than the best so far), and
-// its squared distance in best.
-__device__ __forceinline__ V3<float> cloud_nearest(const SceneArgs<float>& sc, int oc, V3<float> c, float& best) {
-  best = FLT_MAX;
-  V3<float> bp = c;
-  for (int si = sc.super_at[oc]; si < sc.super_at[oc + 1]; ++si) {
-    const CloudSuper S = sc.supers[si];
-    if (box_dist2(S.lb, S.ub, c) > best) continue;
-    for (int t = S.first; t < S.first + S.count; ++t) {
-      const CloudTile T = sc.tiles[t];
-      if (box_dist2(T.lb, T.ub, c) > best) continue;
-      const V3<float> cl{c.x - T.o[0], c.y - T.o[1], c.z - T.o[2]};
-      const float off = dot(cl, cl);
-      const float* Bt = sc.tileB + (int64_t)t * 4 * kCloudTile;
-      for (int j = 0; j < kCloudTile; ++j) {
-        const float* col = Bt + (j / 16) * 64 + (j % 16);
-        const float bx = col[0], by = col[16], bz = col[32], bw = col[48];
-        const float d2 = fmaf(bx, cl.x, fmaf(by, cl.y, fmaf(bz, cl.z, bw))) + off;
-        if (d2 < best) {
-          best = d2;
-          bp = V3<float>{T.o[0] - 0.5f * bx, T.o[1] - 0.5f * by, T.o[2] - 0.5f * bz};
-        }
-      }
-    }
-  }
-  return bp;
-}
 
 // ------------------------------------------------------------------ centres
 template <class T>
@@ -508,7 +330,7 @@ struct ValidVis32T {
       const float rc = Pc.p0;
       const float reach = bk.G * n2_hi + rc + band + 1e-5f;
       float hi[kBlockSpheres], lo[kBlockSpheres];
-      cloud_block_min<true>(sc, (Pc.flags >> 4) & 15, c, n, g, reach * reach, alive(), hi, lo);
+      cloud_block_min<true, kBlockSpheres>(sc, (Pc.flags >> 4) & 15, c, n, g, reach * reach, alive(), hi, lo);
 #pragma unroll
       for (int k = 0; k < kBlockSpheres; ++k) {
         if (k < n) {
@@ -1158,30 +980,6 @@ __global__ void __launch_bounds__(64 * kRecheckWaves) edges_recheck_kernel(KinAr
 //   revolute: a_j x (c - o_j)      prismatic: a_j
 // (KinematicModel::get_attached_point_jacobian, kinematics/algorithm.cpp:346-433;
 // the base columns are the analytic form of its finite differences).
-// The base's own q columns (a planar or floating base), as (column, axis,
-// origin) frames: translations along x, y, z, then the roll / pitch / yaw
-// axes of the base's Rz(yaw) Ry(pitch) Rx(roll) rotation.
-template <class QS, class F>
-__device__ __forceinline__ void base_columns(const KinArgs<float>& ka, const Pose<float>& base, const QS& qs, F&& f) {
-  const int n = ka.n_q_cols;
-  if (ka.base_type == PMP_BASE_PLANAR) {
-    f(n, V3<float>{1.f, 0.f, 0.f}, base.t);
-    f(n + 1, V3<float>{0.f, 1.f, 0.f}, base.t);
-    f(n + 2, V3<float>{0.f, 0.f, 1.f}, base.t);
-  } else if (ka.base_type == PMP_BASE_FLOATING) {
-    const float pitch = (float)qs.get(n + 4), yaw = (float)qs.get(n + 5);
-    float sp, cp, sy, cy;
-    sincosf(pitch, &sp, &cp);
-    sincosf(yaw, &sy, &cy);
-    f(n, V3<float>{1.f, 0.f, 0.f}, base.t);
-    f(n + 1, V3<float>{0.f, 1.f, 0.f}, base.t);
-    f(n + 2, V3<float>{0.f, 0.f, 1.f}, base.t);
-    f(n + 3, V3<float>{cy * cp, sy * cp, -sp}, base.t);  // Rz(yaw) Ry(pitch) x
-    f(n + 4, V3<float>{-sy, cy, 0.f}, base.t);           // Rz(yaw) y
-    f(n + 5, V3<float>{0.f, 0.f, 1.f}, base.t);
-  }
-}
-
 template <int MAXC>
 struct Frames {
   float ax[MAXC], ay[MAXC], az[MAXC], ox[MAXC], oy[MAXC], oz[MAXC];
@@ -1215,14 +1013,12 @@ struct Frames {
 
 // ------------------------------------------------------------ evaluate rows
 // evaluate_ext_collision / evaluate_self_collision
-// (constraints/primitive_sphere_collision.cpp:256-383) split into units: a
-// unit is a sphere item (the external minimum over its spheres x every
-// primitive, visited in the reference's (group, primitive, sphere) key order)
-// or a self group pair (minimum over its sphere pairs in visiting order).  A
-// wave evaluates one unit for 64 consecutive configurations and leaves
-// (value, winner) per lane; the last wave to finish a chunk (device-scope
-// counter after a release fence) reduces the units in visiting order and
-// recomputes the winning Jacobian rows with one more FK walk.
+// (constraints/primitive_sphere_collision.cpp:256-383), a lane per
+// configuration: the form for robots whose tables do not fit a staged
+// workgroup (eval.hip) or that drive two joints with one q column.  A unit is
+// a range of sphere blocks (the external minimum over their spheres x every
+// primitive, in the reference's (group, primitive, sphere) key order) and of
+// self group pairs (minimum over their sphere pairs in visiting order).
 template <int MAXC>
 struct EvalUnitVis {
   static constexpr bool kSelf = true;
@@ -1343,7 +1139,7 @@ struct EvalUnitVis {
       const float rc = Pc.p0;
       const float reach = bk.G * n2_hi + rc + kCutoff + 1e-5f;
       float d2[kBlockSpheres], unused[kBlockSpheres];
-      cloud_block_min<false>(sc, (Pc.flags >> 4) & 15, c, n, g, all ? FLT_MAX : reach * reach, true, d2, unused);
+      cloud_block_min<false, kBlockSpheres>(sc, (Pc.flags >> 4) & 15, c, n, g, all ? FLT_MAX : reach * reach, true, d2, unused);
 #pragma unroll
       for (int k = 0; k < kBlockSpheres; ++k) {
         if (k < n) {
@@ -1379,47 +1175,6 @@ struct EvalUnitVis {
       sc2 = cj;
     }
   }
-};
-
-// FK walk for the Jacobian rows of the winners: it keeps the joint frames
-// and computes the world centres of just the (up to three) winning spheres,
-// and stops at the last node any lane of the wave needs.
-template <int MAXC>
-struct EvalRowVis {
-  static constexpr bool kSelf = false;
-  static constexpr bool kRanged = true;
-  static constexpr bool kBlocks = true;
-  const KinArgs<float>& ka;
-  Frames<MAXC> fr;
-  int s0 = -1, s1 = -1, s2 = -1;
-  int last = 0;  // wave-uniform
-  V3<float> c0{0.f, 0.f, 0.f}, c1{0.f, 0.f, 0.f}, c2{0.f, 0.f, 0.f};
-  __device__ bool alive() const { return true; }
-  __device__ int last_node() const { return last; }
-  __device__ int pair_lo() const { return 0; }
-  __device__ int pair_hi() const { return 0; }
-  template <class QS>
-  __device__ void begin(const Pose<float>& base, const QS& qs) { fr.set_base(ka, base, qs); }
-  __device__ void node(int, const DevNode<float>& nd, const Pose<float>& P) {
-    if (nd.q_col < 0) return;
-    fr.set(nd.q_col, qrot(P.q, V3<float>{nd.axis[0], nd.axis[1], nd.axis[2]}), P.t);
-  }
-  __device__ void sphere(int, V3<float>, float) {}
-  __device__ void blocks(const DevNode<float>& nd, const Pose<float>& P) {
-    const bool h0 = s0 >= nd.sphere_begin && s0 < nd.sphere_end;
-    const bool h1 = s1 >= nd.sphere_begin && s1 < nd.sphere_end;
-    const bool h2 = s2 >= nd.sphere_begin && s2 < nd.sphere_end;
-    if (!wave_any(h0 || h1 || h2)) return;
-    const M3<float> R = qmat(P.q);
-    auto centre = [&](int s) {
-      const DevSphere<float> sp = ka.spheres[s];  // per-lane index: a vector load
-      return add(mv(R, V3<float>{sp.x, sp.y, sp.z}), P.t);
-    };
-    if (h0) c0 = centre(s0);
-    if (h1) c1 = centre(s1);
-    if (h2) c2 = centre(s2);
-  }
-  __device__ void self(const DevSelfPair&, int, int, V3<float>, V3<float>, float) {}
 };
 
 // FK walk that builds the Jacobian rows of the winners column by column as
@@ -1474,8 +1229,7 @@ struct EvalOut {
   float* vals;  // [cst_dim][ld]
   float* jac;   // [cst_dim][D][ld]
   int64_t ld;
-  const DevEvalUnit* units;
-  int n_units;
+  const DevEvalUnit* units;  // one unit: everything
   // trajectories (offsets == nullptr: plain evaluate)
   const int64_t* offsets;
   int n_traj;
@@ -1520,99 +1274,6 @@ __device__ void smooth_terms(const double* X, int64_t ldx, int64_t n, int D, con
       }
     o.cost[lo] = c;
   }
-}
-
-// Reduction of a configuration's unit results in the reference's order
-// (external minimum by (group, primitive, sphere) key, self minimum by
-// visiting order; units hold increasing self-pair ranges, so unit order is
-// visiting order), then the Jacobian rows of the winners from one more FK
-// walk, and for trajectories the smoothness terms.  Unit k's results are at
-// xv[k * stride], xi, sv, si (any address space); (best, bidx, sbest, sidx)
-// start the reduction.
-template <int MAXC, class QS>
-__device__ __forceinline__ void eval_finish(const KinArgs<float>& ka, const SceneArgs<float>& sc, const QS& qs, const double* q,
-                            int64_t ldq, int64_t b, const EvalOut& o, float best, int bidx, float sbest, int sidx,
-                            const float* xv, const int* xi, const float* sv, const int* si, int64_t stride,
-                            int n_red) {
-  const int D = ka.n_cols, NP = sc.n_prims;
-  int bkey = 0x7fffffff;
-  for (int k = 0; k < n_red; ++k) {
-    const float val = xv[k * stride];
-    const int idx = xi[k * stride];
-    if (idx >= 0) {
-      const DevSphereMeta m = cload(ka.meta, idx / kMaxPrims);
-      const int key = (m.group * NP + idx % kMaxPrims) * ka.n_spheres + m.out;
-      if (val < best || (bidx >= 0 && val == best && key < bkey)) {
-        best = val;
-        bkey = key;
-        bidx = idx;
-      }
-    }
-    const float sval = sv[k * stride];
-    const int sid = si[k * stride];
-    if (sid >= 0 && sval < sbest) {
-      sbest = sval;
-      sidx = sid;
-    }
-  }
-  EvalRowVis<MAXC> rv{ka};
-  int need = -1;  // the last node this lane's winners need
-  if (bidx >= 0) {
-    rv.s0 = bidx / kMaxPrims;
-    need = cload(ka.meta, rv.s0).node;
-  }
-  if (sidx >= 0) {
-    rv.s1 = sidx / kMaxSpheres;
-    rv.s2 = sidx % kMaxSpheres;
-    need = max(need, max(cload(ka.meta, rv.s1).node, cload(ka.meta, rv.s2).node));
-  }
-  // lanes of the wave that reach this point walk together (inactive lanes
-  // have returned); no winner in the wave: the rows are zero without FK
-  const int last = wave_max_i(need);
-  if (last >= 0) {
-    rv.last = last;
-    run_fk(ka, qs, false, rv);
-  }
-  int row = 0;
-  if (NP > 0) {
-    o.vals[b] = best;
-    V3<float> g{0.f, 0.f, 0.f};
-    uint64_t mask = 0;
-    if (bidx >= 0) {
-      const DevPrim<float> P = prim_at(sc, bidx % kMaxPrims);
-      if (P.type == PMP_PRIM_CLOUD) {
-        // the gradient of sqrt(min |c - p|^2) at the nearest point, which the
-        // reference's forward difference (eps 1e-6) approximates
-        float d2;
-        const V3<float> d = sub(rv.c0, cloud_nearest(sc, (P.flags >> 4) & 15, rv.c0, d2));
-        g = scale(1.0f / sqrtf(dot(d, d)), d);
-      } else {
-        g = sdf_grad(P, rv.c0);
-      }
-      mask = cload(ka.nodes, cload(ka.meta, rv.s0).node).col_mask;
-    }
-#pragma unroll
-    for (int j = 0; j < MAXC; ++j)
-      if (j < D) o.jac[(int64_t)j * o.ld + b] = dot(g, rv.fr.col(j, mask, ka.rev_mask, rv.c0));
-    row = 1;
-  }
-  if (ka.n_pairs > 0) {
-    o.vals[(int64_t)row * o.ld + b] = sbest;
-    V3<float> n{0.f, 0.f, 0.f};
-    uint64_t m1 = 0, m2 = 0;
-    if (sidx >= 0) {
-      const V3<float> d = sub(rv.c1, rv.c2);
-      n = scale(1.0f / sqrtf(dot(d, d)), d);
-      m1 = cload(ka.nodes, cload(ka.meta, rv.s1).node).col_mask;
-      m2 = cload(ka.nodes, cload(ka.meta, rv.s2).node).col_mask;
-    }
-#pragma unroll
-    for (int j = 0; j < MAXC; ++j)
-      if (j < D)
-        o.jac[((int64_t)row * D + j) * o.ld + b] =
-            dot(n, sub(rv.fr.col(j, m1, ka.rev_mask, rv.c1), rv.fr.col(j, m2, ka.rev_mask, rv.c2)));
-  }
-  if (o.offsets) smooth_terms<MAXC>(q, ldq, b, D, o);
 }
 
 // The rows of one walk's winners (whole mode, where the unit walk kept the
@@ -1690,42 +1351,6 @@ __global__ void __launch_bounds__(64) eval_units_kernel(KinArgs<float> ka, Scene
   run_fk(ka, qs, false, v);
   if (!active) return;
   eval_finish_whole<MAXC>(ka, sc, qs, q, ldq, b, o, v);
-}
-
-// Split mode: one workgroup per chunk of 64 configurations; its waves take
-// the units in turn, leave their results in LDS, and after a barrier the
-// first wave reduces them (no device-scope fence or atomic: a version with a
-// wave per (chunk, unit) that met through a device-scope counter took
-// longer).  LDS holds
-// 16 B x 64 x n_units.
-constexpr int kEvalGroupWaves = 8;
-constexpr int kEvalGroupMaxUnits = 64;  // 64 KiB of LDS
-template <int MAXC>
-__global__ void __launch_bounds__(64 * kEvalGroupWaves) eval_group_kernel(KinArgs<float> ka, SceneArgs<float> sc,
-                                                                          const double* q, int64_t ldq, int64_t B,
-                                                                          EvalOut o) {
-  HIP_DYNAMIC_SHARED(int32_t, eval_lds)
-  const int U = o.n_units;
-  float* xv = reinterpret_cast<float*>(eval_lds);
-  int* xi = eval_lds + U * 64;
-  float* sv = reinterpret_cast<float*>(eval_lds + 2 * U * 64);
-  int* si = eval_lds + 3 * U * 64;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, W = blockDim.x >> 6;
-  const int64_t b = (int64_t)blockIdx.x * 64 + lane;
-  const bool active = b < B;
-  BatchQ qs{q, ldq, active ? b : B - 1};
-  for (int u = w; u < U; u += W) {
-    EvalUnitVis<MAXC> v{ka, sc, cload(o.units, u)};
-    run_fk(ka, qs, false, v);
-    xv[u * 64 + lane] = v.best;
-    xi[u * 64 + lane] = v.bidx;
-    sv[u * 64 + lane] = v.sbest;
-    si[u * 64 + lane] = v.sidx;
-  }
-  __syncthreads();
-  if (w != 0 || !active) return;
-  eval_finish<MAXC>(ka, sc, qs, q, ldq, b, o, kCutoff, -1, kCutoff, -1, xv + lane, xi + lane, sv + lane, si + lane, 64,
-                    U);
 }
 
 // The pair and adjoint kernels give each (configuration, sphere item) its
@@ -2262,22 +1887,13 @@ hipError_t launch_fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t st) {
 }
 hipError_t launch_eval_units(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq,
                              int64_t B, const EvalArgs& e, hipStream_t st) {
-  const int64_t chunks = (B + 63) / 64;
+  hipError_t err;
+  if (launch_eval_staged(ka, sc, q, ldq, B, e, st, &err)) return err;
   EvalOut o{};
   o.vals = e.vals;
   o.jac = e.jac;
   o.ld = B;
-  // Small batches give each configuration many units (one per sphere block
-  // and per self pair, the units of a chunk in one workgroup) so that the
-  // launch fills the GPU; from kWholeUnitChunks chunks on (or beyond
-  // kEvalGroupMaxUnits units), one unit walks the whole configuration.
-  const int64_t whole = e.whole_chunks > 0 ? e.whole_chunks : kWholeUnitChunks;
-  const int waves = ka.n_units < kEvalGroupWaves ? ka.n_units : kEvalGroupWaves;
-  const size_t own = sizeof(int32_t) * 4 * 64 * (size_t)ka.n_units;  // (value, winner) pairs per unit and lane
-  const bool split = chunks < whole && ka.n_units > 1 && ka.n_units <= kEvalGroupMaxUnits &&
-                     own + slot_bytes(ka, 64 * waves) <= (size_t)ka.lds_limit;
-  o.units = split ? ka.units : ka.unit_all;
-  o.n_units = split ? ka.n_units : 1;
+  o.units = ka.unit_all;
   o.offsets = e.offsets;
   o.n_traj = e.n_traj;
   o.w2 = e.w2;
@@ -2287,15 +1903,8 @@ hipError_t launch_eval_units(const KinArgs<float>& ka, const SceneArgs<float>& s
     hipLaunchKernelGGL(fill_f32_kernel, dim3(blocks_for(e.n_traj, 256)), dim3(256), 0, st, e.cost, 0.0f,
                        (int64_t)e.n_traj);
   if (B == 0) return hipGetLastError();
-  if (split) {
-    KinArgs<float> kg = ka;  // slots after the unit partials
-    kg.slot_off = (int32_t)own;
-    PMP_DISPATCH_MAXC(ka.n_cols, eval_group_kernel, dim3((unsigned)chunks), dim3(64 * waves),
-                      own + slot_bytes(ka, 64 * waves), st, kg, sc, q, ldq, B, o);
-  } else {
-    PMP_DISPATCH_MAXC(ka.n_cols, eval_units_kernel, dim3((unsigned)chunks), dim3(64), slot_bytes(ka, 64), st, ka, sc,
-                      q, ldq, B, o);
-  }
+  PMP_DISPATCH_MAXC(ka.n_cols, eval_units_kernel, dim3((unsigned)((B + 63) / 64)), dim3(64), slot_bytes(ka, 64), st, ka,
+                    sc, q, ldq, B, o);
   return hipGetLastError();
 }
 // Waves the pair launch aims for: four per SIMD of a 256-CU MI355X.

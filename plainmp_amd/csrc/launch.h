@@ -117,10 +117,14 @@ struct EvalArgs {
   const double* w2;
   float* cost;
   float* grad;
-  int whole_chunks;  // 0: default
+  int whole_chunks;  // pmp_schedule.eval_whole_chunks; 0: default
 };
 hipError_t launch_eval_units(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq,
                              int64_t B, const EvalArgs& e, hipStream_t st);
+// eval.hip: the staged form of launch_eval_units (its status in *err); false
+// when the robot's tables do not fit a workgroup's LDS.
+bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq, int64_t B,
+                        const EvalArgs& e, hipStream_t st, hipError_t* err);
 // shares: primitive shares (grid z), 0 = about four waves per SIMD
 hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq,
                         int64_t B, float* dist, float* grad, int shares, hipStream_t st);

@@ -1,0 +1,194 @@
+// Staged workgroups: C = 64 / H configurations shared by the W waves of a
+// workgroup, with everything that depends only on the configuration computed
+// once and kept in LDS.
+//
+//   1. every joint's local rotation (a lane per (configuration, joint)),
+//   2. FK along the robot's paths, one wave per path: the poses of the
+//      sphere-carrying and joint nodes,
+//   3. the caller's work (sphere blocks, pairs, rows) split over all waves,
+//      each reading the poses it needs.
+//
+// A lane-per-configuration walk of everything leaves a batch of B
+// configurations B / 64 waves; here the walk that cannot be split (FK) runs
+// once and the rest has W waves per C configurations.  H > 1 gives each
+// configuration H lanes of a wave (lane = sub * C + configuration), which
+// share the spheres of a block, so that a batch of a few thousand
+// configurations still gives every CU a workgroup.
+//
+// All tables are laid out [index][configuration], so the lanes of a wave read
+// consecutive words.  The arithmetic of a pose is that of run_fk (fk.hpp).
+#pragma once
+
+#include "device.hpp"
+
+namespace pmp {
+
+// Offsets (in floats) of a staged workgroup's LDS tables.
+struct StageLds {
+  int joints, poses, end;
+};
+inline StageLds stage_lds(const KinArgs<float>& ka, int C) {
+  StageLds L;
+  L.joints = 0;
+  L.poses = 4 * ka.n_joints * C;
+  L.end = L.poses + 7 * ka.n_poses * C;
+  return L;
+}
+
+// Touches [p, p + bytes) through the scalar data cache, a line in n_parts: for
+// waves that would otherwise wait while another one walks, so that the tables
+// the whole workgroup is about to read are in the cache it shares.
+__device__ __forceinline__ void warm_scalar(const void* p, int bytes, int part, int n_parts) {
+  const int32_t* w = reinterpret_cast<const int32_t*>(p);
+  for (int i = part * 16; i < bytes / 4; i += n_parts * 16) {
+    const int v = cload(w, i);
+    asm volatile("" ::"s"(v));
+  }
+}
+
+template <int H>
+struct Stage {
+  static constexpr int C = 64 / H;           // configurations of the workgroup
+  static constexpr int NK = kBlockSpheres / H;  // spheres of a block a lane takes
+  float* lds;
+  StageLds L;
+  int lane, w, W, cfg, sub;
+  __device__ __forceinline__ Stage(float* base, const StageLds& lay)
+      : lds(base),
+        L(lay),
+        lane(threadIdx.x & 63),
+        w(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))),
+        W(blockDim.x >> 6),
+        cfg(lane & (C - 1)),
+        sub(H == 1 ? 0 : lane / C) {}
+
+  // Every joint's local rotation (origin times joint), or its displacement in
+  // word 0 of a prismatic one.
+  template <class QS>
+  __device__ __forceinline__ void joints(const KinArgs<float>& ka, const QS& qs, bool taylor) const {
+    for (int i = w * H + sub; i < ka.n_joints; i += W * H) {
+      const DevJoint jt = H == 1 ? cload(ka.joints, i) : ka.joints[i];
+      const double v = qs.get(jt.q_col);
+      Q4<float> lq{(float)v, 0.0f, 0.0f, 0.0f};
+      if (jt.revolute) {
+        const float x = (float)v * 0.5f;
+        float s, c;
+        if (taylor)
+          taylor_sincos<float>(x, s, c);
+        else
+          exact_sincos(x, s, c);
+        const Q4<float> jq{s * jt.axis[0], s * jt.axis[1], s * jt.axis[2], c};
+        lq = jt.identity ? jq : qmul(Q4<float>{jt.quat[0], jt.quat[1], jt.quat[2], jt.quat[3]}, jq);
+      }
+      float* p = lds + L.joints + 4 * i * C + cfg;
+      p[0] = lq.x;
+      p[C] = lq.y;
+      p[2 * C] = lq.z;
+      p[3 * C] = lq.w;
+    }
+  }
+
+  // The paths of this wave (path p goes to wave p mod W); joints() of every
+  // wave must be complete.
+  template <class QS>
+  __device__ __forceinline__ void walk(const KinArgs<float>& ka, const QS& qs) const {
+    for (int p = w; p < ka.n_paths; p += W) {
+      Pose<float> P = base_pose(ka, qs);
+      const int e_end = cload(ka.path_at, p + 1);
+      int e = cload(ka.path_at, p);
+      DevPathNode next = cload(ka.path, e);
+      for (; e < e_end; ++e) {
+        const DevPathNode pe = next;
+        next = cload(ka.path, e + 1 < e_end ? e + 1 : e);  // one entry ahead of its use
+        const V3<float> lt{pe.trans[0], pe.trans[1], pe.trans[2]};
+        const Q4<float> oq{pe.quat[0], pe.quat[1], pe.quat[2], pe.quat[3]};
+        const float* jc = lds + L.joints + 4 * pe.joint * C + cfg;
+        switch (pe.kind) {
+          case PMP_NODE_ROOT:
+            break;
+          case PMP_NODE_FIXED:
+            P = compose(P, oq, lt, pe.identity != 0);
+            break;
+          case PMP_NODE_REVOLUTE:
+            P = compose(P, Q4<float>{jc[0], jc[C], jc[2 * C], jc[3 * C]}, lt, false);
+            break;
+          case PMP_NODE_PRISMATIC: {
+            const float v = jc[0];
+            const V3<float> t2{lt.x + pe.axis[0] * v, lt.y + pe.axis[1] * v, lt.z + pe.axis[2] * v};
+            P = compose(P, oq, t2, true);
+            break;
+          }
+          default: {  // PMP_NODE_TRANSLATION
+            const M3<float> R = qmat(P.q);
+            P.t = add(P.t, mv(R, lt));
+            break;
+          }
+        }
+        if (pe.pose >= 0) pose_set(pe.pose, P);
+      }
+    }
+  }
+
+  // With H > 1 the lanes of a configuration hold the same value and write it
+  // to the same word.
+  __device__ __forceinline__ void pose_set(int i, const Pose<float>& P) const {
+    float* p = lds + L.poses + 7 * i * C + cfg;
+    p[0] = P.q.x;
+    p[C] = P.q.y;
+    p[2 * C] = P.q.z;
+    p[3 * C] = P.q.w;
+    p[4 * C] = P.t.x;
+    p[5 * C] = P.t.y;
+    p[6 * C] = P.t.z;
+  }
+  // i may differ between lanes
+  __device__ __forceinline__ Pose<float> pose(int i) const {
+    const float* p = lds + L.poses + 7 * i * C + cfg;
+    return {{p[0], p[C], p[2 * C], p[3 * C]}, {p[4 * C], p[5 * C], p[6 * C]}};
+  }
+  // World axis and origin of q column j (wave-uniform or not); false when the
+  // column moves no sphere.
+  template <class QS>
+  __device__ __forceinline__ bool frame(const KinArgs<float>& ka, const QS& qs, int j, V3<float>& a,
+                                        V3<float>& o) const {
+    if (j >= ka.n_q_cols) {
+      base_columns(ka, base_pose(ka, qs), qs, [&](int col, V3<float> ca, V3<float> co) {
+        if (col == j) {
+          a = ca;
+          o = co;
+        }
+      });
+      return true;
+    }
+    const DevColumn col = ka.columns[j];
+    if (col.pose < 0) return false;
+    const Pose<float> P = pose(col.pose);
+    a = qrot(P.q, V3<float>{col.axis[0], col.axis[1], col.axis[2]});
+    o = P.t;
+    return true;
+  }
+
+  // The n (at most NK) spheres of block bk this lane takes: centres and radii.
+  __device__ __forceinline__ void spheres(const KinArgs<float>& ka, int bi, const DevSphereBlock& bk,
+                                          const Pose<float>& P, const M3<float>& R, V3<float> (&c)[NK],
+                                          float (&r)[NK], int& n) const {
+    n = H == 1 ? bk.n : bk.n - sub * NK;
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      c[k] = P.t;
+      r[k] = 0.0f;
+      if constexpr (H == 1) {
+        if (k < n) {
+          c[k] = add(mv(R, V3<float>{bk.s[k][0], bk.s[k][1], bk.s[k][2]}), P.t);
+          r[k] = bk.s[k][3];
+        }
+      } else if (k < n) {
+        const Quad4 s = reinterpret_cast<const Quad4*>(ka.blocks[bi].s)[sub * NK + k];  // a sphere a lane
+        c[k] = add(mv(R, V3<float>{s.v[0], s.v[1], s.v[2]}), P.t);
+        r[k] = s.v[3];
+      }
+    }
+  }
+};
+
+}  // namespace pmp

@@ -18,10 +18,12 @@ constexpr int kMaxPrims = 512;
 constexpr int kMaxSelfPairs = 1024;
 constexpr int kMaxClouds = 4;
 constexpr int kCloudTile = 64;  // points per cloud tile
+constexpr int kSliceCands = 8;  // candidates of a sphere block a staged evaluate wave takes at a time
 constexpr int kBlockSpheres = 8;  // spheres of one link tested together against a primitive
 // XCDs of an MI355X; workgroups of a launch are handed to them in turn.  Only
 // the locality of index mappings depends on it.
 constexpr int kXcds = 8;
+constexpr int kCus = 256;  // compute units of an MI355X (choice of launch shapes only)
 
 // Primitive kinds of the validity pass; the scene keeps a copy of its
 // primitives sorted by kind so that each kind is a loop without branches.
@@ -57,7 +59,9 @@ struct alignas(16) DevSphereBlock {
   int32_t n;
   int32_t ext[kBlockSpheres];  // index among the primitive-checked spheres
   int32_t sph[kBlockSpheres];  // index in the node-sorted sphere tables
-  int32_t pad[3];
+  int32_t group[kBlockSpheres], out[kBlockSpheres];  // group and group-order index
+  int32_t pose;                // pose-table index of the block's node
+  float n2_lo, n2_hi;          // the node's bounds of |q|^2
   float g[3], G;
   float s[kBlockSpheres][4];   // link-frame centre and radius
 };
@@ -82,10 +86,52 @@ static_assert(kNumKinds + 1 == 8, "CullRange holds one offset per kind plus the 
 // adjoint kernels, which give each (configuration, item) its own lane.
 constexpr int kItemSpheres = 8;
 struct alignas(16) DevSphereItem {
-  int32_t node, begin, end, pad;
+  int32_t node, begin, end, pose;  // pose: pose-table index of the node
 };
 
-// A unit of the evaluate kernels: the sphere blocks [b_lo, b_hi) against
+// Staged kernels (stage.hpp): a workgroup walks the kinematic tree once for
+// its configurations, path by path from the root to a node that carries
+// spheres, and keeps the poses it needs later in LDS.  Every node on a path
+// has the entry before it as its parent.
+struct alignas(64) DevPathNode {  // one cache line: the node's local transform and what to keep
+  float quat[4];
+  float trans[3];
+  float axis[3];
+  int32_t kind, identity;
+  int32_t joint;  // its joint in the joint table (its local rotation or displacement is there), else 0
+  int32_t pose;   // pose-table index to write, -1: none (or another path writes it)
+  int32_t pad[2];
+};
+static_assert(sizeof(DevPathNode) == 64, "a path entry is one cache line");
+
+// A joint on some path.
+struct alignas(16) DevJoint {
+  float quat[4];  // origin rotation
+  float axis[3];
+  int32_t q_col, identity, revolute, pad[2];
+};
+// The joint frame of a q column: pose-table index of its node (-1: the column
+// moves no sphere, or belongs to the base) and the axis in that frame.
+struct alignas(16) DevColumn {
+  float axis[3];
+  int32_t pose;
+};
+
+// What a winning sphere's Jacobian row needs, in one gather (group order).
+struct alignas(32) DevSphereRow {
+  float x, y, z;
+  int32_t pose;       // pose-table index of its node
+  uint64_t col_mask;  // q columns that move it
+  uint64_t pad;
+};
+
+// A slice of a sphere block's candidates: cull entries [lo, hi) of block
+// `block`; the first slice of a block also takes what has no candidate list.
+struct alignas(16) DevCullSlice {
+  int32_t block, lo, hi, first;
+};
+
+// A unit of the lane-per-configuration kernels: the sphere blocks [b_lo, b_hi) against
 // their candidate primitives and the self pairs [k_lo, k_hi), walking FK to
 // node `last`.
 struct alignas(16) DevEvalUnit {
@@ -132,6 +178,7 @@ struct alignas(16) DevSelfPair {
   int32_t slot1, begin1, end1, slot2;
   int32_t begin2, end2, node1, node2;
   float bound1[4], bound2[4];  // each group's bounding sphere in its link frame: centre, radius (rounded up)
+  int32_t pose1, pose2, pad[2];  // pose-table indices of node1 and node2
 };
 
 // Kernel arguments describing the robot (passed by value: kernarg -> SGPRs).
@@ -154,6 +201,13 @@ struct KinArgs {
   int32_t slot_off;         // byte offset of the kept-pose slots in the launch's dynamic LDS
   int32_t slot_wave_bytes;  // kept-pose bytes per wave (n_slots * 7 * 64 * sizeof(T), or more)
   int32_t lds_limit;        // LDS bytes one workgroup may use on this device (launch sizing)
+  const DevPathNode* path;  // staged kernels: paths back to back, path i = [path_at[i], path_at[i + 1])
+  const int32_t* path_at;
+  const DevJoint* joints;
+  const DevColumn* columns;  // [n_q_cols]
+  const DevSphereRow* rows;  // [n_spheres], group order
+  int32_t n_paths, n_poses, n_joints;
+  int32_t staged;  // the staged tables describe this robot (no q column drives two joints)
   T base_q[4];
   T base_t[3];
 };
@@ -191,6 +245,8 @@ struct SceneArgs {
   const CullRange* cull_range;  // [n_blocks]
   const CullEntry* ecull;       // the same for evaluate: boxes grown by the 0.1 m cutoff
   const CullRange* ecull_range;
+  const DevCullSlice* eslices;  // the evaluate candidates cut into slices, last block first
+  int32_t n_ecull, n_eslices;
   const int32_t* vorig;         // kind-sorted index -> scene order
 };
 
