@@ -250,12 +250,9 @@ pmp_status pmp_is_valid_batch(pmp_context* ctx, const double* q, int64_t ldq, in
 /* pmp_is_valid_batch without any allocation: no hipMalloc, hipFree or
  * allocating library call, for callers that cannot allocate (code under HIP
  * graph capture, tight serving loops).  No counterpart in the reference.
- * Its workspaces come from a static device array of 32 MiB that every GPU
- * the library runs on holds until the process ends; a batch that needs more
- * (scenes with a point cloud: 28 B per primitive-checked sphere and
- * configuration plus 4 B per configuration) is refused with PMP_ERR_INVALID.
- * All calls on one GPU share that array: calls that overlap on one GPU (from
- * several contexts, or captured into graphs that replay concurrently) race. */
+ * A batch of more than 32 MiB of query data (scenes with a point cloud: 28 B
+ * per primitive-checked sphere and configuration plus 4 B per configuration)
+ * is refused with PMP_ERR_INVALID. */
 pmp_status pmp_is_valid_batch_noalloc(pmp_context* ctx, const double* q, int64_t ldq, int64_t B, uint8_t* valid,
                                       int32_t* n_recheck);
 

@@ -206,8 +206,7 @@ struct pmp_context {
   std::vector<int64_t> h_traj_off;
   std::vector<double> h_traj_w2;
   EdgeBufs eb;  // edge buffers of direct calls
-  DevBuf seq, tmp_prims, tmp_cloud, ws_cen, ws_cloud, ws_flags;
-  DevBuf ws_vunit;  // per-configuration flags of the unit validity pass (kValidUnitsMaxBatch)
+  DevBuf seq, tmp_prims, tmp_cloud, ws_cen, ws_cloud;
   // Cross-stream order of calls (they share the workspaces above): an event
   // recorded on the stream of the last call, waited on by a call on another.
   hipEvent_t call_ev = nullptr;
@@ -434,6 +433,10 @@ void rebuild_cull(pmp_context* ctx) {
   TablePack pk;
   pk.add(ent, &ctx->s32.cull, &ctx->s64.cull);
   pk.add(rng, &ctx->s32.cull_range, &ctx->s64.cull_range);
+  const std::vector<DevCullSlice> vsl = cull_slices(rng, (int)ctx->h_blocks.size());
+  pk.add(vsl, &ctx->s32.slices, &ctx->s64.slices);
+  ctx->s32.n_cull = ctx->s64.n_cull = (int32_t)ent.size();
+  ctx->s32.n_slices = ctx->s64.n_slices = (int32_t)vsl.size();
   build_cull(ctx, 0.1, ent, rng);
   pk.add(ent, &ctx->s32.ecull, &ctx->s64.ecull);
   pk.add(rng, &ctx->s32.ecull_range, &ctx->s64.ecull_range);
@@ -553,7 +556,6 @@ pmp_status pmp_create(int32_t device, pmp_context** out) {
       PMP_HIP(hipGetDeviceProperties(&prop, device));
       ctx->n_cu = prop.multiProcessorCount;
       ctx->max_lds = (int)prop.sharedMemPerBlock;
-      PMP_HIP(noalloc_scratch_init(device));
       PMP_HIP(hipEventCreateWithFlags(&ctx->call_ev, hipEventDisableTiming));
       ctx->seq.upload(sequence_table(), nullptr);
       PMP_HIP(hipDeviceSynchronize());
@@ -573,7 +575,7 @@ pmp_status pmp_destroy(pmp_context* ctx) {
     (void)hipDeviceSynchronize();
     for (DevBuf* b : {&ctx->robot_tables, &ctx->scene_tables, &ctx->cull_tables, &ctx->ws_vjp, &ctx->supers,
                       &ctx->tiles32, &ctx->tiles64, &ctx->tileB, &ctx->pts64, &ctx->seq, &ctx->tmp_prims, &ctx->tmp_cloud,
-                      &ctx->ws_cen, &ctx->cloud_stage, &ctx->cloud_scratch, &ctx->ws_vunit, &ctx->ws_cloud, &ctx->ws_flags,
+                      &ctx->ws_cen, &ctx->cloud_stage, &ctx->cloud_scratch, &ctx->ws_cloud,
                       &ctx->traj_off, &ctx->traj_w2, &ctx->sqp_rows, &ctx->sqp_tables})
       b->release();
     ctx->eb.release();
@@ -1294,34 +1296,8 @@ pmp_status pmp_is_valid_batch(pmp_context* ctx, const double* q, int64_t ldq, in
     PMP_REQUIRE(B == 0 || valid, "null output");
     if (B == 0) return;
     set_device(ctx);
-    CloudWork cw{};
-    int32_t* flags = nullptr;
-    if (ctx->n_clouds) {
-      const int64_t Q = (int64_t)ctx->k32.n_ext_spheres * B;
-      cw.B = B;
-      cw.cen = (float*)ctx->ws_cen.get(sizeof(float) * std::max<int64_t>(3 * Q, 1));
-      float* w = (float*)ctx->ws_cloud.get(sizeof(float) * std::max<int64_t>(4 * Q * ctx->n_clouds, 1));
-      for (int oc = 0; oc < ctx->n_clouds; ++oc) {  // per cloud: cap2, rr, then the d2 bracket (upper, lower)
-        cw.cap2[oc] = w + 4 * Q * oc;
-        cw.rr[oc] = cw.cap2[oc] + Q;
-      }
-      // the cloud pass's flags are zero on entry and left zero: cleared when
-      // the buffer is new
-      const bool fresh_flags = ctx->ws_flags.bytes < sizeof(int32_t) * (size_t)B;
-      flags = (int32_t*)ctx->ws_flags.get(sizeof(int32_t) * B);
-      if (fresh_flags) PMP_HIP(launch_fill_i32(flags, 0, (int64_t)(ctx->ws_flags.bytes / sizeof(int32_t)), st(ctx)));
-    }
-    // batches up to kValidUnitsMaxBatch: a lane per (configuration, unit);
-    // the flags start at zero (cleared when the buffer is new) and the pass
-    // leaves them so
-    int32_t* unit_flags = nullptr;
-    if (B <= kValidUnitsMaxBatch && ctx->k32.n_units > 0) {
-      const bool fresh = ctx->ws_vunit.bytes < sizeof(int32_t) * (size_t)kValidUnitsMaxBatch;
-      unit_flags = (int32_t*)ctx->ws_vunit.get(sizeof(int32_t) * kValidUnitsMaxBatch);
-      if (fresh) PMP_HIP(launch_fill_i32(unit_flags, 0, kValidUnitsMaxBatch, st(ctx)));
-    }
     PMP_HIP(launch_valid(ctx->k32, ctx->k64, ctx->s32, ctx->s64, q, ldq, B, ctx->band, valid, n_recheck,
-                         ctx->sched.block, cw, ctx->clouds.data(), ctx->n_clouds, flags, unit_flags, st(ctx)));
+                         ctx->sched.block, CloudWork{}, nullptr, 0, nullptr, nullptr, st(ctx)));
   });
 }
 
@@ -1331,42 +1307,23 @@ pmp_status pmp_is_valid_batch_noalloc(pmp_context* ctx, const double* q, int64_t
     PMP_BATCH_CHECKS(q, ldq, B);
     PMP_REQUIRE(B == 0 || valid, "null output");
     if (B == 0) return;
-    set_device(ctx);
-    unsigned char* ws = (unsigned char*)noalloc_scratch(ctx->device);
-    PMP_REQUIRE(ws != nullptr, "internal: no-allocation scratch not set up on this device");
-    // The same workspaces as pmp_is_valid_batch, carved from the static
-    // scratch (256-byte aligned pieces).
-    auto carve = [&](size_t& at, size_t bytes) {
-      unsigned char* p = ws + at;
-      at += (bytes + 255) & ~(size_t)255;
-      return p;
-    };
+    // the documented limit of this entry point (256-byte aligned pieces)
     size_t need = 0;
-    CloudWork cw{};
-    int32_t* flags = nullptr;
-    int32_t* unit_flags = nullptr;
+    auto piece = [&](size_t bytes) { need += (bytes + 255) & ~(size_t)255; };
     if (ctx->n_clouds) {
-      const int64_t Q = (int64_t)ctx->k32.n_ext_spheres * B;
-      cw.B = B;
-      cw.cen = (float*)carve(need, sizeof(float) * 3 * (size_t)Q);
-      float* w = (float*)carve(need, sizeof(float) * 4 * (size_t)Q * ctx->n_clouds);
-      for (int oc = 0; oc < ctx->n_clouds; ++oc) {
-        cw.cap2[oc] = w + 4 * Q * oc;
-        cw.rr[oc] = cw.cap2[oc] + Q;
-      }
-      flags = (int32_t*)carve(need, sizeof(int32_t) * (size_t)B);
+      const size_t Q = (size_t)ctx->k32.n_ext_spheres * (size_t)B;
+      piece(sizeof(float) * 3 * Q);
+      piece(sizeof(float) * 4 * Q * ctx->n_clouds);
+      piece(sizeof(int32_t) * (size_t)B);
     }
-    if (B <= kValidUnitsMaxBatch && ctx->k32.n_units > 0) unit_flags = (int32_t*)carve(need, sizeof(int32_t) * (size_t)B);
+    if (B <= 65536 && ctx->k32.n_units > 0) piece(sizeof(int32_t) * (size_t)B);
     PMP_REQUIRE(need <= kNoAllocScratchBytes,
                 "batch needs " + std::to_string(need) + " bytes of scratch, more than the " +
                     std::to_string(kNoAllocScratchBytes) +
                     " bytes pmp_is_valid_batch_noalloc has; split the batch or call pmp_is_valid_batch");
-    // the scratch keeps the previous call's contents: the unit pass and the
-    // cloud pass need their flags at zero (fill kernels, not memset nodes)
-    if (unit_flags) PMP_HIP(launch_fill_i32(unit_flags, 0, B, st(ctx)));
-    if (flags) PMP_HIP(launch_fill_i32(flags, 0, B, st(ctx)));
+    set_device(ctx);
     PMP_HIP(launch_valid(ctx->k32, ctx->k64, ctx->s32, ctx->s64, q, ldq, B, ctx->band, valid, n_recheck,
-                         ctx->sched.block, cw, ctx->clouds.data(), ctx->n_clouds, flags, unit_flags, st(ctx)));
+                         ctx->sched.block, CloudWork{}, nullptr, 0, nullptr, nullptr, st(ctx)));
   });
 }
 

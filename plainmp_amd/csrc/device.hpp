@@ -58,6 +58,28 @@ __device__ __forceinline__ int wave_max_i(int v) {
   return __builtin_amdgcn_readfirstlane(v);
 }
 
+// The FP32 walk's band covers its rounding for joint values within these
+// ranges (an angle's FP32 rounding is |q| 2^-24, so within 4 pi it stays
+// below 1e-6 rad; a translation within 16 m, below 1e-6 m).  A state with
+// a value outside them is decided by the FP64 walk.
+constexpr double kFp32AngleRange = 4.0 * M_PI;
+constexpr double kFp32LinearRange = 16.0;
+__device__ __forceinline__ bool fp32_range_col(uint64_t rev_mask, int col, double v) {
+  return fabs(v) <= (((rev_mask >> col) & 1ull) ? kFp32AngleRange : kFp32LinearRange);
+}
+
+// Orders a wave's own LDS accesses: what its lanes wrote before is what they
+// read after.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// The lane's rank among the lanes of mask m.
+__device__ __forceinline__ int lane_rank(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+}
+
 // Four consecutive floats of a table read as one wave-uniform load.
 struct alignas(16) Quad4 {
   float v[4];

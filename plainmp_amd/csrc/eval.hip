@@ -138,9 +138,7 @@ __device__ __forceinline__ void ext_slice(const Stage<H>& S, const KinArgs<float
       const uint32_t pkey = (uint32_t)(orig * ka.n_spheres);
       int cnt = 0;  // entries collected, wave-uniform
       auto flush = [&]() {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_order();
         if (S.lane < cnt) {
           const float* t = entries + S.lane;
           const V3<float> ec{t[0], t[64], t[128]};
@@ -148,9 +146,7 @@ __device__ __forceinline__ void ext_slice(const Stage<H>& S, const KinArgs<float
           const float v = sdf_eval_kind<K>(Q, ec) - er;
           if (!outside_aabb(Q, ec, er + kCutoff)) offer(best + __float_as_int(t[320]), v, (uint32_t)__float_as_int(t[256]));
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_lds_order();
         cnt = 0;
       };
 #pragma unroll
@@ -162,7 +158,7 @@ __device__ __forceinline__ void ext_slice(const Stage<H>& S, const KinArgs<float
         if (cnt + more > 64) flush();
         const uint32_t key = key_of(k);
         if (pass) {
-          float* t = entries + cnt + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+          float* t = entries + cnt + lane_rank(m);
           t[0] = c[k].x;
           t[64] = c[k].y;
           t[128] = c[k].z;
@@ -460,16 +456,9 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
     o_best = (L.end + (o_scratch ? need : 0) + 1) & ~1;
     return sizeof(float) * (size_t)(o_best + 4 * C + 2 * C + 1);
   };
-  // 16 configurations a workgroup while every CU then gets one at most, else
-  // 32, else 64, with 16 waves each: 32 primitives, 7R arm, 4,096
-  // configurations 19.1 us so, 24 with 64 a workgroup; 8,192: 22.0 with 32,
-  // 24.3 with 64.  Once a CU has several workgroups, 8 waves each (32,768: 35
-  // us, 16 waves 60), and 4 when the robot has so few blocks that most of 8
-  // would wait for the walk (65,536: 50 us, 8 waves 63).
-  const int n_blocks = ka.n_units - ka.n_pairs;
-  int H = B <= 16 * kCus ? 4 : (B <= 32 * kCus ? 2 : 1);
-  const int W = B <= 64 * kCus ? 16 : (B > 128 * kCus && n_blocks <= 8 ? 4 : 8);
-  while (H < 4 && lds_of(H, W) > (size_t)ka.lds_limit) H *= 2;
+  StageShape sh = stage_shape(B, ka.n_units - ka.n_pairs);
+  while (sh.H < 8 && lds_of(sh.H, sh.W) > (size_t)ka.lds_limit) sh.H *= 2;
+  const int H = sh.H, W = sh.W;
   const size_t lds = lds_of(H, W);
   if (lds > (size_t)ka.lds_limit) return false;
   StagedOut o{};
@@ -491,12 +480,16 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   o.best = o_best;
   const dim3 grid((unsigned)(chunks + (o.n_traj + W - 1) / W)), block(64 * W);
   if (grid.x > 0) {
+#define PMP_EVAL(H) hipLaunchKernelGGL(eval_staged_kernel<H>, grid, block, lds, st, ka, sc, q, ldq, B, o, lay)
     if (H == 1)
-      hipLaunchKernelGGL(eval_staged_kernel<1>, grid, block, lds, st, ka, sc, q, ldq, B, o, lay);
+      PMP_EVAL(1);
     else if (H == 2)
-      hipLaunchKernelGGL(eval_staged_kernel<2>, grid, block, lds, st, ka, sc, q, ldq, B, o, lay);
+      PMP_EVAL(2);
+    else if (H == 4)
+      PMP_EVAL(4);
     else
-      hipLaunchKernelGGL(eval_staged_kernel<4>, grid, block, lds, st, ka, sc, q, ldq, B, o, lay);
+      PMP_EVAL(8);
+#undef PMP_EVAL
   }
   *err = hipGetLastError();
   return true;

@@ -493,7 +493,7 @@ PMP_HD bool is_outside_ref(const DevPrim<T>& p, V3<T> c, T r) {
 // by the exact test; for the ground it is part of the decision (its AABB is
 // z in [0, 0]).  NaN centres are the caller's business (see collide_fast).
 template <int K>
-PMP_HD bool collide_kind(const DevPrim<float>& p, V3<float> c, float r, float band, bool& inband) {
+__device__ __forceinline__ bool collide_kind(const DevPrim<float>& p, V3<float> c, float r, float band, bool& inband) {
   const float dx = c.x - p.pos[0], dy = c.y - p.pos[1], dz = c.z - p.pos[2];
   if constexpr (K == kKindBoxAA || K == kKindBoxRot) {
     V3<float> d = {dx, dy, dz};
@@ -515,7 +515,8 @@ PMP_HD bool collide_kind(const DevPrim<float>& p, V3<float> c, float r, float ba
       xa = dx * p.R[0] + dy * p.R[3] + dz * p.R[6];
       ya = dx * p.R[1] + dy * p.R[4] + dz * p.R[7];
     }
-    const float rs = fmaxf(sqrtf(xa * xa + ya * ya) - p.p0, 0.0f);
+    // the root's rounding is far inside the band
+    const float rs = fmaxf(approx_sqrt(xa * xa + ya * ya) - p.p0, 0.0f);
     zs = fmaxf(zs, 0.0f);
     const float m = rs * rs + zs * zs - r * r;
     inband |= fabsf(m) <= band * (2.0f * r + band);
@@ -550,7 +551,7 @@ PMP_HD int prim_kind(const DevPrim<T>& p) {
 
 // Any non-cloud primitive.  A NaN centre collides, as every comparison of the
 // reference is false for NaN.
-PMP_HD bool collide_fast(const DevPrim<float>& p, V3<float> c, float r, float band, bool& inband) {
+__device__ __forceinline__ bool collide_fast(const DevPrim<float>& p, V3<float> c, float r, float band, bool& inband) {
   if (is_nan3(c)) return true;
   switch (prim_kind(p)) {
     case kKindBoxAA:

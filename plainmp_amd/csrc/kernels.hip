@@ -122,9 +122,7 @@ __global__ void __launch_bounds__(256) clearance_kernel(KinArgs<float> ka, Scene
 // FP32 pass: a collision decided outside the band ends the lane's work
 // ("definite"); a decision inside the band marks the configuration for the
 // FP64 re-decision ("uncertain").
-// kInlineCloud: clouds are tested inside the walk (the edge pass, whose
-// states have no batch-wide cloud pass of their own); otherwise the walk
-// writes cloud queries for the matrix-core pass when use_cw is set.
+// kInlineCloud: the scene holds clouds, tested inside the walk.
 // kFirstHit: the lanes are states of one edge and only the first certain
 // collision in visiting order (`key`) matters, so a lane whose key is past
 // the wave's first certain collision so far stops taking part.
@@ -135,9 +133,6 @@ struct ValidVis32T {
   const KinArgs<float>& ka;
   const SceneArgs<float>& sc;
   float band;
-  CloudWork cw{};        // cloud queries are written here when use_cw (the scene holds clouds)
-  bool use_cw = false;
-  int64_t b = 0;
   int key = 0;  // visiting index of the lane's state (kFirstHit)
   bool idle = false;
   bool definite = false;
@@ -254,47 +249,6 @@ struct ValidVis32T {
         uncertain = true;
         n_inb = 2;
       }
-      if (use_cw && !idle) {
-        const int64_t B = cw.B;
-#pragma unroll
-        for (int k = 0; k < kBlockSpheres; ++k) {
-          if (k < n) {
-            const int64_t e = bk.ext[k];
-            cw.cen[(e * 3 + 0) * B + b] = c[k].x;
-            cw.cen[(e * 3 + 1) * B + b] = c[k].y;
-            cw.cen[(e * 3 + 2) * B + b] = c[k].z;
-          }
-        }
-        // clouds: queried by the matrix-core pass unless the AABB pre-test culls it
-        const DevPrim<float>* vp = reinterpret_cast<const DevPrim<float>*>(sc.vprims);
-        for (int p = sc.vrange[kKindCloud]; p < sc.vrange[kKindCloud + 1]; ++p) {
-          const DevPrim<float> Pc = cload(vp, p);
-          const int oc = (Pc.flags >> 4) & 15;
-          // the cloud's output arrays, chosen with constant indices so that
-          // the arguments stay in registers (an indexed kernel argument
-          // would be copied to scratch)
-          float* cap2 = cw.cap2[0];
-          float* rro = cw.rr[0];
-#pragma unroll
-          for (int i = 1; i < kMaxClouds; ++i) {
-            if (oc == i) {
-              cap2 = cw.cap2[i];
-              rro = cw.rr[i];
-            }
-          }
-#pragma unroll
-          for (int k = 0; k < kBlockSpheres; ++k) {
-            if (k < n) {
-              const float r = bk.s[k][3];
-              const bool qd = alive() && !outside_aabb(Pc, c[k], r);
-              const float Rr = r + Pc.p0;
-              const int64_t at = (int64_t)bk.ext[k] * B + b;
-              cap2[at] = qd ? (Rr + band) * (Rr + band) : -1.0f;
-              rro[at] = qd ? Rr : -1.0f;
-            }
-          }
-        }
-      }
       if (!wave_any(alive())) continue;
       const CullRange cr = cload(sc.cull_range, bi);
       reach = bk.G * growf + band + 1e-4f;
@@ -365,23 +319,6 @@ struct ValidVis32T {
     } else if (m < 0.0f) {
       definite = true;
     }
-  }
-};
-
-using ValidVis32 = ValidVis32T<false>;
-
-// The FP32 validity test of one evaluate unit (a sphere block, or a self
-// link pair) of a configuration: FK stops at the unit's last node, blocks
-// and self pairs outside the unit are skipped.  Clouds are not handled (the
-// unit pass runs only for scenes without one).
-struct ValidUnitVis : ValidVis32 {
-  static constexpr bool kRanged = true;
-  DevEvalUnit u{};
-  __device__ int last_node() const { return u.last; }
-  __device__ int pair_lo() const { return u.k_lo; }
-  __device__ int pair_hi() const { return u.k_hi; }
-  __device__ void blocks(const DevNode<float>& nd, const Pose<float>& P) {
-    blocks_range(nd, P, max(nd.block_begin, u.b_lo), min(nd.block_end, u.b_hi));
   }
 };
 
@@ -534,105 +471,6 @@ struct PairVis64 {
   }
   __device__ void self(const DevSelfPair&, int, int, V3<double>, V3<double>, double) {}
 };
-
-// The FP32 walk's band covers its rounding for joint values within these
-// ranges (an angle's FP32 rounding is |q| 2^-24, so within 4 pi it stays
-// below 1e-6 rad; a translation within 16 m, below 1e-6 m).  A state with
-// a value outside them is decided by the FP64 walk.
-constexpr double kFp32AngleRange = 4.0 * M_PI;
-constexpr double kFp32LinearRange = 16.0;
-__device__ __forceinline__ bool fp32_range_col(uint64_t rev_mask, int col, double v) {
-  return fabs(v) <= (((rev_mask >> col) & 1ull) ? kFp32AngleRange : kFp32LinearRange);
-}
-
-// valid[b] of a configuration with a joint value outside the FP32 walk's
-// ranges: the FP64 walk decides it, whatever the FP32 tests said.
-constexpr uint8_t kValidFp64 = 3;
-template <class QS>
-__device__ __forceinline__ bool fp32_range(const KinArgs<float>& ka, const QS& qs) {
-  bool in = true;
-  for (int j = 0; j < ka.n_cols; ++j) in &= fp32_range_col(ka.rev_mask, j, qs.get(j));
-  return in;
-}
-
-// valid[b]: 0 collision, 1 free, 2 pending FP64 re-decision, kValidFp64
-// decided by the FP64 walk only.
-__global__ void __launch_bounds__(256) valid_kernel(KinArgs<float> k32, SceneArgs<float> s32, const double* q,
-                                                    int64_t ldq, int64_t B, float band, uint8_t* valid, CloudWork cw) {
-  const int64_t b = gid();
-  const bool active = b < B;
-  BatchQ qs{q, ldq, active ? b : B - 1};
-  const bool taylor = k32.base_type == PMP_BASE_FIXED;  // constraints/primitive.hpp:59-61
-  ValidVis32 v{k32, s32, band};
-  v.cw = cw;
-  v.use_cw = s32.n_cloud > 0 && active;
-  v.b = b;
-  v.idle = !active;
-  run_fk(k32, qs, taylor, v);
-  if (active) valid[b] = !fp32_range(k32, qs) ? kValidFp64 : (v.definite ? 0 : (v.uncertain ? 2 : 1));
-}
-
-// Batches of up to kValidUnitsMaxBatch configurations: a lane per
-// (configuration, unit), the unit being grid row y, so that a batch of a few
-// thousand configurations still spreads over the GPU.  Each lane ORs its
-// outcome into flags[b] (1: a certain collision, 2: a test in the band);
-// valid_units_finish_kernel turns the flags into the answer valid_kernel
-// gives (a certain collision anywhere decides, else any band test leaves
-// the configuration to the FP64 pass) and clears them for the next launch.
-// With clouds in the scene each lane writes the cloud queries of its unit's
-// sphere blocks (the units' blocks partition the spheres).
-__global__ void __launch_bounds__(64) valid_units_kernel(KinArgs<float> k32, SceneArgs<float> s32, const double* q,
-                                                         int64_t ldq, int64_t B, float band, int32_t* flags,
-                                                         CloudWork cw) {
-  const int64_t b = gid();
-  const bool active = b < B;
-  BatchQ qs{q, ldq, active ? b : B - 1};
-  ValidUnitVis v{{k32, s32, band}};
-  v.u = cload(k32.units, (int)blockIdx.y);
-  v.cw = cw;
-  v.use_cw = s32.n_cloud > 0 && active;
-  v.b = b;
-  v.idle = !active;
-  run_fk(k32, qs, k32.base_type == PMP_BASE_FIXED, v);
-  // unit 0 also reports a joint value outside the FP32 walk's ranges (4)
-  const int f = (v.definite ? 1 : 0) | (v.uncertain ? 2 : 0) | (blockIdx.y == 0 && !fp32_range(k32, qs) ? 4 : 0);
-  if (active && f != 0) atomicOr(flags + b, f);
-}
-
-__global__ void __launch_bounds__(256) valid_units_finish_kernel(int32_t* flags, int64_t B, uint8_t* valid) {
-  const int64_t b = gid();
-  if (b >= B) return;
-  const int f = flags[b];
-  valid[b] = (f & 4) ? kValidFp64 : ((f & 1) ? 0 : ((f & 2) ? 2 : 1));
-  flags[b] = 0;
-}
-
-// FP64 re-decision of the configurations left pending (2) by the FP32 pass
-// and of those it could not decide (kValidFp64).
-// With unit_flags (a scene without clouds, after the unit pass) it first
-// turns the flags into valid[b] as valid_units_finish_kernel does, and
-// clears them.
-__global__ void __launch_bounds__(64) valid_recheck_kernel(KinArgs<double> k64, SceneArgs<double> s64,
-                                                           const double* q, int64_t ldq, int64_t B, uint8_t* valid,
-                                                           int32_t* n_recheck, int32_t* unit_flags) {
-  const int64_t b = gid();
-  if (b >= B) return;
-  if (unit_flags) {
-    const int f = unit_flags[b];
-    unit_flags[b] = 0;
-    if (!(f & 4) && (f & 3) != 2) {
-      valid[b] = (f & 1) ? 0 : 1;
-      return;
-    }
-  } else if (valid[b] < 2) {
-    return;
-  }
-  BatchQ qs{q, ldq, b};
-  ValidVis64 v{k64, s64};
-  run_fk(k64, qs, k64.base_type == PMP_BASE_FIXED, v);
-  valid[b] = v.collided ? 0 : 1;
-  if (n_recheck) atomicAdd(n_recheck, 1);
-}
 
 // ------------------------------------------------------------------ edges
 // Persistent kernel: each wave takes the next edge from a global counter,
@@ -1664,38 +1502,6 @@ hipError_t launch_clearance(const KinArgs<float>& ka, const SceneArgs<float>& sc
   const int bk = slot_block(ka, 256);
   hipLaunchKernelGGL(clearance_kernel, dim3(blocks_for(B, bk)), dim3(bk), slot_bytes(ka, bk), st, ka, sc, q, ldq, B,
                      taylor, out, cen);
-  return hipGetLastError();
-}
-hipError_t launch_valid(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,
-                        const SceneArgs<double>& s64, const double* q, int64_t ldq, int64_t B, float band,
-                        uint8_t* valid, int32_t* n_recheck, int block, const CloudWork& cw,
-                        const CloudRange* clouds, int n_clouds, int32_t* flags, int32_t* unit_flags,
-                        hipStream_t st) {
-  if (block <= 0) block = 256;
-  block = slot_block(k32, block);
-  // the unit flags become answers in the FP64 pass (no clouds) or in the
-  // first cloud's merge
-  const int64_t Q = (int64_t)k32.n_ext_spheres * B;
-  const bool units = unit_flags && k32.n_units > 0;
-  const bool fused = units && n_clouds == 0;
-  const bool merged = units && n_clouds > 0 && Q > 0;
-  if (units) {
-    hipLaunchKernelGGL(valid_units_kernel, dim3(blocks_for(B, 64), (unsigned)k32.n_units), dim3(64),
-                       slot_bytes(k32, 64), st, k32, s32, q, ldq, B, band, unit_flags, cw);
-    if (!fused && !merged)
-      hipLaunchKernelGGL(valid_units_finish_kernel, dim3(blocks_for(B, 256)), dim3(256), 0, st, unit_flags, B, valid);
-  } else {
-    hipLaunchKernelGGL(valid_kernel, dim3(blocks_for(B, block)), dim3(block), slot_bytes(k32, block), st, k32, s32, q,
-                       ldq, B, band, valid, cw);
-  }
-  // sphere-vs-cloud queries on the matrix cores, one pass per cloud
-  for (int oc = 0; oc < n_clouds && Q > 0; ++oc) {
-    hipError_t e = launch_cloud_valid(s32.tiles, s32.tileB, s32.supers, clouds[oc], cw.cen, cw.cap2[oc], cw.rr[oc],
-                                      B, Q, band, valid, flags, merged && oc == 0 ? unit_flags : nullptr, st);
-    if (e != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL(valid_recheck_kernel, dim3(blocks_for(B, 64)), dim3(64), slot_bytes(k64, 64), st, k64, s64, q,
-                     ldq, B, valid, n_recheck, fused ? unit_flags : nullptr);
   return hipGetLastError();
 }
 hipError_t launch_edges(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,

@@ -77,28 +77,16 @@ struct CloudRange {
 
 hipError_t launch_clearance(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq,
                             int64_t B, int taylor, float* out, float* cen, hipStream_t st);
+// valid.hip.  block, cw, clouds, n_clouds, flags and unit_flags are not used:
+// the staged form keeps everything in LDS.
 hipError_t launch_valid(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,
                         const SceneArgs<double>& s64, const double* q, int64_t ldq, int64_t B, float band,
                         uint8_t* valid, int32_t* n_recheck, int block, const CloudWork& cw,
                         const CloudRange* clouds, int n_clouds, int32_t* flags, int32_t* unit_flags,
                         hipStream_t st);
-// Batches up to this size take the pass with a lane per (configuration,
-// evaluate unit); unit_flags: [B] int32, zero on entry and left zero.
-constexpr int64_t kValidUnitsMaxBatch = 65536;
-// noalloc.hip: the scratch of pmp_is_valid_batch_noalloc, a static device
-// array of kNoAllocScratchBytes per GPU.  noalloc_scratch_init looks up this
-// device's copy (call with `device` current); noalloc_scratch returns it
-// (null before the lookup).
+// Workspace bytes above which pmp_is_valid_batch_noalloc refuses a batch.
 constexpr size_t kNoAllocScratchBytes = (size_t)32 << 20;
-hipError_t noalloc_scratch_init(int device);
-void* noalloc_scratch(int device);
 // cloud.hip
-// unit_flags (optional): valid[] is formed from the unit pass's words by
-// this pass (and the words cleared), instead of by valid_units_finish_kernel.
-hipError_t launch_cloud_valid(const CloudTile* tiles, const float* tileB, const CloudSuper* supers,
-                              const CloudRange& cr, const float* cen, const float* cap2, const float* rr, int64_t B,
-                              int64_t Q, float band, uint8_t* valid, int32_t* flags, int32_t* unit_flags,
-                              hipStream_t st);
 hipError_t launch_cloud_min(const CloudTile* tiles, const float* tileB, const CloudSuper* supers,
                             const CloudRange& cr, const float* cen, const float* cap2, int64_t B, int64_t Q,
                             float* out_d2, hipStream_t st);

@@ -35,6 +35,25 @@ inline StageLds stage_lds(const KinArgs<float>& ka, int C) {
   return L;
 }
 
+// Configurations (64 / H) and waves (W) of a workgroup for a batch of B: the
+// fewest configurations while every CU then gets one workgroup at most, with
+// 16 waves each; once a CU has several workgroups, 8 waves, and 4 when the
+// robot has so few sphere blocks that most of 8 would wait for the walk.
+// Measured (us), 7R arm, 32 primitives: evaluate of 4,096 configurations 19.1
+// with H = 4, 24 with H = 1; of 8,192 22.0 with H = 2, 24.3 with H = 1; of
+// 32,768 35 with 8 waves, 60 with 16; of 65,536 50 with 4 waves, 63 with 8.
+// Validity of 1,000: 13.5 with H = 8, 14.1 with H = 4, 16.7 with H = 1; of
+// 32,768 24 with 8 waves, 32 with 16; of 131,072 55 with 4 waves, 65 with 8.
+struct StageShape {
+  int H, W;
+};
+inline StageShape stage_shape(int64_t B, int n_blocks) {
+  StageShape s;
+  s.H = B <= 8 * kCus ? 8 : (B <= 16 * kCus ? 4 : (B <= 32 * kCus ? 2 : 1));
+  s.W = B <= 64 * kCus ? 16 : (B > 128 * kCus && n_blocks <= 8 ? 4 : 8);
+  return s;
+}
+
 // Touches [p, p + bytes) through the scalar data cache, a line in n_parts: for
 // waves that would otherwise wait while another one walks, so that the tables
 // the whole workgroup is about to read are in the cache it shares.

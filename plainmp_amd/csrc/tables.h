@@ -245,8 +245,10 @@ struct SceneArgs {
   const CullRange* cull_range;  // [n_blocks]
   const CullEntry* ecull;       // the same for evaluate: boxes grown by the 0.1 m cutoff
   const CullRange* ecull_range;
-  const DevCullSlice* eslices;  // the evaluate candidates cut into slices, last block first
-  int32_t n_ecull, n_eslices;
+  // the candidates of either table cut into slices, last block first
+  const DevCullSlice* slices;
+  const DevCullSlice* eslices;
+  int32_t n_cull, n_slices, n_ecull, n_eslices;
   const int32_t* vorig;         // kind-sorted index -> scene order
 };
 

@@ -64,3 +64,31 @@ def test_trajectory_costs_in_the_evaluate_launch(lengths):
         # one rounding of the FP64 sum; the gradient's terms likewise
         assert abs(cost[i] - (acc ** 2).sum()) <= 1e-6 * (acc ** 2).sum()
         assert np.abs(grad[a:b] - g).max(initial=0.0) <= 1e-6 * max(1.0, np.abs(g).max(initial=0.0))
+
+
+@pytest.mark.parametrize("robot", sorted(ROBOTS))
+@pytest.mark.parametrize("B", [1, 65, 2049, 4097, 8193, 16385, 32769])
+def test_validity_batch_sizes(robot, B):
+    wl = _workload(robot, B, n_prims=6)
+    got = product_cst(wl).is_valid_batch(wl.Q)
+    idx = _sample(B, 2048)
+    assert np.array_equal(got[idx], oracle_cst(wl).is_valid_batch(wl.Q[idx], 8).astype(bool))
+
+
+@pytest.mark.parametrize("band", [0.0, 1e-5, 2e-3, 0.2])
+@pytest.mark.parametrize("B", [37, 3000])
+def test_validity_pending_pairs(band, B):
+    """Solid, cloud and self pairs on the pending list, from none to far more
+    than it holds (then whole configurations are re-decided): the answer is
+    that of the FP64 tests at every band."""
+    r = synth.fetch_like(0)
+    Q = synth.uniform_configs(r, B, 8)
+    wl = synth.Workload("pending", r, synth.mixed_primitives(5, 8), cloud=synth.shelf_cloud(3000, 8), Q=Q)
+    oc, pc = oracle_cst(wl), product_cst(wl)
+    pc.set_band(band)
+    got, n = pc.is_valid_batch_stats(Q)
+    ref = oc.is_valid_batch(Q, 8).astype(bool)
+    assert 0.02 < ref.mean() < 0.98 or B < 100
+    if band > 0:  # with no band the FP32 decisions stand, a few ulps of the distances off
+        assert np.array_equal(got, ref)
+    assert 0 <= n <= B and (band < 0.1 or n > 0)
