@@ -136,10 +136,10 @@ typedef struct pmp_schedule {
                                  the waves of a workgroup, smaller ones slices of a
                                  block's primitives; 0 = default (slices up to 16,384
                                  configurations)                                      */
-  int32_t pair_shares;      /* pair distances: the primitives are split into this many
-                               shares, each walked by its own waves (more stores in
-                               flight for a small batch); 0 = default (about four
-                               waves per SIMD), clamped to half the primitive count */
+  int32_t pair_shares;      /* pair distances: workgroups that share a chunk of 64
+                               configurations, each taking its share of the (sphere,
+                               primitive) pairs; 0 = default (a task or two a wave),
+                               clamped to the number of tasks                       */
 } pmp_schedule;
 
 typedef struct pmp_context pmp_context;

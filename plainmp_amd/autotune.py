@@ -7,8 +7,8 @@ Two knobs decide how the persistent kernels map onto the MI355X:
 * ``eval_whole_chunks``: from how many 64-configuration chunks on an evaluate
   or trajectory batch hands out whole sphere blocks instead of slices of a
   block's primitives;
-* ``pair_shares``: into how many shares the pair-distance launch splits the
-  primitives (grid z), each share walked by its own waves.
+* ``pair_shares``: how many workgroups of the pair-distance launch share 64
+  configurations, each taking its share of the (sphere, primitive) pairs.
 
 ``tune_edges``, ``tune_evaluate`` and ``tune_pairs`` time every candidate on
 the caller's own device buffers (HIP events around the edge kernel; stream

@@ -957,7 +957,7 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
     pk.add(path, &a.path, &d.path);
     std::vector<DevSphereRow> rows(S);
     for (int k = 0; k < S; ++k)
-      rows[meta[k].out] = {sp32[k].x, sp32[k].y, sp32[k].z, pose_of[meta[k].node], mask[meta[k].node], 0};
+      rows[meta[k].out] = {sp32[k].x, sp32[k].y, sp32[k].z, sp32[k].r, mask[meta[k].node], pose_of[meta[k].node], 0};
     pk.add(rows, &a.rows, &d.rows);
     pk.add(path_at, &a.path_at, &d.path_at);
     a.n_paths = d.n_paths = (int32_t)path_at.size() - 1;

@@ -179,7 +179,8 @@ __device__ __forceinline__ void cloud_block_min(const SceneArgs<float>& sc, int 
 
 // The nearest point of cloud oc to c, per lane (an exhaustive search over
 // the tiles, skipping those whose box is farther than the best so far), and
-// its squared distance in best.
+// its squared distance in best.  kNamed: with named roundings.
+template <bool kNamed = false>
 __device__ __forceinline__ V3<float> cloud_nearest(const SceneArgs<float>& sc, int oc, V3<float> c, float& best) {
   best = FLT_MAX;
   V3<float> bp = c;
@@ -190,7 +191,7 @@ __device__ __forceinline__ V3<float> cloud_nearest(const SceneArgs<float>& sc, i
       const CloudTile T = sc.tiles[t];
       if (box_dist2(T.lb, T.ub, c) > best) continue;
       const V3<float> cl{c.x - T.o[0], c.y - T.o[1], c.z - T.o[2]};
-      const float off = dot(cl, cl);
+      const float off = kNamed ? dot3(cl, cl) : dot(cl, cl);
       const float* Bt = sc.tileB + (int64_t)t * 4 * kCloudTile;
       for (int j = 0; j < kCloudTile; ++j) {
         const float* col = Bt + (j / 16) * 64 + (j % 16);

@@ -399,6 +399,96 @@ PMP_HD V3<T> sdf_grad(const DevPrim<T>& p, V3<T> c) {
   return {T(0), T(0), T(0)};
 }
 
+// Sums of products with named roundings.  Left to the compiler's contraction,
+// which product is rounded on its own depends on the kernel around it, and the
+// same point then differs by an ulp from kernel to kernel.
+__device__ __forceinline__ float sum3(float ax, float bx, float ay, float by, float az, float bz) {
+  return fmaf(az, bz, fmaf(ax, bx, ay * by));
+}
+__device__ __forceinline__ float sum2sq(float a, float b) { return fmaf(b, b, a * a); }
+__device__ __forceinline__ float dot3(V3<float> a, V3<float> b) { return sum3(a.x, b.x, a.y, b.y, a.z, b.z); }
+__device__ __forceinline__ V3<float> mv3(const M3<float>& R, V3<float> v) {
+  return {sum3(R.a00, v.x, R.a01, v.y, R.a02, v.z), sum3(R.a10, v.x, R.a11, v.y, R.a12, v.z),
+          sum3(R.a20, v.x, R.a21, v.y, R.a22, v.z)};
+}
+
+// sqrt(x) and 1 / sqrt(x) of x >= 0 in FP32 from the hardware's reciprocal
+// root: one Newton step for the reciprocal (about half an ulp, where a
+// correctly rounded root and division make up to one), and the root's residual
+// through it (Markstein), which rounds correctly but for rare last-place ties.
+// sqrt(0) = 0; the reciprocal of 0 is finite.
+__device__ __forceinline__ void root_and_reciprocal(float x, float& s, float& inv) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  float r = __builtin_amdgcn_rsqf(fmaxf(x, 1e-36f));
+  const float h = 0.5f * r;
+  r = fmaf(fmaf(-x * r, r, 1.0f), h, r);
+  inv = r;
+  s = x * r;
+  s = fmaf(fmaf(-s, s, x), 0.5f * r, s);
+#else
+  s = sqrtf(x);  // host pass: never executed, only type-checked
+  inv = 1.0f / s;
+#endif
+}
+
+// sdf_eval_kind<K> and (kGrad) sdf_grad of an FP32 primitive together
+// (clouds excluded): the local coordinates and roots are shared, the roots
+// cost a third of correctly rounded ones, and a cylinder's gradient is formed
+// from its local coordinates.
+template <int K, bool kGrad>
+__device__ __forceinline__ void sdf_value_grad(const DevPrim<float>& p, V3<float> c, float& dist, V3<float>& g) {
+  const V3<float> dc = sub(c, V3<float>{p.pos[0], p.pos[1], p.pos[2]});
+  if constexpr (K == kKindBoxAA || K == kKindBoxRot) {
+    const V3<float> d = K == kKindBoxRot ? mv3(load_m3(p.Rinv), dc) : dc;
+    const float sx = fabsf(d.x) - p.p0, sy = fabsf(d.y) - p.p1, sz = fabsf(d.z) - p.p2;
+    const float mx = fmaxf(sx, 0.0f), my = fmaxf(sy, 0.0f), mz = fmaxf(sz, 0.0f);
+    const float top = fmaxf(fmaxf(sx, sy), sz);
+    float root, inv;
+    root_and_reciprocal(mx * mx + my * my + mz * mz, root, inv);
+    dist = root + fminf(top, 0.0f);
+    if constexpr (kGrad) {
+      V3<float> l{mx * inv, my * inv, mz * inv};
+      if (!(top > 0.0f)) {  // inside: the nearest face
+        l = {sx >= sy && sx >= sz ? 1.0f : 0.0f, 0.0f, 0.0f};
+        if (l.x == 0.0f) l = {0.0f, sy >= sz ? 1.0f : 0.0f, sy >= sz ? 0.0f : 1.0f};
+      }
+      l = {copysignf(l.x, d.x), copysignf(l.y, d.y), copysignf(l.z, d.z)};
+      g = K == kKindBoxRot ? mv3(load_m3(p.R), l) : l;
+    }
+  } else if constexpr (K == kKindCylZ || K == kKindCylRot) {
+    float x = dc.x, y = dc.y, z = dc.z;
+    if constexpr (K == kKindCylRot) {
+      x = dc.x * p.R[0] + dc.y * p.R[3] + dc.z * p.R[6];
+      y = dc.x * p.R[1] + dc.y * p.R[4] + dc.z * p.R[7];
+      z = dc.x * p.R[2] + dc.y * p.R[5] + dc.z * p.R[8];
+    }
+    float rho, inv_rho, root, inv;
+    root_and_reciprocal(sum2sq(x, y), rho, inv_rho);
+    const float rs = rho - p.p0, zs = fabsf(z) - p.p1;
+    const float o0 = fmaxf(rs, 0.0f), o1 = fmaxf(zs, 0.0f);
+    const float top = fmaxf(rs, zs);
+    root_and_reciprocal(sum2sq(o0, o1), root, inv);
+    dist = root + fminf(top, 0.0f);
+    if constexpr (kGrad) {
+      float wr = o0 * inv, wz = o1 * inv;
+      if (!(top > 0.0f)) {
+        wr = rs > zs ? 1.0f : 0.0f;
+        wz = 1.0f - wr;
+      }
+      const float k = wr * inv_rho, gx = k * x, gy = k * y, gz = copysignf(wz, z);
+      g = K == kKindCylRot ? mv3(load_m3(p.R), V3<float>{gx, gy, gz}) : V3<float>{gx, gy, gz};
+    }
+  } else if constexpr (K == kKindSphere) {
+    float root, inv;
+    root_and_reciprocal(dot3(dc, dc), root, inv);
+    dist = root - p.p0;
+    if constexpr (kGrad) g = scale(inv, dc);
+  } else {  // ground
+    dist = c.z + p.p0;
+    if constexpr (kGrad) g = {0.0f, 0.0f, 1.0f};
+  }
+}
+
 // Reference is_outside (primitive_sdf.hpp:313-398, 464-498, 546-552, 246-248)
 // in its own branch structure; used in FP64 for the in-band re-decision.
 // K >= 0 fixes the primitive kind at compile time (kind-sorted loops).

@@ -1191,85 +1191,6 @@ __global__ void __launch_bounds__(64) eval_units_kernel(KinArgs<float> ka, Scene
   eval_finish_whole<MAXC>(ka, sc, qs, q, ldq, b, o, v);
 }
 
-// The pair and adjoint kernels give each (configuration, sphere item) its
-// own lane: the wave's item is uniform (grid y), FK runs only down to the
-// item's node, and the item's spheres meet every primitive.  Lanes b of a
-// wave are consecutive, so every store and gradient load is coalesced.
-// kCloud: the scene holds a point cloud (a separate kernel, so that the
-// cloud search does not weigh on the register allocation of the others).
-template <int MAXC, bool kCloud>
-struct PairVis {
-  static constexpr bool kSelf = false;
-  const KinArgs<float>& ka;
-  const SceneArgs<float>& sc;
-  Frames<MAXC> fr;
-  float* dist;
-  float* grad;
-  int64_t B, b;
-  bool active;
-  DevSphereItem it;
-  int p_lo, p_hi;  // primitives of this lane's share
-  bool done = false;
-  __device__ bool alive() const { return !done; }
-  template <class QS>
-  __device__ void begin(const Pose<float>& base, const QS& qs) { fr.set_base(ka, base, qs); }
-  __device__ void node(int n, const DevNode<float>& nd, const Pose<float>& P) {
-    if (n == it.node) done = true;  // its spheres follow in this same step
-    if (nd.q_col < 0) return;
-    fr.set(nd.q_col, qrot(P.q, V3<float>{nd.axis[0], nd.axis[1], nd.axis[2]}), P.t);
-  }
-  __device__ void sphere(int s, V3<float> c, float r) {
-    if (s < it.begin || s >= it.end) return;
-    const DevSphereMeta m = cload(ka.meta, s);
-    const uint64_t mask = cload(ka.nodes, m.node).col_mask;
-    const int D = ka.n_cols, NP = sc.n_prims;
-    V3<float> J[MAXC];
-#pragma unroll
-    for (int j = 0; j < MAXC; ++j) J[j] = fr.col(j, mask, ka.rev_mask, c);
-    for (int p = p_lo; p < p_hi; ++p) {
-      const DevPrim<float> P = prim_at(sc, p);
-      float d;
-      V3<float> g{0.f, 0.f, 0.f};
-      if (kCloud && P.type == PMP_PRIM_CLOUD) {
-        // CloudSDF::evaluate (primitive_sdf.hpp:585-590): sqrt of the nearest
-        // squared distance minus r_cloud; its gradient at the nearest point
-        float d2;
-        const V3<float> dv = sub(c, cloud_nearest(sc, (P.flags >> 4) & 15, c, d2));
-        d = sqrtf(d2) - P.p0 - r;
-        g = scale(1.0f / sqrtf(dot(dv, dv)), dv);
-      } else {
-        d = sdf_eval(P, c) - r;
-        if (grad) g = sdf_grad(P, c);
-      }
-      // the outputs are written once and not read back here: streaming
-      // (non-temporal) stores keep them from displacing the tables in L2
-      const int64_t row = (int64_t)m.out * NP + p;
-      if (active) __builtin_nontemporal_store(d, dist + row * B + b);
-      if (grad) {
-#pragma unroll
-        for (int j = 0; j < MAXC; ++j)
-          if (j < D && active) __builtin_nontemporal_store(dot(g, J[j]), grad + (row * D + j) * B + b);
-      }
-    }
-  }
-  __device__ void self(const DevSelfPair&, int, int, V3<float>, V3<float>, float) {}
-};
-
-template <int MAXC, bool kCloud>
-__global__ void __launch_bounds__(256) pair_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
-                                                   int64_t ldq, int64_t B, float* dist, float* grad) {
-  const int64_t b = gid();
-  const bool active = b < B;
-  BatchQ qs{q, ldq, active ? b : B - 1};
-  // grid z splits the primitives (p_per each), so that a batch of a few
-  // thousand configurations still puts several waves on every SIMD: the
-  // launch is bound by its stores, and more waves keep more of them in flight
-  const int p_per = (sc.n_prims + (int)gridDim.z - 1) / (int)gridDim.z;
-  const int p_lo = (int)blockIdx.z * p_per, p_hi = min(sc.n_prims, p_lo + p_per);
-  PairVis<MAXC, kCloud> v{ka, sc, {}, dist, grad, B, b, active, cload(ka.items, blockIdx.y), p_lo, p_hi};
-  run_fk(ka, qs, false, v);
-}
-
 // Jacobian of a point fixed to one link (rotation ignored): the joint frames
 // of every node up to the link, then a_j x (p - o_j) (or a_j) for the columns
 // that move it (KinematicModel::get_jacobian / get_attached_point_jacobian,
@@ -1543,18 +1464,6 @@ hipError_t launch_edges(const KinArgs<float>& k32, const KinArgs<double>& k64, c
       hipLaunchKernelGGL(KERNEL<64>, __VA_ARGS__);                                            \
   } while (0)
 
-#define PMP_DISPATCH_MAXC_CLOUD(ncols, KERNEL, CLOUD, ...)                                   \
-  do {                                                                                        \
-    if ((ncols) <= 8)                                                                         \
-      hipLaunchKernelGGL((KERNEL<8, CLOUD>), __VA_ARGS__);                                    \
-    else if ((ncols) <= 16)                                                                   \
-      hipLaunchKernelGGL((KERNEL<16, CLOUD>), __VA_ARGS__);                                   \
-    else if ((ncols) <= 32)                                                                   \
-      hipLaunchKernelGGL((KERNEL<32, CLOUD>), __VA_ARGS__);                                   \
-    else                                                                                      \
-      hipLaunchKernelGGL((KERNEL<64, CLOUD>), __VA_ARGS__);                                   \
-  } while (0)
-
 __global__ void fill_f32_kernel(float* p, float v, int64_t n) {
   const int64_t i = gid();
   if (i < n) p[i] = v;
@@ -1711,25 +1620,6 @@ hipError_t launch_eval_units(const KinArgs<float>& ka, const SceneArgs<float>& s
   if (B == 0) return hipGetLastError();
   PMP_DISPATCH_MAXC(ka.n_cols, eval_units_kernel, dim3((unsigned)((B + 63) / 64)), dim3(64), slot_bytes(ka, 64), st, ka,
                     sc, q, ldq, B, o);
-  return hipGetLastError();
-}
-// Waves the pair launch aims for: four per SIMD of a 256-CU MI355X.
-constexpr int64_t kPairWaves = 4096;
-hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq,
-                        int64_t B, float* dist, float* grad, int shares, hipStream_t st) {
-  if (ka.n_items == 0 || sc.n_prims == 0) return hipSuccess;
-  const int bk = slot_block(ka, 256);
-  const size_t lds = slot_bytes(ka, bk);
-  // primitive shares: the schedule's, or enough for about kPairWaves waves;
-  // at least two primitives a share
-  const int64_t waves = (B + 63) / 64 * ka.n_items;
-  const int64_t want = shares > 0 ? shares : (kPairWaves + waves - 1) / waves, most = (sc.n_prims + 1) / 2;
-  const int nz = (int)(want < most ? want : most) < 1 ? 1 : (int)(want < most ? want : most);
-  const dim3 grid(blocks_for(B, bk), (unsigned)ka.n_items, (unsigned)nz);
-  if (sc.n_cloud > 0)
-    PMP_DISPATCH_MAXC_CLOUD(ka.n_cols, pair_kernel, true, grid, dim3(bk), lds, st, ka, sc, q, ldq, B, dist, grad);
-  else
-    PMP_DISPATCH_MAXC_CLOUD(ka.n_cols, pair_kernel, false, grid, dim3(bk), lds, st, ka, sc, q, ldq, B, dist, grad);
   return hipGetLastError();
 }
 int vjp_shares(const KinArgs<float>& ka, int n_prims, int64_t B, int shares) {

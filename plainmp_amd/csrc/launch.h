@@ -113,7 +113,8 @@ hipError_t launch_eval_units(const KinArgs<float>& ka, const SceneArgs<float>& s
 // when the robot's tables do not fit a workgroup's LDS.
 bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq, int64_t B,
                         const EvalArgs& e, hipStream_t st, hipError_t* err);
-// shares: primitive shares (grid z), 0 = about four waves per SIMD
+// pairs.hip.  shares: workgroups that share a chunk of 64 configurations, 0 =
+// default.
 hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq,
                         int64_t B, float* dist, float* grad, int shares, hipStream_t st);
 // Primitive shares (grid z) of the adjoint launch: the schedule's (shares >

@@ -1,0 +1,274 @@
+// Signed distance of every (sphere, primitive) pair with its derivative, by
+// staged workgroups (stage.hpp).  FK runs once per workgroup; a wave takes up
+// to eight spheres of one link (distances) or one sphere (gradients) and a
+// slice of the primitives, so everything a primitive's evaluation reads is
+// wave-uniform.  Bound by the stores (a gradient batch writes S x P x (D + 1)
+// floats per configuration); the evaluation is resolved per primitive kind,
+// value and gradient together, to stay below that.
+#include <algorithm>
+#include <type_traits>
+
+#include "launch.h"
+#include "stage.hpp"
+
+namespace pmp {
+
+// Runs f with the primitive's kind as a compile-time constant.
+template <class F>
+__device__ __forceinline__ void with_kind(const DevPrim<float>& p, F&& f) {
+  switch (prim_kind(p)) {
+    case kKindBoxAA:
+      f(std::integral_constant<int, kKindBoxAA>{});
+      break;
+    case kKindBoxRot:
+      f(std::integral_constant<int, kKindBoxRot>{});
+      break;
+    case kKindCylZ:
+      f(std::integral_constant<int, kKindCylZ>{});
+      break;
+    case kKindCylRot:
+      f(std::integral_constant<int, kKindCylRot>{});
+      break;
+    case kKindSphere:
+      f(std::integral_constant<int, kKindSphere>{});
+      break;
+    case kKindGround:
+      f(std::integral_constant<int, kKindGround>{});
+      break;
+    default:
+      f(std::integral_constant<int, kKindCloud>{});
+  }
+}
+
+// Distance to a primitive of kind K and its gradient.
+template <int K, bool kGrad>
+__device__ __forceinline__ void pair_eval(const SceneArgs<float>& sc, const DevPrim<float>& P, V3<float> c, float& d,
+                                          V3<float>& g) {
+  if constexpr (K == kKindCloud) {
+    // CloudSDF::evaluate (primitive_sdf.hpp:585-590): sqrt of the nearest
+    // squared distance minus r_cloud; its gradient at the nearest point
+    float d2;
+    const V3<float> dv = sub(c, cloud_nearest<true>(sc, (P.flags >> 4) & 15, c, d2));
+    d = sqrtf(d2) - P.p0;
+    if constexpr (kGrad) g = scale(1.0f / sqrtf(dot3(dv, dv)), dv);
+  } else {
+    sdf_value_grad<K, kGrad>(P, c, d, g);
+  }
+}
+
+// The joint frames of every column, [D][6][C] from `at`, by all waves after
+// the walk.
+template <int H, class QS>
+__device__ __forceinline__ float* stage_frames(const Stage<H>& S, const KinArgs<float>& ka, const QS& qs, int at) {
+  constexpr int C = Stage<H>::C;
+  float* frames = S.lds + at;
+  for (int j = S.w * H + S.sub; j < ka.n_cols; j += S.W * H) {
+    V3<float> a{0.f, 0.f, 0.f}, o{0.f, 0.f, 0.f};
+    S.frame(ka, qs, j, a, o);
+    float* f = frames + 6 * j * C + S.cfg;
+    f[0] = a.x;
+    f[C] = a.y;
+    f[2 * C] = a.z;
+    f[3 * C] = o.x;
+    f[4 * C] = o.y;
+    f[5 * C] = o.z;
+  }
+  return frames;
+}
+template <int C>
+__device__ __forceinline__ void staged_frame(const float* frames, int j, int cfg, V3<float>& a, V3<float>& o) {
+  const float* f = frames + 6 * j * C + cfg;
+  a = {f[0], f[C], f[2 * C]};
+  o = {f[3 * C], f[4 * C], f[5 * C]};
+}
+
+// The (share, chunk of 64 configurations) of a workgroup: workgroups go to the
+// XCDs in turn, and each XCD gets a contiguous range, chunk fastest, so that
+// the chunks that write the same rows (and, in rows that do not start on a
+// cache line, the same lines) share an L2.
+__device__ __forceinline__ void share_and_chunk(int chunks, int& share, int& chunk) {
+  const int g = (int)blockIdx.x, n = (int)gridDim.x, x = g % kXcds;
+  const int at = x * (n / kXcds) + min(x, n % kXcds) + g / kXcds;
+  share = at / chunks;
+  chunk = at % chunks;
+}
+
+// Rows that start on a cache line are written once and in whole lines:
+// streaming stores keep them from displacing one another in L2.  Lines shared
+// by two waves are left to L2 to complete.
+template <bool kStream>
+__device__ __forceinline__ void put(float* p, float v) {
+  if constexpr (kStream)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
+
+// dist[(s * P + p) * B + b]: task t of the launch is item t / n_slices (up to
+// eight spheres of a link, so that a primitive is read once for all of them)
+// against slice t % n_slices of the primitives; workgroups share the tasks.
+template <bool kStream>
+__global__ void __launch_bounds__(512) pair_dist_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
+                                                        int64_t ldq, int64_t B, float* dist, int n_slices, int chunks,
+                                                        StageLds lay) {
+  HIP_DYNAMIC_SHARED(float, staged_lds)
+  const Stage<1> S(staged_lds, lay);
+  int share, chunk;
+  share_and_chunk(chunks, share, chunk);
+  const int shares = (int)gridDim.x / chunks;
+  const int64_t b = (int64_t)chunk * 64 + S.cfg;
+  const bool active = b < B;
+  BatchQ qs{q, ldq, active ? b : B - 1};
+  S.joints(ka, qs, false);
+  if (S.w == S.W - 1) warm_scalar(ka.path, cload(ka.path_at, ka.n_paths) * (int)sizeof(DevPathNode), 0, 1);
+  __syncthreads();
+  S.walk(ka, qs);
+  if (S.w >= ka.n_paths)
+    warm_scalar(sc.prims, sc.n_prims * (int)sizeof(DevPrim<float>), S.w - ka.n_paths, S.W - ka.n_paths);
+  __syncthreads();
+  const int NP = sc.n_prims, T = ka.n_items * n_slices, t_end = (int)((int64_t)T * (share + 1) / shares);
+  for (int t = (int)((int64_t)T * share / shares) + S.w; t < t_end; t += S.W) {
+    const DevSphereItem it = cload(ka.items, t / n_slices);
+    const int sl = t % n_slices, n = it.end - it.begin;
+    const Pose<float> P = S.pose(it.pose);
+    const M3<float> R = qmat(P.q);
+    V3<float> c[kItemSpheres];
+    float r[kItemSpheres];
+    float* row[kItemSpheres];
+#pragma unroll
+    for (int k = 0; k < kItemSpheres; ++k) {
+      const int s = min(it.begin + k, it.end - 1);
+      const DevSphere<float> a = cload(ka.spheres, s);
+      c[k] = add(mv3(R, V3<float>{a.x, a.y, a.z}), P.t);
+      r[k] = a.r;
+      row[k] = dist + (int64_t)cload(ka.meta, s).out * NP * B;
+    }
+    const int p_end = (int)((int64_t)NP * (sl + 1) / n_slices);
+    for (int p = (int)((int64_t)NP * sl / n_slices); p < p_end; ++p) {
+      const DevPrim<float> Q = prim_at(sc, p);
+      with_kind(Q, [&](auto kc) {
+#pragma unroll
+        for (int k = 0; k < kItemSpheres; ++k) {
+          if (k < n) {
+            float d;
+            V3<float> g;
+            pair_eval<decltype(kc)::value, false>(sc, Q, c[k], d, g);
+            if (active) put<kStream>(row[k] + (int64_t)p * B + b, d - r[k]);
+          }
+        }
+      });
+    }
+  }
+}
+
+// dist as above and grad[((s * P + p) * D + j) * B + b]: task t is sphere
+// t / n_slices (group order) against a slice of the primitives, MAXC columns
+// at a time.  Bound by its stores: 8,192 configurations of the 7R arm against
+// 32 primitives write 504 MB in 100 us (124 us with a lane per (configuration,
+// link) before); 256-byte pieces of rows alone take 94 us on this card, a
+// plain fill 73 us.  With rows off the cache lines (8,191 configurations) 142
+// us; 277 us with streaming stores and neighbouring chunks on different XCDs.
+template <int MAXC, bool kStream>
+__global__ void __launch_bounds__(256) pair_grad_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
+                                                        int64_t ldq, int64_t B, float* dist, float* grad, int n_slices,
+                                                        int chunks, StageLds lay) {
+  HIP_DYNAMIC_SHARED(float, staged_lds)
+  const Stage<1> S(staged_lds, lay);
+  int share, chunk;
+  share_and_chunk(chunks, share, chunk);
+  const int shares = (int)gridDim.x / chunks, cfg = S.cfg;
+  const int64_t b = (int64_t)chunk * 64 + cfg;
+  const bool active = b < B;
+  BatchQ qs{q, ldq, active ? b : B - 1};
+  S.joints(ka, qs, false);
+  if (S.w == S.W - 1) warm_scalar(ka.path, cload(ka.path_at, ka.n_paths) * (int)sizeof(DevPathNode), 0, 1);
+  __syncthreads();
+  S.walk(ka, qs);
+  __syncthreads();
+  const float* frames = stage_frames(S, ka, qs, lay.end);
+  __syncthreads();
+  const int D = ka.n_cols, NP = sc.n_prims, T = ka.n_spheres * n_slices;
+  const int t_end = (int)((int64_t)T * (share + 1) / shares);
+  for (int t = (int)((int64_t)T * share / shares) + S.w; t < t_end; t += S.W) {
+    const int s = t / n_slices, sl = t % n_slices;
+    const DevSphereRow row = cload(ka.rows, s);
+    const Pose<float> P = S.pose(row.pose);
+    const V3<float> c = add(mv3(qmat(P.q), V3<float>{row.x, row.y, row.z}), P.t);
+    for (int j0 = 0; j0 < D || j0 == 0; j0 += MAXC) {
+      V3<float> J[MAXC];
+#pragma unroll
+      for (int j = 0; j < MAXC; ++j) {
+        J[j] = {0.f, 0.f, 0.f};
+        if (j0 + j < D && ((row.col_mask >> (j0 + j)) & 1ull)) {
+          V3<float> a, o;
+          staged_frame<64>(frames, j0 + j, cfg, a, o);
+          J[j] = ((ka.rev_mask >> (j0 + j)) & 1ull) ? cross(a, sub(c, o)) : a;
+        }
+      }
+      const int p_end = (int)((int64_t)NP * (sl + 1) / n_slices);
+      for (int p = (int)((int64_t)NP * sl / n_slices); p < p_end; ++p) {
+        const DevPrim<float> Q = prim_at(sc, p);
+        float d = 0.f;
+        V3<float> g{0.f, 0.f, 0.f};
+        with_kind(Q, [&](auto kc) { pair_eval<decltype(kc)::value, true>(sc, Q, c, d, g); });
+        if (!active) continue;
+        const int64_t at = (int64_t)s * NP + p;
+        if (j0 == 0) put<kStream>(dist + at * B + b, d - row.r);
+        float* gp = grad + (at * D + j0) * B + b;
+#pragma unroll
+        for (int j = 0; j < MAXC; ++j) {
+          if (j0 + j < D) {
+            put<kStream>(gp, dot3(g, J[j]));
+            gp += B;
+          }
+        }
+      }
+    }
+  }
+}
+
+constexpr int64_t kPairWorkgroups = 16 * kCus;
+
+hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq,
+                        int64_t B, float* dist, float* grad, int shares, hipStream_t st) {
+  if (ka.n_spheres == 0 || sc.n_prims == 0 || B == 0) return hipSuccess;
+  const StageLds lay = stage_lds(ka, 64);
+  const size_t lds = sizeof(float) * (size_t)(lay.end + (grad ? 6 * ka.n_cols * 64 : 0));
+  if (lds > (size_t)ka.lds_limit) return hipErrorInvalidConfiguration;
+  const int64_t chunks = (B + 63) / 64;
+  // Distances: 4 primitives a task and a task a wave (8,191 configurations of
+  // the 7R arm, 32 primitives: 31 us; 8 primitives 33, 4 tasks a wave 35).
+  // Gradients: 8 primitives, two tasks a wave once the launch fills the GPU
+  // (8,192: 100 us, 4 primitives 106, four tasks 106), else one (1,000: 24 us,
+  // two 28).  More than kPairWorkgroups workgroups only repeat the walk.
+  const int W = grad ? 4 : 8, per = grad ? 8 : 4, tasks_per_wave = grad && chunks > 32 ? 2 : 1;
+  const int n_slices = (sc.n_prims + per - 1) / per;
+  const int64_t tasks = (int64_t)(grad ? ka.n_spheres : ka.n_items) * n_slices;
+  int64_t ny = std::min((tasks + tasks_per_wave * W - 1) / (tasks_per_wave * W),
+                        (kPairWorkgroups + chunks - 1) / chunks);
+  if (shares > 0) ny = std::min<int64_t>(shares, tasks);
+  const bool stream = B % 32 == 0;
+  const dim3 grid((unsigned)(chunks * ny)), block(64 * W);
+#define PMP_DIST(STREAM) \
+  hipLaunchKernelGGL(pair_dist_kernel<STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, n_slices, (int)chunks, lay)
+#define PMP_GRAD(MAXC, STREAM)                                                                                        \
+  hipLaunchKernelGGL((pair_grad_kernel<MAXC, STREAM>), grid, block, lds, st, ka, sc, q, ldq, B, dist, grad, n_slices, \
+                     (int)chunks, lay)
+  if (!grad && stream)
+    PMP_DIST(true);
+  else if (!grad)
+    PMP_DIST(false);
+  else if (ka.n_cols <= 8 && stream)
+    PMP_GRAD(8, true);
+  else if (ka.n_cols <= 8)
+    PMP_GRAD(8, false);
+  else if (stream)
+    PMP_GRAD(16, true);
+  else
+    PMP_GRAD(16, false);
+#undef PMP_DIST
+#undef PMP_GRAD
+  return hipGetLastError();
+}
+
+}  // namespace pmp

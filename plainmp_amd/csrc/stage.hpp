@@ -139,7 +139,7 @@ struct Stage {
           }
           default: {  // PMP_NODE_TRANSLATION
             const M3<float> R = qmat(P.q);
-            P.t = add(P.t, mv(R, lt));
+            P.t = add(P.t, mv3(R, lt));
             break;
           }
         }
@@ -198,12 +198,12 @@ struct Stage {
       r[k] = 0.0f;
       if constexpr (H == 1) {
         if (k < n) {
-          c[k] = add(mv(R, V3<float>{bk.s[k][0], bk.s[k][1], bk.s[k][2]}), P.t);
+          c[k] = add(mv3(R, V3<float>{bk.s[k][0], bk.s[k][1], bk.s[k][2]}), P.t);
           r[k] = bk.s[k][3];
         }
       } else if (k < n) {
         const Quad4 s = reinterpret_cast<const Quad4*>(ka.blocks[bi].s)[sub * NK + k];  // a sphere a lane
-        c[k] = add(mv(R, V3<float>{s.v[0], s.v[1], s.v[2]}), P.t);
+        c[k] = add(mv3(R, V3<float>{s.v[0], s.v[1], s.v[2]}), P.t);
         r[k] = s.v[3];
       }
     }

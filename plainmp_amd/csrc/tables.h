@@ -117,12 +117,11 @@ struct alignas(16) DevColumn {
   int32_t pose;
 };
 
-// What a winning sphere's Jacobian row needs, in one gather (group order).
+// A sphere with what its Jacobian columns need, in one read (group order).
 struct alignas(32) DevSphereRow {
-  float x, y, z;
-  int32_t pose;       // pose-table index of its node
+  float x, y, z, r;
   uint64_t col_mask;  // q columns that move it
-  uint64_t pad;
+  int32_t pose, pad;  // pose-table index of its node
 };
 
 // A slice of a sphere block's candidates: cull entries [lo, hi) of block

@@ -92,3 +92,51 @@ def test_validity_pending_pairs(band, B):
     if band > 0:  # with no band the FP32 decisions stand, a few ulps of the distances off
         assert np.array_equal(got, ref)
     assert 0 <= n <= B and (band < 0.1 or n > 0)
+
+
+def _pair_case(robot, B, n_prims):
+    wl = _workload(robot, B, n_prims=n_prims)
+    return wl, oracle_cst(wl), product_cst(wl)
+
+
+@pytest.mark.parametrize("robot,B,n_prims", [("panda", 1, 1), ("panda", 65, 3), ("panda", 2049, 9), ("panda", 2080, 8),
+                                             ("fetch", 97, 33), ("dual_arm", 64, 5), ("dual_arm", 1001, 2)])
+def test_pair_distances_gradients_and_adjoint(robot, B, n_prims):
+    """Whole and odd rows, primitive counts that leave a slice short; gradients
+    by central differences of the oracle's distances away from kinks, the
+    adjoint as the weighted sum of the gradients."""
+    import torch
+
+    wl, oc, pc = _pair_case(robot, B, n_prims)
+    dist, grad = pc.pair_clearance_batch(wl.Q, True)
+    dist_only = pc.pair_clearance_batch(wl.Q, False)
+    assert np.array_equal(dist, dist_only[0] if isinstance(dist_only, tuple) else dist_only)
+    idx = _sample(B, 24)
+    Q = wl.Q[idx]
+    assert np.abs(dist[idx] - oc.pair_clearance_batch(Q, True, 8)).max() <= 5e-6
+    D, h = wl.robot.dof, 1e-5
+    fd = np.empty((len(Q),) + dist.shape[1:] + (D,))
+    sd = np.empty_like(fd)
+    for j in range(D):
+        e = np.zeros(D)
+        e[j] = h
+        up, mid, dn = (oc.pair_clearance_batch(Q + k * e, True, 8) for k in (1, 0, -1))
+        fd[..., j], sd[..., j] = (up - dn) / (2 * h), np.abs(up - 2 * mid + dn)
+    # central differences are off by about h^2 / 6 times the third derivative
+    # (below 1e-6 here) unless a kink lies in between, which the second
+    # difference shows (a smooth one is about h^2 times the curvature)
+    smooth = sd.max(axis=-1) < 1e-8
+    assert smooth.mean() > 0.95
+    err = np.abs(grad[idx] - fd).max(axis=-1)
+    assert err[smooth].max() <= 1e-4
+    w = np.random.default_rng(1).uniform(size=dist.shape).astype(np.float32)
+    q = torch.from_numpy(np.ascontiguousarray(wl.Q.T)).to("cuda")
+    wt = torch.from_numpy(np.ascontiguousarray(w.transpose(1, 2, 0))).to("cuda")
+    out = torch.empty((D, B), device="cuda")
+    torch.cuda.synchronize()
+    pc._dev_pair_clearance_vjp(q.data_ptr(), B, B, wt.data_ptr(), out.data_ptr(), 0)
+    torch.cuda.synchronize()
+    ref = np.einsum("bsp,bspj->bj", w.astype(np.float64), grad.astype(np.float64))
+    scale = np.einsum("bsp,bspj->bj", w.astype(np.float64), np.abs(grad).astype(np.float64)).max()
+    # FP32 sums of S * P terms: a few roundings of the largest partial sum
+    assert np.abs(out.T.cpu().numpy() - ref).max() <= 64 * 6e-8 * max(scale, 1.0)
