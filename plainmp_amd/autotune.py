@@ -3,7 +3,8 @@
 Two knobs decide how the persistent kernels map onto the MI355X:
 
 * ``block`` / ``waves_per_cu`` of the edge kernel: workgroup size and how many
-  persistent waves each CU holds (the grid never exceeds one wave per edge);
+  persistent waves each CU holds (never more than one wave per edge, or one
+  workgroup per edge where a workgroup checks an edge);
 * ``eval_whole_chunks``: from how many 64-configuration chunks on an evaluate
   or trajectory batch hands out whole sphere blocks instead of slices of a
   block's primitives;

@@ -117,10 +117,13 @@ class TablePack {
 // cannot change what a replay reads.
 struct EdgeBufs {
   DevBuf width, inv_width, pend, counter;
+  int32_t slot = 0;                // EdgeArgs::slot of the last staged launch
+  int32_t count_at = kCntRecheck;  // the counter that holds the last launch's FP64 decisions
   std::vector<double> h_width;  // what width / inv_width hold, so a repeated call uploads nothing
   void release() {
     for (DevBuf* b : {&width, &inv_width, &pend, &counter}) b->release();
     h_width.clear();
+    count_at = kCntRecheck;
   }
 };
 
@@ -1599,6 +1602,14 @@ void prepare_edges(pmp_context* ctx, const double* s1, const double* s2, int64_t
   const bool fresh = eb.counter.bytes < sizeof(int32_t) * kNumEdgeCounters;  // new (or grown) buffer
   ea.counter = (int32_t*)eb.counter.get(sizeof(int32_t) * kNumEdgeCounters);
   if (fresh) PMP_HIP(launch_fill_i32(ea.counter, 0, kNumEdgeCounters, st(ctx)));
+  if (E > 0 && edges_staged(ctx->k32, ctx->s32, E)) {
+    ea.slot = eb.slot ^= 1;
+    eb.count_at = kCntStaged + ea.slot;
+    ea.valid = valid;
+    ea.n_checked = n_checked;
+    return;
+  }
+  if (E > 0) eb.count_at = kCntRecheck;
   const int64_t Ea = std::max<int64_t>(E, 1);
   int32_t* pend = (int32_t*)eb.pend.get(sizeof(int32_t) * Ea * (3 * kPendStates + 3));
   ea.pend = pend;
@@ -1615,12 +1626,19 @@ void prepare_edges(pmp_context* ctx, const double* s1, const double* s2, int64_t
 // hold at once, so a grid with a wave for every edge (whose waves take their
 // edge by index) is launched only when all of it is resident; otherwise the
 // resident grid pulls edges from the counter.
-int edge_grid(pmp_context* ctx, int block, int64_t E) {
+// The staged form takes the schedule's waves and workgroup size as they are.
+void edge_grid(pmp_context* ctx, int64_t E, int& grid, int& block) {
+  if (edges_staged(ctx->k32, ctx->s32, E)) {
+    grid = ctx->n_cu * ctx->sched.waves_per_cu;
+    block = ctx->sched.block;
+    return;
+  }
+  block = slot_block(ctx->k64, ctx->sched.block > 0 ? ctx->sched.block : 256);
   const int occ = edges_resident_waves_per_cu(ctx->s32.n_cloud > 0, block, slot_bytes(ctx->k64, block));
   int wpc = ctx->sched.waves_per_cu > 0 ? ctx->sched.waves_per_cu : 16;
   if (occ > 0) wpc = std::min(wpc, occ);
   const int64_t by_edges = (E * 64 + block - 1) / block;
-  return (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)ctx->n_cu * wpc * 64 / block, by_edges));
+  grid = (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)ctx->n_cu * wpc * 64 / block, by_edges));
 }
 
 }  // namespace
@@ -1633,13 +1651,14 @@ pmp_status pmp_check_edges_batch(pmp_context* ctx, const double* s1, const doubl
     EdgeArgs ea{};
     prepare_edges(ctx, s1, s2, lds, E, v, valid, n_checked, ctx->eb, ea);
     if (E == 0) return;
-    const int block = slot_block(ctx->k64, ctx->sched.block > 0 ? ctx->sched.block : 256);
+    int grid, block;
+    edge_grid(ctx, E, grid, block);
     if (!ctx->edge_ev0) {
       PMP_HIP(hipEventCreate(&ctx->edge_ev0));
       PMP_HIP(hipEventCreate(&ctx->edge_ev1));
     }
-    PMP_HIP(launch_edges(ctx->k32, ctx->k64, ctx->s32, ctx->s64, ea, ctx->band, edge_grid(ctx, block, E), block,
-                         st(ctx), ctx->edge_ev0, ctx->edge_ev1));
+    PMP_HIP(launch_edges(ctx->k32, ctx->k64, ctx->s32, ctx->s64, ea, ctx->band, grid, block, st(ctx),
+                         ctx->edge_ev0, ctx->edge_ev1));
   });
 }
 
@@ -1654,11 +1673,11 @@ pmp_status pmp_check_edges_graph(pmp_context* ctx, const double* s1, const doubl
       prepare_edges(ctx, s1, s2, lds, E, v, valid, n_checked, g->eb, ea);
       PMP_HIP(hipStreamSynchronize(st(ctx)));  // width tables are in place before capture
       hipStream_t cs = graph_stream(ctx);
-      const int block = slot_block(ctx->k64, ctx->sched.block > 0 ? ctx->sched.block : 256);
+      int grid, block;
+      edge_grid(ctx, E, grid, block);
       g->stream = cs;
       PMP_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-      hipError_t le = launch_edges(ctx->k32, ctx->k64, ctx->s32, ctx->s64, ea, ctx->band, edge_grid(ctx, block, E),
-                                   block, cs);
+      hipError_t le = launch_edges(ctx->k32, ctx->k64, ctx->s32, ctx->s64, ea, ctx->band, grid, block, cs);
       hipError_t ce = hipStreamEndCapture(cs, &g->graph);
       PMP_HIP(le);
       PMP_HIP(ce);
@@ -1704,8 +1723,8 @@ pmp_status pmp_edge_recheck_count(pmp_context* ctx, int32_t* n) {
     PMP_REQUIRE(ctx != nullptr && n != nullptr, "null argument");
     PMP_REQUIRE(ctx->eb.counter.ptr != nullptr, "no edge batch has run on this context");
     set_device(ctx);
-    PMP_HIP(hipMemcpyAsync(n, (const int32_t*)ctx->eb.counter.ptr + kCntRecheck, sizeof(int32_t), hipMemcpyDeviceToHost,
-                           st(ctx)));
+    PMP_HIP(hipMemcpyAsync(n, (const int32_t*)ctx->eb.counter.ptr + ctx->eb.count_at, sizeof(int32_t),
+                           hipMemcpyDeviceToHost, st(ctx)));
     PMP_HIP(hipStreamSynchronize(st(ctx)));
   });
 }

@@ -68,6 +68,20 @@ __device__ __forceinline__ bool fp32_range_col(uint64_t rev_mask, int col, doubl
   return fabs(v) <= (((rev_mask >> col) & 1ull) ? kFp32AngleRange : kFp32LinearRange);
 }
 
+// The kernel's one argument struct, read again from memory: a phase that takes
+// its arguments through this leaves no scalar registers held (or spilled) for
+// them in the phases around it.
+template <class A>
+__device__ __forceinline__ const A& args_again() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const A*)p;
+#else
+  return *(const A*)nullptr;  // host pass: never executed, only type-checked
+#endif
+}
+
 // Orders a wave's own LDS accesses: what its lanes wrote before is what they
 // read after.
 __device__ __forceinline__ void wave_lds_order() {

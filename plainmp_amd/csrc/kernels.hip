@@ -122,18 +122,16 @@ __global__ void __launch_bounds__(256) clearance_kernel(KinArgs<float> ka, Scene
 // FP32 pass: a collision decided outside the band ends the lane's work
 // ("definite"); a decision inside the band marks the configuration for the
 // FP64 re-decision ("uncertain").
-// kInlineCloud: the scene holds clouds, tested inside the walk.
-// kFirstHit: the lanes are states of one edge and only the first certain
-// collision in visiting order (`key`) matters, so a lane whose key is past
-// the wave's first certain collision so far stops taking part.
-template <bool kInlineCloud, bool kFirstHit = false>
-struct ValidVis32T {
+// The lanes are states of one edge and only the first certain collision in
+// visiting order (`key`) matters, so a lane whose key is past the wave's first
+// certain collision so far stops taking part.
+struct ValidVis32 {
   static constexpr bool kSelf = true;
   static constexpr bool kBlocks = true;
   const KinArgs<float>& ka;
   const SceneArgs<float>& sc;
   float band;
-  int key = 0;  // visiting index of the lane's state (kFirstHit)
+  int key = 0;  // visiting index of the lane's state
   bool idle = false;
   bool definite = false;
   bool uncertain = false;
@@ -221,11 +219,9 @@ struct ValidVis32T {
     const bool tfin = fabsf(P.t.x) <= FLT_MAX && fabsf(P.t.y) <= FLT_MAX && fabsf(P.t.z) <= FLT_MAX;
     const bool nan_test = n_solid > 0 && wave_any(alive() && !(n2 >= nd.n2_lo && n2 <= nd.n2_hi && tfin));
     for (int bi = lo; bi < hi; ++bi) {
-      if constexpr (kFirstHit) {
-        if (wave_any(definite && !idle)) {
-          const int first = wave_min(definite && !idle ? key : INT_MAX);
-          if (key > first) idle = true;
-        }
+      if (wave_any(definite && !idle)) {
+        const int first = wave_min(definite && !idle ? key : INT_MAX);
+        if (key > first) idle = true;
       }
       if (!wave_any(alive())) return;
       const DevSphereBlock bk = cload(ka.blocks, bi);
@@ -258,48 +254,6 @@ struct ValidVis32T {
       kind_loop<kKindCylRot>(c, bk, n, g, cr, bi);
       kind_loop<kKindSphere>(c, bk, n, g, cr, bi);
       kind_loop<kKindGround>(c, bk, n, g, cr, bi);
-      if constexpr (kInlineCloud) cloud_inline(c, bk, n, g, nd.n2_hi, growf);
-    }
-  }
-
-  // Every cloud against the spheres of a block, for the edge pass.  Super-
-  // tiles, then tiles, are skipped when no live lane's block bounding sphere
-  // (centre g, radius G, stretched by the rotation's norm bound) comes
-  // within rc + band of their box; the points of a kept tile are compared
-  // in tile-local coordinates, |c - p|^2 = |c'|^2 + (|p'|^2 - 2 c'.p'), from
-  // the same operands as the matrix-core pass.  The decision is that of the
-  // cloud pass (CloudSDF::is_outside, primitive_sdf.hpp:597-603, after the
-  // AABB pre-test): collide iff min |c - p|^2 <= (r + rc)^2, with the band
-  // around it, widened by the tile-local form's error bound, left to the
-  // FP64 walk.
-  __device__ __forceinline__ void cloud_inline(const V3<float> (&c)[kBlockSpheres], const DevSphereBlock& bk, int n,
-                                               V3<float> g, float n2_hi, float growf) {
-    const DevPrim<float>* vp = reinterpret_cast<const DevPrim<float>*>(sc.vprims);
-    for (int p = sc.vrange[kKindCloud]; p < sc.vrange[kKindCloud + 1]; ++p) {
-      if (!wave_any(alive())) return;
-      const DevPrim<float> Pc = cload(vp, p);
-      // every sphere of the block fails the reference's AABB pre-test when
-      // the bounding centre is outside the AABB grown by the block's reach
-      if (!wave_any(alive() && !outside_aabb(Pc, g, bk.G * growf + band + 1e-4f))) continue;
-      const float rc = Pc.p0;
-      const float reach = bk.G * n2_hi + rc + band + 1e-5f;
-      float hi[kBlockSpheres], lo[kBlockSpheres];
-      cloud_block_min<true, kBlockSpheres>(sc, (Pc.flags >> 4) & 15, c, n, g, reach * reach, alive(), hi, lo);
-#pragma unroll
-      for (int k = 0; k < kBlockSpheres; ++k) {
-        if (k < n) {
-          const float r = bk.s[k][3];
-          if (!alive() || outside_aabb(Pc, c[k], r)) continue;
-          // the exact minimum lies in [lo, hi]: certain outside the band around R^2
-          const float R = r + rc, R2 = R * R, w = band * (2.0f * R + band);
-          if (hi[k] - R2 < -w) {
-            definite = true;
-          } else if (!(lo[k] - R2 > w)) {
-            uncertain = true;
-            n_inb = 2;
-          }
-        }
-      }
     }
   }
 
@@ -365,28 +319,6 @@ struct ValidVis64 {
     }
   }
 
-  // CloudSDF::is_outside: sqrt(min |p - c|^2) - rc > r (primitive_sdf.hpp:597-603),
-  // the minimum taken over the tiles that can reach within r + rc.
-  __device__ void cloud(const DevPrim<double>& P, V3<double> c, double r) {
-    if (outside_aabb(P, c, r)) return;
-    const double R = r + P.p0, lim = R * R * (1.0 + 1e-12) + 1e-300;
-    double best = DBL_MAX;
-    for (int t = 0; t < P.cloud_count; ++t) {
-      const CloudTile64 T = cload(sc.tiles64, P.cloud_begin + t);
-      const double dx = fmax(fmax(T.lb[0] - c.x, c.x - T.ub[0]), 0.0);
-      const double dy = fmax(fmax(T.lb[1] - c.y, c.y - T.ub[1]), 0.0);
-      const double dz = fmax(fmax(T.lb[2] - c.z, c.z - T.ub[2]), 0.0);
-      if (dx * dx + dy * dy + dz * dz > lim) continue;
-      const double* pt = sc.pts64 + (int64_t)(P.cloud_begin + t) * kCloudTile * 4;
-      for (int j = 0; j < kCloudTile; ++j) {
-        const double ex = pt[4 * j] - c.x, ey = pt[4 * j + 1] - c.y, ez = pt[4 * j + 2] - c.z;
-        const double d2 = ex * ex + ey * ey + ez * ez;
-        if (d2 < best) best = d2;
-      }
-    }
-    if (!(sqrt(best) - P.p0 > r)) collided = true;
-  }
-
   __device__ void blocks(const DevNode<double>& nd, const Pose<double>& P) {
     if (nd.block_begin >= nd.block_end) return;
     const M3<double> R = qmat(P.q);
@@ -421,13 +353,6 @@ struct ValidVis64 {
       kind_loop<kKindCylRot>(c, r, n, g, cr, nocull);
       kind_loop<kKindSphere>(c, r, n, g, cr, nocull);
       kind_loop<kKindGround>(c, r, n, g, cr, nocull);
-      const DevPrim<double>* vp = reinterpret_cast<const DevPrim<double>*>(sc.vprims);
-      for (int p = sc.vrange[kKindCloud] + split; p < sc.vrange[kKindCloud + 1]; p += n_split) {
-        const DevPrim<double> Pc = cload(vp, p);
-#pragma unroll
-        for (int k = 0; k < kBlockSpheres; ++k)
-          if (k < n && !collided) cloud(Pc, c[k], r[k]);
-      }
     }
   }
   __device__ void self(const DevSelfPair&, int, int, V3<double> ci, V3<double> cj, double rs) {
@@ -582,11 +507,12 @@ __device__ __forceinline__ EdgeQv edge_waypoint(const EdgeArgs& ea, const EdgeEn
 // more than kMaxEdgeStates states).  A pending edge queues its in-band states
 // that can matter (all of them, or those before the first certain collision)
 // and that collision's index; the FP64 pass decides from them.
-// Register budget: four waves per SIMD without clouds (the by-index grid
-// of the autotuned schedule holds four per SIMD), three with them.
-template <bool kCloud>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCloud ? 3 : 4))) edges_kernel(KinArgs<float> k32, SceneArgs<float> s32, KinArgs<double> k64,
-                                                    SceneArgs<double> s64, EdgeArgs ea, float band) {
+// The form for scenes without clouds once its waves fill the GPU (edges.hip
+// has the other one).  Register budget: four waves per SIMD (the by-index
+// grid of the autotuned schedule holds four per SIMD).
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+edges_kernel(KinArgs<float> k32, SceneArgs<float> s32, KinArgs<double> k64, SceneArgs<double> s64, EdgeArgs ea,
+             float band) {
   const int lane = threadIdx.x & 63;
   const bool taylor = k32.base_type == PMP_BASE_FIXED;
   // A grid with a wave for every edge gives each wave its edge by index:
@@ -635,7 +561,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCloud
         for (int64_t base = 0; base < n_wp; base += 64) {
           const int64_t k = base + lane;
           const bool has = k < n_wp;
-          ValidVis32T<kCloud, true> v{k32, s32, band};
+          ValidVis32 v{k32, s32, band};
           v.idle = !has;
           v.key = (int)k;
           run_fk(k32, edge_waypoint(ea, ends, n_test, ratio, has ? k : 0), taylor, v);
@@ -1428,20 +1354,18 @@ hipError_t launch_clearance(const KinArgs<float>& ka, const SceneArgs<float>& sc
 hipError_t launch_edges(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,
                         const SceneArgs<double>& s64, const EdgeArgs& ea, float band, int grid, int block,
                         hipStream_t st, hipEvent_t ev_before, hipEvent_t ev_after) {
+  if (edges_staged(k32, s32, ea.E))
+    return launch_edges_staged(k32, k64, s32, s64, ea, band, grid, block, st, ev_before, ev_after);
   if (ev_before) {
     hipError_t e = hipEventRecord(ev_before, st);
     if (e != hipSuccess) return e;
   }
-  // scenes with a point cloud take the variant that tests clouds in the walk;
   // a wave's FP32 walk and its FP64 re-decisions after it share the wave's
   // kept-pose chunk, sized for FP64
   KinArgs<float> kw = k32;
   kw.slot_wave_bytes = k64.slot_wave_bytes;
   const size_t lds = slot_bytes(k64, block);
-  if (s32.n_cloud > 0)
-    hipLaunchKernelGGL(edges_kernel<true>, dim3(grid), dim3(block), lds, st, kw, s32, k64, s64, ea, band);
-  else
-    hipLaunchKernelGGL(edges_kernel<false>, dim3(grid), dim3(block), lds, st, kw, s32, k64, s64, ea, band);
+  hipLaunchKernelGGL(edges_kernel, dim3(grid), dim3(block), lds, st, kw, s32, k64, s64, ea, band);
   if (ev_after) {
     hipError_t e = hipEventRecord(ev_after, st);
     if (e != hipSuccess) return e;
@@ -1580,11 +1504,9 @@ hipError_t launch_link_jacobian(const KinArgs<float>& ka, const double* q, int64
   return hipGetLastError();
 }
 
-int edges_resident_waves_per_cu(bool cloud, int block, size_t lds) {
+int edges_resident_waves_per_cu(bool, int block, size_t lds) {
   int n = 0;
-  const hipError_t err =
-      cloud ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, edges_kernel<true>, block, lds)
-            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, edges_kernel<false>, block, lds);
+  const hipError_t err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, edges_kernel, block, lds);
   return err == hipSuccess ? n * (block / 64) : 0;
 }
 

@@ -16,7 +16,17 @@ constexpr int kPendStates = 16;  // in-band states an edge may queue for the FP6
 // sets the others back to zero, so a launch leaves them as it found them
 // (zero when the buffer is allocated) and no clearing node is needed in a
 // captured graph.
-enum EdgeCounter { kCntWork = 0, kCntRecheck = 1, kCntPending = 2, kCntDone = 3, kCntInline = 4, kNumEdgeCounters = 5 };
+// The staged form counts its FP64 decisions in one of two words in turn
+// (EdgeArgs::slot) and clears the other one for the next launch.
+enum EdgeCounter {
+  kCntWork = 0,
+  kCntRecheck = 1,
+  kCntPending = 2,
+  kCntDone = 3,
+  kCntInline = 4,
+  kCntStaged = 5,  // and 6
+  kNumEdgeCounters = 7
+};
 
 struct EdgeArgs {
   const double* s1;
@@ -28,6 +38,7 @@ struct EdgeArgs {
   const double* inv_width;  // device [n_cols], 1 / width as the reference precomputes
   const uint8_t* seq;       // device [128 * 128] farthest-first sequence table
   int32_t* counter;         // device [kNumEdgeCounters], see EdgeCounter
+  int32_t slot;             // staged form: the word of this launch's count, 0 or 1
   int32_t* pend;            // [E][kPendStates] in-band visiting indices of pending edges
   int32_t* pend_info;       // [E][2] number queued (-1: more than kPendStates), first certain collision
   int32_t* plist;           // [E] the pending edges, in the order edges_kernel finished them
@@ -92,6 +103,22 @@ hipError_t launch_cloud_min(const CloudTile* tiles, const float* tileB, const Cl
                             float* out_d2, hipStream_t st);
 hipError_t launch_cloud_clearance(float* clearance, const float* d2, const float* radius_out, float rc, int64_t B,
                                   int64_t S, hipStream_t st);
+// edges.hip: whether a batch of E motions takes the staged form (a workgroup
+// per motion) or edges_kernel (a wave per motion).  The staged form shortens a
+// motion's chain and shares its work; a wave per motion repeats less once the
+// motions alone fill the GPU.  Measured (us, staged and not), motions across
+// the joint range: 7R arm, 512 45 and 61, 1,024 60 and 61, 2,048 93 and 62;
+// with self pairs, 14 joints, 1,024 119 and 211, 8,192 543 and 540, 32,768
+// 1,909 and 1,410; Fetch-like 1,024 95 and 181, 8,192 379 and 603.  With a
+// cloud its queries are answered by whole waves: 4,096 607 and 1,036.
+inline bool edges_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, int64_t E) {
+  return sc.n_cloud > 0 || E <= (ka.n_pairs > 0 ? 32 * kCus : 4 * kCus);
+}
+// waves: resident at most (0 = a workgroup per motion), block: threads of a
+// workgroup (0 = default).
+hipError_t launch_edges_staged(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,
+                               const SceneArgs<double>& s64, const EdgeArgs& ea, float band, int waves, int block,
+                               hipStream_t st, hipEvent_t ev_before, hipEvent_t ev_after);
 // ev_before / ev_after (optional) are recorded around the FP32 edge kernel.
 hipError_t launch_edges(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,
                         const SceneArgs<double>& s64, const EdgeArgs& ea, float band, int grid, int block,

@@ -1,0 +1,436 @@
+// Validity tests of staged workgroups (stage.hpp), shared by the batch of
+// configurations and the motion check: what the waves of a workgroup do with
+// the staged poses.
+//
+// The waves take slices (a run of one sphere block's candidate primitives; the
+// block's first slice also takes the clouds) and self pairs from a queue and
+// test them in FP32.  A test decided outside the band marks the configuration
+// as colliding, and later items skip it; a test inside the band is put on the
+// workgroup's pending list as the one (sphere, primitive), (sphere, cloud) or
+// (sphere, sphere) pair it concerns.  At the end the first wave re-decides the
+// pending pairs of configurations not yet colliding in FP64, a lane per pair:
+// every other pair was decided outside the band, so the pairs decide the
+// configuration.  A configuration the FP32 walk cannot decide at all (joint
+// values outside its ranges, a rotation outside the cull table's bounds, NaN
+// centres, a full pending list) is walked in FP64 whole.
+//
+// Sphere-vs-cloud queries (spheres inside the cloud's AABB pre-test) are
+// compacted by the wave and answered one at a time by all its lanes: 64
+// super-tiles, then the tiles of four surviving super-tiles, then 64 points a
+// step, stopping at the first point certainly inside.
+#pragma once
+
+#include <float.h>
+
+#include <type_traits>
+
+#include "stage.hpp"
+
+namespace pmp {
+
+// Per configuration: a certain collision; FP64 decides all of it; FP64 decided
+// it or a pending pair of it.
+enum ValidFlag { kHit = 1, kWhole = 2, kPended = 4 };
+constexpr int kPendMax = 64;     // pending pairs a workgroup keeps
+constexpr int kQueryWords = 6;   // a compacted query: centre, reach, sphere, configuration
+
+// The workgroup's results under way, in LDS.  kFirst: its configurations are
+// the states of one motion in visiting order and only the first colliding one
+// matters, so those past the first certain collision count as decided.
+template <bool kFirst>
+struct ValidLds {
+  int* flags;  // [C]
+  int* first;  // kFirst: the first certain collision
+  int* pend;   // [3][kPendMax]: configuration, sphere, primitive (>= 0, kind-sorted) or -1 - second sphere
+  int* count;  // pending pairs
+  __device__ __forceinline__ void mark(int cfg, int f) const {
+    atomicOr(flags + cfg, f);
+    if (kFirst && (f & kHit)) atomicMin(first, cfg);
+  }
+  __device__ __forceinline__ int state(int cfg) const {
+    int f = *reinterpret_cast<volatile int*>(flags + cfg);
+    if (kFirst && cfg > *reinterpret_cast<volatile int*>(first)) f |= kHit;
+    return f;
+  }
+  __device__ __forceinline__ void defer(int cfg, int sphere, int other) const {
+    const int i = atomicAdd(count, 1);
+    if (i < kPendMax) {
+      pend[i] = cfg;
+      pend[kPendMax + i] = sphere;
+      pend[2 * kPendMax + i] = other;
+    } else {
+      mark(cfg, kWhole);
+    }
+  }
+};
+
+// One sphere against a cloud, by the whole wave: 1 when some point is
+// certainly inside R = r + rc, 2 when one may be (within the band, widened by
+// the tile-local form's error), else 0 (CloudSDF::is_outside,
+// primitive_sdf.hpp:597-603: collide iff min |c - p|^2 <= R^2).
+__device__ __forceinline__ int cloud_query(const SceneArgs<float>& sc, int oc, V3<float> c, float R, float band,
+                                           int lane) {
+  const float R2 = R * R, w = band * (2.0f * R + band), cap = (R + band) * (R + band);
+  int res = 0;
+  const int s_end = sc.super_at[oc + 1];
+  for (int s0 = sc.super_at[oc]; s0 < s_end; s0 += 64) {
+    bool near = false;
+    int first = 0, count = 0;
+    if (s0 + lane < s_end) {
+      const CloudSuper S = sc.supers[s0 + lane];
+      near = box_dist2(S.lb, S.ub, c) <= cap;
+      first = S.first;
+      count = S.count;
+    }
+    uint64_t smask = __ballot(near);
+    while (smask) {
+      // the tiles of up to four super-tiles, sixteen lanes each
+      int tile = -1;
+#pragma unroll
+      for (int u = 0; u < 64 / kCloudSuper; ++u) {
+        const int j = smask ? __builtin_ctzll(smask) : 0;
+        const int f = __builtin_amdgcn_readlane(first, j), n = smask ? __builtin_amdgcn_readlane(count, j) : 0;
+        smask &= smask - 1;
+        if (lane / kCloudSuper == u && lane % kCloudSuper < n) tile = f + lane % kCloudSuper;
+      }
+      bool tnear = false;
+      if (tile >= 0) {
+        const CloudTile T = sc.tiles[tile];
+        tnear = box_dist2(T.lb, T.ub, c) <= cap;
+      }
+      for (uint64_t tmask = __ballot(tnear); tmask; tmask &= tmask - 1) {
+        const int t = __builtin_amdgcn_readlane(tile, __builtin_ctzll(tmask));
+        const CloudTile T = cload(sc.tiles, t);
+        const float* col = sc.tileB + (int64_t)t * 4 * kCloudTile + (lane >> 4) * 64 + (lane & 15);
+        const V3<float> cl{c.x - T.o[0], c.y - T.o[1], c.z - T.o[2]};
+        const float off = dot(cl, cl);
+        const float d2 = fmaf(col[0], cl.x, fmaf(col[16], cl.y, fmaf(col[32], cl.z, col[48]))) + off;
+        const float err = kCloudGemmErr * (off + tile_rho2(T));
+        if (__any(d2 + err - R2 < -w)) return 1;
+        if (__any(!(d2 - err - R2 > w))) res = 2;
+      }
+    }
+  }
+  return res;
+}
+
+// One slice of block candidates for the configurations still `live`.
+template <int H, bool kFirst>
+__device__ __forceinline__ void valid_slice(const Stage<H>& S, const KinArgs<float>& ka, const SceneArgs<float>& sc,
+                                            const DevCullSlice& it, float band, const ValidLds<kFirst>& out,
+                                            float* queries) {
+  constexpr int NK = Stage<H>::NK;
+  bool live = (out.state(S.cfg) & (kHit | kWhole)) == 0;
+  if (!wave_any(live)) return;
+  const DevSphereBlock bk = cload(ka.blocks, it.block);
+  const Pose<float> P = S.pose(bk.pose);
+  const M3<float> R = qmat(P.q);
+  // The cull table assumes |q|^2 of this rotation within [n2_lo, n2_hi] (so
+  // that |R v| <= grow |v|), and with a finite translation no centre of such
+  // a rotation is NaN; any other configuration is left to the FP64 walk.
+  const float n2 = P.q.x * P.q.x + P.q.y * P.q.y + P.q.z * P.q.z + P.q.w * P.q.w;
+  const bool sound = n2 >= bk.n2_lo && n2 <= bk.n2_hi && fabsf(P.t.x) <= FLT_MAX && fabsf(P.t.y) <= FLT_MAX &&
+                     fabsf(P.t.z) <= FLT_MAX;
+  if (live && !sound) out.mark(S.cfg, kWhole);
+  live = live && sound;
+  const float growf = 1.0f + 2.0f * fmaxf(0.0f, fmaxf(bk.n2_hi - 1.0f, 1.0f - bk.n2_lo)) + 1e-6f;
+  const float reach = bk.G * growf + band + 1e-4f;
+  V3<float> c[NK];
+  float r[NK];
+  int n;
+  S.spheres(ka, it.block, bk, P, R, c, r, n);
+  auto sphere_of = [&](int k) {
+    return H == 1 ? cload(ka.blocks[it.block].sph, k) : ka.blocks[it.block].sph[S.sub * NK + k];
+  };
+  const V3<float> g = add(mv(R, V3<float>{bk.g[0], bk.g[1], bk.g[2]}), P.t);
+  const CullRange cr = cload(sc.cull_range, it.block);
+  const DevPrim<float>* vp = reinterpret_cast<const DevPrim<float>*>(sc.vprims);
+  auto kind = [&](auto kc) {
+    constexpr int K = decltype(kc)::value;
+    const int hi = min(it.hi, cr.at[K + 1]);
+    for (int i = max(it.lo, cr.at[K]); i < hi; ++i) {
+      const CullEntry ce = cload(sc.cull, i);
+      // every member sphere is outside the primitive's AABB inflated by its
+      // radius plus the band when the bounding centre is outside the grown box
+      const bool near = live && !(g.x < ce.lb[0] || g.x > ce.ub[0] || g.y < ce.lb[1] || g.y > ce.ub[1] ||
+                                  g.z < ce.lb[2] || g.z > ce.ub[2]);
+      if (!wave_any(near)) continue;
+      const DevPrim<float> Q = cload(vp, ce.prim);
+      if constexpr (K != kKindGround) {  // the ground's test is not a pure distance
+        bool nb = false;
+        if (!wave_any(near && collide_kind<K>(Q, g, reach, 0.0f, nb))) continue;
+      }
+      bool hit = false;
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        if (k < n) {
+          bool inb = false;
+          const bool col = collide_kind<K>(Q, c[k], r[k], band, inb);
+          hit |= live && col && !inb;
+          if (live && inb) out.defer(S.cfg, sphere_of(k), ce.prim);
+        }
+      }
+      if (hit) {
+        out.mark(S.cfg, kHit);
+        live = false;
+      }
+      if (kFirst && wave_any(hit)) live = live && (out.state(S.cfg) & kHit) == 0;
+      if (!wave_any(live)) return;
+    }
+  };
+  kind(std::integral_constant<int, kKindBoxAA>{});
+  kind(std::integral_constant<int, kKindBoxRot>{});
+  kind(std::integral_constant<int, kKindCylZ>{});
+  kind(std::integral_constant<int, kKindCylRot>{});
+  kind(std::integral_constant<int, kKindSphere>{});
+  kind(std::integral_constant<int, kKindGround>{});
+  if (!it.first) return;
+  for (int p = sc.vrange[kKindCloud]; p < sc.vrange[kKindCloud + 1]; ++p) {
+    const DevPrim<float> Pc = cload(vp, p);
+    live = live && (out.state(S.cfg) & kHit) == 0;
+    if (!wave_any(live && !outside_aabb(Pc, g, reach))) continue;
+    int cnt = 0;  // queries collected, wave-uniform
+    auto flush = [&]() {
+      wave_lds_order();
+      for (int e = 0; e < cnt; ++e) {
+        const float* t = queries + e;
+        const int cfg = __builtin_amdgcn_readfirstlane(__float_as_int(t[320]));
+        if (__builtin_amdgcn_readfirstlane(out.state(cfg)) & kHit) continue;
+        auto rd = [&](int at) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(t[at]))); };
+        const int res = cloud_query(sc, (Pc.flags >> 4) & 15, V3<float>{rd(0), rd(64), rd(128)}, rd(192), band, S.lane);
+        if (S.lane == 0) {
+          if (res == 1) out.mark(cfg, kHit);
+          if (res == 2) out.defer(cfg, __float_as_int(t[256]), p);
+        }
+      }
+      wave_lds_order();
+      cnt = 0;
+    };
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      const bool ask = live && k < n && !outside_aabb(Pc, c[k], r[k]);
+      const uint64_t m = __ballot(ask);
+      if (m == 0) continue;
+      const int more = __popcll(m);
+      if (cnt + more > 64) flush();
+      if (ask) {
+        float* t = queries + cnt + lane_rank(m);
+        t[0] = c[k].x;
+        t[64] = c[k].y;
+        t[128] = c[k].z;
+        t[192] = r[k] + Pc.p0;
+        t[256] = __int_as_float(sphere_of(k));
+        t[320] = __int_as_float(S.cfg);
+      }
+      cnt += more;
+    }
+    if (cnt > 0) flush();
+  }
+}
+
+// One self pair (check_self_collision, primitive_sphere_collision.cpp:222-254).
+template <int H, bool kFirst>
+__device__ __forceinline__ void valid_pair(const Stage<H>& S, const KinArgs<float>& ka, int k, float band,
+                                           const ValidLds<kFirst>& out) {
+  bool live = (out.state(S.cfg) & (kHit | kWhole)) == 0;
+  if (!wave_any(live)) return;
+  const DevSelfPair pr = cload(ka.pairs, k);
+  const Pose<float> P1 = S.pose(pr.pose1), P2 = S.pose(pr.pose2);
+  const M3<float> R1 = qmat(P1.q), R2 = qmat(P2.q);
+  const V3<float> g1 = add(mv(R1, V3<float>{pr.bound1[0], pr.bound1[1], pr.bound1[2]}), P1.t);
+  const V3<float> g2 = add(mv(R2, V3<float>{pr.bound2[0], pr.bound2[1], pr.bound2[2]}), P2.t);
+  const float n1 = P1.q.x * P1.q.x + P1.q.y * P1.q.y + P1.q.z * P1.q.z + P1.q.w * P1.q.w;
+  const float n2 = P2.q.x * P2.q.x + P2.q.y * P2.q.y + P2.q.z * P2.q.z + P2.q.w * P2.q.w;
+  const float grow = 1.0f + 2.0f * fmaxf(fabsf(n1 - 1.0f), fabsf(n2 - 1.0f));
+  const V3<float> dg = sub(g1, g2);
+  const float far = (pr.bound1[3] + pr.bound2[3]) * grow + band + 1e-4f;
+  if (!wave_any(live && !(dot(dg, dg) > far * far * 1.0001f))) return;
+  bool hit = false;
+  for (int i0 = pr.begin1; i0 < pr.end1; i0 += H) {
+    const int i = H == 1 ? i0 : i0 + S.sub;
+    DevSphere<float> a{};
+    if constexpr (H == 1)
+      a = cload(ka.spheres, i);
+    else if (i < pr.end1)
+      a = ka.spheres[i];
+    const V3<float> ci = add(mv(R1, V3<float>{a.x, a.y, a.z}), P1.t);
+    for (int j = pr.begin2; j < pr.end2; ++j) {
+      const DevSphere<float> bb = cload(ka.spheres, j);
+      const V3<float> d = sub(ci, add(mv(R2, V3<float>{bb.x, bb.y, bb.z}), P2.t));
+      const float rs = a.r + bb.r, m = dot(d, d) - rs * rs;
+      const bool inb = !(fabsf(m) > band * (2.0f * rs + band));  // NaN too
+      if (i < pr.end1 && live) {
+        if (inb) out.defer(S.cfg, i, -1 - j);
+        hit |= !inb && m < 0.0f;
+      }
+    }
+  }
+  if (hit) out.mark(S.cfg, kHit);
+}
+
+// A point cloud against one sphere in FP64, by the whole wave (uniform
+// arguments): CloudSDF::is_outside after the AABB pre-test, the minimum taken
+// over the tiles that can reach within r + rc.
+__device__ __forceinline__ bool cloud_hit64(const SceneArgs<double>& sc, const DevPrim<double>& P, V3<double> c, double r,
+                                            int lane) {
+  const double R = r + P.p0, lim = R * R * (1.0 + 1e-12) + 1e-300;
+  auto far = [&](auto& lb, auto& ub) {
+    const double dx = fmax(fmax((double)lb[0] - c.x, c.x - (double)ub[0]), 0.0);
+    const double dy = fmax(fmax((double)lb[1] - c.y, c.y - (double)ub[1]), 0.0);
+    const double dz = fmax(fmax((double)lb[2] - c.z, c.z - (double)ub[2]), 0.0);
+    return dx * dx + dy * dy + dz * dz > lim;
+  };
+  double best = DBL_MAX;
+  const int oc = (P.flags >> 4) & 15;
+  for (int s0 = sc.super_at[oc]; s0 < sc.super_at[oc + 1]; s0 += 64) {
+    bool near = false;
+    if (s0 + lane < sc.super_at[oc + 1]) {
+      const CloudSuper S = sc.supers[s0 + lane];
+      near = !far(S.lb, S.ub);
+    }
+    for (uint64_t smask = __ballot(near); smask; smask &= smask - 1) {
+      const CloudSuper S = cload(sc.supers, s0 + __builtin_ctzll(smask));
+      bool tnear = false;
+      if (lane < S.count) {
+        const CloudTile64 T = sc.tiles64[S.first + lane];
+        tnear = !far(T.lb, T.ub);
+      }
+      for (uint64_t tmask = __ballot(tnear); tmask; tmask &= tmask - 1) {
+        const double* pt = sc.pts64 + ((int64_t)(S.first + __builtin_ctzll(tmask)) * kCloudTile + lane) * 4;
+        const double ex = pt[0] - c.x, ey = pt[1] - c.y, ez = pt[2] - c.z;
+        best = fmin(best, ex * ex + ey * ey + ez * ez);
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) best = fmin(best, __shfl_xor(best, s, 64));
+  return !(sqrt(best) - P.p0 > r);
+}
+
+__device__ __forceinline__ double readlane64(double v, int i) {
+  const long long u = __builtin_bit_cast(long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, i);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), i);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// Cloud `P` (wave-uniform) against the spheres of the lanes that `ask`, one
+// lane at a time; whether this lane's collides.
+__device__ __forceinline__ bool cloud_hits64(const SceneArgs<double>& sc, const DevPrim<double>& P, V3<double> c, double r,
+                                             bool ask, int lane) {
+  bool hit = false;
+  for (uint64_t m = __ballot(ask && !outside_aabb(P, c, r)); m; m &= m - 1) {
+    const int i = __builtin_ctzll(m);
+    const bool h = cloud_hit64(sc, P, V3<double>{readlane64(c.x, i), readlane64(c.y, i), readlane64(c.z, i)},
+                               readlane64(r, i), lane);
+    if (lane == i) hit = h;
+  }
+  return hit;
+}
+
+// FP64 walk that keeps the poses of two nodes per lane.
+struct TwoPoses64 {
+  static constexpr bool kSelf = false;
+  static constexpr bool kBlocks = true;
+  int node1, node2;
+  bool idle;
+  Pose<double> P1{}, P2{};
+  int last = -1;
+  __device__ bool alive() const { return !idle && last < max(node1, node2); }
+  template <class QS>
+  __device__ void begin(const Pose<double>&, const QS&) {}
+  __device__ void node(int n, const DevNode<double>&, const Pose<double>& P) {
+    if (n == node1) P1 = P;
+    if (n == node2) P2 = P;
+    last = n;
+  }
+  __device__ void sphere(int, V3<double>, double) {}
+  __device__ void blocks(const DevNode<double>&, const Pose<double>&) {}
+  __device__ void self(const DevSelfPair&, int, int, V3<double>, V3<double>, double) {}
+};
+
+// FP64 walk of whole configurations with the reference's own tests: per
+// primitive-checked sphere the AABB pre-test and is_outside, per self pair
+// the strict squared-distance test.  The group-sphere broad phase of the
+// reference only culls, so it is not needed for the result.
+struct WholeVis64 {
+  static constexpr bool kSelf = true;
+  const KinArgs<double>& ka;
+  const SceneArgs<double>& sc;
+  int lane;
+  bool collided;
+  __device__ bool alive() const { return !collided; }
+  template <class QS>
+  __device__ void begin(const Pose<double>&, const QS&) {}
+  __device__ void node(int, const DevNode<double>&, const Pose<double>&) {}
+  __device__ void sphere(int s, V3<double> c, double r) {
+    if (cload(ka.meta, s).ext < 0) return;
+    const DevPrim<double>* vp = reinterpret_cast<const DevPrim<double>*>(sc.vprims);
+    // a NaN centre collides with every primitive but a cloud, whose nearest
+    // point then decides (nothing is nearer than infinity: it does not)
+    if (sc.vrange[kKindCloud] > 0 && is_nan3(c)) collided = true;
+    for (int p = 0; p < sc.vrange[kKindCloud]; ++p) {
+      const DevPrim<double> P = cload(vp, p);
+      if (!collided && !outside_aabb(P, c, r) && !is_outside_ref<double>(P, c, r)) collided = true;
+    }
+    for (int p = sc.vrange[kKindCloud]; p < sc.vrange[kKindCloud + 1]; ++p)
+      if (cloud_hits64(sc, cload(vp, p), c, r, !collided, lane)) collided = true;
+  }
+  __device__ void self(const DevSelfPair&, int, int, V3<double> ci, V3<double> cj, double rs) {
+    const V3<double> d = sub(ci, cj);
+    if (dot(d, d) < rs * rs) collided = true;
+  }
+};
+
+// FP64 decision of what the FP32 items left open, by the first wave: the
+// pending pairs of configurations not yet colliding, a lane each, then whole
+// configurations (H lanes hold one; the first of them walks).  point(cfg) is
+// the joint-value source of a configuration.  The kept poses of the walks take
+// the workgroup's LDS from its start: the results lie past it.  Whether this
+// lane decided anything.
+template <bool kFirst, class F>
+__device__ __forceinline__ bool decide64(int lane, int cfg, int part, const KinArgs<float>& ka,
+                                         const KinArgs<double>& k64, const SceneArgs<double>& s64, bool taylor,
+                                         bool active, const ValidLds<kFirst>& out, F&& point) {
+  const int n_pend = min(*out.count, kPendMax);
+  bool any = false;
+  if (n_pend > 0) {
+    const int pc = lane < n_pend ? out.pend[lane] : 0, s1 = lane < n_pend ? out.pend[kPendMax + lane] : 0,
+              other = lane < n_pend ? out.pend[2 * kPendMax + lane] : 0;
+    const bool has = lane < n_pend && (out.state(pc) & (kHit | kWhole)) == 0;
+    const int s2 = other < 0 ? -1 - other : s1;
+    TwoPoses64 v{has ? ka.meta[s1].node : 0, has ? ka.meta[s2].node : 0, !has};
+    run_fk(k64, point(has ? pc : cfg), taylor, v);
+    const DevSphere<double> a = k64.spheres[s1];
+    const V3<double> c1 = add(mv(qmat(v.P1.q), V3<double>{a.x, a.y, a.z}), v.P1.t);
+    bool hit = false;
+    bool cloud = false;
+    if (has && other < 0) {
+      const DevSphere<double> bb = k64.spheres[s2];
+      const V3<double> d = sub(c1, add(mv(qmat(v.P2.q), V3<double>{bb.x, bb.y, bb.z}), v.P2.t));
+      const double rs = a.r + bb.r;
+      hit = dot(d, d) < rs * rs;
+    } else if (has) {
+      cloud = other >= s64.vrange[kKindCloud];
+      const DevPrim<double>& P = reinterpret_cast<const DevPrim<double>*>(s64.vprims)[other];
+      hit = !cloud && !outside_aabb(P, c1, a.r) && !is_outside_ref<double>(P, c1, a.r);
+    }
+    for (int p = s64.vrange[kKindCloud]; p < s64.vrange[kKindCloud + 1]; ++p)
+      hit |= cloud_hits64(s64, cload(reinterpret_cast<const DevPrim<double>*>(s64.vprims), p), c1, a.r,
+                          cloud && other == p, lane);
+    if (has) out.mark(pc, kPended | (hit ? kHit : 0));
+    any = has;
+    wave_lds_order();
+  }
+  const int f = out.state(cfg);
+  const bool whole = active && (f & kWhole) && !(f & kHit) && part == 0;
+  if (wave_any(whole)) {
+    WholeVis64 v{k64, s64, lane, !whole};
+    run_fk(k64, point(cfg), taylor, v);
+    if (whole) out.mark(cfg, kPended | (v.collided ? kHit : 0));
+    wave_lds_order();
+  }
+  return any || whole;
+}
+
+}  // namespace pmp

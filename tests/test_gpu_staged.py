@@ -140,3 +140,44 @@ def test_pair_distances_gradients_and_adjoint(robot, B, n_prims):
     scale = np.einsum("bsp,bspj->bj", w.astype(np.float64), np.abs(grad).astype(np.float64)).max()
     # FP32 sums of S * P terms: a few roundings of the largest partial sum
     assert np.abs(out.T.cpu().numpy() - ref).max() <= 64 * 6e-8 * max(scale, 1.0)
+
+
+def _motions(robot, E, spans, seed=9):
+    """Motions whose lengths run through `spans` (of the joint range) in turn,
+    some of no length and some with a joint eight turns out of range."""
+    r = ROBOTS[robot](0)
+    rng = np.random.default_rng(seed)
+    a, b = (rng.uniform(r.lower, r.upper, size=(E, r.dof)) for _ in range(2))
+    b = a + np.resize(spans, E)[:, None] * (b - a)
+    b[5::23] = a[5::23]
+    a[7::31, -1] += 16 * np.pi
+    b[7::31, -1] += 16 * np.pi
+    return r, a, b
+
+
+@pytest.mark.parametrize("robot,E", [("panda", 1), ("panda", 1024), ("panda", 1025), ("fetch", 257), ("dual_arm", 300)])
+@pytest.mark.parametrize("schedule", [(0, 0), (64, 1), (256, 2)])
+@pytest.mark.parametrize("band", [None, 0.02])
+def test_motions_by_workgroups(robot, E, schedule, band):
+    """Motions of 1 to over 128 states (1, 2, 4 and 8 lanes a state, several
+    chunks), a workgroup each or a few workgroups for all, on both sides of the
+    form's bound; the wide band sends states to the FP64 decisions and more of
+    them than a pending list holds."""
+    from plainmp_amd.ompl import BoxMotionValidator
+
+    r, a, b = _motions(robot, E, [1.0, 0.02, 0.1, 0.2, 0.4, 3.0])
+    wl = synth.Workload("motions", r, synth.mixed_primitives(12, 2))
+    oc, pc = oracle_cst(wl), product_cst(wl)
+    pc._dev_set_schedule(*schedule, 0, 0)
+    if band is not None:
+        pc.set_band(band)
+    w = [0.05] * r.dof
+    ref, n_ref = oc.check_motions(a, b, True, w, 0.0, 8)
+    mv = BoxMotionValidator(pc, w)
+    for _ in range(2):  # the second call's count starts from zero again
+        got, n_got = mv.check_motions(a, b)
+        assert np.array_equal(got, ref.astype(bool))
+        assert np.array_equal(n_got, n_ref)
+        assert 0 <= mv.last_recheck_count() <= E
+    if band is not None and E > 1:
+        assert mv.last_recheck_count() > 0
