@@ -156,11 +156,10 @@ hipError_t launch_nearest(const double* pts, int64_t N, const double* qry, int64
                           hipStream_t st);
 
 // Device build of one cloud's tile tables (cloud_build.hip).
-constexpr int kSortChunk = 512;  // keys sorted per workgroup in LDS
 struct CloudBuildSizes {
   int64_t n_tiles, n_supers;
-  int64_t n_keys;         // sort length: a power of two >= max(n, kSortChunk)
-  int64_t scratch_bytes;  // keys and bounds
+  int64_t n_keys;         // keys of one sort buffer
+  int64_t scratch_bytes;  // keys, bounds and counts
 };
 CloudBuildSizes cloud_build_sizes(int64_t n);
 // pts: device [n][3] FP64.  Writes n_tiles records to t32 / t64, n_tiles *

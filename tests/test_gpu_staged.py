@@ -181,3 +181,20 @@ def test_motions_by_workgroups(robot, E, schedule, band):
         assert 0 <= mv.last_recheck_count() <= E
     if band is not None and E > 1:
         assert mv.last_recheck_count() > 0
+
+
+@pytest.mark.parametrize("n", [64, 2048, 2049, 4096, 524288, 524289])
+def test_cloud_build_sizes(n):
+    """One workgroup's keys, the first that take several, and both sides of the
+    bound from which the digit counts are summed by a launch of their own; every
+    table bit-exact, with runs of equal codes across wave and workgroup borders."""
+    from oracle import _oracle
+    from plainmp_amd import kdtree as kd
+
+    P = np.random.default_rng(n).uniform(-1, 1, (n, 3))
+    P[n // 3 : n // 3 + min(n // 2, 5000)] = P[7]
+    got, ref = dict(kd.build_cloud_tiles(P)), dict(_oracle.cloud_tiles(P))
+    for d in (got, ref):  # the 8 padding bytes of each 48-byte tile record carry no value
+        d["tiles"] = np.frombuffer(d["tiles"], np.uint8).reshape(-1, 48)[:, :40].tobytes()
+    for k in ref:
+        assert got[k] == ref[k], k
