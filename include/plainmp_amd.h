@@ -350,8 +350,8 @@ pmp_status pmp_traj_cost_grad_graph(pmp_context* ctx, const double* X, int64_t l
                                     int32_t n_traj, const double* weights, float* vals, float* jac, float* cost,
                                     float* grad, pmp_graph** out);
 /* Duration of the FP32 edge kernel of the most recent pmp_check_edges_batch
- * on this context, from HIP events recorded around it on the context stream
- * (waits for that kernel).  No reference counterpart: it serves throughput
+ * on this context, from the device clock's readings at its first start and
+ * last end (waits for that kernel).  No reference counterpart: it serves throughput
  * measurement. */
 pmp_status pmp_edge_kernel_ms(pmp_context* ctx, float* ms);
 /* Edges the most recent edge batch on this context re-decided in FP64

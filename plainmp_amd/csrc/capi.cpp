@@ -117,15 +117,20 @@ class TablePack {
 // cannot change what a replay reads.
 struct EdgeBufs {
   DevBuf width, inv_width, pend, counter;
-  int32_t slot = 0;                // EdgeArgs::slot of the last staged launch
+  int32_t slot = 0;                // EdgeArgs::slot of the last launch
+  bool launched = false;
   int32_t count_at = kCntRecheck;  // the counter that holds the last launch's FP64 decisions
   std::vector<double> h_width;  // what width / inv_width hold, so a repeated call uploads nothing
   void release() {
     for (DevBuf* b : {&width, &inv_width, &pend, &counter}) b->release();
     h_width.clear();
     count_at = kCntRecheck;
+    launched = false;
   }
 };
+// The buffer holds the counters, then the clocks.
+constexpr size_t kEdgeClockAt = 64;
+uint64_t* edge_clocks(const EdgeBufs& eb) { return (uint64_t*)((char*)eb.counter.ptr + kEdgeClockAt); }
 
 // Farthest-first visiting order of the motion validators
 // (ompl/generate_sequence.py:11-63): element i+1 maximises the minimum
@@ -175,7 +180,6 @@ struct pmp_context {
   int device = 0;
   hipStream_t stream = nullptr;
   hipStream_t capture_stream = nullptr;  // used for graph capture when no stream is set
-  hipEvent_t edge_ev0 = nullptr, edge_ev1 = nullptr;  // around the last direct edge kernel
   float band = 1e-5f;
   pmp_schedule sched{0, 0, 0};
   int n_cu = 256;
@@ -212,6 +216,7 @@ struct pmp_context {
   DevBuf seq, tmp_prims, tmp_cloud, ws_cen, ws_cloud;
   // Cross-stream order of calls (they share the workspaces above): an event
   // recorded on the stream of the last call, waited on by a call on another.
+  // Where a kernel ended the call its stop event is that event (call_end).
   hipEvent_t call_ev = nullptr;
   hipStream_t call_stream = nullptr;
   bool call_recorded = false;
@@ -248,6 +253,11 @@ void set_device(pmp_context* ctx) {
     PMP_HIP(hipStreamWaitEvent(ctx->stream, ctx->call_ev, 0));
 }
 hipStream_t st(pmp_context* ctx) { return ctx->stream; }
+// Lets the launcher called next end the call with its last kernel; for entry
+// points that enqueue nothing after it.
+void ends_call(pmp_context* ctx) {
+  if (!capturing(ctx->stream)) call_end.ask = ctx->call_ev;
+}
 
 // The stream a graph is captured on and replayed on: the context stream, or
 // with none set (the null stream) a stream of the context's own created
@@ -532,9 +542,13 @@ void require_robot(pmp_context* ctx) {
 namespace {
 // End of an entry point that enqueued work: remember it for set_device.
 void record_call(pmp_context* ctx) noexcept {
-  if (capturing(ctx->stream)) return;
-  if (!ctx->call_ev) return;  // created with the context
-  if (hipEventRecord(ctx->call_ev, ctx->stream) != hipSuccess) return;
+  const bool done = call_end.done != nullptr;
+  call_end = CallEnd{};
+  if (!done) {
+    if (capturing(ctx->stream)) return;
+    if (!ctx->call_ev) return;  // created with the context
+    if (hipEventRecord(ctx->call_ev, ctx->stream) != hipSuccess) return;
+  }
   ctx->call_recorded = true;
   ctx->call_stream = ctx->stream;
 }
@@ -583,8 +597,6 @@ pmp_status pmp_destroy(pmp_context* ctx) {
       b->release();
     ctx->eb.release();
     if (ctx->capture_stream) (void)hipStreamDestroy(ctx->capture_stream);
-    if (ctx->edge_ev0) (void)hipEventDestroy(ctx->edge_ev0);
-    if (ctx->edge_ev1) (void)hipEventDestroy(ctx->edge_ev1);
     if (ctx->call_ev) (void)hipEventDestroy(ctx->call_ev);
     delete ctx;
   });
@@ -1299,6 +1311,7 @@ pmp_status pmp_is_valid_batch(pmp_context* ctx, const double* q, int64_t ldq, in
     PMP_REQUIRE(B == 0 || valid, "null output");
     if (B == 0) return;
     set_device(ctx);
+    ends_call(ctx);
     PMP_HIP(launch_valid(ctx->k32, ctx->k64, ctx->s32, ctx->s64, q, ldq, B, ctx->band, valid, n_recheck,
                          ctx->sched.block, CloudWork{}, nullptr, 0, nullptr, nullptr, st(ctx)));
   });
@@ -1325,6 +1338,7 @@ pmp_status pmp_is_valid_batch_noalloc(pmp_context* ctx, const double* q, int64_t
                     std::to_string(kNoAllocScratchBytes) +
                     " bytes pmp_is_valid_batch_noalloc has; split the batch or call pmp_is_valid_batch");
     set_device(ctx);
+    ends_call(ctx);
     PMP_HIP(launch_valid(ctx->k32, ctx->k64, ctx->s32, ctx->s64, q, ldq, B, ctx->band, valid, n_recheck,
                          ctx->sched.block, CloudWork{}, nullptr, 0, nullptr, nullptr, st(ctx)));
   });
@@ -1340,6 +1354,7 @@ pmp_status pmp_evaluate_batch(pmp_context* ctx, const double* q, int64_t ldq, in
     e.vals = vals;
     e.jac = jac;
     e.whole_chunks = ctx->sched.eval_whole_chunks;
+    ends_call(ctx);
     PMP_HIP(launch_eval_units(ctx->k32, ctx->s32, q, ldq, B, e, st(ctx)));
   });
 }
@@ -1435,6 +1450,7 @@ pmp_status pmp_traj_cost_grad_batch(pmp_context* ctx, const double* X, int64_t l
     e.cost = cost;
     e.grad = grad;
     e.whole_chunks = ctx->sched.eval_whole_chunks;
+    ends_call(ctx);
     PMP_HIP(launch_eval_units(ctx->k32, ctx->s32, X, ldx, N, e, st(ctx)));
   });
 }
@@ -1538,6 +1554,7 @@ pmp_status pmp_pair_clearance_batch(pmp_context* ctx, const double* q, int64_t l
     PMP_REQUIRE(B == 0 || dist, "null output");
     if (B == 0 || ctx->n_spheres == 0 || ctx->s32.n_prims == 0) return;
     set_device(ctx);
+    ends_call(ctx);
     PMP_HIP(launch_pairs(ctx->k32, ctx->s32, q, ldq, B, dist, grad, ctx->sched.pair_shares, st(ctx)));
   });
 }
@@ -1552,6 +1569,7 @@ pmp_status pmp_pair_clearance_vjp(pmp_context* ctx, const double* q, int64_t ldq
     const int shares = vjp_shares(ctx->k32, ctx->s32.n_prims, B, ctx->sched.pair_shares);
     float* part = (float*)ctx->ws_vjp.get(
         sizeof(float) * std::max<int64_t>(1, (int64_t)ctx->k32.n_items * shares * ctx->n_cols * B));
+    ends_call(ctx);
     PMP_HIP(launch_vjp(ctx->k32, ctx->s32, q, ldq, B, grad_dist, part, grad_q, ctx->sched.pair_shares, st(ctx)));
   });
 }
@@ -1599,11 +1617,16 @@ void prepare_edges(pmp_context* ctx, const double* s1, const double* s2, int64_t
   ea.seq = (const uint8_t*)ctx->seq.ptr;
   // The kernels leave the counters at zero after every launch; a new buffer
   // starts there.
-  const bool fresh = eb.counter.bytes < sizeof(int32_t) * kNumEdgeCounters;  // new (or grown) buffer
-  ea.counter = (int32_t*)eb.counter.get(sizeof(int32_t) * kNumEdgeCounters);
-  if (fresh) PMP_HIP(launch_fill_i32(ea.counter, 0, kNumEdgeCounters, st(ctx)));
-  if (E > 0 && edges_staged(ctx->k32, ctx->s32, E)) {
+  const size_t words = kEdgeClockAt / sizeof(int32_t) + 4 * kEdgeClocks * sizeof(uint64_t) / sizeof(int32_t);
+  const bool fresh = eb.counter.bytes < sizeof(int32_t) * words;  // new buffer
+  ea.counter = (int32_t*)eb.counter.get(sizeof(int32_t) * words);
+  if (fresh) PMP_HIP(launch_fill_i32(ea.counter, 0, (int64_t)words, st(ctx)));
+  ea.clock = edge_clocks(eb);
+  if (E > 0) {
     ea.slot = eb.slot ^= 1;
+    eb.launched = true;
+  }
+  if (E > 0 && edges_staged(ctx->k32, ctx->s32, E)) {
     eb.count_at = kCntStaged + ea.slot;
     ea.valid = valid;
     ea.n_checked = n_checked;
@@ -1653,12 +1676,8 @@ pmp_status pmp_check_edges_batch(pmp_context* ctx, const double* s1, const doubl
     if (E == 0) return;
     int grid, block;
     edge_grid(ctx, E, grid, block);
-    if (!ctx->edge_ev0) {
-      PMP_HIP(hipEventCreate(&ctx->edge_ev0));
-      PMP_HIP(hipEventCreate(&ctx->edge_ev1));
-    }
-    PMP_HIP(launch_edges(ctx->k32, ctx->k64, ctx->s32, ctx->s64, ea, ctx->band, grid, block, st(ctx),
-                         ctx->edge_ev0, ctx->edge_ev1));
+    ends_call(ctx);
+    PMP_HIP(launch_edges(ctx->k32, ctx->k64, ctx->s32, ctx->s64, ea, ctx->band, grid, block, st(ctx)));
   });
 }
 
@@ -1732,10 +1751,18 @@ pmp_status pmp_edge_recheck_count(pmp_context* ctx, int32_t* n) {
 pmp_status pmp_edge_kernel_ms(pmp_context* ctx, float* ms) {
   return guarded([&] {
     PMP_REQUIRE(ctx != nullptr && ms != nullptr, "null argument");
-    PMP_REQUIRE(ctx->edge_ev0 != nullptr, "no edge batch has run on this context");
+    PMP_REQUIRE(ctx->eb.launched, "no edge batch has run on this context");
     set_device(ctx);
-    PMP_HIP(hipEventSynchronize(ctx->edge_ev1));
-    PMP_HIP(hipEventElapsedTime(ms, ctx->edge_ev0, ctx->edge_ev1));
+    uint64_t t[2][kEdgeClocks];
+    PMP_HIP(hipMemcpyAsync(t, edge_clocks(ctx->eb) + 2 * kEdgeClocks * ctx->eb.slot, sizeof(t), hipMemcpyDeviceToHost,
+                           st(ctx)));
+    PMP_HIP(hipStreamSynchronize(st(ctx)));
+    uint64_t first = UINT64_MAX, last = 0;
+    for (int i = 0; i < kEdgeClocks; ++i) {
+      if (t[0][i]) first = std::min(first, t[0][i]);  // 0: no workgroup
+      last = std::max(last, t[1][i]);
+    }
+    *ms = last > first ? (float)((double)(last - first) / kEdgeClockKhz) : 0.0f;
   });
 }
 

@@ -6,6 +6,7 @@
 #include <limits.h>
 
 #include "fk.hpp"
+#include "launch.h"
 
 namespace pmp {
 
@@ -80,6 +81,26 @@ __device__ __forceinline__ const A& args_again() {
 #else
   return *(const A*)nullptr;  // host pass: never executed, only type-checked
 #endif
+}
+
+// The edge kernels' running time, from the device's constant-rate clock: the
+// first workgroups' starts and, in as many words, the latest ends; the host
+// takes the span when it is asked.  (Events around the kernel cost 7 us a call,
+// 12 more where the call is then waited for.)  Also clears what the next
+// launch adds to.
+__device__ __forceinline__ void edge_clock_begin(const EdgeArgs& ea) {
+  uint64_t* mine = ea.clock + ea.slot * 2 * kEdgeClocks;
+  uint64_t* next = ea.clock + (1 - ea.slot) * 2 * kEdgeClocks;
+  if (blockIdx.x < kEdgeClocks && threadIdx.x == 0) mine[blockIdx.x] = (uint64_t)wall_clock64();
+  if (blockIdx.x == 0) {
+    for (int i = threadIdx.x; i < 2 * kEdgeClocks; i += blockDim.x) next[i] = 0;
+    if (threadIdx.x == 0) ea.counter[kCntStaged + 1 - ea.slot] = 0;
+  }
+}
+// By one lane of a wave, after its last edge.
+__device__ __forceinline__ void edge_clock_end(const EdgeArgs& ea) {
+  unsigned long long* end = reinterpret_cast<unsigned long long*>(ea.clock) + (ea.slot * 2 + 1) * kEdgeClocks;
+  atomicMax(end + blockIdx.x % kEdgeClocks, (unsigned long long)wall_clock64());
 }
 
 // Orders a wave's own LDS accesses: what its lanes wrote before is what they

@@ -14,7 +14,7 @@
 // band and its FP64 test walked every tile).
 #include <limits.h>
 
-#include "launch.h"
+#include "last_launch.hpp"
 #include "valid_stage.hpp"
 
 namespace pmp {
@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(1024) edges_staged_kernel(EdgeKernelArgs args)
   out.first = queue + 1;
   out.pend = out.first + 1;
   double* ends = reinterpret_cast<double*>(staged_lds + el.flags + 64 + 4 + 3 * kPendMax);
-  if (blockIdx.x == 0 && threadIdx.x == 0) args.ea.counter[kCntStaged + 1 - args.ea.slot] = 0;  // the next launch's
+  edge_clock_begin(args.ea);
   // Workgroups go to the XCDs in turn; each XCD takes a contiguous range of a
   // round's motions, whose endpoints share cache lines.
   const int g = (int)blockIdx.x, n = (int)gridDim.x, x = g % kXcds;
@@ -230,11 +230,12 @@ __global__ void __launch_bounds__(1024) edges_staged_kernel(EdgeKernelArgs args)
       if (redone) atomicAdd(args.ea.counter + kCntStaged + args.ea.slot, 1);
     }
   }
+  if (threadIdx.x == 0) edge_clock_end(args.ea);
 }
 
 hipError_t launch_edges_staged(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,
                                const SceneArgs<double>& s64, const EdgeArgs& ea, float band, int waves, int block,
-                               hipStream_t st, hipEvent_t ev_before, hipEvent_t ev_after) {
+                               hipStream_t st) {
   EdgeLds el{};
   size_t lds = 0;
   // 8 waves while a motion has a CU to itself or self pairs to share out, else 4
@@ -255,13 +256,8 @@ hipError_t launch_edges_staged(const KinArgs<float>& k32, const KinArgs<double>&
     if (el.h_min == 8) return hipErrorInvalidConfiguration;  // 8 states of any robot fit
   }
   const int64_t most = waves > 0 ? (waves < W ? 1 : waves / W) : 1 << 20;
-  if (ev_before)
-    if (hipError_t e = hipEventRecord(ev_before, st)) return e;
-  hipLaunchKernelGGL(edges_staged_kernel, dim3((unsigned)(ea.E < most ? ea.E : most)), dim3(64 * W), lds, st,
+  return launch_last(edges_staged_kernel, dim3((unsigned)(ea.E < most ? ea.E : most)), dim3(64 * W), lds, st,
                      EdgeKernelArgs{k32, s32, k64, s64, ea, el, band});
-  if (ev_after)
-    if (hipError_t e = hipEventRecord(ev_after, st)) return e;
-  return hipGetLastError();
 }
 
 }  // namespace pmp

@@ -21,7 +21,7 @@
 // centres and directions, and all waves write the rows' columns.
 #include <type_traits>
 
-#include "launch.h"
+#include "last_launch.hpp"
 #include "stage.hpp"
 
 namespace pmp {
@@ -479,8 +479,9 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   o.scratch = o_scratch;
   o.best = o_best;
   const dim3 grid((unsigned)(chunks + (o.n_traj + W - 1) / W)), block(64 * W);
+  *err = hipSuccess;
   if (grid.x > 0) {
-#define PMP_EVAL(H) hipLaunchKernelGGL(eval_staged_kernel<H>, grid, block, lds, st, ka, sc, q, ldq, B, o, lay)
+#define PMP_EVAL(H) *err = launch_last(eval_staged_kernel<H>, grid, block, lds, st, ka, sc, q, ldq, B, o, lay)
     if (H == 1)
       PMP_EVAL(1);
     else if (H == 2)
@@ -491,7 +492,6 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
       PMP_EVAL(8);
 #undef PMP_EVAL
   }
-  *err = hipGetLastError();
   return true;
 }
 

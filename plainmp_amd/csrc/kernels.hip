@@ -9,7 +9,7 @@
 #include <limits.h>
 
 #include "device.hpp"
-#include "launch.h"
+#include "last_launch.hpp"
 
 namespace pmp {
 
@@ -522,6 +522,7 @@ edges_kernel(KinArgs<float> k32, SceneArgs<float> s32, KinArgs<double> k64, Scen
   // edges from the counter.  Every lane takes part in the atomic (lane 0
   // adds 1, the others 0) and the index is read from the first lane into a
   // scalar register, so it and every branch on it are wave-uniform.
+  edge_clock_begin(ea);
   const int W = blockDim.x >> 6;
   const bool by_index = (int64_t)gridDim.x * W >= ea.E;
   int e;
@@ -637,6 +638,7 @@ edges_kernel(KinArgs<float> k32, SceneArgs<float> s32, KinArgs<double> k64, Scen
       }
     }
   }
+  if (lane == 0) edge_clock_end(ea);
 }
 
 // FP64 decision of the edges left pending by edges_kernel, read from its
@@ -1353,27 +1355,18 @@ hipError_t launch_clearance(const KinArgs<float>& ka, const SceneArgs<float>& sc
 }
 hipError_t launch_edges(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,
                         const SceneArgs<double>& s64, const EdgeArgs& ea, float band, int grid, int block,
-                        hipStream_t st, hipEvent_t ev_before, hipEvent_t ev_after) {
+                        hipStream_t st, hipEvent_t, hipEvent_t) {
   if (edges_staged(k32, s32, ea.E))
-    return launch_edges_staged(k32, k64, s32, s64, ea, band, grid, block, st, ev_before, ev_after);
-  if (ev_before) {
-    hipError_t e = hipEventRecord(ev_before, st);
-    if (e != hipSuccess) return e;
-  }
+    return launch_edges_staged(k32, k64, s32, s64, ea, band, grid, block, st);
   // a wave's FP32 walk and its FP64 re-decisions after it share the wave's
   // kept-pose chunk, sized for FP64
   KinArgs<float> kw = k32;
   kw.slot_wave_bytes = k64.slot_wave_bytes;
   const size_t lds = slot_bytes(k64, block);
   hipLaunchKernelGGL(edges_kernel, dim3(grid), dim3(block), lds, st, kw, s32, k64, s64, ea, band);
-  if (ev_after) {
-    hipError_t e = hipEventRecord(ev_after, st);
-    if (e != hipSuccess) return e;
-  }
   const unsigned rgrid = (unsigned)(ea.E < kRecheckGrid ? ea.E : kRecheckGrid);
   const int rblock = slot_block(k64, 64 * kRecheckWaves, sizeof(int));
-  hipLaunchKernelGGL(edges_recheck_kernel, dim3(rgrid), dim3(rblock), slot_bytes(k64, rblock), st, k64, s64, ea);
-  return hipGetLastError();
+  return launch_last(edges_recheck_kernel, dim3(rgrid), dim3(rblock), slot_bytes(k64, rblock), st, k64, s64, ea);
 }
 
 #define PMP_DISPATCH_MAXC(ncols, KERNEL, ...)                                                 \
@@ -1560,9 +1553,8 @@ hipError_t launch_vjp(const KinArgs<float>& ka, const SceneArgs<float>& sc, cons
     PMP_DISPATCH_MAXC(ka.n_cols, vjp_kernel, dim3(blocks_for(B, bk), (unsigned)ka.n_items, (unsigned)nz), dim3(bk),
                       slot_bytes(ka, bk), st, ka, sc, q, ldq, B, gd, part);
   }
-  hipLaunchKernelGGL(vjp_reduce_kernel, dim3(blocks_for((int64_t)ka.n_cols * B, 256)), dim3(256), 0, st, part,
+  return launch_last(vjp_reduce_kernel, dim3(blocks_for((int64_t)ka.n_cols * B, 256)), dim3(256), 0, st, part,
                      ka.n_items * nz, ka.n_cols, B, grad_q);
-  return hipGetLastError();
 }
 hipError_t launch_prims_eval(const DevPrim<double>* prims, int n, const double* cloud_xyz, const double* pts,
                              int64_t N, int mode, double radius, double* out, hipStream_t st) {

@@ -17,7 +17,7 @@ constexpr int kPendStates = 16;  // in-band states an edge may queue for the FP6
 // (zero when the buffer is allocated) and no clearing node is needed in a
 // captured graph.
 // The staged form counts its FP64 decisions in one of two words in turn
-// (EdgeArgs::slot) and clears the other one for the next launch.
+// (EdgeArgs::slot); every launch clears the other word for the next one.
 enum EdgeCounter {
   kCntWork = 0,
   kCntRecheck = 1,
@@ -27,6 +27,17 @@ enum EdgeCounter {
   kCntStaged = 5,  // and 6
   kNumEdgeCounters = 7
 };
+
+// The event that marks the end of the current entry point's call: `ask` is set
+// while a launcher may give it to the call's last kernel (never while the
+// stream is captured), `done` is the event that was given.
+struct CallEnd {
+  hipEvent_t ask = nullptr, done = nullptr;
+};
+inline thread_local CallEnd call_end;
+
+constexpr int kEdgeClocks = 64;
+constexpr double kEdgeClockKhz = 1e5;  // wall_clock64 of gfx950
 
 struct EdgeArgs {
   const double* s1;
@@ -38,7 +49,8 @@ struct EdgeArgs {
   const double* inv_width;  // device [n_cols], 1 / width as the reference precomputes
   const uint8_t* seq;       // device [128 * 128] farthest-first sequence table
   int32_t* counter;         // device [kNumEdgeCounters], see EdgeCounter
-  int32_t slot;             // staged form: the word of this launch's count, 0 or 1
+  uint64_t* clock;          // device [2][2][kEdgeClocks], see edge_clock_begin
+  int32_t slot;             // which of the two words and clock sets this launch uses
   int32_t* pend;            // [E][kPendStates] in-band visiting indices of pending edges
   int32_t* pend_info;       // [E][2] number queued (-1: more than kPendStates), first certain collision
   int32_t* plist;           // [E] the pending edges, in the order edges_kernel finished them
@@ -118,8 +130,8 @@ inline bool edges_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, i
 // workgroup (0 = default).
 hipError_t launch_edges_staged(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,
                                const SceneArgs<double>& s64, const EdgeArgs& ea, float band, int waves, int block,
-                               hipStream_t st, hipEvent_t ev_before, hipEvent_t ev_after);
-// ev_before / ev_after (optional) are recorded around the FP32 edge kernel.
+                               hipStream_t st);
+// The events are not used: the kernels stamp their own time (EdgeArgs::clock).
 hipError_t launch_edges(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,
                         const SceneArgs<double>& s64, const EdgeArgs& ea, float band, int grid, int block,
                         hipStream_t st, hipEvent_t ev_before = nullptr, hipEvent_t ev_after = nullptr);

@@ -8,7 +8,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "launch.h"
+#include "last_launch.hpp"
 #include "stage.hpp"
 
 namespace pmp {
@@ -250,25 +250,15 @@ hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   const bool stream = B % 32 == 0;
   const dim3 grid((unsigned)(chunks * ny)), block(64 * W);
 #define PMP_DIST(STREAM) \
-  hipLaunchKernelGGL(pair_dist_kernel<STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, n_slices, (int)chunks, lay)
+  launch_last(pair_dist_kernel<STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, n_slices, (int)chunks, lay)
 #define PMP_GRAD(MAXC, STREAM)                                                                                        \
-  hipLaunchKernelGGL((pair_grad_kernel<MAXC, STREAM>), grid, block, lds, st, ka, sc, q, ldq, B, dist, grad, n_slices, \
+  launch_last(pair_grad_kernel<MAXC, STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, grad, n_slices,            \
                      (int)chunks, lay)
-  if (!grad && stream)
-    PMP_DIST(true);
-  else if (!grad)
-    PMP_DIST(false);
-  else if (ka.n_cols <= 8 && stream)
-    PMP_GRAD(8, true);
-  else if (ka.n_cols <= 8)
-    PMP_GRAD(8, false);
-  else if (stream)
-    PMP_GRAD(16, true);
-  else
-    PMP_GRAD(16, false);
+  if (!grad) return stream ? PMP_DIST(true) : PMP_DIST(false);
+  if (ka.n_cols <= 8) return stream ? PMP_GRAD(8, true) : PMP_GRAD(8, false);
+  return stream ? PMP_GRAD(16, true) : PMP_GRAD(16, false);
 #undef PMP_DIST
 #undef PMP_GRAD
-  return hipGetLastError();
 }
 
 }  // namespace pmp

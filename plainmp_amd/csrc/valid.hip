@@ -1,7 +1,7 @@
 // Validity of a batch of configurations by staged workgroups (stage.hpp,
 // valid_stage.hpp): SphereCollisionCst::is_valid_dirty
 // (constraints/primitive_sphere_collision.cpp:181-254) per configuration.
-#include "launch.h"
+#include "last_launch.hpp"
 #include "valid_stage.hpp"
 
 namespace pmp {
@@ -98,17 +98,9 @@ hipError_t launch_valid(const KinArgs<float>& k32, const KinArgs<double>& k64, c
   const StageLds lay = stage_lds(k32, C);
   const dim3 grid((unsigned)((B + C - 1) / C)), block(64 * sh.W);
 #define PMP_VALID(H) \
-  hipLaunchKernelGGL(valid_staged_kernel<H>, grid, block, lds, st, k32, s32, k64, s64, q, ldq, B, o, lay)
-  if (sh.H == 1)
-    PMP_VALID(1);
-  else if (sh.H == 2)
-    PMP_VALID(2);
-  else if (sh.H == 4)
-    PMP_VALID(4);
-  else
-    PMP_VALID(8);
+  launch_last(valid_staged_kernel<H>, grid, block, lds, st, k32, s32, k64, s64, q, ldq, B, o, lay)
+  return sh.H == 1 ? PMP_VALID(1) : sh.H == 2 ? PMP_VALID(2) : sh.H == 4 ? PMP_VALID(4) : PMP_VALID(8);
 #undef PMP_VALID
-  return hipGetLastError();
 }
 
 }  // namespace pmp
