@@ -5,6 +5,7 @@
 // tree flattened at set_sdf time with primitives shared by pointer.
 #pragma once
 
+#include <cstring>
 #include <random>
 
 #include "host.hpp"
@@ -560,29 +561,20 @@ class MotionValidator {
   // S1, S2 row-major (E, q_dim)
   std::vector<uint8_t> check_motions(const double* S1, const double* S2, int64_t E, std::vector<int32_t>* n_checked) {
     cst_->sync_batch_tables();
-    pmp_context* ctx = cst_->device_context(nullptr);
-    const int D = (int)cst_->q_dim();
-    std::vector<uint8_t> out(E);
-    if (E == 0) return out;
-    double* d1 = dev_.upload_soa(0, S1, E, D);
-    double* d2 = dev_.upload_soa(1, S2, E, D);
-    uint8_t* dv = (uint8_t*)dev_.buf(2, E);
-    int32_t* dn = (int32_t*)dev_.buf(3, sizeof(int32_t) * E);
-    pmp_validator_desc v = desc();
-    check(pmp_check_edges_batch(ctx, d1, d2, E, E, &v, dv, dn));
-    dev_.d2h(out.data(), dv, E);
-    if (n_checked) {
-      n_checked->resize(E);
-      dev_.d2h(n_checked->data(), dn, sizeof(int32_t) * E);
-    }
-    return out;
+    (void)cst_->device_context(nullptr);
+    if (E == 0) return {};
+    const double* d = dev_.upload_soa(0, S1, E, S2, E, (int)cst_->q_dim());
+    return check_uploaded(d, d + E, 2 * E, E, n_checked);
   }
   // Validity of every segment of a path (row-major (n, q_dim) states), all
   // n - 1 segments in one batched launch: the check OMPL's path utilities
   // make one checkMotion at a time (ompl_thin_wrap.hpp:130-170).
   std::vector<uint8_t> check_path(const double* P, int64_t n) {
     if (n < 2) return {};
-    return check_motions(P, P + cst_->q_dim(), n - 1, nullptr);
+    cst_->sync_batch_tables();
+    // segment i runs from state i to state i + 1 of one array
+    const double* d = dev_.upload_soa(0, P, n, (int)cst_->q_dim());
+    return check_uploaded(d, d + 1, n, n - 1, nullptr);
   }
 
   // Batched shortcutting, the planner's path simplification
@@ -663,6 +655,27 @@ class MotionValidator {
   }
 
  private:
+  // E motions between uploaded states (ld apart per coordinate), one copy in
+  // (the caller's) and one out: a copy costs about 10 us, as much as the check
+  // of a short path (65 states: 69 us with both ends of every segment uploaded
+  // and both results fetched).
+  std::vector<uint8_t> check_uploaded(const double* d1, const double* d2, int64_t ld, int64_t E,
+                                      std::vector<int32_t>* n_checked) {
+    const size_t counts = n_checked ? sizeof(int32_t) * (size_t)E : 0;
+    uint8_t* out = (uint8_t*)dev_.buf(1, counts + (size_t)E);
+    const pmp_validator_desc v = desc();
+    check(pmp_check_edges_batch(cst_->device_context(nullptr), d1, d2, ld, E, &v, out + counts,
+                                n_checked ? (int32_t*)out : nullptr));
+    std::vector<uint8_t> h(counts + (size_t)E);
+    dev_.d2h(h.data(), out, h.size());
+    if (n_checked) {
+      n_checked->resize(E);
+      std::memcpy(n_checked->data(), h.data(), counts);
+      h.erase(h.begin(), h.begin() + (int64_t)counts);
+    }
+    return h;
+  }
+
   std::shared_ptr<SphereCollisionCst> cst_;
   ValidatorConfig vc_;
   Device dev_;  // edge staging buffers (the tables live in the constraint's context)

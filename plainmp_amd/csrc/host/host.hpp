@@ -79,10 +79,16 @@ class Device {
     if (n) hip_check(hipMemcpy(h, d, n, hipMemcpyDeviceToHost), "hipMemcpy D2H");
   }
   // Column-major upload of a row-major (B, D) host array: dst[d * B + b].
-  double* upload_soa(int slot, const double* rows, int64_t B, int D) {
-    std::vector<double> t((size_t)B * D);
-    for (int64_t b = 0; b < B; ++b)
-      for (int d = 0; d < D; ++d) t[(size_t)d * B + b] = rows[(size_t)b * D + d];
+  double* upload_soa(int slot, const double* rows, int64_t B, int D) { return upload_soa(slot, rows, B, nullptr, 0, D); }
+  // Two arrays' states side by side in one copy: dst[d * (A + B) + i], the rows
+  // of `b` from i = A on.
+  double* upload_soa(int slot, const double* a, int64_t A, const double* b, int64_t B, int D) {
+    const int64_t n = A + B;
+    std::vector<double> t((size_t)n * D);
+    for (int64_t i = 0; i < n; ++i) {
+      const double* row = i < A ? a + (size_t)i * D : b + (size_t)(i - A) * D;
+      for (int d = 0; d < D; ++d) t[(size_t)d * n + i] = row[d];
+    }
     double* p = (double*)buf(slot, t.size() * sizeof(double));
     h2d(p, t.data(), t.size() * sizeof(double));
     return p;
