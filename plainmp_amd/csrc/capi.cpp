@@ -976,6 +976,7 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
     pk.add(rows, &a.rows, &d.rows);
     pk.add(path_at, &a.path_at, &d.path_at);
     a.n_paths = d.n_paths = (int32_t)path_at.size() - 1;
+    a.n_path_entries = d.n_path_entries = path_at.back();
     a.n_poses = d.n_poses = n_poses;
     pk.add(joints, &a.joints, &d.joints);
     pk.add(columns, &a.columns, &d.columns);

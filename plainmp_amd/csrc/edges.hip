@@ -103,10 +103,7 @@ __device__ __forceinline__ void edge_chunk(float* lds, const EdgeStates& es, int
   const SceneArgs<float>& sc = A.sc;
   const bool taylor = ka.base_type == PMP_BASE_FIXED;  // constraints/primitive.hpp:59-61
   constexpr int C = 64 / H;
-  StageLds lay;
-  lay.joints = 0;
-  lay.poses = 4 * ka.n_joints * C;
-  lay.end = lay.poses + 7 * ka.n_poses * C;
+  const StageLds lay = stage_lds(ka, C);
   const Stage<H> S(lds, lay);
   const int lane = S.lane, w = S.w, W = S.W, cfg = S.cfg;
   const bool active = base + cfg < es.n_wp;
@@ -118,7 +115,6 @@ __device__ __forceinline__ void edge_chunk(float* lds, const EdgeStates& es, int
     *out.first = INT_MAX;
   }
   S.joints(ka, qs, taylor);
-  if (w == W - 1) warm_scalar(ka.path, cload(ka.path_at, ka.n_paths) * (int)sizeof(DevPathNode), 0, 1);
   __syncthreads();
   for (int col = w * H + S.sub; col < ka.n_cols; col += W * H)
     if (!fp32_range_col(ka.rev_mask, col, qs.get(col))) out.mark(cfg, kWhole);

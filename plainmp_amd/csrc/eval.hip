@@ -294,7 +294,6 @@ __global__ void __launch_bounds__(1024) eval_staged_kernel(KinArgs<float> ka, Sc
   int* queue = tr + 2 * C;
   const int n_blocks = ka.n_units - ka.n_pairs;
   S.joints(ka, qs, false);
-  if (w == W - 1) warm_scalar(ka.path, cload(ka.path_at, ka.n_paths) * (int)sizeof(DevPathNode), 0, 1);
   if (threadIdx.x < 2 * C) best[threadIdx.x] = no_winner();
   if (threadIdx.x == 0) *queue = 0;
   __syncthreads();

@@ -23,15 +23,23 @@
 
 namespace pmp {
 
-// Offsets (in floats) of a staged workgroup's LDS tables.
+// Offsets (in floats) of a staged workgroup's LDS tables: the joints' words,
+// the poses, and a copy of the path entries (16 words each; path < 0: too many,
+// read from memory).
+constexpr int kStagedEntries = 256;
 struct StageLds {
-  int joints, poses, end;
+  int joints, poses, path, end;
 };
-inline StageLds stage_lds(const KinArgs<float>& ka, int C) {
+__host__ __device__ __forceinline__ StageLds stage_lds(const KinArgs<float>& ka, int C) {
   StageLds L;
   L.joints = 0;
   L.poses = 4 * ka.n_joints * C;
   L.end = L.poses + 7 * ka.n_poses * C;
+  L.path = -1;
+  if (ka.n_path_entries <= kStagedEntries) {
+    L.path = L.end;
+    L.end += 16 * ka.n_path_entries;
+  }
   return L;
 }
 
@@ -82,9 +90,12 @@ struct Stage {
         sub(H == 1 ? 0 : lane / C) {}
 
   // Every joint's local rotation (origin times joint), or its displacement in
-  // word 0 of a prismatic one.
+  // word 0 of a prismatic one; and the path entries.
   template <class QS>
   __device__ __forceinline__ void joints(const KinArgs<float>& ka, const QS& qs, bool taylor) const {
+    if (L.path >= 0)
+      for (int i = threadIdx.x; i < 4 * ka.n_path_entries; i += blockDim.x)
+        reinterpret_cast<float4*>(lds + L.path)[i] = reinterpret_cast<const float4*>(ka.path)[i];
     for (int i = w * H + sub; i < ka.n_joints; i += W * H) {
       const DevJoint jt = H == 1 ? cload(ka.joints, i) : ka.joints[i];
       const double v = qs.get(jt.q_col);
@@ -108,32 +119,54 @@ struct Stage {
   }
 
   // The paths of this wave (path p goes to wave p mod W); joints() of every
-  // wave must be complete.
+  // wave must be complete.  A node costs its dependent chain (about 65 vector
+  // instructions of one wave): the entries are read from LDS two ahead and the
+  // joints' words one ahead.  (Entries read by scalar loads meet the LDS reads
+  // in one wait counter, which then waits for both: 1,000 configurations of the
+  // 14-joint robot 16.8 us, so 15.5; 512 motions of it 50.9 and 48.2.)
+  struct Entry {
+    float4 quat, trans_axis0, axis12_kind_identity, joint_pose;
+  };
+  __device__ __forceinline__ Entry entry(const KinArgs<float>& ka, int e) const {
+    if (L.path >= 0) {
+      const float4* p = reinterpret_cast<const float4*>(lds + L.path) + 4 * e;
+      return {p[0], p[1], p[2], p[3]};
+    }
+    const float4* p = reinterpret_cast<const float4*>(ka.path + e);
+    return {p[0], p[1], p[2], p[3]};
+  }
+  __device__ __forceinline__ Q4<float> joint_words(const Entry& e) const {
+    const float* p = lds + L.joints + 4 * __float_as_int(e.joint_pose.x) * C + cfg;
+    return {p[0], p[C], p[2 * C], p[3 * C]};
+  }
   template <class QS>
   __device__ __forceinline__ void walk(const KinArgs<float>& ka, const QS& qs) const {
     for (int p = w; p < ka.n_paths; p += W) {
       Pose<float> P = base_pose(ka, qs);
-      const int e_end = cload(ka.path_at, p + 1);
-      int e = cload(ka.path_at, p);
-      DevPathNode next = cload(ka.path, e);
-      for (; e < e_end; ++e) {
-        const DevPathNode pe = next;
-        next = cload(ka.path, e + 1 < e_end ? e + 1 : e);  // one entry ahead of its use
-        const V3<float> lt{pe.trans[0], pe.trans[1], pe.trans[2]};
-        const Q4<float> oq{pe.quat[0], pe.quat[1], pe.quat[2], pe.quat[3]};
-        const float* jc = lds + L.joints + 4 * pe.joint * C + cfg;
-        switch (pe.kind) {
+      const int e_end = cload(ka.path_at, p + 1), e_begin = cload(ka.path_at, p);
+      Entry cur = entry(ka, e_begin), next = entry(ka, min(e_begin + 1, e_end - 1));
+      Q4<float> jq = joint_words(cur);
+      for (int e = e_begin; e < e_end; ++e) {
+        const Q4<float> jq_next = joint_words(next);
+        const Entry after = entry(ka, min(e + 2, e_end - 1));
+        const V3<float> lt{cur.trans_axis0.x, cur.trans_axis0.y, cur.trans_axis0.z};
+        const Q4<float> oq{cur.quat.x, cur.quat.y, cur.quat.z, cur.quat.w};
+        const int kind = __builtin_amdgcn_readfirstlane(__float_as_int(cur.axis12_kind_identity.z));
+        const int pose = __builtin_amdgcn_readfirstlane(__float_as_int(cur.joint_pose.y));
+        switch (kind) {
           case PMP_NODE_ROOT:
             break;
           case PMP_NODE_FIXED:
-            P = compose(P, oq, lt, pe.identity != 0);
+            P = compose(P, oq, lt,
+                        __builtin_amdgcn_readfirstlane(__float_as_int(cur.axis12_kind_identity.w)) != 0);
             break;
           case PMP_NODE_REVOLUTE:
-            P = compose(P, Q4<float>{jc[0], jc[C], jc[2 * C], jc[3 * C]}, lt, false);
+            P = compose(P, jq, lt, false);
             break;
           case PMP_NODE_PRISMATIC: {
-            const float v = jc[0];
-            const V3<float> t2{lt.x + pe.axis[0] * v, lt.y + pe.axis[1] * v, lt.z + pe.axis[2] * v};
+            const float v = jq.x;
+            const V3<float> t2{lt.x + cur.trans_axis0.w * v, lt.y + cur.axis12_kind_identity.x * v,
+                               lt.z + cur.axis12_kind_identity.y * v};
             P = compose(P, oq, t2, true);
             break;
           }
@@ -143,7 +176,10 @@ struct Stage {
             break;
           }
         }
-        if (pe.pose >= 0) pose_set(pe.pose, P);
+        if (pose >= 0) pose_set(pose, P);
+        cur = next;
+        next = after;
+        jq = jq_next;
       }
     }
   }

@@ -205,7 +205,7 @@ struct KinArgs {
   const DevJoint* joints;
   const DevColumn* columns;  // [n_q_cols]
   const DevSphereRow* rows;  // [n_spheres], group order
-  int32_t n_paths, n_poses, n_joints;
+  int32_t n_paths, n_path_entries, n_poses, n_joints;
   int32_t staged;  // the staged tables describe this robot (no q column drives two joints)
   T base_q[4];
   T base_t[3];

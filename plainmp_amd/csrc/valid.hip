@@ -40,7 +40,6 @@ __global__ void __launch_bounds__(1024) valid_staged_kernel(KinArgs<float> ka, S
   if (threadIdx.x < C) out.flags[threadIdx.x] = active ? 0 : kHit;  // past the batch: nothing to do
   if (threadIdx.x == 0) *out.count = *queue = 0;
   S.joints(ka, qs, taylor);
-  if (w == W - 1) warm_scalar(ka.path, cload(ka.path_at, ka.n_paths) * (int)sizeof(DevPathNode), 0, 1);
   __syncthreads();
   // joint values outside the FP32 walk's ranges
   for (int col = w * H + S.sub; col < ka.n_cols; col += W * H)
