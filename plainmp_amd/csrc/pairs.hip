@@ -107,20 +107,19 @@ __device__ __forceinline__ void put(float* p, float v) {
 // dist[(s * P + p) * B + b]: task t of the launch is item t / n_slices (up to
 // eight spheres of a link, so that a primitive is read once for all of them)
 // against slice t % n_slices of the primitives; workgroups share the tasks.
-template <bool kStream>
+template <int H, bool kStream>
 __global__ void __launch_bounds__(512) pair_dist_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
                                                         int64_t ldq, int64_t B, float* dist, int n_slices, int chunks,
                                                         StageLds lay) {
   HIP_DYNAMIC_SHARED(float, staged_lds)
-  const Stage<1> S(staged_lds, lay);
+  const Stage<H> S(staged_lds, lay);
   int share, chunk;
   share_and_chunk(chunks, share, chunk);
   const int shares = (int)gridDim.x / chunks;
-  const int64_t b = (int64_t)chunk * 64 + S.cfg;
-  const bool active = b < B;
-  BatchQ qs{q, ldq, active ? b : B - 1};
+  const int64_t b = (int64_t)chunk * Stage<H>::C + S.cfg;
+  const bool active = b < B && S.sub == 0;
+  BatchQ qs{q, ldq, b < B ? b : B - 1};
   S.joints(ka, qs, false);
-  if (S.w == S.W - 1) warm_scalar(ka.path, cload(ka.path_at, ka.n_paths) * (int)sizeof(DevPathNode), 0, 1);
   __syncthreads();
   S.walk(ka, qs);
   if (S.w >= ka.n_paths)
@@ -168,20 +167,19 @@ __global__ void __launch_bounds__(512) pair_dist_kernel(KinArgs<float> ka, Scene
 // link) before); 256-byte pieces of rows alone take 94 us on this card, a
 // plain fill 73 us.  With rows off the cache lines (8,191 configurations) 142
 // us; 277 us with streaming stores and neighbouring chunks on different XCDs.
-template <int MAXC, bool kStream>
+template <int H, int MAXC, bool kStream>
 __global__ void __launch_bounds__(256) pair_grad_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
                                                         int64_t ldq, int64_t B, float* dist, float* grad, int n_slices,
                                                         int chunks, StageLds lay) {
   HIP_DYNAMIC_SHARED(float, staged_lds)
-  const Stage<1> S(staged_lds, lay);
+  const Stage<H> S(staged_lds, lay);
   int share, chunk;
   share_and_chunk(chunks, share, chunk);
   const int shares = (int)gridDim.x / chunks, cfg = S.cfg;
-  const int64_t b = (int64_t)chunk * 64 + cfg;
-  const bool active = b < B;
-  BatchQ qs{q, ldq, active ? b : B - 1};
+  const int64_t b = (int64_t)chunk * Stage<H>::C + cfg;
+  const bool active = b < B && S.sub == 0;
+  BatchQ qs{q, ldq, b < B ? b : B - 1};
   S.joints(ka, qs, false);
-  if (S.w == S.W - 1) warm_scalar(ka.path, cload(ka.path_at, ka.n_paths) * (int)sizeof(DevPathNode), 0, 1);
   __syncthreads();
   S.walk(ka, qs);
   __syncthreads();
@@ -201,7 +199,7 @@ __global__ void __launch_bounds__(256) pair_grad_kernel(KinArgs<float> ka, Scene
         J[j] = {0.f, 0.f, 0.f};
         if (j0 + j < D && ((row.col_mask >> (j0 + j)) & 1ull)) {
           V3<float> a, o;
-          staged_frame<64>(frames, j0 + j, cfg, a, o);
+          staged_frame<Stage<H>::C>(frames, j0 + j, cfg, a, o);
           J[j] = ((ka.rev_mask >> (j0 + j)) & 1ull) ? cross(a, sub(c, o)) : a;
         }
       }
@@ -232,10 +230,17 @@ constexpr int64_t kPairWorkgroups = 16 * kCus;
 hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq,
                         int64_t B, float* dist, float* grad, int shares, hipStream_t st) {
   if (ka.n_spheres == 0 || sc.n_prims == 0 || B == 0) return hipSuccess;
-  const StageLds lay = stage_lds(ka, 64);
-  const size_t lds = sizeof(float) * (size_t)(lay.end + (grad ? 6 * ka.n_cols * 64 : 0));
-  if (lds > (size_t)ka.lds_limit) return hipErrorInvalidConfiguration;
-  const int64_t chunks = (B + 63) / 64;
+  // 64 configurations a workgroup; robots whose tables do not fit take fewer
+  // (H lanes hold a configuration, one of them works)
+  int H = 1;
+  auto lds_of = [&](int H) {
+    return sizeof(float) * (size_t)(stage_lds(ka, 64 / H).end + (grad ? 6 * ka.n_cols * (64 / H) : 0));
+  };
+  while (H < 8 && lds_of(H) > (size_t)ka.lds_limit) H *= 2;
+  const size_t lds = lds_of(H);
+  if (lds > (size_t)ka.lds_limit) return hipErrorInvalidConfiguration;  // 8 configurations of any robot fit
+  const StageLds lay = stage_lds(ka, 64 / H);
+  const int64_t chunks = (B + 64 / H - 1) / (64 / H);
   // Distances: 4 primitives a task and a task a wave (8,191 configurations of
   // the 7R arm, 32 primitives: 31 us; 8 primitives 33, 4 tasks a wave 35).
   // Gradients: 8 primitives, two tasks a wave once the launch fills the GPU
@@ -249,14 +254,17 @@ hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   if (shares > 0) ny = std::min<int64_t>(shares, tasks);
   const bool stream = B % 32 == 0;
   const dim3 grid((unsigned)(chunks * ny)), block(64 * W);
-#define PMP_DIST(STREAM) \
-  launch_last(pair_dist_kernel<STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, n_slices, (int)chunks, lay)
-#define PMP_GRAD(MAXC, STREAM)                                                                                        \
-  launch_last(pair_grad_kernel<MAXC, STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, grad, n_slices,            \
-                     (int)chunks, lay)
-  if (!grad) return stream ? PMP_DIST(true) : PMP_DIST(false);
-  if (ka.n_cols <= 8) return stream ? PMP_GRAD(8, true) : PMP_GRAD(8, false);
-  return stream ? PMP_GRAD(16, true) : PMP_GRAD(16, false);
+#define PMP_DIST(H, STREAM)                                                                                           \
+  launch_last(pair_dist_kernel<H, STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, n_slices, (int)chunks, lay)
+#define PMP_GRAD(H, MAXC, STREAM)                                                                                     \
+  launch_last(pair_grad_kernel<H, MAXC, STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, grad, n_slices,       \
+              (int)chunks, lay)
+  if (H == 2) return grad ? PMP_GRAD(2, 16, false) : PMP_DIST(2, false);
+  if (H == 4) return grad ? PMP_GRAD(4, 16, false) : PMP_DIST(4, false);
+  if (H == 8) return grad ? PMP_GRAD(8, 16, false) : PMP_DIST(8, false);
+  if (!grad) return stream ? PMP_DIST(1, true) : PMP_DIST(1, false);
+  if (ka.n_cols <= 8) return stream ? PMP_GRAD(1, 8, true) : PMP_GRAD(1, 8, false);
+  return stream ? PMP_GRAD(1, 16, true) : PMP_GRAD(1, 16, false);
 #undef PMP_DIST
 #undef PMP_GRAD
 }

@@ -198,3 +198,51 @@ def test_cloud_build_sizes(n):
         d["tiles"] = np.frombuffer(d["tiles"], np.uint8).reshape(-1, 48)[:, :40].tobytes()
     for k in ref:
         assert got[k] == ref[k], k
+
+
+def _comb(n=60):
+    """A chain of n joints whose links each carry a sphere, every third one a side
+    link with another: more poses than 64 configurations' tables fit LDS with, and more
+    path entries than are staged."""
+    rng = np.random.default_rng(4)
+    links, joints, urdf, specs = ["base"], [], "", []
+    for i in range(n):
+        prev, ln, side = "base" if i == 0 else f"l{i - 1}", f"l{i}", f"s{i}"
+        axis = ((0, 0, 1), (0, 1, 0), (1, 0, 0))[i % 3]
+        urdf += synth._joint(f"j{i}", "revolute", prev, ln, (0, 0, 0.05), (0, 0, 0), axis=axis, lower=-0.3, upper=0.3)
+        links.append(ln)
+        joints.append(f"j{i}")
+        specs.append((ln, np.zeros((1, 3)), np.array([0.03]), False))
+        if i % 3 == 2:
+            urdf += synth._joint(f"f{i}", "fixed", ln, side, (0.04, 0, 0), (0.1, 0.2, 0.3))
+            links.append(side)
+            specs.append((side, rng.normal(0, 0.01, (1, 3)), np.array([0.02]), False))
+    urdf = '<?xml version="1.0"?>\n<robot name="comb">\n' + "".join(synth._link(x) for x in links) + urdf + "</robot>\n"
+    return synth.Robot(urdf, joints, specs, [("l0", f"s{n - 1}")], np.full(n, -0.3), np.full(n, 0.3))
+
+
+def test_a_robot_whose_tables_do_not_fit_64_configurations():
+    from plainmp_amd.ompl import BoxMotionValidator
+
+    r = _comb()
+    Q = synth.uniform_configs(r, 70, 8)
+    wl = synth.Workload("comb", r, synth.mixed_primitives(6, 3), Q=Q)
+    oc, pc = oracle_cst(wl), product_cst(wl)
+    assert np.array_equal(pc.is_valid_batch(Q), oc.is_valid_batch(Q, 8).astype(bool))
+    assert np.abs(pc.evaluate_batch(Q)[0] - oc.evaluate_batch(Q, 8)[0]).max() <= 1e-5
+    dist, grad = pc.pair_clearance_batch(Q, True)
+    ref = oc.pair_clearance_batch(Q, True, 8)
+    assert np.abs(dist - ref).max() <= 1e-5  # 60 compositions: ten times the roundings of a 7-joint arm
+    assert np.array_equal(dist, pc.pair_clearance_batch(Q, False)[0])
+    h = 1e-5
+    for j in (0, 31, 59):
+        e = np.zeros(r.dof)
+        e[j] = h
+        up, dn = (oc.pair_clearance_batch(Q + k * e, True, 8) for k in (1, -1))
+        smooth = np.abs(up - 2 * ref + dn) < 1e-8
+        assert smooth.mean() > 0.95
+        assert np.abs(grad[..., j] - (up - dn) / (2 * h))[smooth].max() <= 1e-4
+    w = [0.05] * r.dof
+    ok, n_ok = oc.check_motions(Q[:-1], Q[1:], True, w, 0.0, 8)
+    got, n_got = BoxMotionValidator(pc, w).check_motions(Q[:-1], Q[1:])
+    assert np.array_equal(got, ok.astype(bool)) and np.array_equal(n_got, n_ok)
