@@ -8,9 +8,9 @@
 //
 // Bound by the latency of a motion's chain (endpoints, step ratio, states,
 // FK, tests).  Against a wave per motion that walks its states alone: 64
-// motions of the 7R arm a tenth of the joint range long 42 -> 28 us, 1,024 of
+// motions of the 7R arm a tenth of the joint range long 42 -> 17 us, 1,024 of
 // the 14-joint robot across the range 211 -> 115 us; 4,096 motions against a
-// 65,536-point cloud 1,036 -> 607 us (2,600 before when a state fell in the
+// 65,536-point cloud 1,036 -> 583 us (2,600 before when a state fell in the
 // band and its FP64 test walked every tile).
 #include <limits.h>
 
@@ -26,7 +26,7 @@ constexpr double kMaxEdgeStates = 16777216.0;
 // LDS offsets (floats), and the lanes a state gets at least (robots whose
 // tables do not fit 64 states).
 struct EdgeLds {
-  int scratch, flags, h_min;
+  int flags, h_min;
 };
 
 // State t of the way between the endpoints, which are staged as [2][D].
@@ -95,7 +95,7 @@ struct EdgeKernelArgs {
 
 // The FP32 items of states [base, base + 64 / H) of a motion.  Every thread
 // takes part; the results are complete on return.
-template <int H>
+template <bool kCloud, int H>
 __device__ __forceinline__ void edge_chunk(float* lds, const EdgeStates& es, int base, const ValidLds<true>& out,
                                            int* queue) {
   const EdgeKernelArgs& A = args_again<EdgeKernelArgs>();
@@ -126,17 +126,7 @@ __device__ __forceinline__ void edge_chunk(float* lds, const EdgeStates& es, int
     warm_scalar(sc.cull, sc.n_cull * (int)sizeof(CullEntry), part, parts);
   }
   __syncthreads();
-  const int n_ext = sc.n_prims == 0 ? 0 : sc.n_slices, n_items = n_ext + ka.n_pairs;
-  for (;;) {
-    int it = 0;
-    if (lane == 0) it = atomicAdd(queue, 1);
-    it = __builtin_amdgcn_readfirstlane(it);
-    if (it >= n_items) break;
-    if (it < n_ext)
-      valid_slice(S, ka, sc, cload(sc.slices, it), A.band, out, lds + A.el.scratch + w * 64 * kQueryWords);
-    else
-      valid_pair(S, ka, it - n_ext, A.band, out);
-  }
+  valid_items<kCloud>(S, ka, sc, A.band, out, queue);
   __syncthreads();
 }
 
@@ -151,6 +141,7 @@ __device__ __noinline__ bool edge_decide64(const EdgeKernelArgs* args, const Edg
                            [&](int i) { return es.at(A.ea, min(base + i, es.n_wp - 1)); }));
 }
 
+template <bool kCloud>
 __global__ void __launch_bounds__(1024) edges_staged_kernel(EdgeKernelArgs args) {
   HIP_DYNAMIC_SHARED(float, staged_lds)
   const int D = args.ka.n_cols, lane = threadIdx.x & 63;
@@ -198,13 +189,13 @@ __global__ void __launch_bounds__(1024) edges_staged_kernel(EdgeKernelArgs args)
           const int left = es.n_wp - base, h = max(el.h_min, left <= 8 ? 8 : (left <= 16 ? 4 : (left <= 32 ? 2 : 1)));
           const int C = 64 / h, cfg = lane & (C - 1);
           if (h == 1)
-            edge_chunk<1>(staged_lds, es, base, out, queue);
+            edge_chunk<kCloud, 1>(staged_lds, es, base, out, queue);
           else if (h == 2)
-            edge_chunk<2>(staged_lds, es, base, out, queue);
+            edge_chunk<kCloud, 2>(staged_lds, es, base, out, queue);
           else if (h == 4)
-            edge_chunk<4>(staged_lds, es, base, out, queue);
+            edge_chunk<kCloud, 4>(staged_lds, es, base, out, queue);
           else
-            edge_chunk<8>(staged_lds, es, base, out, queue);
+            edge_chunk<kCloud, 8>(staged_lds, es, base, out, queue);
           if (threadIdx.x < 64 && edge_decide64(&args_again<EdgeKernelArgs>(), es, base, C, out))
             redone = true;
           // only the first wave needs the last chunk's answer
@@ -242,17 +233,15 @@ hipError_t launch_edges_staged(const KinArgs<float>& k32, const KinArgs<double>&
   const int W = block > 0 ? block / 64 : (wide ? 8 : 4);
   for (el.h_min = 1;; el.h_min *= 2) {
     const StageLds L = stage_lds(k32, 64 / el.h_min);
-    const int need = s32.n_cloud > 0 ? W * kQueryWords * 64 : 0;
-    el.scratch = need <= 4 * k32.n_joints * 8 ? 0 : L.end;  // the joints' words again, if they are enough
-    el.flags = L.end + (el.scratch ? need : 0);
     const int keep = k64.slot_wave_bytes / (int)sizeof(float);  // one wave's FP64 kept poses
-    el.flags = (el.flags < keep ? keep : el.flags) + 1 & ~1;
+    el.flags = ((L.end < keep ? keep : L.end) + 1) & ~1;
     lds = sizeof(float) * (size_t)(el.flags + 64 + 4 + 3 * kPendMax + 4 * k32.n_cols);
     if (lds <= (size_t)k32.lds_limit) break;
     if (el.h_min == 8) return hipErrorInvalidConfiguration;  // 8 states of any robot fit
   }
   const int64_t most = waves > 0 ? (waves < W ? 1 : waves / W) : 1 << 20;
-  return launch_last(edges_staged_kernel, dim3((unsigned)(ea.E < most ? ea.E : most)), dim3(64 * W), lds, st,
+  return launch_last(s32.n_cloud > 0 ? edges_staged_kernel<true> : edges_staged_kernel<false>,
+                     dim3((unsigned)(ea.E < most ? ea.E : most)), dim3(64 * W), lds, st,
                      EdgeKernelArgs{k32, s32, k64, s64, ea, el, band});
 }
 

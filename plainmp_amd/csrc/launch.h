@@ -122,7 +122,7 @@ hipError_t launch_cloud_clearance(float* clearance, const float* d2, const float
 // the joint range: 7R arm, 512 45 and 61, 1,024 60 and 61, 2,048 93 and 62;
 // with self pairs, 14 joints, 1,024 119 and 211, 8,192 543 and 540, 32,768
 // 1,909 and 1,410; Fetch-like 1,024 95 and 181, 8,192 379 and 603.  With a
-// cloud its queries are answered by whole waves: 4,096 607 and 1,036.
+// cloud its queries are answered by whole waves: 4,096 583 and 1,036.
 inline bool edges_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, int64_t E) {
   return sc.n_cloud > 0 || E <= (ka.n_pairs > 0 ? 32 * kCus : 4 * kCus);
 }

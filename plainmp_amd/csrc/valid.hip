@@ -10,16 +10,18 @@ struct ValidOut {
   uint8_t* valid;
   int32_t* n_recheck;
   float band;
-  int scratch, flags;  // LDS offsets (floats)
+  int flags;  // LDS offset (floats)
 };
 
 // Bound by latency, like evaluate.  Against a launch with a lane per
 // configuration or per (configuration, block) and a second one re-deciding
 // whole configurations in FP64: 100,003 configurations of the Fetch-like robot
-// 263 -> 101 us (128 us of it the FP64 walks), 1,024 of the 7R arm 15.0 -> 11.5
-// us; 16,384 configurations against a 65,536-point cloud 92 -> 40 us (queries
+// 263 -> 93 us (128 us of it the FP64 walks), 1,024 of the 7R arm 15.0 -> 8.5
+// us; 16,384 configurations against a 65,536-point cloud 92 -> 31 us (queries
 // through memory, 98,304 waves and four launches before).
-template <int H>
+// kCloud: the scene holds clouds (their code costs the others registers: 97.5 us
+// instead of 94 for the 100,003).
+template <int H, bool kCloud>
 __global__ void __launch_bounds__(1024) valid_staged_kernel(KinArgs<float> ka, SceneArgs<float> sc, KinArgs<double> k64,
                                                             SceneArgs<double> s64, const double* q, int64_t ldq,
                                                             int64_t B, ValidOut o, StageLds lay) {
@@ -52,17 +54,7 @@ __global__ void __launch_bounds__(1024) valid_staged_kernel(KinArgs<float> ka, S
     warm_scalar(sc.cull, sc.n_cull * (int)sizeof(CullEntry), part, parts);
   }
   __syncthreads();
-  const int n_ext = sc.n_prims == 0 ? 0 : sc.n_slices, n_items = n_ext + ka.n_pairs;
-  for (;;) {
-    int it = 0;
-    if (lane == 0) it = atomicAdd(queue, 1);
-    it = __builtin_amdgcn_readfirstlane(it);
-    if (it >= n_items) break;
-    if (it < n_ext)
-      valid_slice(S, ka, sc, cload(sc.slices, it), o.band, out, staged_lds + o.scratch + w * 64 * kQueryWords);
-    else
-      valid_pair(S, ka, it - n_ext, o.band, out);
-  }
+  valid_items<kCloud>(S, ka, sc, o.band, out, queue);
   __syncthreads();
   if (w != 0) return;
   decide64(lane, cfg, S.sub, ka, k64, s64, taylor, active, out,
@@ -78,26 +70,25 @@ hipError_t launch_valid(const KinArgs<float>& k32, const KinArgs<double>& k64, c
                         const SceneArgs<double>& s64, const double* q, int64_t ldq, int64_t B, float band,
                         uint8_t* valid, int32_t* n_recheck, int, const CloudWork&, const CloudRange*, int, int32_t*,
                         int32_t*, hipStream_t st) {
-  ValidOut o{valid, n_recheck, band, 0, 0};
-  auto lds_of = [&](int H, int W) {
+  ValidOut o{valid, n_recheck, band, 0};
+  auto lds_of = [&](int H) {
     const int C = 64 / H;
     const StageLds L = stage_lds(k32, C);
-    const int need = s32.n_cloud > 0 ? W * kQueryWords * 64 : 0;
-    o.scratch = need <= L.poses ? 0 : L.end;  // the joints' words again, if they are enough
-    o.flags = L.end + (o.scratch ? need : 0);
+    o.flags = L.end;
     const int keep = k64.slot_wave_bytes / (int)sizeof(float);  // one wave's FP64 kept poses
     if (o.flags < keep) o.flags = keep;
     return sizeof(float) * (size_t)(o.flags + C + 2 + 3 * kPendMax);
   };
   StageShape sh = stage_shape(B, k32.n_units - k32.n_pairs);
-  while (sh.H < 8 && lds_of(sh.H, sh.W) > (size_t)k32.lds_limit) sh.H *= 2;
-  const size_t lds = lds_of(sh.H, sh.W);
+  while (sh.H < 8 && lds_of(sh.H) > (size_t)k32.lds_limit) sh.H *= 2;
+  const size_t lds = lds_of(sh.H);
   if (lds > (size_t)k32.lds_limit) return hipErrorInvalidConfiguration;  // 8 configurations of any robot fit
   const int C = 64 / sh.H;
   const StageLds lay = stage_lds(k32, C);
   const dim3 grid((unsigned)((B + C - 1) / C)), block(64 * sh.W);
 #define PMP_VALID(H) \
-  launch_last(valid_staged_kernel<H>, grid, block, lds, st, k32, s32, k64, s64, q, ldq, B, o, lay)
+  launch_last(s32.n_cloud > 0 ? valid_staged_kernel<H, true> : valid_staged_kernel<H, false>, grid, block, lds, st, \
+              k32, s32, k64, s64, q, ldq, B, o, lay)
   return sh.H == 1 ? PMP_VALID(1) : sh.H == 2 ? PMP_VALID(2) : sh.H == 4 ? PMP_VALID(4) : PMP_VALID(8);
 #undef PMP_VALID
 }

@@ -2,9 +2,9 @@
 // configurations and the motion check: what the waves of a workgroup do with
 // the staged poses.
 //
-// The waves take slices (a run of one sphere block's candidate primitives; the
-// block's first slice also takes the clouds) and self pairs from a queue and
-// test them in FP32.  A test decided outside the band marks the configuration
+// The waves take slices (a run of one sphere block's candidate primitives),
+// self pairs and, with clouds, a few spheres of a block from a queue and test
+// them in FP32.  A test decided outside the band marks the configuration
 // as colliding, and later items skip it; a test inside the band is put on the
 // workgroup's pending list as the one (sphere, primitive), (sphere, cloud) or
 // (sphere, sphere) pair it concerns.  At the end the first wave re-decides the
@@ -15,7 +15,7 @@
 // centres, a full pending list) is walked in FP64 whole.
 //
 // Sphere-vs-cloud queries (spheres inside the cloud's AABB pre-test) are
-// compacted by the wave and answered one at a time by all its lanes: 64
+// answered one at a time by all lanes of a wave: 64
 // super-tiles, then the tiles of four surviving super-tiles, then 64 points a
 // step, stopping at the first point certainly inside.
 #pragma once
@@ -32,7 +32,6 @@ namespace pmp {
 // it or a pending pair of it.
 enum ValidFlag { kHit = 1, kWhole = 2, kPended = 4 };
 constexpr int kPendMax = 64;     // pending pairs a workgroup keeps
-constexpr int kQueryWords = 6;   // a compacted query: centre, reach, sphere, configuration
 
 // The workgroup's results under way, in LDS.  kFirst: its configurations are
 // the states of one motion in visiting order and only the first colliding one
@@ -114,25 +113,28 @@ __device__ __forceinline__ int cloud_query(const SceneArgs<float>& sc, int oc, V
   return res;
 }
 
+// The cull table assumes |q|^2 of a rotation within [n2_lo, n2_hi] (so that
+// |R v| <= grow |v|), and with a finite translation no centre of such a rotation
+// is NaN; any other configuration is left to the FP64 walk.
+__device__ __forceinline__ bool sound_pose(const Pose<float>& P, float n2_lo, float n2_hi) {
+  const float n2 = P.q.x * P.q.x + P.q.y * P.q.y + P.q.z * P.q.z + P.q.w * P.q.w;
+  return n2 >= n2_lo && n2 <= n2_hi && fabsf(P.t.x) <= FLT_MAX && fabsf(P.t.y) <= FLT_MAX && fabsf(P.t.z) <= FLT_MAX;
+}
+
 // One slice of block candidates for the configurations still `live`.
 template <int H, bool kFirst>
 __device__ __forceinline__ void valid_slice(const Stage<H>& S, const KinArgs<float>& ka, const SceneArgs<float>& sc,
-                                            const DevCullSlice& it, float band, const ValidLds<kFirst>& out,
-                                            float* queries) {
+                                            const DevCullSlice& it, float band, const ValidLds<kFirst>& out) {
   constexpr int NK = Stage<H>::NK;
   bool live = (out.state(S.cfg) & (kHit | kWhole)) == 0;
   if (!wave_any(live)) return;
   const DevSphereBlock bk = cload(ka.blocks, it.block);
   const Pose<float> P = S.pose(bk.pose);
   const M3<float> R = qmat(P.q);
-  // The cull table assumes |q|^2 of this rotation within [n2_lo, n2_hi] (so
-  // that |R v| <= grow |v|), and with a finite translation no centre of such
-  // a rotation is NaN; any other configuration is left to the FP64 walk.
-  const float n2 = P.q.x * P.q.x + P.q.y * P.q.y + P.q.z * P.q.z + P.q.w * P.q.w;
-  const bool sound = n2 >= bk.n2_lo && n2 <= bk.n2_hi && fabsf(P.t.x) <= FLT_MAX && fabsf(P.t.y) <= FLT_MAX &&
-                     fabsf(P.t.z) <= FLT_MAX;
-  if (live && !sound) out.mark(S.cfg, kWhole);
-  live = live && sound;
+  if (live && !sound_pose(P, bk.n2_lo, bk.n2_hi)) {
+    out.mark(S.cfg, kWhole);
+    live = false;
+  }
   const float growf = 1.0f + 2.0f * fmaxf(0.0f, fmaxf(bk.n2_hi - 1.0f, 1.0f - bk.n2_lo)) + 1e-6f;
   const float reach = bk.G * growf + band + 1e-4f;
   V3<float> c[NK];
@@ -184,47 +186,53 @@ __device__ __forceinline__ void valid_slice(const Stage<H>& S, const KinArgs<flo
   kind(std::integral_constant<int, kKindCylRot>{});
   kind(std::integral_constant<int, kKindSphere>{});
   kind(std::integral_constant<int, kKindGround>{});
-  if (!it.first) return;
+}
+
+// Spheres [k0, k0 + kCloudSpheres) of each lane's share of a block against the
+// clouds: the lanes whose sphere is inside a cloud's AABB pre-test are answered
+// one at a time by all of them.
+// (4,096 motions 585 us with two spheres an item, 597 with four, 654 with eight
+// and 637 with one; 512 of the Fetch-like robot 117, 133, 133 and 104.)
+constexpr int kCloudSpheres = 2;
+template <int H, bool kFirst>
+__device__ __forceinline__ void valid_cloud(const Stage<H>& S, const KinArgs<float>& ka, const SceneArgs<float>& sc,
+                                            int block, int k0, float band, const ValidLds<kFirst>& out) {
+  constexpr int NK = Stage<H>::NK, G = NK < kCloudSpheres ? NK : kCloudSpheres;
+  bool live = (out.state(S.cfg) & (kHit | kWhole)) == 0;
+  if (!wave_any(live)) return;
+  const DevSphereBlock bk = cload(ka.blocks, block);
+  const Pose<float> P = S.pose(bk.pose);
+  if (live && !sound_pose(P, bk.n2_lo, bk.n2_hi)) {
+    out.mark(S.cfg, kWhole);
+    live = false;
+  }
+  const M3<float> R = qmat(P.q);
+  const int at = S.sub * NK + k0;
+  V3<float> c[G];
+  float r[G];
+#pragma unroll
+  for (int k = 0; k < G; ++k) {
+    const Quad4 s = reinterpret_cast<const Quad4*>(ka.blocks[block].s)[at + k];
+    c[k] = add(mv3(R, V3<float>{s.v[0], s.v[1], s.v[2]}), P.t);
+    r[k] = s.v[3];
+  }
   for (int p = sc.vrange[kKindCloud]; p < sc.vrange[kKindCloud + 1]; ++p) {
-    const DevPrim<float> Pc = cload(vp, p);
-    live = live && (out.state(S.cfg) & kHit) == 0;
-    if (!wave_any(live && !outside_aabb(Pc, g, reach))) continue;
-    int cnt = 0;  // queries collected, wave-uniform
-    auto flush = [&]() {
-      wave_lds_order();
-      for (int e = 0; e < cnt; ++e) {
-        const float* t = queries + e;
-        const int cfg = __builtin_amdgcn_readfirstlane(__float_as_int(t[320]));
+    const DevPrim<float> Pc = cload(reinterpret_cast<const DevPrim<float>*>(sc.vprims), p);
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+      const bool ask = live && at + k < bk.n && !outside_aabb(Pc, c[k], r[k]);
+      for (uint64_t m = __ballot(ask); m; m &= m - 1) {
+        const int i = __builtin_ctzll(m), cfg = i & (Stage<H>::C - 1);
         if (__builtin_amdgcn_readfirstlane(out.state(cfg)) & kHit) continue;
-        auto rd = [&](int at) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(t[at]))); };
-        const int res = cloud_query(sc, (Pc.flags >> 4) & 15, V3<float>{rd(0), rd(64), rd(128)}, rd(192), band, S.lane);
-        if (S.lane == 0) {
+        auto rd = [&](float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i)); };
+        const int res = cloud_query(sc, (Pc.flags >> 4) & 15, V3<float>{rd(c[k].x), rd(c[k].y), rd(c[k].z)},
+                                    rd(r[k]) + Pc.p0, band, S.lane);
+        if (S.lane == i) {
           if (res == 1) out.mark(cfg, kHit);
-          if (res == 2) out.defer(cfg, __float_as_int(t[256]), p);
+          if (res == 2) out.defer(cfg, ka.blocks[block].sph[at + k], p);
         }
       }
-      wave_lds_order();
-      cnt = 0;
-    };
-#pragma unroll
-    for (int k = 0; k < NK; ++k) {
-      const bool ask = live && k < n && !outside_aabb(Pc, c[k], r[k]);
-      const uint64_t m = __ballot(ask);
-      if (m == 0) continue;
-      const int more = __popcll(m);
-      if (cnt + more > 64) flush();
-      if (ask) {
-        float* t = queries + cnt + lane_rank(m);
-        t[0] = c[k].x;
-        t[64] = c[k].y;
-        t[128] = c[k].z;
-        t[192] = r[k] + Pc.p0;
-        t[256] = __int_as_float(sphere_of(k));
-        t[320] = __int_as_float(S.cfg);
-      }
-      cnt += more;
     }
-    if (cnt > 0) flush();
   }
 }
 
@@ -266,6 +274,28 @@ __device__ __forceinline__ void valid_pair(const Stage<H>& S, const KinArgs<floa
     }
   }
   if (hit) out.mark(S.cfg, kHit);
+}
+
+// The items of a workgroup: slices, self pairs, then some spheres of a block
+// against the clouds, whose configurations the cheaper tests may have decided.
+template <bool kCloud, int H, bool kFirst>
+__device__ __forceinline__ void valid_items(const Stage<H>& S, const KinArgs<float>& ka, const SceneArgs<float>& sc,
+                                            float band, const ValidLds<kFirst>& out, int* queue) {
+  constexpr int G = Stage<H>::NK < kCloudSpheres ? 1 : Stage<H>::NK / kCloudSpheres;  // cloud items of a block
+  const int n_ext = sc.n_prims == 0 ? 0 : sc.n_slices, n_solid = n_ext + ka.n_pairs;
+  const int n_items = n_solid + (kCloud ? (ka.n_units - ka.n_pairs) * G : 0);
+  for (;;) {
+    int it = 0;
+    if (S.lane == 0) it = atomicAdd(queue, 1);
+    it = __builtin_amdgcn_readfirstlane(it);
+    if (it >= n_items) break;
+    if (it < n_ext)
+      valid_slice(S, ka, sc, cload(sc.slices, it), band, out);
+    else if (!kCloud || it < n_solid)
+      valid_pair(S, ka, it - n_ext, band, out);
+    else if constexpr (kCloud)
+      valid_cloud(S, ka, sc, (it - n_solid) / G, (it - n_solid) % G * kCloudSpheres, band, out);
+  }
 }
 
 // A point cloud against one sphere in FP64, by the whole wave (uniform
