@@ -27,6 +27,7 @@ constexpr double kMaxEdgeStates = 16777216.0;
 // tables do not fit 64 states).
 struct EdgeLds {
   int flags, h_min;
+  bool sliced;
 };
 
 // State t of the way between the endpoints, which are staged as [2][D].
@@ -126,7 +127,7 @@ __device__ __forceinline__ void edge_chunk(float* lds, const EdgeStates& es, int
     warm_scalar(sc.cull, sc.n_cull * (int)sizeof(CullEntry), part, parts);
   }
   __syncthreads();
-  valid_items<kCloud>(S, ka, sc, A.band, out, queue);
+  valid_items<kCloud>(S, ka, sc, A.band, out, queue, A.el.sliced);
   __syncthreads();
 }
 
@@ -231,6 +232,7 @@ hipError_t launch_edges_staged(const KinArgs<float>& k32, const KinArgs<double>&
   // 1,024: 119 with 8, 144 with 4; 8,192: 544 with 4, 559 with 8)
   const bool wide = ea.E <= kCus || s32.n_cloud > 0 || (k32.n_pairs > 0 && ea.E <= 8 * kCus);
   const int W = block > 0 ? block / 64 : (wide ? 8 : 4);
+  el.sliced = slice_blocks(k32, W);
   for (el.h_min = 1;; el.h_min *= 2) {
     const StageLds L = stage_lds(k32, 64 / el.h_min);
     const int keep = k64.slot_wave_bytes / (int)sizeof(float);  // one wave's FP64 kept poses

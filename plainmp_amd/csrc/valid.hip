@@ -11,6 +11,7 @@ struct ValidOut {
   int32_t* n_recheck;
   float band;
   int flags;  // LDS offset (floats)
+  bool sliced;
 };
 
 // Bound by latency, like evaluate.  Against a launch with a lane per
@@ -54,7 +55,7 @@ __global__ void __launch_bounds__(1024) valid_staged_kernel(KinArgs<float> ka, S
     warm_scalar(sc.cull, sc.n_cull * (int)sizeof(CullEntry), part, parts);
   }
   __syncthreads();
-  valid_items<kCloud>(S, ka, sc, o.band, out, queue);
+  valid_items<kCloud>(S, ka, sc, o.band, out, queue, o.sliced);
   __syncthreads();
   if (w != 0) return;
   decide64(lane, cfg, S.sub, ka, k64, s64, taylor, active, out,
@@ -70,7 +71,7 @@ hipError_t launch_valid(const KinArgs<float>& k32, const KinArgs<double>& k64, c
                         const SceneArgs<double>& s64, const double* q, int64_t ldq, int64_t B, float band,
                         uint8_t* valid, int32_t* n_recheck, int, const CloudWork&, const CloudRange*, int, int32_t*,
                         int32_t*, hipStream_t st) {
-  ValidOut o{valid, n_recheck, band, 0};
+  ValidOut o{valid, n_recheck, band, 0, true};
   auto lds_of = [&](int H) {
     const int C = 64 / H;
     const StageLds L = stage_lds(k32, C);
@@ -81,6 +82,7 @@ hipError_t launch_valid(const KinArgs<float>& k32, const KinArgs<double>& k64, c
   };
   StageShape sh = stage_shape(B, k32.n_units - k32.n_pairs);
   while (sh.H < 8 && lds_of(sh.H) > (size_t)k32.lds_limit) sh.H *= 2;
+  o.sliced = slice_blocks(k32, sh.W);
   const size_t lds = lds_of(sh.H);
   if (lds > (size_t)k32.lds_limit) return hipErrorInvalidConfiguration;  // 8 configurations of any robot fit
   const int C = 64 / sh.H;

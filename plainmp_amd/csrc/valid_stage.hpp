@@ -276,21 +276,29 @@ __device__ __forceinline__ void valid_pair(const Stage<H>& S, const KinArgs<floa
   if (hit) out.mark(S.cfg, kHit);
 }
 
+// Whether a workgroup of W waves takes slices of the blocks' candidates or,
+// sparing the repeated set-up, whole blocks: slices while there are too few
+// blocks and self pairs to balance it.  (48 primitives: 7R arm, 8 blocks, 16,384
+// configurations with 16 waves 17.7 us by slices, 22.5 by blocks; 131,072 with 4
+// waves 60 and 57; 14 joints and self pairs, 16,384 42 and 38; Fetch-like, 16
+// primitives, 100,003 94 and 90; 1,024 motions of the 14-joint robot 96 and 90.)
+inline bool slice_blocks(const KinArgs<float>& ka, int W) { return ka.n_units < 2 * W; }
+
 // The items of a workgroup: slices, self pairs, then some spheres of a block
 // against the clouds, whose configurations the cheaper tests may have decided.
 template <bool kCloud, int H, bool kFirst>
 __device__ __forceinline__ void valid_items(const Stage<H>& S, const KinArgs<float>& ka, const SceneArgs<float>& sc,
-                                            float band, const ValidLds<kFirst>& out, int* queue) {
+                                            float band, const ValidLds<kFirst>& out, int* queue, bool sliced) {
   constexpr int G = Stage<H>::NK < kCloudSpheres ? 1 : Stage<H>::NK / kCloudSpheres;  // cloud items of a block
-  const int n_ext = sc.n_prims == 0 ? 0 : sc.n_slices, n_solid = n_ext + ka.n_pairs;
-  const int n_items = n_solid + (kCloud ? (ka.n_units - ka.n_pairs) * G : 0);
+  const int n_blocks = ka.n_units - ka.n_pairs, n_ext = sc.n_prims == 0 ? 0 : (sliced ? sc.n_slices : n_blocks);
+  const int n_solid = n_ext + ka.n_pairs, n_items = n_solid + (kCloud ? n_blocks * G : 0);
   for (;;) {
     int it = 0;
     if (S.lane == 0) it = atomicAdd(queue, 1);
     it = __builtin_amdgcn_readfirstlane(it);
     if (it >= n_items) break;
     if (it < n_ext)
-      valid_slice(S, ka, sc, cload(sc.slices, it), band, out);
+      valid_slice(S, ka, sc, sliced ? cload(sc.slices, it) : DevCullSlice{n_blocks - 1 - it, 0, INT_MAX, 0}, band, out);
     else if (!kCloud || it < n_solid)
       valid_pair(S, ka, it - n_ext, band, out);
     else if constexpr (kCloud)
