@@ -12,7 +12,7 @@ Two knobs decide how the persistent kernels map onto the MI355X:
   configurations, each taking its share of the (sphere, primitive) pairs.
 
 ``tune_edges``, ``tune_evaluate`` and ``tune_pairs`` time every candidate on
-the caller's own device buffers (HIP events around the edge kernel; stream
+the caller's own device buffers (the edge kernel's own clock; stream
 events around the evaluate and pair calls), keep the fastest, apply it to the constraint's context and
 record it in a JSON cache keyed by device name and workload signature, so a
 later run with the same workload applies the cached schedule without timing.
@@ -26,8 +26,8 @@ from typing import Dict, Iterable, Optional, Tuple
 
 import numpy as np
 
-EDGE_BLOCKS = (64, 128, 256)  # the edge kernel is built for workgroups of at most 256
-EDGE_WAVES_PER_CU = (4, 8, 12, 16, 20, 24, 32)
+EDGE_BLOCKS = (0, 64, 128, 256)  # 0: the launch's own choice
+EDGE_WAVES_PER_CU = (0, 4, 8, 12, 16, 20, 24, 32)
 EVAL_WHOLE_CHUNKS = (16, 32, 64, 128, 256, 512, 1024, 4096)
 PAIR_SHARES = (1, 2, 3, 4, 6, 8, 12, 16, 24, 32)
 

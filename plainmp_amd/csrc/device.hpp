@@ -121,10 +121,10 @@ struct alignas(16) Quad4 {
 };
 
 // One kept tile t of cloud_block_min: the spheres' minima over its points.
-template <bool kBounds, int NK>
+template <int NK>
 __device__ __forceinline__ void cloud_tile_min(const SceneArgs<float>& sc, int t, const CloudTile& T,
                                                const V3<float> (&c)[NK], int n,
-                                               float (&best)[NK], float (&lo)[NK]) {
+                                               float (&best)[NK]) {
   V3<float> cl[NK];
   float tb[NK];
 #pragma unroll
@@ -148,18 +148,8 @@ __device__ __forceinline__ void cloud_tile_min(const SceneArgs<float>& sc, int t
       }
     }
   }
-  const float rho2 = kBounds ? tile_rho2(T) : 0.f;
 #pragma unroll
-  for (int k = 0; k < NK; ++k) {
-    const float off = dot(cl[k], cl[k]);
-    if constexpr (kBounds) {
-      const float err = kCloudGemmErr * (off + rho2);
-      best[k] = fminf(best[k], tb[k] + off + err);
-      lo[k] = fminf(lo[k], tb[k] + off - err);
-    } else {
-      best[k] = fminf(best[k], tb[k] + off);
-    }
-  }
+  for (int k = 0; k < NK; ++k) best[k] = fminf(best[k], tb[k] + dot(cl[k], cl[k]));
 }
 
 // Per sphere k < n of a block, min |c_k - p|^2 over the points of cloud oc
@@ -169,16 +159,13 @@ __device__ __forceinline__ void cloud_tile_min(const SceneArgs<float>& sc, int t
 // first tested against the box around the live lanes' g, a box a lane, and
 // the survivors of that ballot are tested lane by lane.  A kept tile's points
 // are compared in tile-local coordinates, |c - p|^2 = |c'|^2 + (|p'|^2 -
-// 2 c'.p'), from the matrix-core pass's operands (-2 p', |p'|^2).  With
-// kBounds the minimum is bracketed: best = min over tiles of (d2 + err), lo =
-// min over tiles of (d2 - err), err = kCloudGemmErr (|c'|^2 + rho^2) of the
-// tile.
-template <bool kBounds, int NK>
+// 2 c'.p'), from the matrix-core pass's operands (-2 p', |p'|^2).
+template <int NK>
 __device__ __forceinline__ void cloud_block_min(const SceneArgs<float>& sc, int oc, const V3<float> (&c)[NK],
                                                 int n, V3<float> g, float reach2, bool live,
-                                                float (&best)[NK], float (&lo)[NK]) {
+                                                float (&best)[NK]) {
 #pragma unroll
-  for (int k = 0; k < NK; ++k) best[k] = lo[k] = FLT_MAX;
+  for (int k = 0; k < NK; ++k) best[k] = FLT_MAX;
   if (!wave_any(live)) return;
   const V3<float> gl{wave_minf(live ? g.x : FLT_MAX), wave_minf(live ? g.y : FLT_MAX), wave_minf(live ? g.z : FLT_MAX)};
   const V3<float> gu{wave_maxf(live ? g.x : -FLT_MAX), wave_maxf(live ? g.y : -FLT_MAX),
@@ -205,7 +192,7 @@ __device__ __forceinline__ void cloud_block_min(const SceneArgs<float>& sc, int 
           const int t = t0 + __builtin_ctzll(tmask);
           const CloudTile T = cload(sc.tiles, t);
           if (!wave_any(live && box_dist2(T.lb, T.ub, g) <= reach2)) continue;
-          cloud_tile_min<kBounds, NK>(sc, t, T, c, n, best, lo);
+          cloud_tile_min<NK>(sc, t, T, c, n, best);
         }
       }
     }

@@ -189,8 +189,8 @@ __device__ __forceinline__ void ext_slice(const Stage<H>& S, const KinArgs<float
     const uint32_t pkey = (uint32_t)(cload(sc.vorig, p) * ka.n_spheres);
     const float rc = Pc.p0;
     const float reach = bk.G * bk.n2_hi + rc + kCutoff + 1e-5f;
-    float d2[NK], unused[NK];
-    cloud_block_min<false, NK>(sc, (Pc.flags >> 4) & 15, c, n, g, all ? FLT_MAX : reach * reach, true, d2, unused);
+    float d2[NK];
+    cloud_block_min<NK>(sc, (Pc.flags >> 4) & 15, c, n, g, all ? FLT_MAX : reach * reach, true, d2);
 #pragma unroll
     for (int k = 0; k < NK; ++k)
       if (k < n && d2[k] != FLT_MAX && !outside_aabb(Pc, c[k], r[k] + kCutoff))

@@ -904,8 +904,8 @@ struct EvalUnitVis {
       const int orig = cload(sc.vorig, p);
       const float rc = Pc.p0;
       const float reach = bk.G * n2_hi + rc + kCutoff + 1e-5f;
-      float d2[kBlockSpheres], unused[kBlockSpheres];
-      cloud_block_min<false, kBlockSpheres>(sc, (Pc.flags >> 4) & 15, c, n, g, all ? FLT_MAX : reach * reach, true, d2, unused);
+      float d2[kBlockSpheres];
+      cloud_block_min<kBlockSpheres>(sc, (Pc.flags >> 4) & 15, c, n, g, all ? FLT_MAX : reach * reach, true, d2);
 #pragma unroll
       for (int k = 0; k < kBlockSpheres; ++k) {
         if (k < n) {

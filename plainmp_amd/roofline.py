@@ -138,8 +138,8 @@ def _counter_rows(path):
 
 def _kernel_base(name: str) -> str:
     """A kernel's name without return type, namespaces and argument list
-    (template arguments kept): 'void pmp::edges_kernel<false>(...)' ->
-    'edges_kernel<false>'."""
+    (template arguments kept): 'void pmp::eval_staged_kernel<8>(...)' ->
+    'eval_staged_kernel<8>'."""
     n = name.replace("(anonymous namespace)::", "")
     if n.startswith("void "):
         n = n[5:]
