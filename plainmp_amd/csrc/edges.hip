@@ -9,7 +9,7 @@
 // Bound by the latency of a motion's chain (endpoints, step ratio, states,
 // FK, tests).  Against a wave per motion that walks its states alone: 64
 // motions of the 7R arm a tenth of the joint range long 42 -> 17 us, 1,024 of
-// the 14-joint robot across the range 211 -> 115 us; 4,096 motions against a
+// the 14-joint robot across the range 211 -> 101 us; 4,096 motions against a
 // 65,536-point cloud 1,036 -> 583 us (2,600 before when a state fell in the
 // band and its FP64 test walked every tile).
 #include <limits.h>
@@ -27,7 +27,6 @@ constexpr double kMaxEdgeStates = 16777216.0;
 // tables do not fit 64 states).
 struct EdgeLds {
   int flags, h_min;
-  bool sliced;
 };
 
 // State t of the way between the endpoints, which are staged as [2][D].
@@ -127,7 +126,9 @@ __device__ __forceinline__ void edge_chunk(float* lds, const EdgeStates& es, int
     warm_scalar(sc.cull, sc.n_cull * (int)sizeof(CullEntry), part, parts);
   }
   __syncthreads();
-  valid_items<kCloud>(S, ka, sc, A.band, out, queue, A.el.sliced);
+  // whole blocks, or with clouds slices (of the solids beside them): a choice at
+  // run time spills 20 to 50 more registers (against a cloud 583 -> 830 us)
+  valid_items<kCloud>(S, ka, sc, A.band, out, queue, kCloud);
   __syncthreads();
 }
 
@@ -232,7 +233,6 @@ hipError_t launch_edges_staged(const KinArgs<float>& k32, const KinArgs<double>&
   // 1,024: 119 with 8, 144 with 4; 8,192: 544 with 4, 559 with 8)
   const bool wide = ea.E <= kCus || s32.n_cloud > 0 || (k32.n_pairs > 0 && ea.E <= 8 * kCus);
   const int W = block > 0 ? block / 64 : (wide ? 8 : 4);
-  el.sliced = slice_blocks(k32, W);
   for (el.h_min = 1;; el.h_min *= 2) {
     const StageLds L = stage_lds(k32, 64 / el.h_min);
     const int keep = k64.slot_wave_bytes / (int)sizeof(float);  // one wave's FP64 kept poses

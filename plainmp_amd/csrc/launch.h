@@ -119,9 +119,9 @@ hipError_t launch_cloud_clearance(float* clearance, const float* d2, const float
 // per motion) or edges_kernel (a wave per motion).  The staged form shortens a
 // motion's chain and shares its work; a wave per motion repeats less once the
 // motions alone fill the GPU.  Measured (us, staged and not), motions across
-// the joint range: 7R arm, 512 45 and 61, 1,024 60 and 61, 2,048 93 and 62;
-// with self pairs, 14 joints, 1,024 119 and 211, 8,192 543 and 540, 32,768
-// 1,909 and 1,410; Fetch-like 1,024 95 and 181, 8,192 379 and 603.  With a
+// the joint range: 7R arm, 512 32 and 61, 1,024 41 and 61, 2,048 (before its
+// last speed-ups) 93 and 62; with self pairs, 14 joints, 1,024 101 and 211,
+// 32,768 (before) 1,909 and 1,410; Fetch-like 1,024 80 and 181, 8,192 379 and 603.  With a
 // cloud its queries are answered by whole waves: 4,096 583 and 1,036.
 inline bool edges_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, int64_t E) {
   return sc.n_cloud > 0 || E <= (ka.n_pairs > 0 ? 32 * kCus : 4 * kCus);

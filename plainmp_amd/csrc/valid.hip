@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(1024) valid_staged_kernel(KinArgs<float> ka, S
     warm_scalar(sc.cull, sc.n_cull * (int)sizeof(CullEntry), part, parts);
   }
   __syncthreads();
-  valid_items<kCloud>(S, ka, sc, o.band, out, queue, o.sliced);
+  valid_items<kCloud>(S, ka, sc, o.band, out, queue, kCloud || o.sliced);
   __syncthreads();
   if (w != 0) return;
   decide64(lane, cfg, S.sub, ka, k64, s64, taylor, active, out,

@@ -289,9 +289,6 @@ inline bool slice_blocks(const KinArgs<float>& ka, int W) { return ka.n_units < 
 template <bool kCloud, int H, bool kFirst>
 __device__ __forceinline__ void valid_items(const Stage<H>& S, const KinArgs<float>& ka, const SceneArgs<float>& sc,
                                             float band, const ValidLds<kFirst>& out, int* queue, bool sliced) {
-  // with clouds always slices: the choice spills 20 more registers of the motion
-  // check (4,096 motions 583 -> 830 us)
-  if constexpr (kCloud) sliced = true;
   constexpr int G = Stage<H>::NK < kCloudSpheres ? 1 : Stage<H>::NK / kCloudSpheres;  // cloud items of a block
   const int n_blocks = ka.n_units - ka.n_pairs, n_ext = sc.n_prims == 0 ? 0 : (sliced ? sc.n_slices : n_blocks);
   const int n_solid = n_ext + ka.n_pairs, n_items = n_solid + (kCloud ? n_blocks * G : 0);
