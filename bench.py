@@ -9,8 +9,8 @@ replay of the persistent edge kernel.  Inputs are resident in HBM.
 counts them: the states checkMotion evaluates in its visiting order, up to
 and including each edge's first invalid state (the kernel reports this count
 per edge, exact).  The same line carries edges/s, the other workloads' rates,
-the roofline figures of the edge kernel (its duration from HIP events
-recorded around it on the stream, in direct launches of the same work) and the CPU baseline (the FP64 oracle on
+the roofline figures of the edge kernel (its duration by the device clock, in
+direct launches of the same work) and the CPU baseline (the FP64 oracle on
 this box's host cores, on a bounded sample, counted the same way).
 
 Usage: python bench.py [--gpus 1] [--steps K] [--warmup W]
@@ -103,7 +103,7 @@ def main():
     wall = time.perf_counter() - t0
     ms_step = ev0.elapsed_time(ev1) / args.steps
     # the edge kernel alone: the same launch made directly on the stream, with
-    # HIP events recorded around the kernel itself
+    # the kernel's own first start and last end
     kernel_ms = []
     for _ in range(max(args.steps, 5)):
         mv._dev_check_motions(s1.data_ptr(), s2.data_ptr(), E, E, valid.data_ptr(), nchk.data_ptr(), sh)
@@ -123,7 +123,7 @@ def main():
     n_wp_total = _total_waypoints(wl)
     wp_flops = roofline.waypoint_flops(wl.robot, wl.prims)
     achieved_tflops = checked * wp_flops / (kernel_ms * 1e-3) / 1e12
-    traffic, traffic_note = _traffic_per_launch("edges_kernel<false>")
+    traffic, traffic_note = _traffic_per_launch("edges_kernel")
 
     out = {
         "metric": "collision-checked configs/sec + Jacobian evals/sec on 1 MI355X vs plain GPU & CPU",
@@ -208,25 +208,6 @@ def _traffic_per_launch(kernel):
     if rec is None:
         return None, "kernel not in the traffic table"
     return rec.get("bytes_per_launch"), "profiles/traffic.json, this build's sources"
-
-
-def _matrix_cores(kernel):
-    """Matrix-core counters and rocprof duration of `kernel`'s largest grid
-    from the committed table, or None when it was measured on other kernel
-    sources than these."""
-    from plainmp_amd import roofline
-
-    path = os.path.join(ROOT, "profiles", "traffic.json")
-    if not os.path.exists(path):
-        return None
-    with open(path) as f:
-        table = json.load(f)
-    if table.get("_calibration", {}).get("sources_digest") != roofline.sources_digest():
-        return None
-    grids = table.get("_matrix_cores", {}).get(kernel)
-    if not grids:
-        return None
-    return grids[max(grids, key=int)]
 
 
 def _parity_headline(wl, got_valid, got_n):
@@ -339,7 +320,7 @@ def _extra(torch, stream, dev):
         "autotune": tune_pair,
     }
     rl = {}
-    rl["pair_kernel"] = {"workload": "grad_mixed32 pair distances + d/dq, 8192 configs", "bound": "hbm",
+    rl["pair_grad_kernel"] = {"workload": "grad_mixed32 pair distances + d/dq, 8192 configs", "bound": "hbm",
                          "achieved": bytes_out / (ms * 1e-3) / 1e9, "peak": roofline.PEAK_HBM_GBS, "unit": "GB/s",
                          "frac": bytes_out / (ms * 1e-3) / 1e9 / roofline.PEAK_HBM_GBS,
                          "bytes_per_launch": bytes_out, "launch_ms": ms,
@@ -362,7 +343,7 @@ def _extra(torch, stream, dev):
     res["grad_mixed32_evaluate"] = {"configs": B, "ms": ms, "jacobians_per_s": B / (ms * 1e-3),
                                     "autotune": tune_eval}
     ev_flops = roofline.evaluate_flops(wl.robot, wl.prims)
-    rl["eval_group_kernel"] = {"workload": "grad_mixed32 evaluate (value + row), 8192 configs", "bound": "valu",
+    rl["eval_staged_kernel"] = {"workload": "grad_mixed32 evaluate (value + row), 8192 configs", "bound": "valu",
                                "achieved": B * ev_flops / (ms * 1e-3) / 1e12, "peak": roofline.PEAK_FP32_VALU_TFLOPS,
                                "unit": "TFLOP/s", "frac": B * ev_flops / (ms * 1e-3) / 1e12 / roofline.PEAK_FP32_VALU_TFLOPS,
                                "flops_per_config": ev_flops, "launch_ms": ms}
@@ -391,7 +372,7 @@ def _extra(torch, stream, dev):
     res["traj_dual_arm_cost_grad"] = {"trajectories": T, "waypoints": N, "ms": ms,
                                       "waypoints_per_s": N / (ms * 1e-3), "trajectories_per_s": T / (ms * 1e-3)}
     tw = roofline.traj_waypoint_flops(wl.robot, wl.prims, synth.self_pair_count(wl.robot))
-    rl["eval_units_kernel"] = {"workload": "traj_dual_arm cost + gradient, 122138 waypoints", "bound": "valu",
+    rl["eval_staged_kernel_trajectories"] = {"workload": "traj_dual_arm cost + gradient, 122138 waypoints", "bound": "valu",
                                "achieved": N * tw / (ms * 1e-3) / 1e12, "peak": roofline.PEAK_FP32_VALU_TFLOPS,
                                "unit": "TFLOP/s", "frac": N * tw / (ms * 1e-3) / 1e12 / roofline.PEAK_FP32_VALU_TFLOPS,
                                "flops_per_waypoint": tw, "launch_ms": ms}
@@ -413,7 +394,7 @@ def _extra(torch, stream, dev):
                                     "note": "includes the evaluate rows of every waypoint (same launch as "
                                             "traj_dual_arm_cost_grad without the smoothness terms)"}
     # cloud_shelves: 16,384 configurations of an 8-DOF arm with 90 spheres against a
-    # 65,536-point cloud (sphere-vs-cloud distances on the matrix cores)
+    # 65,536-point cloud
     wl = synth.workload("cloud_shelves")
     cst = product_cst(wl)
     B = len(wl.Q)
@@ -425,24 +406,10 @@ def _extra(torch, stream, dev):
     res["cloud_shelves_is_valid"] = {
         "configs": B, "cloud_points": n_pts, "spheres": cst.n_spheres(), "ms": ms, "configs_per_s": B / (ms * 1e-3),
         "valid_frac": float(valid.float().mean().item()),
-        "note": "whole validity call (FP32 walk, matrix-core cloud pass, decisions, FP64 re-decisions); the "
-                "cloud kernel's matrix-core utilisation is measured with counters (profiles/)",
+        "note": "whole validity call, one launch (FP32 walk, cloud queries, decisions, FP64 re-decisions)",
     }
-    mc = _matrix_cores("cloud_min_kernel<true>")
-    if mc is not None:
-        flop = mc["mfma_f32_insts"] * roofline.MFMA_F32_16X16X4_FLOP
-        simd_cycles = roofline.N_SIMD * mc["duration_us"] * 1e-6 * roofline.CLOCK_GHZ * 1e9
-        rl["cloud_min_kernel"] = {
-            "workload": "cloud_shelves: 16,384 configs x 90 spheres vs 65,536 points", "bound": "mfma",
-            "achieved": flop / (mc["duration_us"] * 1e-6) / 1e12, "peak": roofline.PEAK_FP32_MFMA_TFLOPS,
-            "unit": "TFLOP/s", "frac": flop / (mc["duration_us"] * 1e-6) / 1e12 / roofline.PEAK_FP32_MFMA_TFLOPS,
-            "mfma_busy": mc["mfma_busy_cycles"] / simd_cycles, "mfma_insts": mc["mfma_f32_insts"],
-            "launch_us": mc["duration_us"],
-            "note": "executed matrix-core work (SQ_INSTS_VALU_MFMA_F32 x 2,048 flop) over the kernel's rocprof "
-                    "duration, and SQ_VALU_MFMA_BUSY_CYCLES over the launch's SIMD-cycles, from the counter "
-                    "runs of this build's sources (profiles/traffic.json); the kernel is bound by its culling"}
     # the same arm and cloud, 4,096 motions between consecutive configurations
-    # (box validator 0.05 rad): the cloud variant of the edge kernel
+    # (box validator 0.05 rad), a workgroup per motion
     from plainmp_amd.ompl import BoxMotionValidator
 
     E = 4096
