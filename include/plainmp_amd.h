@@ -75,7 +75,9 @@ typedef struct pmp_robot_desc {
   int32_t n_nodes;
   const int32_t* node_parent;        /* [n_nodes] parent node, -1 for the root          */
   const int32_t* node_kind;          /* [n_nodes] PMP_NODE_*                           */
-  const int32_t* node_q_col;         /* [n_nodes] column of q for joints, else -1       */
+  const int32_t* node_q_col;         /* [n_nodes] column of q for joints, else -1;
+                                        several joints may share one: its derivative
+                                        is the sum over them                           */
   const double* node_quat;           /* [n_nodes*4] local rotation x,y,z,w              */
   const double* node_trans;          /* [n_nodes*3] local translation                  */
   const double* node_axis;           /* [n_nodes*3] joint axis (not normalised)        */

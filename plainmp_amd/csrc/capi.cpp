@@ -768,7 +768,13 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
     std::vector<DevJoint> joints;
     std::vector<DevColumn> columns(n_q, DevColumn{{0.f, 0.f, 0.f}, -1});
     int n_poses = 0;
-    bool staged = true;
+    bool staged = true, shared = false;
+    std::vector<bool> driven(n_q, false);
+    for (int i = 1; i < N; ++i)
+      if (r->node_kind[i] == PMP_NODE_REVOLUTE || r->node_kind[i] == PMP_NODE_PRISMATIC) {
+        shared = shared || driven[r->node_q_col[i]];
+        driven[r->node_q_col[i]] = true;
+      }
     {
       std::vector<bool> has(N, false), below(N, false);
       std::vector<int> joint_of(N, -1);
@@ -800,10 +806,10 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
             j.q_col = r->node_q_col[i];
             j.identity = e.identity;
             j.revolute = e.kind == PMP_NODE_REVOLUTE;
+            j.pose = pose_of[i];
+            j.node = i;
             joints.push_back(j);
-            DevColumn& col = columns[j.q_col];
-            staged = staged && col.pose < 0;
-            col = {{e.axis[0], e.axis[1], e.axis[2]}, pose_of[i]};
+            columns[j.q_col] = {{e.axis[0], e.axis[1], e.axis[2]}, pose_of[i]};
           }
           e.joint = joint ? joint_of[i] : 0;
           path.push_back(e);
@@ -972,7 +978,7 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
     pk.add(path, &a.path, &d.path);
     std::vector<DevSphereRow> rows(S);
     for (int k = 0; k < S; ++k)
-      rows[meta[k].out] = {sp32[k].x, sp32[k].y, sp32[k].z, sp32[k].r, mask[meta[k].node], pose_of[meta[k].node], 0};
+      rows[meta[k].out] = {sp32[k].x, sp32[k].y, sp32[k].z, sp32[k].r, mask[meta[k].node], pose_of[meta[k].node], meta[k].node};
     pk.add(rows, &a.rows, &d.rows);
     pk.add(path_at, &a.path_at, &d.path_at);
     a.n_paths = d.n_paths = (int32_t)path_at.size() - 1;
@@ -982,6 +988,11 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
     pk.add(columns, &a.columns, &d.columns);
     a.n_joints = d.n_joints = (int32_t)joints.size();
     a.staged = d.staged = staged ? 1 : 0;
+    a.shared = d.shared = shared ? 1 : 0;
+    std::vector<uint32_t> above(shared ? (size_t)N * kNodeWords : 0, 0u);
+    for (int i = 0; shared && i < N; ++i)
+      for (int n = i; n >= 0; n = n == 0 ? -1 : r->node_parent[n]) above[i * kNodeWords + (n >> 5)] |= 1u << (n & 31);
+    pk.add(above, &a.above, &d.above);
     // evaluate units: one per sphere item, then one per self pair; and the whole configuration
     std::vector<DevEvalUnit> units;
     for (int b = 0; b < (int)blocks.size(); ++b) units.push_back({b, b + 1, 0, 0, block_node[b], {0, 0, 0}});

@@ -16,6 +16,11 @@ __device__ __forceinline__ DevPrim<T> prim_at(const SceneArgs<T>& sc, int p) {
   return cload(reinterpret_cast<const DevPrim<T>*>(sc.prims), p);
 }
 
+// Whether node a is n or above it (robots with ka.shared).
+__device__ __forceinline__ bool moves_node(const KinArgs<float>& ka, int a, int n) {
+  return (ka.above[n * kNodeWords + (a >> 5)] >> (a & 31)) & 1u;
+}
+
 __device__ __forceinline__ int64_t gid() { return (int64_t)blockIdx.x * blockDim.x + threadIdx.x; }
 
 // Squared distance from c to the box [lb, ub] (0 inside).

@@ -268,9 +268,10 @@ __device__ __forceinline__ void traj_cost(const StagedOut& o, const double* X, i
 // the 7R arm among 32 primitives 51 -> 22 us, 256 among two bars 28 -> 15 us,
 // each against a lane per configuration (a workgroup of 8 waves with a block
 // each, every wave walking FK again) before.
-template <int H>
-__global__ void __launch_bounds__(1024) eval_staged_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
-                                                           int64_t ldq, int64_t B, StagedOut o, StageLds lay) {
+// kShared: the robot's q columns drive several joints (ka.shared).
+template <int H, bool kShared>
+__device__ __forceinline__ void eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q,
+                                            int64_t ldq, int64_t B, const StagedOut& o, const StageLds& lay) {
   HIP_DYNAMIC_SHARED(float, staged_lds)
   const Stage<H> S(staged_lds, lay);
   constexpr int C = Stage<H>::C;
@@ -424,10 +425,40 @@ __global__ void __launch_bounds__(1024) eval_staged_kernel(KinArgs<float> ka, Sc
       if (!get_bit(at, j)) return V3<float>{0.f, 0.f, 0.f};
       return rev ? cross(a, sub(c, og)) : a;
     };
+    // the winners' nodes again from their keys
+    auto joints_col = [&](int node, V3<float> c) {
+      V3<float> r{0.f, 0.f, 0.f};
+      S.joint_columns(ka, node, c, [&](int at, V3<float> v) {
+        if (at == j) r = add(r, v);
+      });
+      return r;
+    };
     if (!active) continue;
-    if (NP > 0) o.jac[(int64_t)j * B + b] = dot(get3(3), col(6, get3(0)));
-    if (ka.n_pairs > 0)
-      o.jac[((NP > 0 ? (int64_t)D : 0) + j) * B + b] = dot(get3(14), sub(col(17, get3(8)), col(19, get3(11))));
+    const bool by_joint = kShared && j < ka.n_q_cols;
+    if (NP > 0) {
+      if (by_joint) {
+        const Best e = best[cfg];
+        float v = 0.f;
+        if (has_winner(e)) v = dot(get3(3), joints_col(ka.rows[(uint32_t)e % (uint32_t)ka.n_spheres].node, get3(0)));
+        o.jac[(int64_t)j * B + b] = v;
+      } else {
+        o.jac[(int64_t)j * B + b] = dot(get3(3), col(6, get3(0)));
+      }
+    }
+    if (ka.n_pairs > 0) {
+      float* row = o.jac + ((NP > 0 ? (int64_t)D : 0) + j) * B + b;
+      if (by_joint) {
+        const Best e = best[C + cfg];
+        float v = 0.f;
+        if (has_winner(e)) {
+          const DevSelfPair& pr = ka.pairs[(uint32_t)e >> (2 * kSelfPosBits)];
+          v = dot(get3(14), sub(joints_col(pr.node1, get3(8)), joints_col(pr.node2, get3(11))));
+        }
+        *row = v;
+      } else {
+        *row = dot(get3(14), sub(col(17, get3(8)), col(19, get3(11))));
+      }
+    }
     if (o.offsets) {
       // smoothness gradient: d cost / d x_t = 2 w^2 (a_{t-1} - 2 a_t + a_{t+1}),
       // terms of interior indices only; the differences in FP64 (they cancel)
@@ -440,6 +471,17 @@ __global__ void __launch_bounds__(1024) eval_staged_kernel(KinArgs<float> ka, Sc
       o.grad[(int64_t)j * B + b] = (float)(2.0 * o.w2[j] * g);
     }
   }
+}
+
+template <int H>
+__global__ void __launch_bounds__(1024) eval_staged_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
+                                                           int64_t ldq, int64_t B, StagedOut o, StageLds lay) {
+  eval_staged<H, false>(ka, sc, q, ldq, B, o, lay);
+}
+template <int H>
+__global__ void __launch_bounds__(1024) eval_shared_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
+                                                           int64_t ldq, int64_t B, StagedOut o, StageLds lay) {
+  eval_staged<H, true>(ka, sc, q, ldq, B, o, lay);
 }
 
 bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq, int64_t B,
@@ -457,6 +499,7 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   };
   StageShape sh = stage_shape(B, ka.n_units - ka.n_pairs);
   while (sh.H < 8 && lds_of(sh.H, sh.W) > (size_t)ka.lds_limit) sh.H *= 2;
+  if (ka.shared && sh.H > 1) sh.H = 8;
   const int H = sh.H, W = sh.W;
   const size_t lds = lds_of(H, W);
   if (lds > (size_t)ka.lds_limit) return false;
@@ -481,7 +524,10 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   *err = hipSuccess;
   if (grid.x > 0) {
 #define PMP_EVAL(H) *err = launch_last(eval_staged_kernel<H>, grid, block, lds, st, ka, sc, q, ldq, B, o, lay)
-    if (H == 1)
+    if (ka.shared)
+      *err = launch_last(H == 1 ? eval_shared_kernel<1> : eval_shared_kernel<8>, grid, block, lds, st, ka, sc, q, ldq, B,
+                         o, lay);
+    else if (H == 1)
       PMP_EVAL(1);
     else if (H == 2)
       PMP_EVAL(2);

@@ -777,14 +777,65 @@ struct Frames {
   }
 };
 
+// The same for robots with ka.shared: a column holds the sum over its joints
+// set so far, as J = A x c + M with A = sum a_k and M = sum o_k x a_k over the
+// rotating ones, M += a_k for the others.
+template <int MAXC>
+struct FrameSums {
+  float ax[MAXC] = {}, ay[MAXC] = {}, az[MAXC] = {}, mx[MAXC] = {}, my[MAXC] = {}, mz[MAXC] = {};
+  __device__ __forceinline__ void put(int col, V3<float> a, V3<float> m) {
+#pragma unroll
+    for (int j = 0; j < MAXC; ++j)
+      if (j == col) {
+        ax[j] += a.x;
+        ay[j] += a.y;
+        az[j] += a.z;
+        mx[j] += m.x;
+        my[j] += m.y;
+        mz[j] += m.z;
+      }
+  }
+  __device__ __forceinline__ void joint(int col, bool revolute, V3<float> a, V3<float> o) {
+    if (revolute)
+      put(col, a, cross(o, a));
+    else
+      put(col, V3<float>{0.f, 0.f, 0.f}, a);
+  }
+  template <class QS>
+  __device__ __forceinline__ void set_base(const KinArgs<float>& ka, const Pose<float>& base, const QS& qs) {
+    base_columns(ka, base, qs,
+                 [&](int col, V3<float> a, V3<float> o) { joint(col, (ka.rev_mask >> col) & 1ull, a, o); });
+  }
+  __device__ __forceinline__ V3<float> col(int j, uint64_t mask, uint64_t, V3<float> c) const {
+    V3<float> r{0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < MAXC; ++k)
+      if (k == j && ((mask >> k) & 1ull))
+        r = add(cross(V3<float>{ax[k], ay[k], az[k]}, c), V3<float>{mx[k], my[k], mz[k]});
+    return r;
+  }
+};
+
+// The joint frame of node n for a point of node `target`, in either form.
+template <int MAXC>
+__device__ __forceinline__ void joint_frame(Frames<MAXC>& fr, const KinArgs<float>&, int, int,
+                                            const DevNode<float>& nd, const Pose<float>& P) {
+  if (nd.q_col >= 0) fr.set(nd.q_col, qrot(P.q, V3<float>{nd.axis[0], nd.axis[1], nd.axis[2]}), P.t);
+}
+template <int MAXC>
+__device__ __forceinline__ void joint_frame(FrameSums<MAXC>& fr, const KinArgs<float>& ka, int n, int target,
+                                            const DevNode<float>& nd, const Pose<float>& P) {
+  if (nd.q_col >= 0 && moves_node(ka, n, target))
+    fr.joint(nd.q_col, nd.kind == PMP_NODE_REVOLUTE, qrot(P.q, V3<float>{nd.axis[0], nd.axis[1], nd.axis[2]}), P.t);
+}
+
 // ------------------------------------------------------------ evaluate rows
 // evaluate_ext_collision / evaluate_self_collision
 // (constraints/primitive_sphere_collision.cpp:256-383), a lane per
-// configuration: the form for robots whose tables do not fit a staged
-// workgroup (eval.hip) or that drive two joints with one q column.  A unit is
-// a range of sphere blocks (the external minimum over their spheres x every
-// primitive, in the reference's (group, primitive, sphere) key order) and of
-// self group pairs (minimum over their sphere pairs in visiting order).
+// configuration: the form for robots beyond the staged form's limits (eval.hip).
+// A unit is a range of sphere blocks (the external minimum over their spheres x
+// every primitive, in the reference's (group, primitive, sphere) key order) and
+// of self group pairs (minimum over their sphere pairs in visiting order).
 template <int MAXC>
 struct EvalUnitVis {
   static constexpr bool kSelf = true;
@@ -958,33 +1009,38 @@ struct EvalRowAccVis {
   int last = 0;  // wave-uniform
   V3<float> c0{0.f, 0.f, 0.f}, c1{0.f, 0.f, 0.f}, c2{0.f, 0.f, 0.f}, g0{0.f, 0.f, 0.f}, n{0.f, 0.f, 0.f};
   uint64_t m0 = 0, m1 = 0, m2 = 0;  // column masks of the winners' nodes (0: no winner)
+  int n0 = 0, n1 = 0, n2 = 0;       // and the nodes
   float re[MAXC], rs[MAXC];
   __device__ bool alive() const { return true; }
   __device__ int last_node() const { return last; }
   __device__ int pair_lo() const { return 0; }
   __device__ int pair_hi() const { return 0; }
-  __device__ __forceinline__ void column(int col, V3<float> a, V3<float> o) {
-    const bool rev = (ka.rev_mask >> col) & 1ull;
+  // node: the joint's, -1: a base column
+  __device__ __forceinline__ void column(int node, int col, bool rev, V3<float> a, V3<float> o) {
     auto cv = [&](V3<float> c) { return rev ? cross(a, sub(c, o)) : a; };
-    const float ve = ((m0 >> col) & 1ull) ? dot(g0, cv(c0)) : 0.f;
-    const float v1 = ((m1 >> col) & 1ull) ? dot(n, cv(c1)) : 0.f;
-    const float v2 = ((m2 >> col) & 1ull) ? dot(n, cv(c2)) : 0.f;
+    auto moves = [&](uint64_t m, int target) {
+      return ((m >> col) & 1ull) && (!ka.shared || node < 0 || moves_node(ka, node, target));
+    };
+    const float ve = moves(m0, n0) ? dot(g0, cv(c0)) : 0.f;
+    const float v1 = moves(m1, n1) ? dot(n, cv(c1)) : 0.f;
+    const float v2 = moves(m2, n2) ? dot(n, cv(c2)) : 0.f;
 #pragma unroll
     for (int j = 0; j < MAXC; ++j)
       if (j == col) {
-        re[j] = ve;
-        rs[j] = v1 - v2;
+        re[j] += ve;
+        rs[j] += v1 - v2;
       }
   }
   template <class QS>
   __device__ void begin(const Pose<float>& base, const QS& qs) {
 #pragma unroll
     for (int j = 0; j < MAXC; ++j) re[j] = rs[j] = 0.f;
-    base_columns(ka, base, qs, [&](int col, V3<float> a, V3<float> o) { column(col, a, o); });
+    base_columns(ka, base, qs,
+                 [&](int col, V3<float> a, V3<float> o) { column(-1, col, (ka.rev_mask >> col) & 1ull, a, o); });
   }
-  __device__ void node(int, const DevNode<float>& nd, const Pose<float>& P) {
+  __device__ void node(int n, const DevNode<float>& nd, const Pose<float>& P) {
     if (nd.q_col < 0) return;
-    column(nd.q_col, qrot(P.q, V3<float>{nd.axis[0], nd.axis[1], nd.axis[2]}), P.t);
+    column(n, nd.q_col, nd.kind == PMP_NODE_REVOLUTE, qrot(P.q, V3<float>{nd.axis[0], nd.axis[1], nd.axis[2]}), P.t);
   }
   __device__ void sphere(int, V3<float>, float) {}
   __device__ void blocks(const DevNode<float>&, const Pose<float>&) {}
@@ -1059,6 +1115,7 @@ __device__ __forceinline__ void eval_finish_whole(const KinArgs<float>& ka, cons
     need = node0;
     rv.c0 = v.bc;
     rv.m0 = cload(ka.nodes, node0).col_mask;
+    rv.n0 = node0;
     const DevPrim<float> P = prim_at(sc, v.bidx % kMaxPrims);
     if (P.type == PMP_PRIM_CLOUD) {
       // the gradient of sqrt(min |c - p|^2) at the nearest point, which the
@@ -1079,6 +1136,8 @@ __device__ __forceinline__ void eval_finish_whole(const KinArgs<float>& ka, cons
     rv.n = scale(1.0f / sqrtf(dot(d, d)), d);
     rv.m1 = cload(ka.nodes, n1).col_mask;
     rv.m2 = cload(ka.nodes, n2).col_mask;
+    rv.n1 = n1;
+    rv.n2 = n2;
   }
   // lanes of the wave that reach this point walk together (inactive lanes
   // have returned); no winner in the wave: the rows are zero without FK
@@ -1123,11 +1182,11 @@ __global__ void __launch_bounds__(64) eval_units_kernel(KinArgs<float> ka, Scene
 // of every node up to the link, then a_j x (p - o_j) (or a_j) for the columns
 // that move it (KinematicModel::get_jacobian / get_attached_point_jacobian,
 // kinematics/algorithm.cpp:212-433).
-template <int MAXC>
+template <int MAXC, class Fr>
 struct LinkJacVis {
   static constexpr bool kSelf = false;
   const KinArgs<float>& ka;
-  Frames<MAXC> fr;
+  Fr fr;
   int target;
   V3<float> off;
   V3<float> p{0.f, 0.f, 0.f};
@@ -1138,7 +1197,7 @@ struct LinkJacVis {
   template <class QS>
   __device__ void begin(const Pose<float>& base, const QS& qs) { fr.set_base(ka, base, qs); }
   __device__ void node(int n, const DevNode<float>& nd, const Pose<float>& P) {
-    if (nd.q_col >= 0) fr.set(nd.q_col, qrot(P.q, V3<float>{nd.axis[0], nd.axis[1], nd.axis[2]}), P.t);
+    joint_frame(fr, ka, n, target, nd, P);
     if (n == target) {
       p = add(qrot(P.q, off), P.t);
       lp = P;
@@ -1150,14 +1209,13 @@ struct LinkJacVis {
   __device__ void self(const DevSelfPair&, int, int, V3<float>, V3<float>, float) {}
 };
 
-template <int MAXC>
-__global__ void __launch_bounds__(256) link_jac_kernel(KinArgs<float> ka, const double* q, int64_t ldq, int64_t B,
-                                                       int target, float ox, float oy, float oz, float* jac,
-                                                       float* pose) {
+template <int MAXC, class Fr>
+__device__ __forceinline__ void link_jac(const KinArgs<float>& ka, const double* q, int64_t ldq, int64_t B, int target,
+                                         float ox, float oy, float oz, float* jac, float* pose) {
   const int64_t b = gid();
   const bool active = b < B;
   BatchQ qs{q, ldq, active ? b : B - 1};
-  LinkJacVis<MAXC> v{ka, {}, target, V3<float>{ox, oy, oz}};
+  LinkJacVis<MAXC, Fr> v{ka, {}, target, V3<float>{ox, oy, oz}};
   run_fk(ka, qs, false, v);
   if (!active) return;
   const int D = ka.n_cols;
@@ -1177,17 +1235,30 @@ __global__ void __launch_bounds__(256) link_jac_kernel(KinArgs<float> ka, const 
   }
 }
 
+template <int MAXC>
+__global__ void __launch_bounds__(256) link_jac_kernel(KinArgs<float> ka, const double* q, int64_t ldq, int64_t B,
+                                                       int target, float ox, float oy, float oz, float* jac,
+                                                       float* pose) {
+  link_jac<MAXC, Frames<MAXC>>(ka, q, ldq, B, target, ox, oy, oz, jac, pose);
+}
+template <int MAXC>
+__global__ void __launch_bounds__(256) link_jac_shared_kernel(KinArgs<float> ka, const double* q, int64_t ldq,
+                                                              int64_t B, int target, float ox, float oy, float oz,
+                                                              float* jac, float* pose) {
+  link_jac<MAXC, FrameSums<MAXC>>(ka, q, ldq, B, target, ox, oy, oz, jac, pose);
+}
+
 // Reverse mode: per sphere the upstream weights of its primitive distances
 // are folded into one world-space force g = sum_p w_p grad sdf_p(c); each
 // q column then receives g . (a_j x (c - o_j)) (or g . a_j).  Each
 // (configuration, item) lane writes its partial column sums; a second pass
 // adds the items in a fixed order.
-template <int MAXC>
+template <int MAXC, class Fr>
 struct VjpVis {
   static constexpr bool kSelf = false;
   const KinArgs<float>& ka;
   const SceneArgs<float>& sc;
-  Frames<MAXC> fr;
+  Fr fr;
   const float* gd;
   int64_t B, b;
   DevSphereItem it;
@@ -1199,8 +1270,7 @@ struct VjpVis {
   __device__ void begin(const Pose<float>& base, const QS& qs) { fr.set_base(ka, base, qs); }
   __device__ void node(int n, const DevNode<float>& nd, const Pose<float>& P) {
     if (n == it.node) done = true;
-    if (nd.q_col < 0) return;
-    fr.set(nd.q_col, qrot(P.q, V3<float>{nd.axis[0], nd.axis[1], nd.axis[2]}), P.t);
+    joint_frame(fr, ka, n, it.node, nd, P);
   }
   __device__ void sphere(int s, V3<float> c, float) {
     if (s < it.begin || s >= it.end) return;
@@ -1227,18 +1297,18 @@ struct VjpVis {
   __device__ void self(const DevSelfPair&, int, int, V3<float>, V3<float>, float) {}
 };
 
-template <int MAXC>
-__global__ void __launch_bounds__(256) vjp_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
-                                                  int64_t ldq, int64_t B, const float* gd, float* part) {
+template <int MAXC, class Fr>
+__device__ __forceinline__ void vjp(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq,
+                                    int64_t B, const float* gd, float* part) {
   const int64_t b = gid();
   const bool active = b < B;
   const int64_t bb = active ? b : B - 1;
   BatchQ qs{q, ldq, bb};
-  // grid z splits the primitives into shares, as in pair_kernel; each
-  // (item, share) writes its own partial column sums
+  // grid z splits the primitives into shares; each (item, share) writes its
+  // own partial column sums
   const int p_per = (sc.n_prims + (int)gridDim.z - 1) / (int)gridDim.z;
   const int p_lo = (int)blockIdx.z * p_per, p_hi = min(sc.n_prims, p_lo + p_per);
-  VjpVis<MAXC> v{ka, sc, {}, gd, B, bb, cload(ka.items, blockIdx.y), p_lo, p_hi};
+  VjpVis<MAXC, Fr> v{ka, sc, {}, gd, B, bb, cload(ka.items, blockIdx.y), p_lo, p_hi};
 #pragma unroll
   for (int j = 0; j < MAXC; ++j) v.acc[j] = 0.f;
   run_fk(ka, qs, false, v);
@@ -1248,6 +1318,17 @@ __global__ void __launch_bounds__(256) vjp_kernel(KinArgs<float> ka, SceneArgs<f
 #pragma unroll
   for (int j = 0; j < MAXC; ++j)
     if (j < D) part[(part_row * D + j) * B + b] = v.acc[j];
+}
+
+template <int MAXC>
+__global__ void __launch_bounds__(256) vjp_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
+                                                  int64_t ldq, int64_t B, const float* gd, float* part) {
+  vjp<MAXC, Frames<MAXC>>(ka, sc, q, ldq, B, gd, part);
+}
+template <int MAXC>
+__global__ void __launch_bounds__(256) vjp_shared_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
+                                                         int64_t ldq, int64_t B, const float* gd, float* part) {
+  vjp<MAXC, FrameSums<MAXC>>(ka, sc, q, ldq, B, gd, part);
 }
 
 // Sum of the n_parts partial column sums (items x shares, in that order:
@@ -1491,8 +1572,13 @@ hipError_t launch_link_jacobian(const KinArgs<float>& ka, const double* q, int64
                                 const float (&off)[3], float* jac, float* pose, hipStream_t st) {
   if (B > 0) {
     const int bk = slot_block(ka, 256);
-    PMP_DISPATCH_MAXC(ka.n_cols, link_jac_kernel, dim3(blocks_for(B, bk)), dim3(bk), slot_bytes(ka, bk), st, ka, q,
-                      ldq, B, link, off[0], off[1], off[2], jac, pose);
+    const dim3 grid(blocks_for(B, bk));
+    if (ka.shared)
+      PMP_DISPATCH_MAXC(ka.n_cols, link_jac_shared_kernel, grid, dim3(bk), slot_bytes(ka, bk), st, ka, q, ldq, B, link,
+                        off[0], off[1], off[2], jac, pose);
+    else
+      PMP_DISPATCH_MAXC(ka.n_cols, link_jac_kernel, grid, dim3(bk), slot_bytes(ka, bk), st, ka, q, ldq, B, link, off[0],
+                        off[1], off[2], jac, pose);
   }
   return hipGetLastError();
 }
@@ -1550,8 +1636,11 @@ hipError_t launch_vjp(const KinArgs<float>& ka, const SceneArgs<float>& sc, cons
   const int nz = vjp_shares(ka, sc.n_prims, B, shares);
   if (ka.n_items > 0) {
     const int bk = slot_block(ka, 256);
-    PMP_DISPATCH_MAXC(ka.n_cols, vjp_kernel, dim3(blocks_for(B, bk), (unsigned)ka.n_items, (unsigned)nz), dim3(bk),
-                      slot_bytes(ka, bk), st, ka, sc, q, ldq, B, gd, part);
+    const dim3 grid(blocks_for(B, bk), (unsigned)ka.n_items, (unsigned)nz);
+    if (ka.shared)
+      PMP_DISPATCH_MAXC(ka.n_cols, vjp_shared_kernel, grid, dim3(bk), slot_bytes(ka, bk), st, ka, sc, q, ldq, B, gd, part);
+    else
+      PMP_DISPATCH_MAXC(ka.n_cols, vjp_kernel, grid, dim3(bk), slot_bytes(ka, bk), st, ka, sc, q, ldq, B, gd, part);
   }
   return launch_last(vjp_reduce_kernel, dim3(blocks_for((int64_t)ka.n_cols * B, 256)), dim3(256), 0, st, part,
                      ka.n_items * nz, ka.n_cols, B, grad_q);

@@ -167,10 +167,11 @@ __global__ void __launch_bounds__(512) pair_dist_kernel(KinArgs<float> ka, Scene
 // link) before); 256-byte pieces of rows alone take 94 us on this card, a
 // plain fill 73 us.  With rows off the cache lines (8,191 configurations) 142
 // us; 277 us with streaming stores and neighbouring chunks on different XCDs.
-template <int H, int MAXC, bool kStream>
-__global__ void __launch_bounds__(256) pair_grad_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
-                                                        int64_t ldq, int64_t B, float* dist, float* grad, int n_slices,
-                                                        int chunks, StageLds lay) {
+// kShared: the robot's q columns drive several joints (ka.shared).
+template <int H, int MAXC, bool kStream, bool kShared>
+__device__ __forceinline__ void pair_grad(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q,
+                                          int64_t ldq, int64_t B, float* dist, float* grad, int n_slices, int chunks,
+                                          const StageLds& lay) {
   HIP_DYNAMIC_SHARED(float, staged_lds)
   const Stage<H> S(staged_lds, lay);
   int share, chunk;
@@ -201,8 +202,15 @@ __global__ void __launch_bounds__(256) pair_grad_kernel(KinArgs<float> ka, Scene
           V3<float> a, o;
           staged_frame<Stage<H>::C>(frames, j0 + j, cfg, a, o);
           J[j] = ((ka.rev_mask >> (j0 + j)) & 1ull) ? cross(a, sub(c, o)) : a;
+          if (kShared && j0 + j < ka.n_q_cols) J[j] = {0.f, 0.f, 0.f};
         }
       }
+      if constexpr (kShared)
+        S.joint_columns(ka, row.node, c, [&](int col, V3<float> v) {
+#pragma unroll
+          for (int j = 0; j < MAXC; ++j)
+            if (j0 + j == col) J[j] = add(J[j], v);
+        });
       const int p_end = (int)((int64_t)NP * (sl + 1) / n_slices);
       for (int p = (int)((int64_t)NP * sl / n_slices); p < p_end; ++p) {
         const DevPrim<float> Q = prim_at(sc, p);
@@ -225,6 +233,19 @@ __global__ void __launch_bounds__(256) pair_grad_kernel(KinArgs<float> ka, Scene
   }
 }
 
+template <int H, int MAXC, bool kStream>
+__global__ void __launch_bounds__(256) pair_grad_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
+                                                        int64_t ldq, int64_t B, float* dist, float* grad, int n_slices,
+                                                        int chunks, StageLds lay) {
+  pair_grad<H, MAXC, kStream, false>(ka, sc, q, ldq, B, dist, grad, n_slices, chunks, lay);
+}
+template <int H>
+__global__ void __launch_bounds__(256) pair_grad_shared_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
+                                                               int64_t ldq, int64_t B, float* dist, float* grad,
+                                                               int n_slices, int chunks, StageLds lay) {
+  pair_grad<H, 16, false, true>(ka, sc, q, ldq, B, dist, grad, n_slices, chunks, lay);
+}
+
 constexpr int64_t kPairWorkgroups = 16 * kCus;
 
 hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q, int64_t ldq,
@@ -237,6 +258,7 @@ hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
     return sizeof(float) * (size_t)(stage_lds(ka, 64 / H).end + (grad ? 6 * ka.n_cols * (64 / H) : 0));
   };
   while (H < 8 && lds_of(H) > (size_t)ka.lds_limit) H *= 2;
+  if (grad && ka.shared && H > 1) H = 8;
   const size_t lds = lds_of(H);
   if (lds > (size_t)ka.lds_limit) return hipErrorInvalidConfiguration;  // 8 configurations of any robot fit
   const StageLds lay = stage_lds(ka, 64 / H);
@@ -259,6 +281,9 @@ hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
 #define PMP_GRAD(H, MAXC, STREAM)                                                                                     \
   launch_last(pair_grad_kernel<H, MAXC, STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, grad, n_slices,       \
               (int)chunks, lay)
+  if (grad && ka.shared)
+    return launch_last(H == 1 ? pair_grad_shared_kernel<1> : pair_grad_shared_kernel<8>, grid, block, lds, st, ka, sc, q,
+                       ldq, B, dist, grad, n_slices, (int)chunks, lay);
   if (H == 2) return grad ? PMP_GRAD(2, 16, false) : PMP_DIST(2, false);
   if (H == 4) return grad ? PMP_GRAD(4, 16, false) : PMP_DIST(4, false);
   if (H == 8) return grad ? PMP_GRAD(8, 16, false) : PMP_DIST(8, false);

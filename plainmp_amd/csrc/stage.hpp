@@ -223,6 +223,19 @@ struct Stage {
     return true;
   }
 
+  // f(column, its derivative at point c of node `node`) for every joint that
+  // moves the node (robots whose q columns drive several joints).
+  template <class F>
+  __device__ __forceinline__ void joint_columns(const KinArgs<float>& ka, int node, V3<float> c, F&& f) const {
+    for (int i = 0; i < ka.n_joints; ++i) {
+      const DevJoint jt = cload(ka.joints, i);
+      if (!moves_node(ka, jt.node, node)) continue;
+      const Pose<float> P = pose(jt.pose);
+      const V3<float> a = qrot(P.q, V3<float>{jt.axis[0], jt.axis[1], jt.axis[2]});
+      f(jt.q_col, jt.revolute ? cross(a, pmp::sub(c, P.t)) : a);
+    }
+  }
+
   // The n (at most NK) spheres of block bk this lane takes: centres and radii.
   __device__ __forceinline__ void spheres(const KinArgs<float>& ka, int bi, const DevSphereBlock& bk,
                                           const Pose<float>& P, const M3<float>& R, V3<float> (&c)[NK],

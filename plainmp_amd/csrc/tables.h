@@ -13,6 +13,7 @@ namespace pmp {
 constexpr int kMaxSlots = 32;     // live poses kept during FK (LDS; the device's LDS may allow fewer)
 constexpr int kMaxCols = 64;      // q columns (joints + base)
 constexpr int kMaxNodes = 256;
+constexpr int kNodeWords = kMaxNodes / 32;  // a set of nodes
 constexpr int kMaxSpheres = 4096;
 constexpr int kMaxPrims = 512;
 constexpr int kMaxSelfPairs = 1024;
@@ -108,7 +109,8 @@ static_assert(sizeof(DevPathNode) == 64, "a path entry is one cache line");
 struct alignas(16) DevJoint {
   float quat[4];  // origin rotation
   float axis[3];
-  int32_t q_col, identity, revolute, pad[2];
+  int32_t q_col, identity, revolute;
+  int32_t pose, node;  // its pose-table index, its node
 };
 // The joint frame of a q column: pose-table index of its node (-1: the column
 // moves no sphere, or belongs to the base) and the axis in that frame.
@@ -121,7 +123,7 @@ struct alignas(16) DevColumn {
 struct alignas(32) DevSphereRow {
   float x, y, z, r;
   uint64_t col_mask;  // q columns that move it
-  int32_t pose, pad;  // pose-table index of its node
+  int32_t pose, node;  // its node, and that one's pose-table index
 };
 
 // A slice of a sphere block's candidates: cull entries [lo, hi) of block
@@ -206,7 +208,12 @@ struct KinArgs {
   const DevColumn* columns;  // [n_q_cols]
   const DevSphereRow* rows;  // [n_spheres], group order
   int32_t n_paths, n_path_entries, n_poses, n_joints;
-  int32_t staged;  // the staged tables describe this robot (no q column drives two joints)
+  int32_t staged;  // evaluate's self keys hold this robot's groups
+  // Robots whose q columns each drive one joint have one joint frame a column.
+  // The others (two fingers on one column, coupled joints of a chain) take the
+  // sum over the column's joints at or above a point's node.
+  int32_t shared;            // some q column drives several joints
+  const uint32_t* above;     // shared: [n_nodes][kNodeWords], bit a of row n: node a is n or above it
   T base_q[4];
   T base_t[3];
 };
