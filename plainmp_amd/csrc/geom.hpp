@@ -14,6 +14,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <float.h>
 #include <math.h>
 #include <stdint.h>
 
@@ -416,15 +417,18 @@ __device__ __forceinline__ V3<float> mv3(const M3<float>& R, V3<float> v) {
 // root: one Newton step for the reciprocal (about half an ulp, where a
 // correctly rounded root and division make up to one), and the root's residual
 // through it (Markstein), which rounds correctly but for rare last-place ties.
-// sqrt(0) = 0; the reciprocal of 0 is finite.
+// sqrt(0) = 0 and sqrt(inf) = inf, as a NaN's root is NaN; the reciprocal of 0
+// is finite, that of infinity and (its step is NaN) of NaN 0.  Below FLT_MIN
+// (points within 1e-19 m) the root is too small.
 __device__ __forceinline__ void root_and_reciprocal(float x, float& s, float& inv) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  float r = __builtin_amdgcn_rsqf(fmaxf(x, 1e-36f));
+  float r = __builtin_amdgcn_rsqf(fmaxf(x, FLT_MIN));
   const float h = 0.5f * r;
   r = fmaf(fmaf(-x * r, r, 1.0f), h, r);
-  inv = r;
+  inv = fmaxf(r, 0.0f);
   s = x * r;
   s = fmaf(fmaf(-s, s, x), 0.5f * r, s);
+  s = x > FLT_MAX ? x : s;
 #else
   s = sqrtf(x);  // host pass: never executed, only type-checked
   inv = 1.0f / s;
@@ -434,7 +438,9 @@ __device__ __forceinline__ void root_and_reciprocal(float x, float& s, float& in
 // sdf_eval_kind<K> and (kGrad) sdf_grad of an FP32 primitive together
 // (clouds excluded): the local coordinates and roots are shared, the roots
 // cost a third of correctly rounded ones, and a cylinder's gradient is formed
-// from its local coordinates.
+// from its local coordinates.  Infinite and NaN coordinates and points on a
+// kink go the way they do there: a NaN term counts as 0, a zero coordinate as
+// positive, and where no direction is defined the gradient's part is 0.
 template <int K, bool kGrad>
 __device__ __forceinline__ void sdf_value_grad(const DevPrim<float>& p, V3<float> c, float& dist, V3<float>& g) {
   const V3<float> dc = sub(c, V3<float>{p.pos[0], p.pos[1], p.pos[2]});
@@ -445,14 +451,14 @@ __device__ __forceinline__ void sdf_value_grad(const DevPrim<float>& p, V3<float
     const float top = fmaxf(fmaxf(sx, sy), sz);
     float root, inv;
     root_and_reciprocal(mx * mx + my * my + mz * mz, root, inv);
-    dist = root + fminf(top, 0.0f);
+    dist = root + fmaxf(fmaxf(fminf(sx, 0.0f), fminf(sy, 0.0f)), fminf(sz, 0.0f));
     if constexpr (kGrad) {
       V3<float> l{mx * inv, my * inv, mz * inv};
       if (!(top > 0.0f)) {  // inside: the nearest face
         l = {sx >= sy && sx >= sz ? 1.0f : 0.0f, 0.0f, 0.0f};
         if (l.x == 0.0f) l = {0.0f, sy >= sz ? 1.0f : 0.0f, sy >= sz ? 0.0f : 1.0f};
       }
-      l = {copysignf(l.x, d.x), copysignf(l.y, d.y), copysignf(l.z, d.z)};
+      l = {d.x < 0.0f ? -l.x : l.x, d.y < 0.0f ? -l.y : l.y, d.z < 0.0f ? -l.z : l.z};
       g = K == kKindBoxRot ? mv3(load_m3(p.R), l) : l;
     }
   } else if constexpr (K == kKindCylZ || K == kKindCylRot) {
@@ -468,21 +474,22 @@ __device__ __forceinline__ void sdf_value_grad(const DevPrim<float>& p, V3<float
     const float o0 = fmaxf(rs, 0.0f), o1 = fmaxf(zs, 0.0f);
     const float top = fmaxf(rs, zs);
     root_and_reciprocal(sum2sq(o0, o1), root, inv);
-    dist = root + fminf(top, 0.0f);
+    dist = root + fmaxf(fminf(rs, 0.0f), fminf(zs, 0.0f));
     if constexpr (kGrad) {
       float wr = o0 * inv, wz = o1 * inv;
       if (!(top > 0.0f)) {
         wr = rs > zs ? 1.0f : 0.0f;
         wz = 1.0f - wr;
       }
-      const float k = wr * inv_rho, gx = k * x, gy = k * y, gz = copysignf(wz, z);
+      const float k = wr * inv_rho, gz = z < 0.0f ? -wz : wz;
+      const float gx = rho > 0.0f ? k * x : 0.0f, gy = rho > 0.0f ? k * y : 0.0f;
       g = K == kKindCylRot ? mv3(load_m3(p.R), V3<float>{gx, gy, gz}) : V3<float>{gx, gy, gz};
     }
   } else if constexpr (K == kKindSphere) {
     float root, inv;
     root_and_reciprocal(dot3(dc, dc), root, inv);
     dist = root - p.p0;
-    if constexpr (kGrad) g = scale(inv, dc);
+    if constexpr (kGrad) g = root > 0.0f ? scale(inv, dc) : V3<float>{0.0f, 0.0f, 0.0f};
   } else {  // ground
     dist = c.z + p.p0;
     if constexpr (kGrad) g = {0.0f, 0.0f, 1.0f};

@@ -1,0 +1,85 @@
+"""Pair distances and gradients far out and where no direction is defined (GPU).
+
+The distance is that of the primitives' formulas in FP32: infinite beyond the
+square root of the largest float, and a NaN coordinate's terms count as 0 (every
+comparison with them is false)."""
+
+import numpy as np
+import pytest
+
+from cabi_robot import Balls, Context, Robot
+from plainmp_amd import synth
+from support import product_cst
+
+pytestmark = pytest.mark.gpu
+
+_R = synth._rot_rpy(0.3, -0.5, 0.9)
+PRIMS = {
+    "box": {"type": "box", "width": np.array([0.2, 0.3, 0.4]), "position": np.array([0.5, 0.1, 0.4]), "rotation": np.eye(3)},
+    "box_rot": {"type": "box", "width": np.array([0.2, 0.3, 0.4]), "position": np.array([0.5, 0.1, 0.4]), "rotation": _R},
+    "cylinder": {"type": "cylinder", "radius": 0.1, "height": 0.8, "position": np.array([0.5, 0.1, 0.4]), "rotation": np.eye(3)},
+    "cylinder_rot": {"type": "cylinder", "radius": 0.1, "height": 0.8, "position": np.array([0.5, 0.1, 0.4]), "rotation": _R},
+    "sphere": {"type": "sphere", "radius": 0.1, "position": np.array([0.5, 0.1, 0.4]), "rotation": np.eye(3)},
+    "ground": {"type": "ground", "height": 0.1},
+}
+VALUES = [0.3, 1e3, 1e15, 3e19, -3e19, 1e30, -1e30, np.inf, -np.inf, np.nan]
+
+
+def _distance(p, c):
+    """The formula in FP32 (c [..., 3] FP32 centres)."""
+    f = np.float32
+    pos = lambda x: np.where(x > 0, x, f(0))
+    neg = lambda x: np.where(x < 0, x, f(0))
+    if p["type"] == "ground":
+        return c[..., 2] + f(p["height"])
+    d = c - np.asarray(p["position"], f)
+    if p["type"] == "sphere":
+        return np.sqrt((d * d).sum(-1)) - f(p["radius"])
+    if not np.array_equal(p["rotation"], np.eye(3)):
+        R = np.asarray(p["rotation"], f)
+        d = d[..., 0, None] * R[0] + d[..., 1, None] * R[1] + d[..., 2, None] * R[2]
+    if p["type"] == "box":
+        s = np.abs(d) - np.asarray(p["width"], f) / 2
+    else:
+        rho = np.sqrt(d[..., 0] ** 2 + d[..., 1] ** 2)
+        s = np.stack([rho - f(p["radius"]), np.abs(d[..., 2]) - f(p["height"] / 2)], -1)
+    return np.sqrt((pos(s) ** 2).sum(-1)) + neg(s).max(-1)
+
+
+@pytest.mark.parametrize("kind", sorted(PRIMS))
+def test_far_and_nan_bases(kind):
+    from plainmp_amd.kinematics import BaseType
+
+    r, prim = synth.panda_like(0), PRIMS[kind]
+    Q = np.zeros((2 * len(VALUES) + 1, r.dof + 3))
+    Q[:, : r.dof] = synth.uniform_configs(r, len(Q), 1)
+    for i, v in enumerate(VALUES):
+        Q[i, r.dof] = v
+        Q[len(VALUES) + i, r.dof + 1] = v
+    Q[-1, r.dof:r.dof + 2] = 3e19, -3e19
+    pc = product_cst(synth.Workload("far", r, [prim]), base_type=BaseType.PLANAR)
+    radii = -pc.pair_clearance_batch(Q[:1], False)[0][0, :, 0] + _distance(prim, pc.sphere_centers_batch(Q[:1], True)[0])
+    dist, grad = pc.pair_clearance_batch(Q, True)
+    with np.errstate(all="ignore"):
+        ref = _distance(prim, pc.sphere_centers_batch(Q, True)) - radii
+    got = dist[..., 0]
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.isinf(got), np.isinf(ref))
+    ok = np.isfinite(ref)
+    # a few roundings of the largest of the numbers involved
+    assert (np.abs(got[ok] - ref[ok]) <= 1e-6 * np.maximum(1.0, np.abs(ref[ok]))).all()
+    # a translation of the base changes a distance by at most as much, also where
+    # the distance is infinite (a cylinder's radial part is then inf / inf)
+    finite = np.isfinite(Q).all(axis=1)
+    if prim["type"] == "cylinder":
+        finite &= np.isfinite(got).all(axis=1)
+    assert (np.abs(grad[finite][..., r.dof:r.dof + 2]) <= 1 + 1e-5).all()
+
+
+def test_centre_on_centre():
+    """A sphere at a ball's very centre: the distance is minus both radii and no
+    direction is preferred."""
+    robot = Robot([(-1, 0, -1, (0, 0, 0), (0, 0, 0)), (0, 2, 0, (0, 0, 0.5), (0, 0, 1))], [(1, (0, 0, 0), 0.1, 0)], 1)
+    dist, grad = Context(robot, Balls([((0, 0, 0.5), 0.2)])).pairs(np.array([[0.0], [0.7]]))
+    assert np.abs(dist - -0.3).max() <= 1e-7
+    assert np.array_equal(grad, np.zeros_like(grad))
