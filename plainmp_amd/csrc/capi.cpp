@@ -748,6 +748,10 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
     std::vector<DevSphere<float>> sp32(S);
     std::vector<DevSphere<double>> sp64(S);
     std::vector<DevSphereMeta> meta(S);
+    // groups by their rank among those that hold spheres: the tie keys of
+    // evaluate stay below n_spheres^2 n_prims whatever ids the caller uses
+    std::vector<int> group_rank(S, 0);
+    for (int s = 1; s < S; ++s) group_rank[s] = group_rank[s - 1] + (r->sphere_group[s] != r->sphere_group[s - 1]);
     int n_ext = 0;
     for (int k = 0; k < S; ++k) {
       const int s = order[k];
@@ -756,7 +760,7 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
       sp64[k] = {l[0], l[1], l[2], r->sphere_radius[s]};
       const int g = r->sphere_group[s];
       const bool ext = !(r->group_only_self && r->group_only_self[g]);
-      meta[k] = {s, ext ? n_ext : -1, r->sphere_node[s], g};
+      meta[k] = {s, ext ? n_ext : -1, r->sphere_node[s], group_rank[s]};
       n_ext += ext;
     }
     // Staged kernels' paths: one from the root to every sphere-carrying node

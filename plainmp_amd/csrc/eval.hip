@@ -65,7 +65,8 @@ __device__ __forceinline__ float bound_of(const Best* best) {
 }
 
 // Keys: external (group * n_prims + primitive) * n_spheres + sphere (group
-// order); self: pair, then the spheres' positions in their groups.
+// order; fewer groups than spheres, so below n_spheres^2 n_prims); self: pair,
+// then the spheres' positions in their groups.
 constexpr int kSelfPosBits = 11;
 
 // Entries a wave collects before it evaluates them: the sphere's centre and
@@ -96,7 +97,9 @@ __device__ __forceinline__ void ext_slice(const Stage<H>& S, const KinArgs<float
   S.spheres(ka, it.block, bk, P, R, c, r, n);
   // a sphere's part of the key: kept per lane with H > 1, else read when
   // wanted (eight more scalar registers would be spilled)
-  auto sphere_key = [&](int group, int out) { return (uint32_t)(group * sc.n_prims * ka.n_spheres + out); };
+  auto sphere_key = [&](int group, int out) {
+    return (uint32_t)group * (uint32_t)sc.n_prims * (uint32_t)ka.n_spheres + (uint32_t)out;
+  };
   if constexpr (H > 1) {
 #pragma unroll
     for (int k = 0; k < NK; ++k) {
@@ -135,7 +138,7 @@ __device__ __forceinline__ void ext_slice(const Stage<H>& S, const KinArgs<float
       // every member sphere's value is at least the bounding centre's
       // distance minus the block's reach (the SDFs are 1-Lipschitz)
       if (!all && !wave_any(sdf_may_reach<K>(Q, g, bound + ereach))) continue;
-      const uint32_t pkey = (uint32_t)(orig * ka.n_spheres);
+      const uint32_t pkey = (uint32_t)orig * (uint32_t)ka.n_spheres;
       int cnt = 0;  // entries collected, wave-uniform
       auto flush = [&]() {
         wave_lds_order();
@@ -186,7 +189,7 @@ __device__ __forceinline__ void ext_slice(const Stage<H>& S, const KinArgs<float
   if (!it.first) return;
   for (int p = sc.vrange[kKindCloud]; p < sc.vrange[kKindCloud + 1]; ++p) {
     const DevPrim<float> Pc = cload(vp, p);
-    const uint32_t pkey = (uint32_t)(cload(sc.vorig, p) * ka.n_spheres);
+    const uint32_t pkey = (uint32_t)cload(sc.vorig, p) * (uint32_t)ka.n_spheres;
     const float rc = Pc.p0;
     const float reach = bk.G * bk.n2_hi + rc + kCutoff + 1e-5f;
     float d2[NK];
@@ -525,8 +528,8 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   if (grid.x > 0) {
 #define PMP_EVAL(H) *err = launch_last(eval_staged_kernel<H>, grid, block, lds, st, ka, sc, q, ldq, B, o, lay)
     if (ka.shared)
-      *err = launch_last(H == 1 ? eval_shared_kernel<1> : eval_shared_kernel<8>, grid, block, lds, st, ka, sc, q, ldq, B,
-                         o, lay);
+      *err = launch_last(H == 1 ? eval_shared_kernel<1> : eval_shared_kernel<8>, grid, block, lds, st, ka, sc, q, ldq,
+                         B, o, lay);
     else if (H == 1)
       PMP_EVAL(1);
     else if (H == 2)

@@ -845,7 +845,8 @@ struct EvalUnitVis {
   const SceneArgs<float>& sc;
   DevEvalUnit u{};
   float best = kCutoff, sbest = kCutoff;
-  int bkey = 0x7fffffff, bidx = -1, sidx = -1;
+  int64_t bkey = INT64_MAX;  // beyond 32 bits for the robots that come here
+  int bidx = -1, sidx = -1;
   V3<float> bc{0.f, 0.f, 0.f}, sc1{0.f, 0.f, 0.f}, sc2{0.f, 0.f, 0.f};  // the winners' world centres
   float ereach = 0.0f;  // the current block's bounding radius, grown, plus a slack
   __device__ bool alive() const { return true; }
@@ -892,7 +893,7 @@ struct EvalUnitVis {
           if (outside_aabb(P, c[k], r + kCutoff)) continue;
           const float v = sdf_eval_kind<K>(P, c[k]) - r;
           if (v <= best) {  // a new best, or a tie that the visiting order settles
-            const int key = (m[k].group * sc.n_prims + orig) * ka.n_spheres + m[k].out;
+            const int64_t key = ((int64_t)m[k].group * sc.n_prims + orig) * ka.n_spheres + m[k].out;
             if (v < best || (bidx >= 0 && key < bkey)) {
               best = v;
               bkey = key;
@@ -963,7 +964,7 @@ struct EvalUnitVis {
           const float r = bk.s[k][3];
           if (d2[k] == FLT_MAX || outside_aabb(Pc, c[k], r + kCutoff)) continue;
           const float v = sqrtf(d2[k]) - rc - r;
-          const int key = (m[k].group * sc.n_prims + orig) * ka.n_spheres + m[k].out;
+          const int64_t key = ((int64_t)m[k].group * sc.n_prims + orig) * ka.n_spheres + m[k].out;
           if (v < best || (bidx >= 0 && v == best && key < bkey)) {
             best = v;
             bkey = key;

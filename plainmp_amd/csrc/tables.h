@@ -144,7 +144,7 @@ struct alignas(16) DevSphereMeta {
   int32_t out;    // index in SphereCollisionCst group order
   int32_t ext;    // index among the spheres checked against primitives, -1 for only-self groups
   int32_t node;
-  int32_t group;
+  int32_t group;  // its group's rank among those with spheres
 };
 
 // Point-cloud tile: AABB and centre (FP32, for culling and the local frame of
