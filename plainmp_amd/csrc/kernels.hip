@@ -1446,6 +1446,7 @@ hipError_t launch_edges(const KinArgs<float>& k32, const KinArgs<double>& k64, c
   kw.slot_wave_bytes = k64.slot_wave_bytes;
   const size_t lds = slot_bytes(k64, block);
   hipLaunchKernelGGL(edges_kernel, dim3(grid), dim3(block), lds, st, kw, s32, k64, s64, ea, band);
+  if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   const unsigned rgrid = (unsigned)(ea.E < kRecheckGrid ? ea.E : kRecheckGrid);
   const int rblock = slot_block(k64, 64 * kRecheckWaves, sizeof(int));
   return launch_last(edges_recheck_kernel, dim3(rgrid), dim3(rblock), slot_bytes(k64, rblock), st, k64, s64, ea);
@@ -1642,6 +1643,7 @@ hipError_t launch_vjp(const KinArgs<float>& ka, const SceneArgs<float>& sc, cons
       PMP_DISPATCH_MAXC(ka.n_cols, vjp_shared_kernel, grid, dim3(bk), slot_bytes(ka, bk), st, ka, sc, q, ldq, B, gd, part);
     else
       PMP_DISPATCH_MAXC(ka.n_cols, vjp_kernel, grid, dim3(bk), slot_bytes(ka, bk), st, ka, sc, q, ldq, B, gd, part);
+    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   }
   return launch_last(vjp_reduce_kernel, dim3(blocks_for((int64_t)ka.n_cols * B, 256)), dim3(256), 0, st, part,
                      ka.n_items * nz, ka.n_cols, B, grad_q);

@@ -22,7 +22,8 @@ inline hipError_t launch_with_stop(void (*kernel)(P...), dim3 grid, dim3 block, 
   return hipExtLaunchKernel((const void*)kernel, grid, block, ptrs, lds, st, nullptr, stop, 0);
 }
 
-// The last kernel of a call.
+// The last kernel of a call.  Its own status is returned; a launcher with
+// kernels before it asks for theirs first.
 template <class... P, class... A>
 inline hipError_t launch_last(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t st, A&&... a) {
   if (!call_end.ask) {
