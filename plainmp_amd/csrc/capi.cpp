@@ -117,14 +117,12 @@ class TablePack {
 // cannot change what a replay reads.
 struct EdgeBufs {
   DevBuf width, inv_width, pend, counter;
-  int32_t slot = 0;                // EdgeArgs::slot of the last launch
+  int32_t slot = 0;  // EdgeArgs::slot of the last direct launch
   bool launched = false;
-  int32_t count_at = kCntRecheck;  // the counter that holds the last launch's FP64 decisions
   std::vector<double> h_width;  // what width / inv_width hold, so a repeated call uploads nothing
   void release() {
     for (DevBuf* b : {&width, &inv_width, &pend, &counter}) b->release();
     h_width.clear();
-    count_at = kCntRecheck;
     launched = false;
   }
 };
@@ -254,9 +252,11 @@ void set_device(pmp_context* ctx) {
 }
 hipStream_t st(pmp_context* ctx) { return ctx->stream; }
 // Lets the launcher called next end the call with its last kernel; for entry
-// points that enqueue nothing after it.
-void ends_call(pmp_context* ctx) {
-  if (!capturing(ctx->stream)) call_end.ask = ctx->call_ev;
+// points that enqueue nothing after it.  False while the stream is captured.
+bool ends_call(pmp_context* ctx) {
+  if (capturing(ctx->stream)) return false;
+  call_end.ask = ctx->call_ev;
+  return true;
 }
 
 // The stream a graph is captured on and replayed on: the context stream, or
@@ -982,7 +982,8 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
     pk.add(path, &a.path, &d.path);
     std::vector<DevSphereRow> rows(S);
     for (int k = 0; k < S; ++k)
-      rows[meta[k].out] = {sp32[k].x, sp32[k].y, sp32[k].z, sp32[k].r, mask[meta[k].node], pose_of[meta[k].node], meta[k].node};
+      rows[meta[k].out] = {sp32[k].x, sp32[k].y, sp32[k].z, sp32[k].r, mask[meta[k].node],
+                           pose_of[meta[k].node], meta[k].node};
     pk.add(rows, &a.rows, &d.rows);
     pk.add(path_at, &a.path_at, &d.path_at);
     a.n_paths = d.n_paths = (int32_t)path_at.size() - 1;
@@ -1637,26 +1638,16 @@ void prepare_edges(pmp_context* ctx, const double* s1, const double* s2, int64_t
   const bool fresh = eb.counter.bytes < sizeof(int32_t) * words;  // new buffer
   ea.counter = (int32_t*)eb.counter.get(sizeof(int32_t) * words);
   if (fresh) PMP_HIP(launch_fill_i32(ea.counter, 0, (int64_t)words, st(ctx)));
-  ea.clock = edge_clocks(eb);
-  if (E > 0) {
-    ea.slot = eb.slot ^= 1;
-    eb.launched = true;
-  }
-  if (E > 0 && edges_staged(ctx->k32, ctx->s32, E)) {
-    eb.count_at = kCntStaged + ea.slot;
-    ea.valid = valid;
-    ea.n_checked = n_checked;
-    return;
-  }
-  if (E > 0) eb.count_at = kCntRecheck;
+  ea.slot = 1 - eb.slot;  // the last direct launch cleared what this one adds to
+  ea.valid = valid;
+  ea.n_checked = n_checked;
+  if (E > 0 && edges_staged(ctx->k32, ctx->s32, E)) return;
   const int64_t Ea = std::max<int64_t>(E, 1);
   int32_t* pend = (int32_t*)eb.pend.get(sizeof(int32_t) * Ea * (3 * kPendStates + 3));
   ea.pend = pend;
   ea.pend_info = pend + Ea * kPendStates;
   ea.plist = pend + Ea * (kPendStates + 2);
   ea.pend_pair = pend + Ea * (kPendStates + 3);
-  ea.valid = valid;
-  ea.n_checked = n_checked;
 }
 
 // Persistent grid: waves_per_cu waves on every CU (default 16, four per
@@ -1692,8 +1683,20 @@ pmp_status pmp_check_edges_batch(pmp_context* ctx, const double* s1, const doubl
     if (E == 0) return;
     int grid, block;
     edge_grid(ctx, E, grid, block);
-    ends_call(ctx);
+    const bool direct = ends_call(ctx);
+    if (direct) {
+      ea.clock = edge_clocks(ctx->eb);
+    } else {
+      // replays run between direct calls, in no order the host knows
+      ea.slot = kEdgeSlots - 1;
+      if (edges_staged(ctx->k32, ctx->s32, E))
+        PMP_HIP(launch_fill_i32(ea.counter + kCntRecheck, 0, kNumEdgeCounters - kCntRecheck, st(ctx)));
+    }
     PMP_HIP(launch_edges(ctx->k32, ctx->k64, ctx->s32, ctx->s64, ea, ctx->band, grid, block, st(ctx)));
+    if (direct) {
+      ctx->eb.slot = ea.slot;
+      ctx->eb.launched = true;
+    }
   });
 }
 
@@ -1758,9 +1761,11 @@ pmp_status pmp_edge_recheck_count(pmp_context* ctx, int32_t* n) {
     PMP_REQUIRE(ctx != nullptr && n != nullptr, "null argument");
     PMP_REQUIRE(ctx->eb.counter.ptr != nullptr, "no edge batch has run on this context");
     set_device(ctx);
-    PMP_HIP(hipMemcpyAsync(n, (const int32_t*)ctx->eb.counter.ptr + ctx->eb.count_at, sizeof(int32_t),
-                           hipMemcpyDeviceToHost, st(ctx)));
+    int32_t c[kNumEdgeCounters];
+    PMP_HIP(hipMemcpyAsync(c, ctx->eb.counter.ptr, sizeof(c), hipMemcpyDeviceToHost, st(ctx)));
     PMP_HIP(hipStreamSynchronize(st(ctx)));
+    *n = c[kCntRecheck];
+    for (int i = 0; i < kEdgeSlots; ++i) *n += c[kCntStaged + i];
   });
 }
 

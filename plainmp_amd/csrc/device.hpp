@@ -92,18 +92,26 @@ __device__ __forceinline__ const A& args_again() {
 // first workgroups' starts and, in as many words, the latest ends; the host
 // takes the span when it is asked.  (Events around the kernel cost 7 us a call,
 // 12 more where the call is then waited for.)  Also clears what the next
-// launch adds to.
-__device__ __forceinline__ void edge_clock_begin(const EdgeArgs& ea) {
-  uint64_t* mine = ea.clock + ea.slot * 2 * kEdgeClocks;
-  uint64_t* next = ea.clock + (1 - ea.slot) * 2 * kEdgeClocks;
-  if (blockIdx.x < kEdgeClocks && threadIdx.x == 0) mine[blockIdx.x] = (uint64_t)wall_clock64();
-  if (blockIdx.x == 0) {
-    for (int i = threadIdx.x; i < 2 * kEdgeClocks; i += blockDim.x) next[i] = 0;
-    if (threadIdx.x == 0) ea.counter[kCntStaged + 1 - ea.slot] = 0;
+// launch adds to and the counts of earlier ones.  kStaged: the launch counts
+// in its slot's word, otherwise in the recheck count.
+template <bool kStaged>
+__device__ __forceinline__ void edge_begin(const EdgeArgs& ea) {
+  if (ea.clock) {
+    uint64_t* mine = ea.clock + ea.slot * 2 * kEdgeClocks;
+    uint64_t* next = ea.clock + (1 - ea.slot) * 2 * kEdgeClocks;
+    if (blockIdx.x < kEdgeClocks && threadIdx.x == 0) mine[blockIdx.x] = (uint64_t)wall_clock64();
+    if (blockIdx.x == 0)
+      for (int i = threadIdx.x; i < 2 * kEdgeClocks; i += blockDim.x) next[i] = 0;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    for (int i = 0; i < kEdgeSlots; ++i)
+      if (!kStaged || i != ea.slot) ea.counter[kCntStaged + i] = 0;
+    if (kStaged) ea.counter[kCntRecheck] = 0;
   }
 }
 // By one lane of a wave, after its last edge.
 __device__ __forceinline__ void edge_clock_end(const EdgeArgs& ea) {
+  if (!ea.clock) return;
   unsigned long long* end = reinterpret_cast<unsigned long long*>(ea.clock) + (ea.slot * 2 + 1) * kEdgeClocks;
   atomicMax(end + blockIdx.x % kEdgeClocks, (unsigned long long)wall_clock64());
 }

@@ -155,7 +155,7 @@ __global__ void __launch_bounds__(1024) edges_staged_kernel(EdgeKernelArgs args)
   out.first = queue + 1;
   out.pend = out.first + 1;
   double* ends = reinterpret_cast<double*>(staged_lds + el.flags + 64 + 4 + 3 * kPendMax);
-  edge_clock_begin(args.ea);
+  edge_begin<true>(args.ea);
   // Workgroups go to the XCDs in turn; each XCD takes a contiguous range of a
   // round's motions, whose endpoints share cache lines.
   const int g = (int)blockIdx.x, n = (int)gridDim.x, x = g % kXcds;

@@ -522,7 +522,7 @@ edges_kernel(KinArgs<float> k32, SceneArgs<float> s32, KinArgs<double> k64, Scen
   // edges from the counter.  Every lane takes part in the atomic (lane 0
   // adds 1, the others 0) and the index is read from the first lane into a
   // scalar register, so it and every branch on it are wave-uniform.
-  edge_clock_begin(ea);
+  edge_begin<false>(ea);
   const int W = blockDim.x >> 6;
   const bool by_index = (int64_t)gridDim.x * W >= ea.E;
   int e;
@@ -1640,7 +1640,8 @@ hipError_t launch_vjp(const KinArgs<float>& ka, const SceneArgs<float>& sc, cons
     const int bk = slot_block(ka, 256);
     const dim3 grid(blocks_for(B, bk), (unsigned)ka.n_items, (unsigned)nz);
     if (ka.shared)
-      PMP_DISPATCH_MAXC(ka.n_cols, vjp_shared_kernel, grid, dim3(bk), slot_bytes(ka, bk), st, ka, sc, q, ldq, B, gd, part);
+      PMP_DISPATCH_MAXC(ka.n_cols, vjp_shared_kernel, grid, dim3(bk), slot_bytes(ka, bk), st, ka, sc, q, ldq, B, gd,
+                        part);
     else
       PMP_DISPATCH_MAXC(ka.n_cols, vjp_kernel, grid, dim3(bk), slot_bytes(ka, bk), st, ka, sc, q, ldq, B, gd, part);
     if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;

@@ -16,16 +16,19 @@ constexpr int kPendStates = 16;  // in-band states an edge may queue for the FP6
 // sets the others back to zero, so a launch leaves them as it found them
 // (zero when the buffer is allocated) and no clearing node is needed in a
 // captured graph.
-// The staged form counts its FP64 decisions in one of two words in turn
-// (EdgeArgs::slot); every launch clears the other word for the next one.
+// The staged form counts its FP64 decisions in word EdgeArgs::slot: two words
+// in turn for direct calls, the third for launches in a caller's own capture,
+// whose node before it clears them all.  Every launch clears the words it does
+// not count in, so their sum with the recheck count is the last launch's.
 enum EdgeCounter {
   kCntWork = 0,
   kCntRecheck = 1,
   kCntPending = 2,
   kCntDone = 3,
   kCntInline = 4,
-  kCntStaged = 5,  // and 6
-  kNumEdgeCounters = 7
+  kCntStaged = 5,  // to 7
+  kEdgeSlots = 3,
+  kNumEdgeCounters = 8
 };
 
 // The event that marks the end of the current entry point's call: `ask` is set
@@ -49,8 +52,8 @@ struct EdgeArgs {
   const double* inv_width;  // device [n_cols], 1 / width as the reference precomputes
   const uint8_t* seq;       // device [128 * 128] farthest-first sequence table
   int32_t* counter;         // device [kNumEdgeCounters], see EdgeCounter
-  uint64_t* clock;          // device [2][2][kEdgeClocks], see edge_clock_begin
-  int32_t slot;             // which of the two words and clock sets this launch uses
+  uint64_t* clock;          // device [2][2][kEdgeClocks], see edge_begin; nullptr: not kept (captured launches)
+  int32_t slot;             // which word and clock set this launch uses
   int32_t* pend;            // [E][kPendStates] in-band visiting indices of pending edges
   int32_t* pend_info;       // [E][2] number queued (-1: more than kPendStates), first certain collision
   int32_t* plist;           // [E] the pending edges, in the order edges_kernel finished them

@@ -282,8 +282,8 @@ hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   launch_last(pair_grad_kernel<H, MAXC, STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, grad, n_slices,       \
               (int)chunks, lay)
   if (grad && ka.shared)
-    return launch_last(H == 1 ? pair_grad_shared_kernel<1> : pair_grad_shared_kernel<8>, grid, block, lds, st, ka, sc, q,
-                       ldq, B, dist, grad, n_slices, (int)chunks, lay);
+    return launch_last(H == 1 ? pair_grad_shared_kernel<1> : pair_grad_shared_kernel<8>, grid, block, lds, st, ka, sc,
+                       q, ldq, B, dist, grad, n_slices, (int)chunks, lay);
   if (H == 2) return grad ? PMP_GRAD(2, 16, false) : PMP_DIST(2, false);
   if (H == 4) return grad ? PMP_GRAD(4, 16, false) : PMP_DIST(4, false);
   if (H == 8) return grad ? PMP_GRAD(8, 16, false) : PMP_DIST(8, false);

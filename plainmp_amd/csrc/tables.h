@@ -123,7 +123,7 @@ struct alignas(16) DevColumn {
 struct alignas(32) DevSphereRow {
   float x, y, z, r;
   uint64_t col_mask;  // q columns that move it
-  int32_t pose, node;  // its node, and that one's pose-table index
+  int32_t pose, node;  // its node: pose-table index and number
 };
 
 // A slice of a sphere block's candidates: cull entries [lo, hi) of block

@@ -21,7 +21,8 @@ def _values(robot, scene, Q):
     tables = [np.concatenate([np.linalg.norm(c[:, ext] - m, axis=2) - r[ext] - b for m, b in scene.balls], 1)]
     for a, b in robot.pairs:
         ia, ib = np.flatnonzero(group == a), np.flatnonzero(group == b)
-        tables.append((np.linalg.norm(c[:, ia, None] - c[:, None, ib], axis=3) - (r[ia][:, None] + r[ib])).reshape(len(Q), -1))
+        d = np.linalg.norm(c[:, ia, None] - c[:, None, ib], axis=3) - (r[ia][:, None] + r[ib])
+        tables.append(d.reshape(len(Q), -1))
     for d in [tables[0]] + ([np.concatenate(tables[1:], 1)] if robot.pairs else []):
         top = np.partition(d, 1, axis=1)[:, :2]
         out.append(np.minimum(top[:, 0], CUTOFF))
@@ -60,8 +61,9 @@ def test_tie_goes_to_the_smaller_group():
     ids = (2796202, 2796203)  # times 512 primitives times 3 spheres: below and above 2^32
     nodes = [ROOT, (0, PRISMATIC, 0, (0, 0, 0.25), (1, 0, 0))]
     far = [((0.0, 5.0 + i, 5.0), 0.01) for i in range(510)]
-    for balls in ([((0.5, 0, 0.25), 0.125), ((-0.5, 0, 0.25), 0.125)], [((-0.5, 0, 0.25), 0.125), ((0.5, 0, 0.25), 0.125)]):
-        spheres = [(1, (0.25, 0, 0), 0.0625, ids[0]), (1, (-0.25, 0, 0), 0.0625, ids[1]), (1, (0, 3.0, 0), 0.01, ids[1])]
+    spheres = [(1, (0.25, 0, 0), 0.0625, ids[0]), (1, (-0.25, 0, 0), 0.0625, ids[1]), (1, (0, 3.0, 0), 0.01, ids[1])]
+    near = [((0.5, 0, 0.25), 0.125), ((-0.5, 0, 0.25), 0.125)]
+    for balls in (near, near[::-1]):
         v, j = Context(Robot(nodes, spheres, ids[1] + 1), Balls(balls + far)).evaluate(np.zeros((70, 1)))
         assert np.array_equal(v[:, 0], np.full(70, 0.0625, np.float32))
         assert np.abs(j[:, 0, 0] + 1.0).max() <= 1e-6  # the sphere of the first group nears its ball

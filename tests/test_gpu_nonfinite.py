@@ -14,12 +14,15 @@ from support import product_cst
 pytestmark = pytest.mark.gpu
 
 _R = synth._rot_rpy(0.3, -0.5, 0.9)
+_AT = np.array([0.5, 0.1, 0.4])
+_BOX = {"type": "box", "width": np.array([0.2, 0.3, 0.4]), "position": _AT}
+_CYL = {"type": "cylinder", "radius": 0.1, "height": 0.8, "position": _AT}
 PRIMS = {
-    "box": {"type": "box", "width": np.array([0.2, 0.3, 0.4]), "position": np.array([0.5, 0.1, 0.4]), "rotation": np.eye(3)},
-    "box_rot": {"type": "box", "width": np.array([0.2, 0.3, 0.4]), "position": np.array([0.5, 0.1, 0.4]), "rotation": _R},
-    "cylinder": {"type": "cylinder", "radius": 0.1, "height": 0.8, "position": np.array([0.5, 0.1, 0.4]), "rotation": np.eye(3)},
-    "cylinder_rot": {"type": "cylinder", "radius": 0.1, "height": 0.8, "position": np.array([0.5, 0.1, 0.4]), "rotation": _R},
-    "sphere": {"type": "sphere", "radius": 0.1, "position": np.array([0.5, 0.1, 0.4]), "rotation": np.eye(3)},
+    "box": {**_BOX, "rotation": np.eye(3)},
+    "box_rot": {**_BOX, "rotation": _R},
+    "cylinder": {**_CYL, "rotation": np.eye(3)},
+    "cylinder_rot": {**_CYL, "rotation": _R},
+    "sphere": {"type": "sphere", "radius": 0.1, "position": _AT, "rotation": np.eye(3)},
     "ground": {"type": "ground", "height": 0.1},
 }
 VALUES = [0.3, 1e3, 1e15, 3e19, -3e19, 1e30, -1e30, np.inf, -np.inf, np.nan]
@@ -58,8 +61,8 @@ def test_far_and_nan_bases(kind):
         Q[len(VALUES) + i, r.dof + 1] = v
     Q[-1, r.dof:r.dof + 2] = 3e19, -3e19
     pc = product_cst(synth.Workload("far", r, [prim]), base_type=BaseType.PLANAR)
-    radii = -pc.pair_clearance_batch(Q[:1], False)[0][0, :, 0] + _distance(prim, pc.sphere_centers_batch(Q[:1], True)[0])
     dist, grad = pc.pair_clearance_batch(Q, True)
+    radii = _distance(prim, pc.sphere_centers_batch(Q[:1], True)[0]) - dist[0, :, 0]
     with np.errstate(all="ignore"):
         ref = _distance(prim, pc.sphere_centers_batch(Q, True)) - radii
     got = dist[..., 0]
