@@ -503,24 +503,23 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   StageShape sh = stage_shape(B, ka.n_units - ka.n_pairs);
   while (sh.H < 8 && lds_of(sh.H, sh.W) > (size_t)ka.lds_limit) sh.H *= 2;
   if (ka.shared && sh.H > 1) sh.H = 8;
-  const int H = sh.H, W = sh.W;
+  const int64_t chunks = (B + 64 / sh.H - 1) / (64 / sh.H), n_traj = e.offsets ? e.n_traj : 0;
+  const int H = sh.H, W = waves_of_launch(chunks + n_traj, sh.W);
   const size_t lds = lds_of(H, W);
   if (lds > (size_t)ka.lds_limit) return false;
   StagedOut o{};
   o.vals = e.vals;
   o.jac = e.jac;
   o.offsets = e.offsets;
-  o.n_traj = e.offsets ? e.n_traj : 0;
+  o.n_traj = (int)n_traj;
   o.w2 = e.w2;
   o.cost = e.cost;
   o.grad = e.grad;
-  const int C = 64 / H;
-  const int64_t chunks = (B + C - 1) / C;
   o.n_chunks = (int)chunks;
   // slices balance a workgroup's waves; a full GPU does better without their
   // repeated set-up (trajectories of the dual arm: 157 us by blocks, 182 by slices)
   o.sliced = e.whole_chunks > 0 ? (B + 63) / 64 < e.whole_chunks : W == 16;
-  const StageLds lay = stage_lds(ka, C);
+  const StageLds lay = stage_lds(ka, 64 / H);
   o.scratch = o_scratch;
   o.best = o_best;
   const dim3 grid((unsigned)(chunks + (o.n_traj + W - 1) / W)), block(64 * W);

@@ -268,7 +268,7 @@ hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   // Gradients: 8 primitives, two tasks a wave once the launch fills the GPU
   // (8,192: 100 us, 4 primitives 106, four tasks 106), else one (1,000: 24 us,
   // two 28).  More than kPairWorkgroups workgroups only repeat the walk.
-  const int W = grad ? 4 : 8, per = grad ? 8 : 4, tasks_per_wave = grad && chunks > 32 ? 2 : 1;
+  const int W = waves_of_launch(chunks, grad ? 4 : 8), per = grad ? 8 : 4, tasks_per_wave = grad && chunks > 32 ? 2 : 1;
   const int n_slices = (sc.n_prims + per - 1) / per;
   const int64_t tasks = (int64_t)(grad ? ka.n_spheres : ka.n_items) * n_slices;
   int64_t ny = std::min((tasks + tasks_per_wave * W - 1) / (tasks_per_wave * W),

@@ -62,6 +62,13 @@ inline StageShape stage_shape(int64_t B, int n_blocks) {
   return s;
 }
 
+// The waves of a workgroup, at most W, with which a launch of n workgroups stays
+// below the 2^32 threads a launch may have.
+inline int waves_of_launch(int64_t n, int W) {
+  while (W > 1 && n * 64 * W > 0xffffffffll) W /= 2;
+  return W;
+}
+
 // Touches [p, p + bytes) through the scalar data cache, a line in n_parts: for
 // waves that would otherwise wait while another one walks, so that the tables
 // the whole workgroup is about to read are in the cache it shares.
