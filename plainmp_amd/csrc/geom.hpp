@@ -612,8 +612,7 @@ __device__ __forceinline__ bool collide_kind(const DevPrim<float>& p, V3<float> 
       xa = dx * p.R[0] + dy * p.R[3] + dz * p.R[6];
       ya = dx * p.R[1] + dy * p.R[4] + dz * p.R[7];
     }
-    // the root's rounding is far inside the band
-    const float rs = fmaxf(approx_sqrt(xa * xa + ya * ya) - p.p0, 0.0f);
+    const float rs = fmaxf(sqrtf(xa * xa + ya * ya) - p.p0, 0.0f);
     zs = fmaxf(zs, 0.0f);
     const float m = rs * rs + zs * zs - r * r;
     inband |= fabsf(m) <= band * (2.0f * r + band);
