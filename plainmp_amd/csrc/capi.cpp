@@ -118,6 +118,7 @@ class TablePack {
 struct EdgeBufs {
   DevBuf width, inv_width, pend, counter;
   int32_t slot = 0;  // EdgeArgs::slot of the last direct launch
+  int32_t clock_khz = 0;
   bool launched = false;
   std::vector<double> h_width;  // what width / inv_width hold, so a repeated call uploads nothing
   void release() {
@@ -1686,6 +1687,7 @@ pmp_status pmp_check_edges_batch(pmp_context* ctx, const double* s1, const doubl
     const bool direct = ends_call(ctx);
     if (direct) {
       ea.clock = edge_clocks(ctx->eb);
+      ea.clock_khz = &ctx->eb.clock_khz;
     } else {
       // replays run between direct calls, in no order the host knows
       ea.slot = kEdgeSlots - 1;
@@ -1783,7 +1785,7 @@ pmp_status pmp_edge_kernel_ms(pmp_context* ctx, float* ms) {
       if (t[0][i]) first = std::min(first, t[0][i]);  // 0: no workgroup
       last = std::max(last, t[1][i]);
     }
-    *ms = last > first ? (float)((double)(last - first) / kEdgeClockKhz) : 0.0f;
+    *ms = last > first ? (float)((double)(last - first) / ctx->eb.clock_khz) : 0.0f;
   });
 }
 

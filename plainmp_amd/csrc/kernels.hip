@@ -1438,6 +1438,13 @@ hipError_t launch_clearance(const KinArgs<float>& ka, const SceneArgs<float>& sc
 hipError_t launch_edges(const KinArgs<float>& k32, const KinArgs<double>& k64, const SceneArgs<float>& s32,
                         const SceneArgs<double>& s64, const EdgeArgs& ea, float band, int grid, int block,
                         hipStream_t st, hipEvent_t, hipEvent_t) {
+  if (ea.clock && *ea.clock_khz == 0) {
+    int device = 0, khz = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device);
+    if (e != hipSuccess) return e;
+    *ea.clock_khz = khz;
+  }
   if (edges_staged(k32, s32, ea.E))
     return launch_edges_staged(k32, k64, s32, s64, ea, band, grid, block, st);
   // a wave's FP32 walk and its FP64 re-decisions after it share the wave's

@@ -40,7 +40,6 @@ struct CallEnd {
 inline thread_local CallEnd call_end;
 
 constexpr int kEdgeClocks = 64;
-constexpr double kEdgeClockKhz = 1e5;  // wall_clock64 of gfx950
 
 struct EdgeArgs {
   const double* s1;
@@ -54,6 +53,7 @@ struct EdgeArgs {
   int32_t* counter;         // device [kNumEdgeCounters], see EdgeCounter
   uint64_t* clock;          // device [2][2][kEdgeClocks], see edge_begin; nullptr: not kept (captured launches)
   int32_t slot;             // which word and clock set this launch uses
+  int32_t* clock_khz;       // host: the clock's rate, set by the launcher while 0 (with a clock only)
   int32_t* pend;            // [E][kPendStates] in-band visiting indices of pending edges
   int32_t* pend_info;       // [E][2] number queued (-1: more than kPendStates), first certain collision
   int32_t* plist;           // [E] the pending edges, in the order edges_kernel finished them
