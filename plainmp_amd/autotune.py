@@ -14,8 +14,9 @@ Two knobs decide how the persistent kernels map onto the MI355X:
 ``tune_edges``, ``tune_evaluate`` and ``tune_pairs`` time every candidate on
 the caller's own device buffers (the edge kernel's own clock; stream
 events around the evaluate and pair calls), keep the fastest, apply it to the constraint's context and
-record it in a JSON cache keyed by device name and workload signature, so a
-later run with the same workload applies the cached schedule without timing.
+record it in a JSON cache keyed by device name, the version of the schedule's
+meaning and workload signature, so a later run with the same workload applies
+the cached schedule without timing.
 """
 
 from __future__ import annotations
@@ -28,8 +29,12 @@ import numpy as np
 
 EDGE_BLOCKS = (0, 64, 128, 256)  # 0: the launch's own choice
 EDGE_WAVES_PER_CU = (0, 4, 8, 12, 16, 20, 24, 32)
-EVAL_WHOLE_CHUNKS = (16, 32, 64, 128, 256, 512, 1024, 4096)
-PAIR_SHARES = (1, 2, 3, 4, 6, 8, 12, 16, 24, 32)
+EVAL_WHOLE_CHUNKS = (0, 16, 32, 64, 128, 256, 512, 1024, 4096)
+PAIR_SHARES = (0, 1, 2, 3, 4, 6, 8, 12, 16, 24, 32)
+
+# What the values of a schedule mean to the launches; an entry of another
+# version is timed again, not applied.
+SCHEDULE_VERSION = 2
 
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "plainmp_amd", "autotune.json")
 
@@ -38,6 +43,10 @@ def _device_name() -> str:
     import torch
 
     return torch.cuda.get_device_name(0)
+
+
+def _key(kind: str, key: str, size: str) -> str:
+    return f"{_device_name()}|v{SCHEDULE_VERSION}|{kind}|{key}|{size}"
 
 
 def _load(path: str) -> Dict:
@@ -84,7 +93,7 @@ def tune_edges(mv, cst, s1_ptr: int, s2_ptr: int, E: int, valid_ptr: int, nchk_p
     """Pick block / waves_per_cu for the edge batch (device SoA s1, s2 of E
     edges); returns the applied schedule and a report."""
     schedule = schedule or Schedule()
-    ckey = f"{_device_name()}|edges|{key}|E={E}"
+    ckey = _key("edges", key, f"E={E}")
     table = _load(cache) if cache else {}
     if ckey in table:
         schedule.block, schedule.waves_per_cu = table[ckey]["block"], table[ckey]["waves_per_cu"]
@@ -118,7 +127,7 @@ def tune_evaluate(cst, q_ptr: int, B: int, vals_ptr: int, jac_ptr: int, stream, 
     import torch
 
     schedule = schedule or Schedule()
-    ckey = f"{_device_name()}|evaluate|{key}|B={B}"
+    ckey = _key("evaluate", key, f"B={B}")
     table = _load(cache) if cache else {}
     if ckey in table:
         schedule.eval_whole_chunks = table[ckey]["eval_whole_chunks"]
@@ -169,7 +178,7 @@ def tune_pairs(cst, q_ptr: int, B: int, dist_ptr: int, grad_ptr: int, stream, sc
     """Pick pair_shares for a pair-distance batch of B configurations
     (``grad_ptr`` 0: distances only; ``stream`` is a torch.cuda.Stream)."""
     schedule = schedule or Schedule()
-    ckey = f"{_device_name()}|pairs|{key}|B={B}|grad={int(grad_ptr != 0)}"
+    ckey = _key("pairs", key, f"B={B}|grad={int(grad_ptr != 0)}")
     table = _load(cache) if cache else {}
     if ckey in table:
         schedule.pair_shares = table[ckey]["pair_shares"]
