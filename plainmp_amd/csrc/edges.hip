@@ -133,14 +133,21 @@ __device__ __forceinline__ void edge_chunk(float* lds, const EdgeStates& es, int
 }
 
 // The FP64 decisions of a chunk, by the first wave: whether there were any.
-// Out of line: inlined, their registers spill into the FP32 path.
+// Out of line: inlined, their registers spill into the FP32 path.  (Whole states
+// by all waves, as validity has it, take a second call in the motion's loop:
+// 2,000 motions of the 14-joint robot out of range 1,446 -> 1,170 us, but 1,000
+// in range 95 -> 103, and 64 against a cloud 41 -> 49.)
 __device__ __noinline__ bool edge_decide64(const EdgeKernelArgs* args, const EdgeStates es, int base, int C,
                                            const ValidLds<true> out) {
   const EdgeKernelArgs& A = *args;
   const int lane = threadIdx.x & 63, cfg = lane & (C - 1);
-  return wave_any(decide64(lane, cfg, lane / C, A.ka, A.k64, A.s64, A.ka.base_type == PMP_BASE_FIXED,
-                           base + cfg < es.n_wp, out,
-                           [&](int i) { return es.at(A.ea, min(base + i, es.n_wp - 1)); }));
+  const bool taylor = A.ka.base_type == PMP_BASE_FIXED;
+  auto point = [&](int i) { return es.at(A.ea, min(base + i, es.n_wp - 1)); };
+  const bool any = decide_pending(lane, cfg, A.ka, A.k64, A.s64, taylor, out, point);
+  const bool whole = decide_whole(lane, cfg, lane / C, kBlockSpheres * C / 64, 0, 1, A.k64, A.s64, taylor,
+                                  base + cfg < es.n_wp, out, point);
+  wave_lds_order();
+  return wave_any(any || whole);
 }
 
 template <bool kCloud>
@@ -189,7 +196,7 @@ __global__ void __launch_bounds__(1024) edges_staged_kernel(EdgeKernelArgs args)
         checked = es.n_wp;
         for (int base = 0; base < es.n_wp;) {
           const int left = es.n_wp - base, h = max(el.h_min, left <= 8 ? 8 : (left <= 16 ? 4 : (left <= 32 ? 2 : 1)));
-          const int C = 64 / h, cfg = lane & (C - 1);
+          const int C = 64 / h;
           if (h == 1)
             edge_chunk<kCloud, 1>(staged_lds, es, base, out, queue);
           else if (h == 2)

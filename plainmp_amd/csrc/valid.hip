@@ -11,8 +11,30 @@ struct ValidOut {
   int32_t* n_recheck;
   float band;
   int flags;  // LDS offset (floats)
+  int whole_waves;
   bool sliced;
 };
+
+struct ValidKernelArgs {
+  KinArgs<float> ka;
+  SceneArgs<float> sc;
+  KinArgs<double> k64;
+  SceneArgs<double> s64;
+  const double* q;
+  int64_t ldq, B;
+  ValidOut o;
+  StageLds lay;
+};
+
+// Configurations left to FP64 whole, from arguments read again: the others'
+// path keeps its registers.  (Out of line, 2.5 times the time.)
+template <int H>
+__device__ __forceinline__ void valid_whole(const Stage<H>& S, const ValidLds<false>& out) {
+  const ValidKernelArgs& A = args_again<ValidKernelArgs>();
+  const int64_t b0 = (int64_t)blockIdx.x * Stage<H>::C;
+  decide_whole(S.lane, S.cfg, S.sub, Stage<H>::NK, S.w, A.o.whole_waves, A.k64, A.s64, A.ka.base_type == PMP_BASE_FIXED,
+               b0 + S.cfg < A.B, out, [&](int i) { return BatchQ{A.q, A.ldq, min(b0 + i, A.B - 1)}; });
+}
 
 // Bound by latency, like evaluate.  Against a launch with a lane per
 // configuration or per (configuration, block) and a second one re-deciding
@@ -23,10 +45,14 @@ struct ValidOut {
 // kCloud: the scene holds clouds (their code costs the others registers: 97.5 us
 // instead of 94 for the 100,003).
 template <int H, bool kCloud>
-__global__ void __launch_bounds__(1024) valid_staged_kernel(KinArgs<float> ka, SceneArgs<float> sc, KinArgs<double> k64,
-                                                            SceneArgs<double> s64, const double* q, int64_t ldq,
-                                                            int64_t B, ValidOut o, StageLds lay) {
+__global__ void __launch_bounds__(1024) valid_staged_kernel(ValidKernelArgs args) {
   HIP_DYNAMIC_SHARED(float, staged_lds)
+  const KinArgs<float>& ka = args.ka;
+  const SceneArgs<float>& sc = args.sc;
+  const StageLds& lay = args.lay;
+  const ValidOut& o = args.o;
+  const double* q = args.q;
+  const int64_t ldq = args.ldq, B = args.B;
   const Stage<H> S(staged_lds, lay);
   constexpr int C = Stage<H>::C;
   const int lane = S.lane, w = S.w, W = S.W, cfg = S.cfg;
@@ -57,9 +83,16 @@ __global__ void __launch_bounds__(1024) valid_staged_kernel(KinArgs<float> ka, S
   __syncthreads();
   valid_items<kCloud>(S, ka, sc, o.band, out, queue, kCloud || o.sliced);
   __syncthreads();
+  const bool whole = any_whole(out, cfg);
+  if (w == 0)
+    decide_pending(lane, cfg, ka, args.k64, args.s64, taylor, out,
+                   [&](int i) { return BatchQ{q, ldq, min((int64_t)blockIdx.x * C + i, B - 1)}; });
+  if (whole) {
+    __syncthreads();
+    valid_whole(S, out);
+    __syncthreads();
+  }
   if (w != 0) return;
-  decide64(lane, cfg, S.sub, ka, k64, s64, taylor, active, out,
-           [&](int i) { return BatchQ{q, ldq, min((int64_t)blockIdx.x * C + i, B - 1)}; });
   const int f = out.state(cfg);
   if (active && S.sub == 0) {
     o.valid[b] = (f & kHit) ? 0 : 1;
@@ -71,7 +104,7 @@ hipError_t launch_valid(const KinArgs<float>& k32, const KinArgs<double>& k64, c
                         const SceneArgs<double>& s64, const double* q, int64_t ldq, int64_t B, float band,
                         uint8_t* valid, int32_t* n_recheck, int, const CloudWork&, const CloudRange*, int, int32_t*,
                         int32_t*, hipStream_t st) {
-  ValidOut o{valid, n_recheck, band, 0, true};
+  ValidOut o{valid, n_recheck, band, 0, 1, true};
   auto lds_of = [&](int H) {
     const int C = 64 / H;
     const StageLds L = stage_lds(k32, C);
@@ -86,12 +119,13 @@ hipError_t launch_valid(const KinArgs<float>& k32, const KinArgs<double>& k64, c
   o.sliced = slice_blocks(k32, sh.W);
   const size_t lds = lds_of(sh.H);
   if (lds > (size_t)k32.lds_limit) return hipErrorInvalidConfiguration;  // 8 configurations of any robot fit
+  o.whole_waves = whole_waves(k64, sizeof(float) * (size_t)o.flags, sh.W);
   const int C = 64 / sh.H;
   const StageLds lay = stage_lds(k32, C);
   const dim3 grid((unsigned)((B + C - 1) / C)), block(64 * sh.W);
 #define PMP_VALID(H) \
   launch_last(s32.n_cloud > 0 ? valid_staged_kernel<H, true> : valid_staged_kernel<H, false>, grid, block, lds, st, \
-              k32, s32, k64, s64, q, ldq, B, o, lay)
+              ValidKernelArgs{k32, s32, k64, s64, q, ldq, B, o, lay})
   return sh.H == 1 ? PMP_VALID(1) : sh.H == 2 ? PMP_VALID(2) : sh.H == 4 ? PMP_VALID(4) : PMP_VALID(8);
 #undef PMP_VALID
 }

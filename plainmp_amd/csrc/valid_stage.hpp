@@ -390,29 +390,102 @@ struct TwoPoses64 {
 // FP64 walk of whole configurations with the reference's own tests: per
 // primitive-checked sphere the AABB pre-test and is_outside, per self pair
 // the strict squared-distance test.  The group-sphere broad phase of the
-// reference only culls, so it is not needed for the result.
+// reference only culls, so it is not needed for the result.  The waves share
+// the sphere blocks and self pairs and the lanes of a configuration a block's
+// spheres (lane `part` takes nk of them).  A block's candidates are those of
+// the FP32 pass: its grown boxes carry a 1e-4 m slack, far above the FP32/FP64
+// centre difference, so a candidate they drop is outside the AABB pre-test in
+// FP64 too.
+template <bool kFirst>
 struct WholeVis64 {
   static constexpr bool kSelf = true;
+  static constexpr bool kRanged = true;
+  static constexpr bool kBlocks = true;
   const KinArgs<double>& ka;
   const SceneArgs<double>& sc;
-  int lane;
-  bool collided;
+  const ValidLds<kFirst>& out;
+  int lane, cfg, part, nk, wave, n_waves;
+  bool collided;  // or decided by another wave, or nothing to do
   __device__ bool alive() const { return !collided; }
+  __device__ int last_node() const { return ka.n_nodes - 1; }
+  __device__ int pair_lo() const { return ka.n_pairs * wave / n_waves; }
+  __device__ int pair_hi() const { return ka.n_pairs * (wave + 1) / n_waves; }
   template <class QS>
   __device__ void begin(const Pose<double>&, const QS&) {}
   __device__ void node(int, const DevNode<double>&, const Pose<double>&) {}
-  __device__ void sphere(int s, V3<double> c, double r) {
-    if (cload(ka.meta, s).ext < 0) return;
-    const DevPrim<double>* vp = reinterpret_cast<const DevPrim<double>*>(sc.vprims);
-    // a NaN centre collides with every primitive but a cloud, whose nearest
-    // point then decides (nothing is nearer than infinity: it does not)
-    if (sc.vrange[kKindCloud] > 0 && is_nan3(c)) collided = true;
-    for (int p = 0; p < sc.vrange[kKindCloud]; ++p) {
-      const DevPrim<double> P = cload(vp, p);
-      if (!collided && !outside_aabb(P, c, r) && !is_outside_ref<double>(P, c, r)) collided = true;
+  __device__ void sphere(int, V3<double>, double) {}
+  // Candidates i0 + (bits of mask) of kind K.
+  template <int K>
+  __device__ __forceinline__ void kind(V3<double> c, double r, bool has, int i0, uint64_t mask, int lo, int hi,
+                                       bool nocull) {
+    lo = max(lo - i0, 0);
+    hi = min(hi - i0, 64);
+    if (lo >= hi) return;
+    mask &= (~0ull << lo) & (~0ull >> (64 - hi));
+    for (; mask; mask &= mask - 1) {
+      if (!wave_any(has && !collided)) return;
+      const int i = i0 + __builtin_ctzll(mask);
+      const DevPrim<double> P =
+          cload(reinterpret_cast<const DevPrim<double>*>(sc.vprims), nocull ? i : cload(sc.cull, i).prim);
+      if (has && !collided && !outside_aabb(P, c, r) && !is_outside_ref<double, K>(P, c, r)) collided = true;
     }
-    for (int p = sc.vrange[kKindCloud]; p < sc.vrange[kKindCloud + 1]; ++p)
-      if (cloud_hits64(sc, cload(vp, p), c, r, !collided, lane)) collided = true;
+  }
+  __device__ __forceinline__ void block(int bi, const Pose<double>& P, const M3<double>& R, bool nocull) {
+    const DevSphereBlock bk = cload(ka.blocks, bi);
+    auto centre = [&](int k, bool& has, double& r) {
+      const int at = part * nk + k;
+      has = at < bk.n;
+      const DevSphere<double> sp = ka.spheres[ka.blocks[bi].sph[has ? at : 0]];
+      r = sp.r;
+      return add(mv(R, V3<double>{sp.x, sp.y, sp.z}), P.t);
+    };
+    bool has;
+    double r;
+    for (int k = 0; k < nk; ++k) {
+      const V3<double> c = centre(k, has, r);
+      // a NaN centre collides with every primitive but a cloud, whose nearest
+      // point then decides (nothing is nearer than infinity: it does not)
+      if (has && sc.vrange[kKindCloud] > 0 && is_nan3(c)) collided = true;
+      for (int p = sc.vrange[kKindCloud]; p < sc.vrange[kKindCloud + 1]; ++p)
+        if (cloud_hits64(sc, cload(reinterpret_cast<const DevPrim<double>*>(sc.vprims), p), c, r, has && !collided,
+                         lane))
+          collided = true;
+    }
+    const V3<double> g = add(mv(R, V3<double>{bk.g[0], bk.g[1], bk.g[2]}), P.t);
+    const CullRange cr = cload(sc.cull_range, bi);
+    auto at = [&](int k) { return nocull ? sc.vrange[k] : cr.at[k]; };
+    for (int i0 = at(0); i0 < at(kKindCloud); i0 += 64) {
+      uint64_t mask = 0;
+      for (int i = i0; i < min(i0 + 64, at(kKindCloud)); ++i) {
+        bool near = !collided;
+        if (!nocull) {
+          const CullEntry ce = cload(sc.cull, i);
+          near = near && !(g.x < ce.lb[0] || g.x > ce.ub[0] || g.y < ce.lb[1] || g.y > ce.ub[1] || g.z < ce.lb[2] ||
+                           g.z > ce.ub[2]);
+        }
+        if (wave_any(near)) mask |= 1ull << (i - i0);
+      }
+      if (mask == 0) continue;
+      for (int k = 0; k < nk; ++k) {
+        const V3<double> c = centre(k, has, r);
+        kind<kKindBoxAA>(c, r, has, i0, mask, at(kKindBoxAA), at(kKindBoxAA + 1), nocull);
+        kind<kKindBoxRot>(c, r, has, i0, mask, at(kKindBoxRot), at(kKindBoxRot + 1), nocull);
+        kind<kKindCylZ>(c, r, has, i0, mask, at(kKindCylZ), at(kKindCylZ + 1), nocull);
+        kind<kKindCylRot>(c, r, has, i0, mask, at(kKindCylRot), at(kKindCylRot + 1), nocull);
+        kind<kKindSphere>(c, r, has, i0, mask, at(kKindSphere), at(kKindSphere + 1), nocull);
+        kind<kKindGround>(c, r, has, i0, mask, at(kKindGround), at(kKindGround + 1), nocull);
+      }
+    }
+  }
+  __device__ __forceinline__ void blocks(const DevNode<double>& nd, const Pose<double>& P) {
+    if (nd.block_begin >= nd.block_end) return;
+    if (out.state(cfg) & kHit) collided = true;
+    const M3<double> R = qmat(P.q);
+    // outside the norm bounds the cull table assumed: test every primitive
+    const double n2 = P.q.x * P.q.x + P.q.y * P.q.y + P.q.z * P.q.z + P.q.w * P.q.w;
+    const bool nocull = wave_any(alive() && !(n2 >= nd.n2_lo && n2 <= nd.n2_hi));
+    for (int bi = nd.block_begin; bi < nd.block_end; ++bi)
+      if (bi % n_waves == wave && wave_any(alive())) block(bi, P, R, nocull);
   }
   __device__ void self(const DevSelfPair&, int, int, V3<double> ci, V3<double> cj, double rs) {
     const V3<double> d = sub(ci, cj);
@@ -420,55 +493,78 @@ struct WholeVis64 {
   }
 };
 
-// FP64 decision of what the FP32 items left open, by the first wave: the
-// pending pairs of configurations not yet colliding, a lane each, then whole
-// configurations (H lanes hold one; the first of them walks).  point(cfg) is
-// the joint-value source of a configuration.  The kept poses of the walks take
-// the workgroup's LDS from its start: the results lie past it.  Whether this
-// lane decided anything.
+// FP64 decision of what the FP32 items left open.  point(cfg) is the
+// joint-value source of a configuration.  The kept poses of the walks take the
+// workgroup's LDS from its start: the results lie past it.  Both return whether
+// this lane decided anything.
+//
+// The pending pairs of configurations not yet colliding, by the first wave, a
+// lane each.
 template <bool kFirst, class F>
-__device__ __forceinline__ bool decide64(int lane, int cfg, int part, const KinArgs<float>& ka,
-                                         const KinArgs<double>& k64, const SceneArgs<double>& s64, bool taylor,
-                                         bool active, const ValidLds<kFirst>& out, F&& point) {
+__device__ __forceinline__ bool decide_pending(int lane, int cfg, const KinArgs<float>& ka, const KinArgs<double>& k64,
+                                               const SceneArgs<double>& s64, bool taylor, const ValidLds<kFirst>& out,
+                                               F&& point) {
   const int n_pend = min(*out.count, kPendMax);
-  bool any = false;
-  if (n_pend > 0) {
-    const int pc = lane < n_pend ? out.pend[lane] : 0, s1 = lane < n_pend ? out.pend[kPendMax + lane] : 0,
-              other = lane < n_pend ? out.pend[2 * kPendMax + lane] : 0;
-    const bool has = lane < n_pend && (out.state(pc) & (kHit | kWhole)) == 0;
-    const int s2 = other < 0 ? -1 - other : s1;
-    TwoPoses64 v{has ? ka.meta[s1].node : 0, has ? ka.meta[s2].node : 0, !has};
-    run_fk(k64, point(has ? pc : cfg), taylor, v);
-    const DevSphere<double> a = k64.spheres[s1];
-    const V3<double> c1 = add(mv(qmat(v.P1.q), V3<double>{a.x, a.y, a.z}), v.P1.t);
-    bool hit = false;
-    bool cloud = false;
-    if (has && other < 0) {
-      const DevSphere<double> bb = k64.spheres[s2];
-      const V3<double> d = sub(c1, add(mv(qmat(v.P2.q), V3<double>{bb.x, bb.y, bb.z}), v.P2.t));
-      const double rs = a.r + bb.r;
-      hit = dot(d, d) < rs * rs;
-    } else if (has) {
-      cloud = other >= s64.vrange[kKindCloud];
-      const DevPrim<double>& P = reinterpret_cast<const DevPrim<double>*>(s64.vprims)[other];
-      hit = !cloud && !outside_aabb(P, c1, a.r) && !is_outside_ref<double>(P, c1, a.r);
-    }
-    for (int p = s64.vrange[kKindCloud]; p < s64.vrange[kKindCloud + 1]; ++p)
-      hit |= cloud_hits64(s64, cload(reinterpret_cast<const DevPrim<double>*>(s64.vprims), p), c1, a.r,
-                          cloud && other == p, lane);
-    if (has) out.mark(pc, kPended | (hit ? kHit : 0));
-    any = has;
-    wave_lds_order();
+  if (n_pend == 0) return false;
+  const int pc = lane < n_pend ? out.pend[lane] : 0, s1 = lane < n_pend ? out.pend[kPendMax + lane] : 0,
+            other = lane < n_pend ? out.pend[2 * kPendMax + lane] : 0;
+  const bool has = lane < n_pend && (out.state(pc) & (kHit | kWhole)) == 0;
+  const int s2 = other < 0 ? -1 - other : s1;
+  TwoPoses64 v{has ? ka.meta[s1].node : 0, has ? ka.meta[s2].node : 0, !has};
+  run_fk(k64, point(has ? pc : cfg), taylor, v);
+  const DevSphere<double> a = k64.spheres[s1];
+  const V3<double> c1 = add(mv(qmat(v.P1.q), V3<double>{a.x, a.y, a.z}), v.P1.t);
+  bool hit = false;
+  bool cloud = false;
+  if (has && other < 0) {
+    const DevSphere<double> bb = k64.spheres[s2];
+    const V3<double> d = sub(c1, add(mv(qmat(v.P2.q), V3<double>{bb.x, bb.y, bb.z}), v.P2.t));
+    const double rs = a.r + bb.r;
+    hit = dot(d, d) < rs * rs;
+  } else if (has) {
+    cloud = other >= s64.vrange[kKindCloud];
+    const DevPrim<double>& P = reinterpret_cast<const DevPrim<double>*>(s64.vprims)[other];
+    hit = !cloud && !outside_aabb(P, c1, a.r) && !is_outside_ref<double>(P, c1, a.r);
   }
+  for (int p = s64.vrange[kKindCloud]; p < s64.vrange[kKindCloud + 1]; ++p)
+    hit |= cloud_hits64(s64, cload(reinterpret_cast<const DevPrim<double>*>(s64.vprims), p), c1, a.r,
+                        cloud && other == p, lane);
+  if (has) out.mark(pc, kPended | (hit ? kHit : 0));
+  wave_lds_order();
+  return has;
+}
+
+// Whether some configuration is left to the FP64 walk whole: the same in every
+// wave, also while the first one decides pending pairs.
+template <bool kFirst>
+__device__ __forceinline__ bool any_whole(const ValidLds<kFirst>& out, int cfg) {
+  return wave_any((*reinterpret_cast<volatile int*>(out.flags + cfg) & kWhole) != 0);
+}
+// Whole configurations, by the first n_waves waves (whose kept poses fit the
+// tables' LDS), nk = kBlockSpheres / H spheres of a block to each of a
+// configuration's H lanes.  Configurations eight turns out of range: 1,000 of the
+// 7R arm 25 us, 50,000 of it 75, of the 14-joint robot 327, of a floating 31-joint
+// one 465.  (By one wave, a lane a configuration and every sphere against every
+// primitive: 249, 273, 1,364 and 1,508; in a launch of their own with a lane a
+// configuration: 102, 117, 414 and 454.)
+template <bool kFirst, class F>
+__device__ __forceinline__ bool decide_whole(int lane, int cfg, int part, int nk, int wave, int n_waves,
+                                             const KinArgs<double>& k64, const SceneArgs<double>& s64, bool taylor,
+                                             bool active, const ValidLds<kFirst>& out, F&& point) {
   const int f = out.state(cfg);
-  const bool whole = active && (f & kWhole) && !(f & kHit) && part == 0;
+  const bool whole = active && (f & kWhole) && !(f & kHit) && wave < n_waves;
   if (wave_any(whole)) {
-    WholeVis64 v{k64, s64, lane, !whole};
+    WholeVis64<kFirst> v{k64, s64, out, lane, cfg, part, nk, wave, n_waves, !whole};
     run_fk(k64, point(cfg), taylor, v);
     if (whole) out.mark(cfg, kPended | (v.collided ? kHit : 0));
-    wave_lds_order();
   }
-  return any || whole;
+  return whole;
+}
+
+// The waves of a workgroup of W whose FP64 kept poses fit lds bytes.
+inline int whole_waves(const KinArgs<double>& k64, size_t lds, int W) {
+  const int64_t fit = k64.slot_wave_bytes > 0 ? (int64_t)lds / k64.slot_wave_bytes : W;
+  return fit < 1 ? 1 : (fit < W ? (int)fit : W);
 }
 
 }  // namespace pmp
