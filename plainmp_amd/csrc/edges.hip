@@ -234,12 +234,6 @@ hipError_t launch_edges_staged(const KinArgs<float>& k32, const KinArgs<double>&
                                hipStream_t st) {
   EdgeLds el{};
   size_t lds = 0;
-  // 8 waves while a motion has a CU to itself or self pairs to share out, else 4
-  // (7R arm, 512 motions of a tenth of the joint range: 34 us, 36 with 8 waves,
-  // 57 with 16; 64 motions: 28 with 8, 29 with 4; with self pairs, 14 joints,
-  // 1,024: 119 with 8, 144 with 4; 8,192: 544 with 4, 559 with 8)
-  const bool wide = ea.E <= kCus || s32.n_cloud > 0 || (k32.n_pairs > 0 && ea.E <= 8 * kCus);
-  const int W = block > 0 ? block / 64 : (wide ? 8 : 4);
   for (el.h_min = 1;; el.h_min *= 2) {
     const StageLds L = stage_lds(k32, 64 / el.h_min);
     const int keep = k64.slot_wave_bytes / (int)sizeof(float);  // one wave's FP64 kept poses
@@ -248,6 +242,15 @@ hipError_t launch_edges_staged(const KinArgs<float>& k32, const KinArgs<double>&
     if (lds <= (size_t)k32.lds_limit) break;
     if (el.h_min == 8) return hipErrorInvalidConfiguration;  // 8 states of any robot fit
   }
+  // 8 waves while a motion has a CU to itself, self pairs to share out or a cloud,
+  // else 4 (7R arm, 512 motions of a tenth of the joint range: 20 us, 25 with 8
+  // waves, 42 with 16; with self pairs, 14 joints, 1,024: 119 with 8, 145 with 4;
+  // 4,096: 332 with 4, 346 with 8; clouds, 7R arm, 16,384: 584 with 4, 911 with 8;
+  // 14 joints 2,845 and 2,394); 16 where the tables leave a CU one workgroup (31
+  // joints, 1,024: 145 with 16, 167 with 8; 60 joints 273 and 328)
+  const bool wide = ea.E <= kCus || (s32.n_cloud > 0 && (ea.E <= 32 * kCus || staged_fit(k32) < 4)) ||
+                    (k32.n_pairs > 0 && ea.E <= 8 * kCus);
+  const int W = block > 0 ? block / 64 : (2 * lds > (size_t)k32.lds_limit ? 16 : (wide ? 8 : 4));
   const int64_t most = waves > 0 ? (waves < W ? 1 : waves / W) : 1 << 20;
   return launch_last(s32.n_cloud > 0 ? edges_staged_kernel<true> : edges_staged_kernel<false>,
                      dim3((unsigned)(ea.E < most ? ea.E : most)), dim3(64 * W), lds, st,

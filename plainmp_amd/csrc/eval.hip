@@ -503,6 +503,7 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   StageShape sh = stage_shape(B, ka.n_units - ka.n_pairs);
   while (sh.H < 8 && lds_of(sh.H, sh.W) > (size_t)ka.lds_limit) sh.H *= 2;
   if (ka.shared && sh.H > 1) sh.H = 8;
+  if (2 * lds_of(sh.H, sh.W) > (size_t)ka.lds_limit && lds_of(sh.H, 16) <= (size_t)ka.lds_limit) sh.W = 16;
   const int64_t chunks = (B + 64 / sh.H - 1) / (64 / sh.H), n_traj = e.offsets ? e.n_traj : 0;
   const int H = sh.H, W = waves_of_launch(chunks + n_traj, sh.W);
   const size_t lds = lds_of(H, W);
@@ -517,8 +518,11 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   o.grad = e.grad;
   o.n_chunks = (int)chunks;
   // slices balance a workgroup's waves; a full GPU does better without their
-  // repeated set-up (trajectories of the dual arm: 157 us by blocks, 182 by slices)
-  o.sliced = e.whole_chunks > 0 ? (B + 63) / 64 < e.whole_chunks : W == 16;
+  // repeated set-up (trajectories of the dual arm: 157 us by blocks, 182 by slices),
+  // and a block's cloud, all of it in one slice, has nothing to balance (10,000
+  // configurations of the Fetch-like robot 2,828 and 2,946, but fewer with lanes
+  // that share blocks, 1,000 of the 14-joint one among primitives, 35 and 22)
+  o.sliced = e.whole_chunks > 0 ? (B + 63) / 64 < e.whole_chunks : B <= 64 * kCus && !(sc.n_cloud > 0 && H == 1);
   const StageLds lay = stage_lds(ka, 64 / H);
   o.scratch = o_scratch;
   o.best = o_best;

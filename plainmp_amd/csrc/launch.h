@@ -118,16 +118,44 @@ hipError_t launch_cloud_min(const CloudTile* tiles, const float* tileB, const Cl
                             float* out_d2, hipStream_t st);
 hipError_t launch_cloud_clearance(float* clearance, const float* d2, const float* radius_out, float rc, int64_t B,
                                   int64_t S, hipStream_t st);
+// Offsets (in floats) of a staged workgroup's LDS tables: the joints' words,
+// the poses, and a copy of the path entries (16 words each; path < 0: too many,
+// read from memory).
+constexpr int kStagedEntries = 256;
+struct StageLds {
+  int joints, poses, path, end;
+};
+__host__ __device__ __forceinline__ StageLds stage_lds(const KinArgs<float>& ka, int C) {
+  StageLds L;
+  L.joints = 0;
+  L.poses = 4 * ka.n_joints * C;
+  L.end = L.poses + 7 * ka.n_poses * C;
+  L.path = -1;
+  if (ka.n_path_entries <= kStagedEntries) {
+    L.path = L.end;
+    L.end += 16 * ka.n_path_entries;
+  }
+  return L;
+}
+
+// Workgroups of 64 configurations whose tables fit a CU's LDS.
+inline int staged_fit(const KinArgs<float>& ka) {
+  return ka.lds_limit / ((int)sizeof(float) * (stage_lds(ka, 64).end + 1));
+}
 // edges.hip: whether a batch of E motions takes the staged form (a workgroup
 // per motion) or edges_kernel (a wave per motion).  The staged form shortens a
-// motion's chain and shares its work; a wave per motion repeats less once the
-// motions alone fill the GPU.  Measured (us, staged and not), motions across
-// the joint range: 7R arm, 512 32 and 61, 1,024 41 and 61, 2,048 (before its
-// last speed-ups) 93 and 62; with self pairs, 14 joints, 1,024 101 and 211,
-// 32,768 (before) 1,909 and 1,410; Fetch-like 1,024 80 and 181, 8,192 379 and 603.  With a
-// cloud its queries are answered by whole waves: 4,096 583 and 1,036.
+// motion's chain and shares its work, the more with self pairs; a wave per motion
+// repeats less once the motions alone fill the GPU, which robots with large
+// tables need more of (workgroups a CU: Fetch-like 5, 14 joints 3, 31 joints 1).
+// Measured (us, staged and not), motions across the joint range among 16
+// primitives: 7R arm, 1,024 44 and 55, 2,048 78 and 57; on a lift 95 and 131, 168
+// and 139; with self pairs, Fetch-like, 8,192 328 and 519; 14 joints, 4,096 332 and
+// 371, 8,192 588 and 529; 31 joints, 1,024 145 and 166, 2,048 255 and 168.
+// With a cloud its queries are answered by whole waves: 4,096 583 and 1,036.
 inline bool edges_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, int64_t E) {
-  return sc.n_cloud > 0 || E <= (ka.n_pairs > 0 ? 32 * kCus : 4 * kCus);
+  if (sc.n_cloud > 0) return true;
+  const int fit = ka.n_pairs > 0 ? staged_fit(ka) : 1;
+  return E <= (fit >= 4 ? 32 : (fit >= 2 ? 16 : 4)) * kCus;
 }
 // waves: resident at most (0 = a workgroup per motion), block: threads of a
 // workgroup (0 = default).

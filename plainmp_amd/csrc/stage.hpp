@@ -23,26 +23,6 @@
 
 namespace pmp {
 
-// Offsets (in floats) of a staged workgroup's LDS tables: the joints' words,
-// the poses, and a copy of the path entries (16 words each; path < 0: too many,
-// read from memory).
-constexpr int kStagedEntries = 256;
-struct StageLds {
-  int joints, poses, path, end;
-};
-__host__ __device__ __forceinline__ StageLds stage_lds(const KinArgs<float>& ka, int C) {
-  StageLds L;
-  L.joints = 0;
-  L.poses = 4 * ka.n_joints * C;
-  L.end = L.poses + 7 * ka.n_poses * C;
-  L.path = -1;
-  if (ka.n_path_entries <= kStagedEntries) {
-    L.path = L.end;
-    L.end += 16 * ka.n_path_entries;
-  }
-  return L;
-}
-
 // Configurations (64 / H) and waves (W) of a workgroup for a batch of B: the
 // fewest configurations while every CU then gets one workgroup at most, with
 // 16 waves each; once a CU has several workgroups, 8 waves, and 4 when the
@@ -52,6 +32,10 @@ __host__ __device__ __forceinline__ StageLds stage_lds(const KinArgs<float>& ka,
 // 32,768 35 with 8 waves, 60 with 16; of 65,536 50 with 4 waves, 63 with 8.
 // Validity of 1,000: 13.5 with H = 8, 14.1 with H = 4, 16.7 with H = 1; of
 // 32,768 24 with 8 waves, 32 with 16; of 131,072 55 with 4 waves, 65 with 8.
+// A robot whose tables take more than half of a CU's LDS has one workgroup there,
+// which then gets 16 waves (100,000 configurations of 31 joints on a
+// floating base: validity 350 us with 8, 207 with 16; evaluate 488 and 333; of 60
+// joints 1,150 and 761, 1,297 and 842).
 struct StageShape {
   int H, W;
 };

@@ -115,6 +115,7 @@ hipError_t launch_valid(const KinArgs<float>& k32, const KinArgs<double>& k64, c
   };
   StageShape sh = stage_shape(B, k32.n_units - k32.n_pairs);
   while (sh.H < 8 && lds_of(sh.H) > (size_t)k32.lds_limit) sh.H *= 2;
+  if (2 * lds_of(sh.H) > (size_t)k32.lds_limit) sh.W = 16;
   sh.W = waves_of_launch((B + 64 / sh.H - 1) / (64 / sh.H), sh.W);
   o.sliced = slice_blocks(k32, sh.W);
   const size_t lds = lds_of(sh.H);
