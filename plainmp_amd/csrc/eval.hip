@@ -73,6 +73,9 @@ constexpr int kSelfPosBits = 11;
 // radius, its key and its configuration.
 constexpr int kEntryWords = 6;
 
+// Lanes a configuration has at least in scenes with clouds.
+constexpr int kCloudLanes = 4;
+
 // One slice of block candidates.
 // kBoxes: candidates are first tested against their grown box (coherent
 // batches, where it drops most of them before their primitive is read).
@@ -186,7 +189,7 @@ __device__ __forceinline__ void ext_slice(const Stage<H>& S, const KinArgs<float
   // a sphere can give a value below the cutoff, so the minimum is taken over
   // the tiles within that reach of the block (all tiles when the rotation is
   // outside the norm bounds).
-  if (!it.first) return;
+  if (H < kCloudLanes || !it.first) return;
   for (int p = sc.vrange[kKindCloud]; p < sc.vrange[kKindCloud + 1]; ++p) {
     const DevPrim<float> Pc = cload(vp, p);
     const uint32_t pkey = (uint32_t)cload(sc.vorig, p) * (uint32_t)ka.n_spheres;
@@ -501,6 +504,11 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
     return sizeof(float) * (size_t)(o_best + 4 * C + 2 * C + 1);
   };
   StageShape sh = stage_shape(B, ka.n_units - ka.n_pairs);
+  // a block's cloud is one wave's work: with four lanes a configuration more of
+  // its tiles are too far for all of a wave's configurations (10,000 of the
+  // Fetch-like robot against 20,000 points 2,277 us, 2,926 with one lane, 2,785
+  // before the staged form; 100,000 of the 7R arm 744, 1,105 and 1,646)
+  if (sc.n_cloud > 0 && sh.H < kCloudLanes) sh.H = kCloudLanes;
   while (sh.H < 8 && lds_of(sh.H, sh.W) > (size_t)ka.lds_limit) sh.H *= 2;
   if (ka.shared && sh.H > 1) sh.H = 8;
   if (2 * lds_of(sh.H, sh.W) > (size_t)ka.lds_limit && lds_of(sh.H, 16) <= (size_t)ka.lds_limit) sh.W = 16;
@@ -518,11 +526,8 @@ bool launch_eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   o.grad = e.grad;
   o.n_chunks = (int)chunks;
   // slices balance a workgroup's waves; a full GPU does better without their
-  // repeated set-up (trajectories of the dual arm: 157 us by blocks, 182 by slices),
-  // and a block's cloud, all of it in one slice, has nothing to balance (10,000
-  // configurations of the Fetch-like robot 2,828 and 2,946, but fewer with lanes
-  // that share blocks, 1,000 of the 14-joint one among primitives, 35 and 22)
-  o.sliced = e.whole_chunks > 0 ? (B + 63) / 64 < e.whole_chunks : B <= 64 * kCus && !(sc.n_cloud > 0 && H == 1);
+  // repeated set-up (trajectories of the dual arm: 157 us by blocks, 182 by slices)
+  o.sliced = e.whole_chunks > 0 ? (B + 63) / 64 < e.whole_chunks : B <= 64 * kCus;
   const StageLds lay = stage_lds(ka, 64 / H);
   o.scratch = o_scratch;
   o.best = o_best;
