@@ -13,7 +13,7 @@
 
 namespace pmp {
 
-// Runs f with the primitive's kind as a compile-time constant.
+// Runs f with the primitive's kind as a compile-time constant (clouds excluded).
 template <class F>
 __device__ __forceinline__ void with_kind(const DevPrim<float>& p, F&& f) {
   switch (prim_kind(p)) {
@@ -32,28 +32,19 @@ __device__ __forceinline__ void with_kind(const DevPrim<float>& p, F&& f) {
     case kKindSphere:
       f(std::integral_constant<int, kKindSphere>{});
       break;
-    case kKindGround:
-      f(std::integral_constant<int, kKindGround>{});
-      break;
     default:
-      f(std::integral_constant<int, kKindCloud>{});
+      f(std::integral_constant<int, kKindGround>{});
   }
 }
 
-// Distance to a primitive of kind K and its gradient.
-template <int K, bool kGrad>
-__device__ __forceinline__ void pair_eval(const SceneArgs<float>& sc, const DevPrim<float>& P, V3<float> c, float& d,
-                                          V3<float>& g) {
-  if constexpr (K == kKindCloud) {
-    // CloudSDF::evaluate (primitive_sdf.hpp:585-590): sqrt of the nearest
-    // squared distance minus r_cloud; its gradient at the nearest point
-    float d2;
-    const V3<float> dv = sub(c, cloud_nearest<true>(sc, (P.flags >> 4) & 15, c, d2));
-    d = sqrtf(d2) - P.p0;
-    if constexpr (kGrad) g = scale(1.0f / sqrtf(dot3(dv, dv)), dv);
-  } else {
-    sdf_value_grad<K, kGrad>(P, c, d, g);
-  }
+// CloudSDF::evaluate (primitive_sdf.hpp:585-590): sqrt of the nearest squared
+// distance minus r_cloud; its gradient at the nearest point.
+__device__ __forceinline__ float cloud_eval(const SceneArgs<float>& sc, const DevPrim<float>& P, V3<float> c,
+                                            V3<float>& g) {
+  float d2;
+  const V3<float> dv = sub(c, cloud_nearest<true>(sc, (P.flags >> 4) & 15, c, d2));
+  g = scale(1.0f / sqrtf(dot3(dv, dv)), dv);
+  return sqrtf(d2) - P.p0;
 }
 
 // The joint frames of every column, [D][6][C] from `at`, by all waves after
@@ -151,7 +142,7 @@ __global__ void __launch_bounds__(512) pair_dist_kernel(KinArgs<float> ka, Scene
           if (k < n) {
             float d;
             V3<float> g;
-            pair_eval<decltype(kc)::value, false>(sc, Q, c[k], d, g);
+            sdf_value_grad<decltype(kc)::value, false>(Q, c[k], d, g);
             if (active) put<kStream>(row[k] + (int64_t)p * B + b, d - r[k]);
           }
         }
@@ -168,7 +159,13 @@ __global__ void __launch_bounds__(512) pair_dist_kernel(KinArgs<float> ka, Scene
 // plain fill 73 us.  With rows off the cache lines (8,191 configurations) 142
 // us; 277 us with streaming stores and neighbouring chunks on different XCDs.
 // kShared: the robot's q columns drive several joints (ka.shared).
-template <int H, int MAXC, bool kStream, bool kShared>
+// kCloud: the scene holds clouds.  Finding the nearest point costs more than all
+// else, so it is done once a sphere, before the columns, and distances alone
+// (grad == nullptr) come here too, a sphere a task.  (2,000 configurations
+// against 20,000 points: 31 joints, a search for every 16 of 37 columns 6,579 us,
+// now 1,036, 3,027 before the staged form; 60 joints 28,221, 3,315 and 3,420;
+// distances of the 7R arm, eight spheres a task 1,250, now 202, before 1,301.)
+template <int H, int MAXC, bool kStream, bool kShared, bool kCloud>
 __device__ __forceinline__ void pair_grad(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q,
                                           int64_t ldq, int64_t B, float* dist, float* grad, int n_slices, int chunks,
                                           const StageLds& lay) {
@@ -184,15 +181,32 @@ __device__ __forceinline__ void pair_grad(const KinArgs<float>& ka, const SceneA
   __syncthreads();
   S.walk(ka, qs);
   __syncthreads();
-  const float* frames = stage_frames(S, ka, qs, lay.end);
-  __syncthreads();
-  const int D = ka.n_cols, NP = sc.n_prims, T = ka.n_spheres * n_slices;
+  const int D = kCloud && !grad ? 0 : ka.n_cols, NP = sc.n_prims, T = ka.n_spheres * n_slices;
+  const float* frames = nullptr;
+  if (!kCloud || grad) {
+    frames = stage_frames(S, ka, qs, lay.end);
+    __syncthreads();
+  }
   const int t_end = (int)((int64_t)T * (share + 1) / shares);
   for (int t = (int)((int64_t)T * share / shares) + S.w; t < t_end; t += S.W) {
     const int s = t / n_slices, sl = t % n_slices;
     const DevSphereRow row = cload(ka.rows, s);
     const Pose<float> P = S.pose(row.pose);
     const V3<float> c = add(mv3(qmat(P.q), V3<float>{row.x, row.y, row.z}), P.t);
+    const int p_begin = (int)((int64_t)NP * sl / n_slices), p_end = (int)((int64_t)NP * (sl + 1) / n_slices);
+    V3<float> near[kMaxClouds];
+    if constexpr (kCloud) {
+      for (int p = p_begin; p < p_end; ++p) {
+        const DevPrim<float> Q = prim_at(sc, p);
+        if (Q.type != PMP_PRIM_CLOUD) continue;
+        V3<float> g;
+        const float d = cloud_eval(sc, Q, c, g);
+#pragma unroll
+        for (int k = 0; k < kMaxClouds; ++k)
+          if (k == ((Q.flags >> 4) & 15)) near[k] = g;
+        if (active) put<kStream>(dist + ((int64_t)s * NP + p) * B + b, d - row.r);
+      }
+    }
     for (int j0 = 0; j0 < D || j0 == 0; j0 += MAXC) {
       V3<float> J[MAXC];
 #pragma unroll
@@ -211,15 +225,21 @@ __device__ __forceinline__ void pair_grad(const KinArgs<float>& ka, const SceneA
           for (int j = 0; j < MAXC; ++j)
             if (j0 + j == col) J[j] = add(J[j], v);
         });
-      const int p_end = (int)((int64_t)NP * (sl + 1) / n_slices);
-      for (int p = (int)((int64_t)NP * sl / n_slices); p < p_end; ++p) {
+      for (int p = p_begin; p < p_end; ++p) {
         const DevPrim<float> Q = prim_at(sc, p);
         float d = 0.f;
         V3<float> g{0.f, 0.f, 0.f};
-        with_kind(Q, [&](auto kc) { pair_eval<decltype(kc)::value, true>(sc, Q, c, d, g); });
+        const bool cloud = kCloud && Q.type == PMP_PRIM_CLOUD;
+        if (cloud) {
+#pragma unroll
+          for (int k = 0; k < kMaxClouds; ++k)
+            if (k == ((Q.flags >> 4) & 15)) g = near[k];
+        } else {
+          with_kind(Q, [&](auto kc) { sdf_value_grad<decltype(kc)::value, true>(Q, c, d, g); });
+        }
         if (!active) continue;
         const int64_t at = (int64_t)s * NP + p;
-        if (j0 == 0) put<kStream>(dist + at * B + b, d - row.r);
+        if (j0 == 0 && !cloud) put<kStream>(dist + at * B + b, d - row.r);
         float* gp = grad + (at * D + j0) * B + b;
 #pragma unroll
         for (int j = 0; j < MAXC; ++j) {
@@ -237,13 +257,25 @@ template <int H, int MAXC, bool kStream>
 __global__ void __launch_bounds__(256) pair_grad_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
                                                         int64_t ldq, int64_t B, float* dist, float* grad, int n_slices,
                                                         int chunks, StageLds lay) {
-  pair_grad<H, MAXC, kStream, false>(ka, sc, q, ldq, B, dist, grad, n_slices, chunks, lay);
+  pair_grad<H, MAXC, kStream, false, false>(ka, sc, q, ldq, B, dist, grad, n_slices, chunks, lay);
 }
 template <int H>
 __global__ void __launch_bounds__(256) pair_grad_shared_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
                                                                int64_t ldq, int64_t B, float* dist, float* grad,
                                                                int n_slices, int chunks, StageLds lay) {
-  pair_grad<H, 16, false, true>(ka, sc, q, ldq, B, dist, grad, n_slices, chunks, lay);
+  pair_grad<H, 16, false, true, false>(ka, sc, q, ldq, B, dist, grad, n_slices, chunks, lay);
+}
+template <int H>
+__global__ void __launch_bounds__(1024) pair_cloud_kernel(KinArgs<float> ka, SceneArgs<float> sc, const double* q,
+                                                          int64_t ldq, int64_t B, float* dist, float* grad,
+                                                          int n_slices, int chunks, StageLds lay) {
+  pair_grad<H, 16, false, false, true>(ka, sc, q, ldq, B, dist, grad, n_slices, chunks, lay);
+}
+template <int H>
+__global__ void __launch_bounds__(1024) pair_cloud_shared_kernel(KinArgs<float> ka, SceneArgs<float> sc,
+                                                                 const double* q, int64_t ldq, int64_t B, float* dist,
+                                                                 float* grad, int n_slices, int chunks, StageLds lay) {
+  pair_grad<H, 16, false, true, true>(ka, sc, q, ldq, B, dist, grad, n_slices, chunks, lay);
 }
 
 constexpr int64_t kPairWorkgroups = 16 * kCus;
@@ -263,14 +295,22 @@ hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
   if (lds > (size_t)ka.lds_limit) return hipErrorInvalidConfiguration;  // 8 configurations of any robot fit
   const StageLds lay = stage_lds(ka, 64 / H);
   const int64_t chunks = (B + 64 / H - 1) / (64 / H);
+  // With clouds a task a wave, of more primitives once there are waves enough
+  // (those of a slice without a cloud end at once), four waves a workgroup while
+  // that gives every CU one at most, and later as many as make 16 on a CU.
   // Distances: 4 primitives a task and a task a wave (8,191 configurations of
   // the 7R arm, 32 primitives: 31 us; 8 primitives 33, 4 tasks a wave 35).
   // Gradients: 8 primitives, two tasks a wave once the launch fills the GPU
   // (8,192: 100 us, 4 primitives 106, four tasks 106), else one (1,000: 24 us,
   // two 28).  More than kPairWorkgroups workgroups only repeat the walk.
-  const int W = waves_of_launch(chunks, grad ? 4 : 8), per = grad ? 8 : 4, tasks_per_wave = grad && chunks > 32 ? 2 : 1;
+  const bool cloud = sc.n_cloud > 0, by_sphere = grad || cloud;
+  const size_t fit = (size_t)ka.lds_limit / lds;
+  const int per = cloud && chunks * ka.n_spheres > 4 * kCus ? 32 : (by_sphere ? 8 : 4);
+  const int tasks_per_wave = grad && !cloud && chunks > 32 ? 2 : 1;
   const int n_slices = (sc.n_prims + per - 1) / per;
-  const int64_t tasks = (int64_t)(grad ? ka.n_spheres : ka.n_items) * n_slices;
+  const int64_t tasks = (int64_t)(by_sphere ? ka.n_spheres : ka.n_items) * n_slices;
+  const int few = chunks * ((tasks + 3) / 4) <= kCus || fit >= 4 ? 4 : (fit >= 2 ? 8 : 16);
+  const int W = waves_of_launch(chunks, cloud ? few : (grad ? 4 : 8));
   int64_t ny = std::min((tasks + tasks_per_wave * W - 1) / (tasks_per_wave * W),
                         (kPairWorkgroups + chunks - 1) / chunks);
   if (shares > 0) ny = std::min<int64_t>(shares, tasks);
@@ -281,6 +321,13 @@ hipError_t launch_pairs(const KinArgs<float>& ka, const SceneArgs<float>& sc, co
 #define PMP_GRAD(H, MAXC, STREAM)                                                                                     \
   launch_last(pair_grad_kernel<H, MAXC, STREAM>, grid, block, lds, st, ka, sc, q, ldq, B, dist, grad, n_slices,       \
               (int)chunks, lay)
+#define PMP_CLOUD(KERNEL) \
+  launch_last(KERNEL, grid, block, lds, st, ka, sc, q, ldq, B, dist, grad, n_slices, (int)chunks, lay)
+  if (cloud && grad && ka.shared) return PMP_CLOUD((H == 1 ? pair_cloud_shared_kernel<1> : pair_cloud_shared_kernel<8>));
+  if (cloud)
+    return PMP_CLOUD((H == 1 ? pair_cloud_kernel<1> : H == 2 ? pair_cloud_kernel<2> : H == 4 ? pair_cloud_kernel<4>
+                                                                                             : pair_cloud_kernel<8>));
+#undef PMP_CLOUD
   if (grad && ka.shared)
     return launch_last(H == 1 ? pair_grad_shared_kernel<1> : pair_grad_shared_kernel<8>, grid, block, lds, st, ka, sc,
                        q, ldq, B, dist, grad, n_slices, (int)chunks, lay);

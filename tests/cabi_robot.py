@@ -95,22 +95,31 @@ def _rot(axis, angle):
 
 
 class Balls:
-    """A scene of spheres (centre, radius)."""
+    """A scene of spheres (centre, radius), then point clouds (points, radius)."""
 
-    def __init__(self, balls):
+    def __init__(self, balls, clouds=()):
         self.balls = [(np.asarray(c, float), float(r)) for c, r in balls]
-        self._prims = (PrimDesc * max(1, len(balls)))()
+        self.clouds = [(np.ascontiguousarray(p, float), float(r)) for p, r in clouds]
+        self._prims = (PrimDesc * max(1, len(balls) + len(clouds)))()
         for p, (c, r) in zip(self._prims, self.balls):
             p.type, p.axis_aligned, p.z_axis_aligned = 3, 1, 1
             p.position[:], p.size[:] = list(c), [r, 0.0, 0.0]
             p.rotation[:] = p.rotation_inv[:] = [1.0, 0, 0, 0, 1.0, 0, 0, 0, 1.0]
             p.lb[:], p.ub[:] = list(c - r), list(c + r)
-        self.desc = SceneDesc(len(balls), self._prims)
+        for p, (points, r) in zip(self._prims[len(balls):], self.clouds):
+            p.type, p.axis_aligned, p.z_axis_aligned = 5, 1, 1
+            p.rotation[:] = p.rotation_inv[:] = [1.0, 0, 0, 0, 1.0, 0, 0, 0, 1.0]
+            p.size[:] = [r, 0.0, 0.0]
+            p.lb[:], p.ub[:] = list(points.min(0) - r), list(points.max(0) + r)
+            p.points, p.n_points = points.ctypes.data, len(points)
+        self.n_prims = len(balls) + len(clouds)
+        self.desc = SceneDesc(self.n_prims, self._prims)
 
     def distances(self, robot, Q):
         """[B][S][P] signed distances in FP64."""
         c = robot.centres(Q)
         d = [np.linalg.norm(c - m, axis=2) - r for m, r in self.balls]
+        d += [np.linalg.norm(c[:, :, None] - p, axis=3).min(2) - r for p, r in self.clouds]
         return np.stack(d, 2) - robot.radii()[None, :, None]
 
 
@@ -167,7 +176,7 @@ class Context:
         return np.moveaxis(t.cpu().numpy(), -1, 0)
 
     def pairs(self, Q, grad=True):
-        B, S, P = len(Q), len(self.robot.spheres), len(self.scene.balls)
+        B, S, P = len(Q), len(self.robot.spheres), self.scene.n_prims
         q, dist, g = self._q(Q), self._out(S, P, B), self._out(S, P, self.robot.D, B)
         self.ok(self.lib.pmp_pair_clearance_batch(self.ctx, self._ptr(q), i64(B), i64(B), self._ptr(dist),
                                                   self._ptr(g) if grad else None))
