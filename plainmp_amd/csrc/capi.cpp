@@ -995,6 +995,12 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
     a.n_joints = d.n_joints = (int32_t)joints.size();
     a.staged = d.staged = staged ? 1 : 0;
     a.shared = d.shared = shared ? 1 : 0;
+    double links = 0.0;  // how far the links can reach, the prismatic ones at 0
+    for (int i = 0; i < N; ++i)
+      for (int k = 0; k < 3; ++k) links += std::fabs(r->node_trans[3 * i + k]);
+    for (int k = 0; r->base_type == PMP_BASE_FIXED && k < 7; ++k) links += std::fabs(r->base_pose[k]);
+    for (const DevSphere<double>& s : sp64) links += std::fabs(s.x) + std::fabs(s.y) + std::fabs(s.z) + std::fabs(s.r);
+    a.far = d.far = !(links < 0.1 * kFar);
     std::vector<uint32_t> above(shared ? (size_t)N * kNodeWords : 0, 0u);
     for (int i = 0; shared && i < N; ++i)
       for (int n = i; n >= 0; n = n == 0 ? -1 : r->node_parent[n]) above[i * kNodeWords + (n >> 5)] |= 1u << (n & 31);
@@ -1136,6 +1142,12 @@ pmp_status pmp_upload_scene(pmp_context* ctx, const pmp_scene_desc* sc) {
     a.tiles64 = d.tiles64 = t64;
     a.tileB = d.tileB = tb;
     a.pts64 = d.pts64 = p64c;
+    for (const DevPrim<float>& p : p32) {
+      bool far = false;
+      for (const float v : {p.pos[0], p.pos[1], p.pos[2], p.p0, p.p1, p.p2}) far = far || !(std::fabs(v) < 0.1f * kFar);
+      for (int k = 0; k < 9; ++k) far = far || !(std::fabs(p.R[k]) < 100.f && std::fabs(p.Rinv[k]) < 100.f);
+      if (far && p.type != PMP_PRIM_CLOUD) a.far = d.far = 1;
+    }
     a.n_prims = d.n_prims = sc->n_prims;
     a.n_cloud = d.n_cloud = n_clouds;
     for (int i = 0; i <= kMaxClouds; ++i)

@@ -417,18 +417,19 @@ __device__ __forceinline__ V3<float> mv3(const M3<float>& R, V3<float> v) {
 // root: one Newton step for the reciprocal (about half an ulp, where a
 // correctly rounded root and division make up to one), and the root's residual
 // through it (Markstein), which rounds correctly but for rare last-place ties.
-// sqrt(0) = 0 and sqrt(inf) = inf, as a NaN's root is NaN; the reciprocal of 0
-// is finite, that of infinity and (its step is NaN) of NaN 0.  Below FLT_MIN
-// (points within 1e-19 m) the root is too small.
+// sqrt(0) = 0 and, with kAny, sqrt(inf) = inf, as a NaN's root is NaN; the
+// reciprocal of 0 is finite, that of infinity and (its step is NaN) of NaN 0.
+// Below FLT_MIN (points within 1e-19 m) the root is too small.
+template <bool kAny>
 __device__ __forceinline__ void root_and_reciprocal(float x, float& s, float& inv) {
 #if defined(__HIP_DEVICE_COMPILE__)
   float r = __builtin_amdgcn_rsqf(fmaxf(x, FLT_MIN));
   const float h = 0.5f * r;
   r = fmaf(fmaf(-x * r, r, 1.0f), h, r);
-  inv = fmaxf(r, 0.0f);
+  inv = kAny ? fmaxf(r, 0.0f) : r;
   s = x * r;
   s = fmaf(fmaf(-s, s, x), 0.5f * r, s);
-  s = x > FLT_MAX ? x : s;
+  if (kAny) s = x > FLT_MAX ? x : s;
 #else
   s = sqrtf(x);  // host pass: never executed, only type-checked
   inv = 1.0f / s;
@@ -440,7 +441,10 @@ __device__ __forceinline__ void root_and_reciprocal(float x, float& s, float& in
 // cost a third of correctly rounded ones, and a cylinder's gradient is formed
 // from its local coordinates.  Infinite and NaN coordinates and points on a
 // kink go the way they do there: a NaN term counts as 0, a zero coordinate as
-// positive, and where no direction is defined the gradient's part is 0.
+// positive, and where no direction is defined the gradient's part is 0.  The
+// distance alone takes coordinates and sizes below kFar (bound by its arithmetic
+// where gradients are by their stores).
+constexpr float kFar = 1e15f;  // no square of an entry of R times it overflows
 template <int K, bool kGrad>
 __device__ __forceinline__ void sdf_value_grad(const DevPrim<float>& p, V3<float> c, float& dist, V3<float>& g) {
   const V3<float> dc = sub(c, V3<float>{p.pos[0], p.pos[1], p.pos[2]});
@@ -450,8 +454,8 @@ __device__ __forceinline__ void sdf_value_grad(const DevPrim<float>& p, V3<float
     const float mx = fmaxf(sx, 0.0f), my = fmaxf(sy, 0.0f), mz = fmaxf(sz, 0.0f);
     const float top = fmaxf(fmaxf(sx, sy), sz);
     float root, inv;
-    root_and_reciprocal(mx * mx + my * my + mz * mz, root, inv);
-    dist = root + fmaxf(fmaxf(fminf(sx, 0.0f), fminf(sy, 0.0f)), fminf(sz, 0.0f));
+    root_and_reciprocal<kGrad>(mx * mx + my * my + mz * mz, root, inv);
+    dist = root + (kGrad ? fmaxf(fmaxf(fminf(sx, 0.0f), fminf(sy, 0.0f)), fminf(sz, 0.0f)) : fminf(top, 0.0f));
     if constexpr (kGrad) {
       V3<float> l{mx * inv, my * inv, mz * inv};
       if (!(top > 0.0f)) {  // inside: the nearest face
@@ -469,12 +473,12 @@ __device__ __forceinline__ void sdf_value_grad(const DevPrim<float>& p, V3<float
       z = dc.x * p.R[2] + dc.y * p.R[5] + dc.z * p.R[8];
     }
     float rho, inv_rho, root, inv;
-    root_and_reciprocal(sum2sq(x, y), rho, inv_rho);
+    root_and_reciprocal<kGrad>(sum2sq(x, y), rho, inv_rho);
     const float rs = rho - p.p0, zs = fabsf(z) - p.p1;
     const float o0 = fmaxf(rs, 0.0f), o1 = fmaxf(zs, 0.0f);
     const float top = fmaxf(rs, zs);
-    root_and_reciprocal(sum2sq(o0, o1), root, inv);
-    dist = root + fmaxf(fminf(rs, 0.0f), fminf(zs, 0.0f));
+    root_and_reciprocal<kGrad>(sum2sq(o0, o1), root, inv);
+    dist = root + (kGrad ? fmaxf(fminf(rs, 0.0f), fminf(zs, 0.0f)) : fminf(top, 0.0f));
     if constexpr (kGrad) {
       float wr = o0 * inv, wz = o1 * inv;
       if (!(top > 0.0f)) {
@@ -487,7 +491,7 @@ __device__ __forceinline__ void sdf_value_grad(const DevPrim<float>& p, V3<float
     }
   } else if constexpr (K == kKindSphere) {
     float root, inv;
-    root_and_reciprocal(dot3(dc, dc), root, inv);
+    root_and_reciprocal<kGrad>(dot3(dc, dc), root, inv);
     dist = root - p.p0;
     if constexpr (kGrad) g = root > 0.0f ? scale(inv, dc) : V3<float>{0.0f, 0.0f, 0.0f};
   } else {  // ground

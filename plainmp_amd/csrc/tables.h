@@ -213,6 +213,7 @@ struct KinArgs {
   // The others (two fingers on one column, coupled joints of a chain) take the
   // sum over the column's joints at or above a point's node.
   int32_t shared;            // some q column drives several joints
+  int32_t far;               // the links reach kFar / 10 (or NaN)
   const uint32_t* above;     // shared: [n_nodes][kNodeWords], bit a of row n: node a is n or above it
   T base_q[4];
   T base_t[3];
@@ -255,6 +256,7 @@ struct SceneArgs {
   const DevCullSlice* slices;
   const DevCullSlice* eslices;
   int32_t n_cull, n_slices, n_ecull, n_eslices;
+  int32_t far;                  // a primitive reaches kFar / 10, or its rotation's entries 100 (or NaN)
   const int32_t* vorig;         // kind-sorted index -> scene order
 };
 

@@ -79,6 +79,43 @@ def test_far_and_nan_bases(kind):
     assert (np.abs(grad[finite][..., r.dof:r.dof + 2]) <= 1 + 1e-5).all()
 
 
+@pytest.mark.parametrize("B", [21, 700])
+@pytest.mark.parametrize("kind", sorted(PRIMS))
+def test_far_and_nan_bases_distances_alone(kind, B):
+    """The kernel without gradients, which leaves workgroups with such a base to
+    the formulas; those without one keep the bits they have beside gradients."""
+    from plainmp_amd.kinematics import BaseType
+
+    r, prim = synth.panda_like(0), PRIMS[kind]
+    Q = np.zeros((B, r.dof + 3))
+    Q[:, : r.dof] = synth.uniform_configs(r, B, 1)
+    odd = np.r_[0, np.arange(1, len(VALUES) + 1) * (B // 32 or 1)][: len(VALUES)]
+    Q[odd, r.dof + np.arange(len(odd)) % 2] = VALUES
+    pc = product_cst(synth.Workload("far", r, [prim]), base_type=BaseType.PLANAR)
+    got, beside = pc.pair_clearance_batch(Q, False)[0][..., 0], pc.pair_clearance_batch(Q, True)[0][..., 0]
+    assert np.array_equal(np.isnan(got), np.isnan(beside)) and np.array_equal(np.isinf(got), np.isinf(beside))
+    ok = np.isfinite(got)
+    assert (np.abs(got[ok] - beside[ok]) <= 1e-6 * np.maximum(1.0, np.abs(beside[ok]))).all()
+    clean = np.ones(B, bool)  # configurations more than a workgroup's 64 from an odd one
+    for i in odd:
+        clean[max(0, i - 64): i + 65] = False
+    assert np.array_equal(got[clean], beside[clean]) and (B < 100 or clean.any())
+
+
+@pytest.mark.parametrize("at", [2e14, 1e16, 3e19])
+def test_far_primitives_and_links(at):
+    robot = Robot([(-1, 0, -1, (0, 0, 0), (0, 0, 0)), (0, 2, 0, (0, 0, 0.5), (0, 0, 1))], [(1, (0.1, 0, 0), 0.1, 0)], 1)
+    long = Robot([(-1, 0, -1, (0, 0, 0), (0, 0, 0)), (0, 2, 0, (at, 0, 0.5), (0, 0, 1))], [(1, (0.1, 0, 0), 0.1, 0)], 1)
+    near, far = ((0, 0.3, 0.5), 0.2), ((at, 0, 0), 0.2)
+    with np.errstate(over="ignore"):
+        d = np.float32(np.sqrt(np.float32(at) * np.float32(at)))
+    for ctx, ref in ((Context(robot, Balls([near, far])), d), (Context(long, Balls([near])), d)):
+        for grad in (False, True):
+            dist = ctx.pairs(np.zeros((3, 1)), grad)[0][:, 0, -1]
+            assert np.array_equal(np.isinf(dist), np.full(3, np.isinf(ref)))
+            assert np.isinf(ref) or np.abs(dist - ref).max() <= 1e-6 * ref
+
+
 def test_centre_on_centre():
     """A sphere at a ball's very centre: the distance is minus both radii and no
     direction is preferred."""
