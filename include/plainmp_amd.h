@@ -23,7 +23,9 @@
  *     share its device workspaces: a call made on another stream than the
  *     previous call waits (on the device, through an event) for that call's
  *     work, so consecutive calls never overlap.  Calls recorded into a
- *     caller's own stream capture are not ordered this way.
+ *     caller's own stream capture are not ordered this way, and hold the
+ *     tables of their time: capture them again after pmp_upload_robot,
+ *     pmp_upload_scene or pmp_set_band.
  *   - A context is not re-entrant: use one context per host thread.
  */
 #ifndef PLAINMP_AMD_H_

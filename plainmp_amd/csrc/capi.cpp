@@ -1005,14 +1005,9 @@ pmp_status pmp_upload_robot(pmp_context* ctx, const pmp_robot_desc* r) {
     for (int i = 0; shared && i < N; ++i)
       for (int n = i; n >= 0; n = n == 0 ? -1 : r->node_parent[n]) above[i * kNodeWords + (n >> 5)] |= 1u << (n & 31);
     pk.add(above, &a.above, &d.above);
-    // evaluate units: one per sphere item, then one per self pair; and the whole configuration
-    std::vector<DevEvalUnit> units;
-    for (int b = 0; b < (int)blocks.size(); ++b) units.push_back({b, b + 1, 0, 0, block_node[b], {0, 0, 0}});
-    for (int k = 0; k < (int)pairs.size(); ++k)
-      units.push_back({0, 0, k, k + 1, std::max(pairs[k].node1, pairs[k].node2), {0, 0, 0}});
+    // the whole configuration as one unit of the lane-per-configuration form
     std::vector<DevEvalUnit> whole{{0, (int32_t)blocks.size(), 0, (int32_t)pairs.size(), N - 1, {0, 0, 0}}};
-    pk.add(units, &a.units, &d.units);
-    a.n_units = d.n_units = (int32_t)units.size();
+    a.n_units = d.n_units = (int32_t)(blocks.size() + pairs.size());
     pk.add(whole, &a.unit_all, &d.unit_all);
     std::vector<float> rad(std::max(S, 1), 0.f);
     for (int s2 = 0; s2 < S; ++s2) rad[s2] = (float)r->sphere_radius[s2];
@@ -1353,7 +1348,8 @@ pmp_status pmp_is_valid_batch_noalloc(pmp_context* ctx, const double* q, int64_t
     PMP_BATCH_CHECKS(q, ldq, B);
     PMP_REQUIRE(B == 0 || valid, "null output");
     if (B == 0) return;
-    // the documented limit of this entry point (256-byte aligned pieces)
+    // The documented limit of this entry point, kept as callers size their
+    // batches by it: the launch itself needs no workspace.
     size_t need = 0;
     auto piece = [&](size_t bytes) { need += (bytes + 255) & ~(size_t)255; };
     if (ctx->n_clouds) {
@@ -1364,9 +1360,9 @@ pmp_status pmp_is_valid_batch_noalloc(pmp_context* ctx, const double* q, int64_t
     }
     if (B <= 65536 && ctx->k32.n_units > 0) piece(sizeof(int32_t) * (size_t)B);
     PMP_REQUIRE(need <= kNoAllocScratchBytes,
-                "batch needs " + std::to_string(need) + " bytes of scratch, more than the " +
+                "batch counts as " + std::to_string(need) + " bytes of scratch, more than the " +
                     std::to_string(kNoAllocScratchBytes) +
-                    " bytes pmp_is_valid_batch_noalloc has; split the batch or call pmp_is_valid_batch");
+                    " bytes pmp_is_valid_batch_noalloc accepts; split the batch or call pmp_is_valid_batch");
     set_device(ctx);
     ends_call(ctx);
     PMP_HIP(launch_valid(ctx->k32, ctx->k64, ctx->s32, ctx->s64, q, ldq, B, ctx->band, valid, n_recheck,

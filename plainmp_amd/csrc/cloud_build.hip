@@ -474,7 +474,7 @@ hipError_t launch_cloud_build(const double* pts, int64_t n, int32_t tile_base, C
                               float* tb, double* p64, CloudSuper* sup, void* scratch, hipStream_t st) {
   const CloudBuildSizes z = cloud_build_sizes(n);
   const int64_t nb = (n + kSortKeys - 1) / kSortKeys;
-  uint32_t* counts = (uint32_t*)scratch;  // first: read 16 bytes at a time
+  uint32_t* counts = (uint32_t*)scratch;
   double* part = (double*)(counts + nb * (kDigits / 2));
   uint64_t* keys = (uint64_t*)(part + 6 * kBoundsGrid);
   uint64_t* other = keys + n;

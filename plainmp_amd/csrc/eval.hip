@@ -268,12 +268,11 @@ __device__ __forceinline__ void traj_cost(const StagedOut& o, const double* X, i
   if (lane == 0) o.cost[i] = (float)c;
 }
 
-// Bound by latency (waves wait 57 % of their cycles on scalar table reads and
-// LDS; the vector instructions are half of the time).  Measured: trajectories
-// of the dual arm (123,498 waypoints) 411 -> 162 us, 8,192 configurations of
-// the 7R arm among 32 primitives 51 -> 22 us, 256 among two bars 28 -> 15 us,
-// each against a lane per configuration (a workgroup of 8 waves with a block
-// each, every wave walking FK again) before.
+// Bound by latency: scalar table reads and LDS.  Measured: trajectories of the
+// dual arm (123,498 waypoints) 411 -> 138 us, 8,192 configurations of the 7R arm
+// among 32 primitives 51 -> 17 us, 256 among two bars 28 -> 12 us, each against
+// a lane per configuration (a workgroup of 8 waves with a block each, every wave
+// walking FK again) before.
 // kShared: the robot's q columns drive several joints (ka.shared).
 template <int H, bool kShared>
 __device__ __forceinline__ void eval_staged(const KinArgs<float>& ka, const SceneArgs<float>& sc, const double* q,

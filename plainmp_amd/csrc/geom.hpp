@@ -592,7 +592,7 @@ PMP_HD bool is_outside_ref(const DevPrim<T>& p, V3<T> c, T r) {
 // !is_outside) and raises `inband` when the decision lies within `band`
 // metres of flipping.  For box, cylinder and sphere the AABB test is implied
 // by the exact test; for the ground it is part of the decision (its AABB is
-// z in [0, 0]).  NaN centres are the caller's business (see collide_fast).
+// z in [0, 0]).  NaN centres are the caller's business.
 template <int K>
 __device__ __forceinline__ bool collide_kind(const DevPrim<float>& p, V3<float> c, float r, float band, bool& inband) {
   const float dx = c.x - p.pos[0], dy = c.y - p.pos[1], dz = c.z - p.pos[2];
@@ -647,27 +647,6 @@ PMP_HD int prim_kind(const DevPrim<T>& p) {
       return kKindGround;
   }
   return kKindCloud;
-}
-
-// Any non-cloud primitive.  A NaN centre collides, as every comparison of the
-// reference is false for NaN.
-__device__ __forceinline__ bool collide_fast(const DevPrim<float>& p, V3<float> c, float r, float band, bool& inband) {
-  if (is_nan3(c)) return true;
-  switch (prim_kind(p)) {
-    case kKindBoxAA:
-      return collide_kind<kKindBoxAA>(p, c, r, band, inband);
-    case kKindBoxRot:
-      return collide_kind<kKindBoxRot>(p, c, r, band, inband);
-    case kKindCylZ:
-      return collide_kind<kKindCylZ>(p, c, r, band, inband);
-    case kKindCylRot:
-      return collide_kind<kKindCylRot>(p, c, r, band, inband);
-    case kKindSphere:
-      return collide_kind<kKindSphere>(p, c, r, band, inband);
-    case kKindGround:
-      return collide_kind<kKindGround>(p, c, r, band, inband);
-  }
-  return false;
 }
 
 }  // namespace pmp

@@ -110,7 +110,7 @@ hipError_t launch_valid(const KinArgs<float>& k32, const KinArgs<double>& k64, c
                         uint8_t* valid, int32_t* n_recheck, int block, const CloudWork& cw,
                         const CloudRange* clouds, int n_clouds, int32_t* flags, int32_t* unit_flags,
                         hipStream_t st);
-// Workspace bytes above which pmp_is_valid_batch_noalloc refuses a batch.
+// What pmp_is_valid_batch_noalloc counts a batch as must not be above this.
 constexpr size_t kNoAllocScratchBytes = (size_t)32 << 20;
 // cloud.hip
 hipError_t launch_cloud_min(const CloudTile* tiles, const float* tileB, const CloudSuper* supers,

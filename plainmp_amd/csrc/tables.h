@@ -83,8 +83,9 @@ struct alignas(16) CullRange {
 static_assert(kNumKinds + 1 == 8, "CullRange holds one offset per kind plus the end");
 
 // A run of at most kItemSpheres consecutive node-sorted spheres of one node
-// (every sphere, primitive-checked or not): the unit of work of the pair and
-// adjoint kernels, which give each (configuration, item) its own lane.
+// (every sphere, primitive-checked or not): the unit of work of pair distances,
+// a wave's task, and of the adjoint, which gives each (configuration, item) its
+// own lane.
 constexpr int kItemSpheres = 8;
 struct alignas(16) DevSphereItem {
   int32_t node, begin, end, pose;  // pose: pose-table index of the node
@@ -192,8 +193,7 @@ struct KinArgs {
   const DevSphereBlock* blocks;
   const DevSphereItem* items;
   int32_t n_items;
-  const DevEvalUnit* units;  // one unit per sphere block, then one per self pair
-  int32_t n_units;
+  int32_t n_units;  // sphere blocks and self pairs
   const DevEvalUnit* unit_all;  // one unit: every sphere and self pair
   int32_t n_nodes, n_spheres, n_pairs, n_cols;
   int32_t n_q_cols, base_type, n_ext_spheres;

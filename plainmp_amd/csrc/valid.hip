@@ -39,11 +39,11 @@ __device__ __forceinline__ void valid_whole(const Stage<H>& S, const ValidLds<fa
 // Bound by latency, like evaluate.  Against a launch with a lane per
 // configuration or per (configuration, block) and a second one re-deciding
 // whole configurations in FP64: 100,003 configurations of the Fetch-like robot
-// 263 -> 93 us (128 us of it the FP64 walks), 1,024 of the 7R arm 15.0 -> 8.5
-// us; 16,384 configurations against a 65,536-point cloud 92 -> 31 us (queries
-// through memory, 98,304 waves and four launches before).
-// kCloud: the scene holds clouds (their code costs the others registers: 97.5 us
-// instead of 94 for the 100,003).
+// 263 -> 89 us (128 us of it the FP64 walks), 1,024 of the 7R arm 15.0 -> 9 us;
+// 16,384 configurations against a 65,536-point cloud 92 -> 34 us (queries through
+// memory, 98,304 waves and four launches before).
+// kCloud: the scene holds clouds (their code costs the others registers: 4 % of
+// the time of the 100,003).
 template <int H, bool kCloud>
 __global__ void __launch_bounds__(1024) valid_staged_kernel(ValidKernelArgs args) {
   HIP_DYNAMIC_SHARED(float, staged_lds)

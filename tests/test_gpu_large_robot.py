@@ -21,8 +21,9 @@ def _scene():
     for k in range(18):
         a, z = rng.uniform(0, 2 * np.pi), rng.uniform(1.0, 2.6)
         at = np.array([0.8 * np.cos(a), 0.8 * np.sin(a), z])
-        prims.append([{"type": "sphere", "radius": 0.1}, {"type": "box", "width": np.full(3, 0.15)},
-                      {"type": "cylinder", "radius": 0.08, "height": 0.2}][k % 3] | {"position": at, "rotation": np.eye(3)})
+        shape = [{"type": "sphere", "radius": 0.1}, {"type": "box", "width": np.full(3, 0.15)},
+                 {"type": "cylinder", "radius": 0.08, "height": 0.2}][k % 3]
+        prims.append({**shape, "position": at, "rotation": np.eye(3)})
     return prims
 
 

@@ -16,10 +16,11 @@ def _setup(name):
     """Robot, base type name, extra columns, scene."""
     solids = dict(prims=synth.mixed_primitives(8, 2))
     cloud = dict(prims=synth.mixed_primitives(3, 2), cloud=synth.shelf_cloud(2000, 2))
-    return {"panda_cloud": (synth.panda_like(0), "FIXED", 0, cloud), "dual_arm": (synth.dual_arm(0), "FIXED", 0, solids),
-            "dual_arm_cloud": (synth.dual_arm(0), "FIXED", 0, cloud), "fetch": (synth.fetch_like(0), "FIXED", 0, solids),
-            "humanoid": (synth.humanoid31(0), "FLOATING", 6, solids), "comb": (_comb(), "FIXED", 0, solids),
-            "humanoid_cloud": (synth.humanoid31(0), "FLOATING", 6, cloud)}[name]
+    kind, scene = (name[:-6], cloud) if name.endswith("_cloud") else (name, solids)
+    if kind == "humanoid":
+        return synth.humanoid31(0), "FLOATING", 6, scene
+    return {"panda": synth.panda_like, "dual_arm": synth.dual_arm, "fetch": synth.fetch_like,
+            "comb": lambda _: _comb()}[kind](0), "FIXED", 0, scene
 
 
 def _configs(r, extra, n, seed):
@@ -35,9 +36,10 @@ def _constraints(wl, base):
             product_cst(wl, base_type=getattr(BaseType, base)))
 
 
-@pytest.mark.parametrize("name,E", [("panda_cloud", 8192), ("panda_cloud", 8193), ("dual_arm", 4096), ("dual_arm", 4097),
-                                    ("dual_arm_cloud", 8193), ("fetch", 8192), ("fetch", 8193), ("humanoid", 1024),
-                                    ("humanoid", 1025), ("humanoid_cloud", 3000), ("comb", 1024), ("comb", 1025)])
+@pytest.mark.parametrize("name,E", [
+    ("panda_cloud", 8192), ("panda_cloud", 8193), ("dual_arm", 4096), ("dual_arm", 4097), ("dual_arm_cloud", 8193),
+    ("fetch", 8192), ("fetch", 8193), ("humanoid", 1024), ("humanoid", 1025), ("humanoid_cloud", 3000), ("comb", 1024),
+    ("comb", 1025)])
 def test_motions(name, E):
     from plainmp_amd.ompl import BoxMotionValidator
 

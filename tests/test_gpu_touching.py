@@ -25,7 +25,8 @@ def test_touching_cylinders(tilted):
     axis = (0, 1, 0) if tilted else (0, 0, 1)
     prims = [{"type": "cylinder", "radius": a, "height": 2.0**-7, "position": c * np.array(axis), "rotation": R}
              for c, a in zip(at, radius)]
-    urdf = ('<?xml version="1.0"?>\n<robot name="slider">\n' + "".join(synth._link(x) for x in ("base", "lift", "slide"))
+    urdf = ('<?xml version="1.0"?>\n<robot name="slider">\n'
+            + "".join(synth._link(x) for x in ("base", "lift", "slide"))
             + synth._joint("j0", "prismatic", "base", "lift", (0, 0, 0), (0, 0, 0), axis=axis, lower=-9, upper=9)
             + synth._joint("j1", "prismatic", "lift", "slide", (0, 0, 0), (0, 0, 0), axis=(1, 0, 0), lower=-9, upper=9)
             + "</robot>\n")
